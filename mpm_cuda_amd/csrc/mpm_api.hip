@@ -229,6 +229,8 @@ int mpm_create(const mpm_config *cfg, mpm_sim **out)
     GridP &g = s->g;
     g.nx = cfg->nx; g.ny = cfg->ny; g.nz = cfg->nz;
     g.nbx = (g.nx + BLK - 1) / BLK; g.nby = (g.ny + BLK - 1) / BLK; g.nbz = (g.nz + BLK - 1) / BLK;
+    g.div_nbx = div_recip((uint32_t)g.nbx);
+    g.div_nby = div_recip((uint32_t)g.nby);
     g.h = (float)cfg->h;
     g.inv_h = (float)(1.0 / cfg->h);
     g.ox = (float)cfg->origin[0]; g.oy = (float)cfg->origin[1]; g.oz = (float)cfg->origin[2];
@@ -733,6 +735,7 @@ void mpm_destroy(mpm_sim *s)
                     s->staging, s->blk_tile, s->spill, s->dtc, s->warm_list, s->warm_cnt, s->g2p_perm};
     for (void *p : ptrs) if (p) (void)hipFree(p);
     if (s->spill_host) (void)hipHostFree(s->spill_host);
+    if (s->tiles_host) (void)hipHostFree(s->tiles_host);
     for (auto &t : s->timed) { (void)hipEventDestroy(t.a); (void)hipEventDestroy(t.b); }
     for (hipEvent_t e : s->event_pool) (void)hipEventDestroy(e);
     if (s->stream) (void)hipStreamDestroy(s->stream);

@@ -32,7 +32,7 @@ const int P2G_CAND[NCAND] = {1024, 2048, 4096, 8192};   // one-wave workgroups
 const int GRID_CAND[NCAND] = {1024, 2048, 4096, 8192};
 const int G2P_CAND[NCAND] = {64, 128, 192, 256};
 constexpr int NTILE = 3;
-const int TILE_CAND[NTILE] = {256, 384, 512};            // P2G particles per pass over a tile
+const int TILE_CAND[NTILE] = {256, 384, 512};            // values of p2g_tile; the P2G is the same with each
 
 // What the captured graphs depend on, per scene.
 struct SceneSig {
@@ -63,7 +63,7 @@ struct mpm_batch {
     std::vector<SceneSig> sig;          // signature the tables and graphs were built for
     bool built = false;
     hipGraphExec_t step_exec[2] = {}, sort_exec[2] = {};
-    int captured_p2g = 0, captured_grid = 0, captured_g2p = 0, captured_tile = 0;
+    int captured_p2g = 0, captured_grid = 0, captured_g2p = 0;
     int parity = 0;
     int64_t steps_since_sort = 0;
     int64_t total = 0;
@@ -158,12 +158,12 @@ int fork_materials(mpm_batch *b, L launch)
 // ms: counter reset, P2G, spill scatter, block compaction, grid update, the
 // warm-start inference of each weight set among them, G2P.
 int enqueue_material(mpm_batch *b, hipStream_t ms, int m, const BatchSlice *tab, int s0, int cnt, int p2g, int grid,
-                     int g2p_threads, int tile)
+                     int g2p_threads)
 {
     const BatchSlice *t = tab + s0;
     int rc;
     if ((rc = check(launch_batch_zero(ms, t, cnt), "batch_zero"))) return rc;
-    if ((rc = check(launch_p2g_batch(ms, m, t, b->types.data() + s0, cnt, p2g, tile), "p2g_batch"))) return rc;
+    if ((rc = check(launch_p2g_batch(ms, m, t, b->types.data() + s0, cnt, p2g), "p2g_batch"))) return rc;
     if ((rc = check(launch_spill_batch(ms, t, cnt, SPILL_WGS), "spill_batch"))) return rc;
     if ((rc = check(launch_compact_batch(ms, t, cnt, b->mat_compact_wgs[m]), "compact_batch"))) return rc;
     if ((rc = check(launch_grid_batch(ms, t, cnt, grid), "grid_batch"))) return rc;
@@ -181,7 +181,7 @@ int enqueue_material(mpm_batch *b, hipStream_t ms, int m, const BatchSlice *tab,
 // With `ev` (6 events, the autotuner's stage timing) the stages follow one
 // another on the batch stream, only the materials' P2G and G2P launches side
 // by side, and the P2G, grid-update and G2P stages are bracketed.
-int enqueue_step(mpm_batch *b, int p, int p2g, int grid, int g2p_threads, int tile, hipEvent_t *ev)
+int enqueue_step(mpm_batch *b, int p, int p2g, int grid, int g2p_threads, hipEvent_t *ev)
 {
     hipStream_t st = b->stream;
     const BatchSlice *tab = b->tab[p];
@@ -189,12 +189,12 @@ int enqueue_step(mpm_batch *b, int p, int p2g, int grid, int g2p_threads, int ti
     int rc;
     if (!ev)
         return fork_materials(b, [&](hipStream_t ms, int m) {
-            return enqueue_material(b, ms, m, tab, b->mat_begin[m], b->mat_count[m], p2g, grid, g2p_threads, tile);
+            return enqueue_material(b, ms, m, tab, b->mat_begin[m], b->mat_count[m], p2g, grid, g2p_threads);
         });
     if ((rc = check(launch_batch_zero(st, tab, n), "batch_zero"))) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[0], st));
     rc = fork_materials(b, [&](hipStream_t ms, int m) {
-        return check(launch_p2g_batch(ms, m, tab, b->types.data(), n, p2g, tile), "p2g_batch");
+        return check(launch_p2g_batch(ms, m, tab, b->types.data(), n, p2g), "p2g_batch");
     });
     if (rc) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[1], st));
@@ -261,7 +261,7 @@ int capture(mpm_batch *b, hipGraphExec_t *out, bool sort, int p)
     MPM_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed));
     int rc = sort ? enqueue_sort(b, p)
                   : enqueue_step(b, p, b->shape.p2g_workgroups, b->shape.grid_workgroups, b->shape.g2p_threads,
-                                 b->shape.p2g_tile, nullptr);
+                                 nullptr);
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(b->stream, &graph);
     for (size_t k = 0; k < b->sims.size(); ++k) set_book(b->sims[k], book[k]);
@@ -379,7 +379,6 @@ int build(mpm_batch *b)
     b->captured_p2g = b->shape.p2g_workgroups;
     b->captured_grid = b->shape.grid_workgroups;
     b->captured_g2p = b->shape.g2p_threads;
-    b->captured_tile = b->shape.p2g_tile;
     return MPM_OK;
 }
 
@@ -421,8 +420,7 @@ int prepare(mpm_batch *b)
     for (size_t k = 0; same && k < n; ++k) same = sig_of(b, k) == b->sig[k];
     if (same && b->shape.use_graph)
         same = b->step_exec[0] && b->captured_p2g == b->shape.p2g_workgroups &&
-               b->captured_grid == b->shape.grid_workgroups && b->captured_g2p == b->shape.g2p_threads &&
-               b->captured_tile == b->shape.p2g_tile;
+               b->captured_grid == b->shape.grid_workgroups && b->captured_g2p == b->shape.g2p_threads;
     if (!same) {
         for (mpm_sim *s : b->sims) MPM_HIP(hipStreamSynchronize(s->stream));
         int rc = build(b);
@@ -473,7 +471,7 @@ void after_step(mpm_batch *b)
 }
 
 // Sort when due, then one step; graphs or direct launches.
-int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, int tile, hipEvent_t *ev, bool graphs)
+int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, hipEvent_t *ev, bool graphs)
 {
     if (b->steps_since_sort >= b->shape.sort_every) {
         if (graphs) {
@@ -490,7 +488,7 @@ int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, int tile, hipEven
     if (graphs) {
         MPM_HIP(hipGraphLaunch(b->step_exec[b->parity], b->stream));
     } else {
-        int rc = enqueue_step(b, b->parity, p2g, grid, g2p_threads, tile, ev);
+        int rc = enqueue_step(b, b->parity, p2g, grid, g2p_threads, ev);
         if (rc) return rc;
     }
     after_step(b);
@@ -621,8 +619,7 @@ int mpm_batch_run(mpm_batch *b, int32_t nsteps, float *step_ms)
     const bool graphs = b->shape.use_graph != 0;
     for (int32_t k = 0; k < nsteps; ++k) {
         if (ev) MPM_HIP(hipEventRecord(ev[k], b->stream));
-        rc = one_step(b, b->shape.p2g_workgroups, b->shape.grid_workgroups, b->shape.g2p_threads, b->shape.p2g_tile,
-                      nullptr, graphs);
+        rc = one_step(b, b->shape.p2g_workgroups, b->shape.grid_workgroups, b->shape.g2p_threads, nullptr, graphs);
         if (rc) return rc;
     }
     if (ev) MPM_HIP(hipEventRecord(ev[nsteps], b->stream));
@@ -636,11 +633,11 @@ int mpm_batch_run(mpm_batch *b, int32_t nsteps, float *step_ms)
 
 // Times each stage's launch-width candidates on live steps (rounds of
 // NCAND steps, candidate c in step c of every round) and keeps the fastest
-// median per stage; then, with those widths, the P2G tile shapes (rounds of
-// NTILE steps) and keeps the fastest.  Advances every scene by
+// median per stage; then, with those widths, the values of p2g_tile (rounds of
+// NTILE steps; they select the same kernel) and keeps the fastest.  Advances every scene by
 // reps * (NCAND + NTILE) steps.  ms_out (optional, 3 x NCAND + NTILE):
 // median milliseconds of P2G, grid update and G2P per width candidate, then
-// of P2G per tile shape.
+// of P2G per p2g_tile.
 int mpm_batch_autotune(mpm_batch *b, int32_t reps, float *ms_out)
 {
     if (!b) return set_error(MPM_ERR_INVALID, "batch is null");
@@ -650,11 +647,10 @@ int mpm_batch_autotune(mpm_batch *b, int32_t reps, float *ms_out)
     const size_t per = 6;
     hipEvent_t *ev = timing_events(b, (size_t)reps * (NCAND + NTILE) * per);
     if (!ev) return set_error(MPM_ERR_HIP, "hipEventCreate failed");
-    const int tile0 = tile_shape(b->shape.p2g_tile);
     for (int32_t r = 0; r < reps; ++r)
         for (int c = 0; c < NCAND; ++c) {
             hipEvent_t *e = ev + ((size_t)r * NCAND + c) * per;
-            rc = one_step(b, P2G_CAND[c], GRID_CAND[c], G2P_CAND[c], tile0, e, false);
+            rc = one_step(b, P2G_CAND[c], GRID_CAND[c], G2P_CAND[c], e, false);
             if (rc) return rc;
         }
     MPM_HIP(hipStreamSynchronize(b->stream));
@@ -682,13 +678,12 @@ int mpm_batch_autotune(mpm_batch *b, int32_t reps, float *ms_out)
     b->shape.p2g_workgroups = P2G_CAND[best[0]];
     b->shape.grid_workgroups = GRID_CAND[best[1]];
     b->shape.g2p_threads = G2P_CAND[best[2]];
-    // tile shapes with the chosen widths
+    // values of p2g_tile with the chosen widths
     const size_t t0 = (size_t)reps * NCAND;
     for (int32_t r = 0; r < reps; ++r)
         for (int c = 0; c < NTILE; ++c) {
             hipEvent_t *e = ev + (t0 + (size_t)r * NTILE + c) * per;
-            rc = one_step(b, b->shape.p2g_workgroups, b->shape.grid_workgroups, b->shape.g2p_threads, TILE_CAND[c], e,
-                          false);
+            rc = one_step(b, b->shape.p2g_workgroups, b->shape.grid_workgroups, b->shape.g2p_threads, e, false);
             if (rc) return rc;
         }
     if ((rc = release(b))) return rc;

@@ -8,15 +8,13 @@
 //   * per-group sort of particles by the 4x4x4 node block of their base
 //     node, payload permutation of every SoA plane, and one tile (block,
 //     first particle, count, staging slot) per non-empty block;
-//   * P2G over tiles without atomics: one wave per block bins its particles
-//     by base node in LDS, sums each bin's particles in registers and adds
-//     the sums to an 8^3-node LDS arena by plain read-modify-write, then
-//     writes the arena's nodes with mass, and a mask of them, to a staging
+//   * P2G over tiles without global atomics: a workgroup adds a tile's
+//     particles to an 8^3-node LDS arena of 64-bit fixed-point sums with LDS
+//     integer atomics, then writes the nodes its stencils reached to a staging
 //     slot that the grid update gathers.
-// (On gfx950 an LDS float atomic add costs ~200 cycles per wave instruction
-// even when the 64 lanes hit different addresses, ~15x a float4 plain LDS
-// read-modify-write, and global float atomics at ~77 G/s would dominate a
-// per-node flush.)
+// (A wave's 64-lane LDS atomic add to different words takes ~8 cycles as a
+// 64-bit integer, ~16 as a double and ~200 as a float on gfx950; global float
+// atomics at ~77 G/s would dominate a per-node flush.)
 #include "mpm_g2p.h"
 #include "mpm_launch.h"
 
@@ -24,6 +22,7 @@
 #include <cstring>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 
 namespace mpm {
 
@@ -498,6 +497,71 @@ __global__ void k_emit_tiles(const uint32_t *blk_start, const uint32_t *blk_end,
                  desc_cap, blk_tile, tile_base);
 }
 
+// Order of a tile's particles inside its block: one particle of every cell
+// (base node of the block) that has one, in cell order, then the second of
+// every cell that has two, and so on, so that 64 consecutive particles hold
+// mostly different cells and a P2G batch scatters them without turns.  One
+// wave; skeys / sperm are the sorted keys and the stable order, the tile's
+// slots [d.x, d.x + d.y) of perm are written.  Particles past RANK_LEVELS of
+// one cell follow cell by cell.
+constexpr uint32_t RANK_LEVELS = 64;
+struct RankLds {
+    uint64_t mask[RANK_LEVELS];     // cells with more than r particles
+    uint32_t base[RANK_LEVELS];     // place of the first of them
+    uint32_t begin[64], end[64];    // the cells' runs in the sorted order
+    uint32_t deep[64];              // place of a cell's particle RANK_LEVELS
+};
+__device__ __forceinline__ void rank_tile(const uint32_t *__restrict__ skeys, const uint32_t *__restrict__ sperm,
+                                          const uint4 d, uint32_t n, uint32_t *__restrict__ perm, RankLds &L)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t first = d.x, last = min(d.x + d.y, n);
+    if (first >= last) return;
+    L.begin[lane] = 0u;
+    L.end[lane] = 0u;
+    __asm__ volatile("" ::: "memory");      // one wave: its LDS operations execute in order
+    for (uint32_t i = first + lane; i < last; i += 64) {
+        const uint32_t c = skeys[i] & 63u;
+        if (i == first || (skeys[i - 1] & 63u) != c) L.begin[c] = i;
+        if (i + 1 == last || (skeys[i + 1] & 63u) != c) L.end[c] = i + 1;
+    }
+    __asm__ volatile("" ::: "memory");
+    const uint32_t begin = L.begin[lane], cnt = L.end[lane] - begin;
+    uint32_t run = 0;
+    for (uint32_t r = 0; r < RANK_LEVELS; ++r) {
+        const uint64_t m = __ballot(cnt > r);
+        if (lane == 0) {
+            L.mask[r] = m;
+            L.base[r] = run;
+        }
+        run += (uint32_t)__popcll(m);
+        if (!m) break;
+    }
+    const uint32_t rest = cnt > RANK_LEVELS ? cnt - RANK_LEVELS : 0u;
+    L.deep[lane] = run + wave_incl_scan(rest) - rest;
+    __asm__ volatile("" ::: "memory");
+    for (uint32_t i = first + lane; i < last; i += 64) {
+        const uint32_t c = skeys[i] & 63u, r = i - L.begin[c];
+        uint32_t at;
+        if (r < RANK_LEVELS) at = L.base[r] + (uint32_t)__popcll(L.mask[r] & ((1ull << c) - 1ull));
+        else at = L.deep[c] + (r - RANK_LEVELS);
+        perm[first + at] = sperm[i];
+    }
+}
+
+// One wave per tile; 10-18 us a sort (262k-2M particles).  The number of
+// tiles goes to a pinned host word for the choice of the P2G's width.
+__global__ void __launch_bounds__(256) k_rank_tiles(const uint32_t *__restrict__ skeys, const uint32_t *__restrict__ sperm,
+                                                    int n, const uint4 *__restrict__ desc,
+                                                    const uint32_t *__restrict__ tile_count, uint32_t desc_cap,
+                                                    uint32_t *__restrict__ perm, uint32_t *tiles_host)
+{
+    __shared__ RankLds L[4];
+    const uint32_t w = threadIdx.x >> 6, nt = min(*tile_count, desc_cap);
+    if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(tiles_host, nt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    for (uint32_t t = blockIdx.x * 4 + w; t < nt; t += gridDim.x * 4) rank_tile(skeys, sperm, desc[t], (uint32_t)n, perm, L[w]);
+}
+
 // ---------------------------------------------------------------------------
 // Batched re-sort: every scene of a SortSlice table through each stage of the
 // sort above in one launch per stage (8-bit digits, the same number of
@@ -551,9 +615,8 @@ __global__ void __launch_bounds__(256) k_bsort_spine(const SortSlice *__restrict
 }
 
 // Pass `pass` reads the keys (values: the positions in pass 0) from the
-// buffers of its parity and writes the other ones; the last pass writes the
-// values into the scene's permutation.
-__global__ void __launch_bounds__(RS_T) k_bsort_scatter(const SortSlice *__restrict__ tab, int ns, int pass, int last)
+// buffers of its parity and writes the other ones.
+__global__ void __launch_bounds__(RS_T) k_bsort_scatter(const SortSlice *__restrict__ tab, int ns, int pass)
 {
     __shared__ uint32_t cnt[RS_WAVES][1 << BS_DB];
     __shared__ uint32_t lds[40];
@@ -563,7 +626,7 @@ __global__ void __launch_bounds__(RS_T) k_bsort_scatter(const SortSlice *__restr
     const SortSlice &t = tab[sid];
     const bool odd = (pass & 1) != 0;
     const uint32_t *vin = pass == 0 ? nullptr : (odd ? t.vals_alt : t.vals);
-    uint32_t *vout = last ? t.perm : (odd ? t.vals : t.vals_alt);
+    uint32_t *vout = odd ? t.vals : t.vals_alt;
     rs_scatter_tile<BS_DB>(odd ? t.keys_alt : t.keys, vin, odd ? t.keys : t.keys_alt, vout, t.n, BS_DB * pass, 0xFFu,
                            t.hist, t.scan, t.ntiles, tile, cnt, lds);
 }
@@ -616,41 +679,46 @@ __global__ void __launch_bounds__(256) k_bsort_emit(const SortSlice *__restrict_
                  0u);
 }
 
+// The tiles' particle orders (rank_tile) into the scenes' permutations, one
+// wave per tile of all the scenes' tiles.
+__global__ void __launch_bounds__(256) k_bsort_rank(const SortSlice *__restrict__ tab, int ns, int alt)
+{
+    __shared__ RankLds L[4];
+    SliceScan sc;
+    sc.build(ns, [&](int s) { return min(*gp(tab[s].tile_count), tab[s].desc_cap); });
+    const uint32_t w = threadIdx.x >> 6;
+    for (uint32_t k = blockIdx.x * 4 + w; k < sc.total; k += gridDim.x * 4) {
+        const uint32_t sid = (uint32_t)__builtin_amdgcn_readfirstlane((int)sc.find(k));
+        const SortSlice &t = tab[sid];
+        const uint4 d = gload_u4(t.desc, k - sc.start(sid));
+        rank_tile(alt ? t.keys_alt : t.keys, alt ? t.vals_alt : t.vals, d, (uint32_t)t.n, t.perm, L[w]);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // P2G over blocks without atomics.
 //
-// A tile is one node block's particles (grouped by the last sort).  It is
-// processed in chunks of at most CHUNK particles:
-//   A. one lane per particle (dense and coalesced): FAST loads the position,
-//      FUSED runs the particle's G2P update and writes its record (below)
-//      to LDS; both find the base node.  The base, relative to the block's
-//      8^3-node arena (the block's 4 nodes + 1 below + 3 above per axis),
-//      is one of 6^3 bins.
-//   B. the tile's waves (FAST: its one wave; FUSED: both) sort the chunk by
-//      bin (stable counting sort in LDS) and cut every bin into items of at
-//      most ITEM_CAP particles.
+// A tile is one node block's particles (grouped by the last sort), its arena
+// the 8^3 nodes around the block (its 4 and 1 below, 3 above per axis).
+// FAST: see p2g_tile.  FUSED takes chunks of at most CHUNK particles:
+//   A. one lane per particle (dense and coalesced) runs the particle's G2P
+//      update and writes its record (below) to LDS; its base node, relative
+//      to the arena, is one of 6^3 bins.
+//   B. the two waves sort the chunk by bin (stable counting sort in LDS) and
+//      cut every bin into items of at most ITEM_CAP particles.
 //   C. one lane per item: the item's particles share their base node, so the
-//      lane sums their 27 node contributions in registers (FAST reloads each
-//      particle and builds its record in registers; FUSED reads the LDS
-//      record) and adds them to its wave's LDS arena once, in a fixed node
-//      order.  In each of the 27 read-modify-writes the lanes of different
-//      bins touch different slots; lanes of one bin take turns.
-// The waves' arenas are summed into the tile's staging slot, which the grid
-// update gathers.  Particles whose stencil leaves the arena (or whose tile
-// has no staging slot) are listed for the atomic fallback kernel.
-// (On gfx950 an LDS float atomic runs ~20x slower than a plain LDS
-// read-modify-write; summing in registers first also divides the LDS traffic
-// by the particles per item.)
+//      lane sums their 27 node contributions in registers and adds them to
+//      its wave's LDS arena once, in a fixed node order.  In each of the 27
+//      read-modify-writes the lanes of different bins touch different slots;
+//      lanes of one bin take turns.
+// The arena is written to the tile's staging slot, which the grid update
+// gathers.  Particles whose stencil leaves the arena (or whose tile has no
+// staging slot) are listed for the atomic fallback kernel.
 constexpr int TILE_WAVES = 2;                    // FUSED form: waves per tile
 constexpr int TILE_THREADS = 64 * TILE_WAVES;
-constexpr int P2G_THREADS = 64;                  // FAST form: one wave per tile
 static_assert(ARENA_NODES % TILE_THREADS == 0, "arena nodes per thread must be whole");
 constexpr int CHUNK = 384;          // particles per pass over a tile (a full 4^3-cell block holds ~320 at 5 per cell)
 static_assert(CHUNK % TILE_THREADS == 0, "whole phase-A passes");
-// FAST form: particles per pass over a tile, chosen per simulator
-// (mpm_config.tile) or per batch (its autotuner) among these
-constexpr int TILE_SHAPES[3] = {256, 384, 512};
-constexpr int TILE_DEFAULT = 384;
 constexpr int ITEM_CAP = 4;         // particles per lane item
 constexpr int NBIN = 216;           // 6^3 base positions inside an arena
 constexpr uint32_t NO_BIN = 255u;
@@ -698,23 +766,46 @@ struct TileLds {
     uint32_t nitems;
 };
 
-// LDS of a FAST-form tile (one wave) of CH particles per pass: the
-// particles' fx, bin keys, the sort and the arena (14.5 / 17.1 / 19.8 KB for
-// CH = 256 / 384 / 512; the rest of the particle records stays in HBM /
-// cache).
-template <int CH>
-struct TileKeys {
-    static_assert(CH % 64 == 0 && CH <= 4095, "whole 64-particle passes; 12-bit item positions");
-    float4 arena[A_SLOTS];
-    float fx[3][CH];            // phase A: position relative to the base node, in cells
-    uint32_t items[CH];
-    uint16_t perm[CH];
-    uint16_t rnk[CH];
-    uint16_t cnt[NBIN];
-    uint16_t start[NBIN];       // each bin's first sorted position
-    uint8_t key[CH];
-    uint32_t nitems;
+// LDS of a FAST-form tile worked by W waves: an 8^3-node arena of 64-bit
+// fixed-point sums, one plane per component (mass, then momentum).  Node
+// (x, y, z) of a plane is x + AR_Y y + AR_Z z: linear, so that a stencil's
+// offsets are immediates of the LDS instructions, and AR_Z = 68 spreads the
+// 64 cells of a block evenly over the banks.  17.1 KB.
+constexpr int AR_Y = ARENA, AR_Z = ARENA * ARENA + 4, AR_PLANE = ARENA * AR_Z;
+template <int W>
+struct TileArena {
+    unsigned long long sum[4][AR_PLANE];
+    float bound[W];
+    uint32_t faces[W];
 };
+
+// Fixed-point sums.  x (an FP64 value below 2^50 in magnitude) + FIX_MAGIC
+// has the integer nearest to x in its low mantissa bits, so its bit pattern
+// is that integer plus a constant whose low 51 bits are zero: patterns are
+// added as they are, and the low 51 bits of the total, sign-extended, are the
+// sum of the integers as long as that stays below 2^50.  A tile's unit is
+// 2^-50 of its particle count times the largest contribution any of them can
+// make to a component: for 512 particles 2^-40 of that, where FP32 sums round
+// at 2^-24 of the node's own value.  What the unit loses at a node of little
+// mass comes back to a particle times that node's weight.
+constexpr double FIX_MAGIC = 6755399441055744.0;        // 1.5 * 2^52
+constexpr int FIX_BITS = 50;
+__device__ __forceinline__ double fix_value(unsigned long long s) { return (double)((long long)(s << 13) >> 13); }
+// Largest of non-negative v over the wave, in lane 63 (DPP moves; lanes
+// without a source keep their own value).
+__device__ __forceinline__ float wave_max_dpp(float v)
+{
+#define MPM_MAX_STEP(ctrl, rows)                                                                                         v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), ctrl, rows, 0xf, false)))
+    MPM_MAX_STEP(0x111, 0xf);       // row_shr:1
+    MPM_MAX_STEP(0x112, 0xf);
+    MPM_MAX_STEP(0x114, 0xf);
+    MPM_MAX_STEP(0x118, 0xf);
+    MPM_MAX_STEP(0x142, 0xa);       // row_bcast:15 into rows 1 and 3
+    MPM_MAX_STEP(0x143, 0xc);       // row_bcast:31 into rows 2 and 3
+#undef MPM_MAX_STEP
+    return v;
+}
+__device__ __forceinline__ double pow2(int e) { return __hiloint2double((1023 + e) << 20, 0); }
 
 struct TileGeo {
     int ax, ay, az;     // arena origin (node index of arena slot 0)
@@ -722,19 +813,18 @@ struct TileGeo {
 
 __device__ __forceinline__ TileGeo tile_geo(const GridP &g, uint32_t blk)
 {
-    const int bx = (int)(blk % (uint32_t)g.nbx);
-    const int by = (int)((blk / (uint32_t)g.nbx) % (uint32_t)g.nby);
-    const int bz = (int)(blk / ((uint32_t)g.nbx * (uint32_t)g.nby));
-    return TileGeo{bx * BLK - 1, by * BLK - 1, bz * BLK - 1};
+    const uint32_t row = div_by(blk, (uint32_t)g.nbx, g.div_nbx);
+    const uint32_t bz = div_by(row, (uint32_t)g.nby, g.div_nby);
+    const int bx = (int)(blk - row * (uint32_t)g.nbx), by = (int)(row - bz * (uint32_t)g.nby);
+    return TileGeo{bx * BLK - 1, by * BLK - 1, (int)bz * BLK - 1};
 }
 
-// Phase A tail: the particle's bin key, or NO_BIN and an entry in the list
-// of the atomic fallback (whose node blocks are flagged here when `flags` is
-// given).  Returns true when the particle was listed.
-template <class TL>
-__device__ __forceinline__ bool bin_key(const GridP &g, TL &L, const TileGeo &t, bool active, int slot, int i,
-                                        const int b[3], bool staged, uint32_t *spill, uint32_t *counters,
-                                        uint32_t *flags)
+// Phase A tail: a particle whose base lies outside the arena's bins (or whose
+// tile has no staging slot) gets an entry in the list of the atomic fallback
+// (its node blocks are flagged here when `flags` is given).  Returns true
+// when the particle was listed.
+__device__ __forceinline__ bool list_spill(const GridP &g, const TileGeo &t, bool active, int i, const int b[3],
+                                           bool staged, uint32_t *spill, uint32_t *counters, uint32_t *flags)
 {
     const int lane = threadIdx.x & 63;
     const int lx = b[0] - t.ax, ly = b[1] - t.ay, lz = b[2] - t.az;
@@ -753,8 +843,12 @@ __device__ __forceinline__ bool bin_key(const GridP &g, TL &L, const TileGeo &t,
             if (flags) mark_blocks(g, b, flags);
         }
     }
-    if (active) L.key[slot] = inside ? (uint8_t)(lx + 6 * (ly + 6 * lz)) : (uint8_t)NO_BIN;
     return spill_me;
+}
+// bin of a base node inside the arena
+__device__ __forceinline__ uint32_t bin_of(const TileGeo &t, const int b[3])
+{
+    return (uint32_t)((b[0] - t.ax) + 6 * ((b[1] - t.ay) + 6 * (b[2] - t.az)));
 }
 
 // The particle's P2G record from its stencil and scatter quantities:
@@ -781,7 +875,8 @@ __device__ __forceinline__ bool bin_particle(const GridP &g, TileLds &L, const T
                                              int i, const Stencil &s, const Scatter &sc, bool staged,
                                              uint32_t *spill, uint32_t *counters)
 {
-    const bool spill_me = bin_key(g, L, t, active, slot, i, s.b, staged, spill, counters, nullptr);
+    const bool spill_me = list_spill(g, t, active, i, s.b, staged, spill, counters, nullptr);
+    if (active) L.key[slot] = spill_me ? (uint8_t)NO_BIN : (uint8_t)bin_of(t, s.b);
     if (active && !spill_me) {
         float q0[3], hB[9], Gs[6];
         make_record<MAT>(g, s, sc, q0, hB, Gs);
@@ -889,45 +984,6 @@ __device__ __forceinline__ void sort_chunk(TileLds &L, int nc)
             L.perm[(uint32_t)L.cnt1[key] + off + L.rnk[sl]] = (uint16_t)sl;
         }
     }
-}
-
-// Phase B, FAST form (the tile's one wave): the same sort, in slot order
-// within each bin.  One wave's LDS operations execute in order, so the
-// steps need no barrier; the compiler barriers keep their order.
-template <class TK>
-__device__ __forceinline__ void sort_chunk_wave(TK &L, int nc)
-{
-    const int lane = threadIdx.x & 63;
-    const uint64_t lt = lane ? ((~0ull) >> (64 - lane)) : 0ull;
-    for (int b = lane; b < NBIN; b += 64) L.cnt[b] = 0;
-    __asm__ volatile("" ::: "memory");
-    for (int s0 = 0; s0 < nc; s0 += 64) {
-        const int sl = s0 + lane;
-        const uint32_t key = sl < nc ? (uint32_t)L.key[sl] : NO_BIN;
-        const bool v = key != NO_BIN;
-        const uint64_t m = match_key8(key) & __ballot(v);
-        const uint32_t below = (uint32_t)__popcll(m & lt);
-        uint32_t prev = 0;
-        if (v) prev = L.cnt[key];
-        if (v && below == 0) L.cnt[key] = (uint16_t)(prev + (uint32_t)__popcll(m));
-        if (v) L.rnk[sl] = (uint16_t)(prev + below);
-        __asm__ volatile("" ::: "memory");
-    }
-    uint32_t c[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int b = 4 * lane + j;
-        c[j] = b < NBIN ? (uint32_t)L.cnt[b] : 0u;
-    }
-    __asm__ volatile("" ::: "memory");
-    build_items(c, L.items, L.start, &L.nitems);
-    __asm__ volatile("" ::: "memory");
-    for (int s0 = 0; s0 < nc; s0 += 64) {
-        const int sl = s0 + lane;
-        const uint32_t key = sl < nc ? (uint32_t)L.key[sl] : NO_BIN;
-        if (key != NO_BIN) L.perm[(uint32_t)L.start[key] + L.rnk[sl]] = (uint16_t)sl;
-    }
-    __asm__ volatile("" ::: "memory");
 }
 
 // Phase C, one particle given its record in registers (fx, q0, hB and G as
@@ -1088,37 +1144,8 @@ __device__ __forceinline__ void scatter_items(TileLds &L, float4 *arena, int bat
     flush_item(arena, has, bin, acc);
 }
 
-// The P2G record straight from a loaded particle (FAST form): fx, hB = hm C
-// with hm = h m, q0 = m v - hB fx, and G (xx, yy, zz, xy, xz, yz) = -dt V
-// tau, water: G[0] = dt V p J (MPMCUDA.cu:345-353, 391-414).
-template <int MAT>
-__device__ __forceinline__ void record_from_raw(const MatP &mat, float dt, float hm, const RawP &r,
-                                                const float fx[3], float q0[3], float hB[9], float Gs[6])
-{
-#pragma unroll
-    for (int k = 0; k < 9; ++k) hB[k] = hm * r.C[k];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        float q = mat.mass * r.v[c];
-        q = fmaf(-hB[3 * c], fx[0], q);
-        q = fmaf(-hB[3 * c + 1], fx[1], q);
-        q0[c] = fmaf(-hB[3 * c + 2], fx[2], q);
-    }
-    if (MAT == MPM_WATER) {
-        const float J = r.s[0];
-        const float pr = mat.eos_k * (powf(J, -mat.eos_gamma) - 1.0f);   // MPMCUDA.cu:353
-        Gs[0] = dt * mat.vol * pr * J;
-#pragma unroll
-        for (int k = 1; k < 6; ++k) Gs[k] = 0.0f;
-    } else {
-        const float c = -dt * mat.vol;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) Gs[k] = c * r.s[k];
-    }
-}
-
-// v, C and the stored stress (water: J) of particle i: the FAST P2G's phase
-// C inputs besides fx, which phase A left in LDS.
+// v, C and the stored stress (water: J) of particle i: the FAST P2G's
+// inputs besides the position.
 template <int MAT>
 __device__ __forceinline__ void load_vcs(const PartView &pv, int i, RawP &r)
 {
@@ -1133,53 +1160,6 @@ __device__ __forceinline__ void load_vcs(const PartView &pv, int i, RawP &r)
 #pragma unroll
         for (int k = 0; k < 6; ++k) r.s[k] = ld_plane(pv, PL_TAU + k, u);
     }
-}
-
-// Phase C for one wave, FAST form: the item's particles are loaded again
-// from the particle planes (the tile's lines are in cache from phase A or
-// arrive now; no LDS records) and their records built in registers with the
-// fx phase A computed.
-template <int MAT, class TK>
-__device__ __forceinline__ void scatter_items_reload(TK &L, float4 *arena, int batch, const GridP &g,
-                                                     const MatP &mat, const PartView &pv, int i0, float dt, float hm)
-{
-    const int lane = threadIdx.x & 63;
-    const uint32_t it = (uint32_t)(batch * 64 + lane);
-    const bool has = it < L.nitems;
-    const uint32_t item = has ? L.items[it] : 0u;
-    const uint32_t bin = has ? (item & 255u) : NO_BIN;
-    const uint32_t first = (item >> 8) & 4095u, cnt = has ? (item >> 20) : 0u;
-    float4 acc[27];
-#pragma unroll
-    for (int o = 0; o < 27; ++o) acc[o] = make_float4(0.f, 0.f, 0.f, 0.f);
-    // item counts never increase along the item list (build_items), so the
-    // batch's first lane holds its largest
-    const uint32_t rounds = (uint32_t)__builtin_amdgcn_readfirstlane((int)cnt);
-    // the next round's particle is loaded while this one is accumulated;
-    // lanes without a next particle reload a valid one (one basic block)
-    auto slot_of = [&](uint32_t r) -> int { return cnt ? (int)L.perm[first + min(r, cnt - 1u)] : 0; };
-    RawP nxt;
-    float nfx[3];
-    int sl = slot_of(0);
-    load_vcs<MAT>(pv, i0 + sl, nxt);
-#pragma unroll
-    for (int a = 0; a < 3; ++a) nfx[a] = L.fx[a][sl];
-    for (uint32_t r = 0; r < rounds; ++r) {
-        const RawP raw = nxt;
-        const float fx[3] = {nfx[0], nfx[1], nfx[2]};
-        if (r + 1 < rounds) {
-            sl = slot_of(r + 1);
-            load_vcs<MAT>(pv, i0 + sl, nxt);
-#pragma unroll
-            for (int a = 0; a < 3; ++a) nfx[a] = L.fx[a][sl];
-        }
-        if (r < cnt) {
-            float q0[3], hB[9], Gs[6];
-            record_from_raw<MAT>(mat, dt, hm, raw, fx, q0, hB, Gs);
-            accum_regs<MAT>(fx, q0, hB, Gs, g.inv_h, mat.mass, acc);
-        }
-    }
-    flush_item(arena, has, bin, acc);
 }
 
 // Phases B and C of one chunk (all threads; ends synchronized).
@@ -1229,105 +1209,241 @@ __device__ __forceinline__ void tile_end(const GridP &g, const TileGeo &t, const
     __syncthreads();
 }
 
+// Water: dt V p J / h of a particle.
+__device__ __forceinline__ float water_force(const MatP &mat, const GridP &g, float dt, float J)
+{
+    const float pr = mat.eos_k * (powf(J, -mat.eos_gamma) - 1.0f);   // MPMCUDA.cu:353
+    return dt * mat.vol * pr * J * g.inv_h;
+}
+
+// A bound on the magnitude of a particle's contribution to any component of
+// any node's momentum (see scatter_particle: N <= 3/4, |D| <= 1, offsets at
+// most 2, |fx| <= 1.5; a NaN input gives NaN or infinity).
+template <int MAT>
+__device__ __forceinline__ float contribution_bound(const MatP &mat, const GridP &g, float dt, const RawP &r, float gw)
+{
+    const float hm = 3.5f * g.h * mat.mass, cg = dt * mat.vol * g.inv_h;
+    float s = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        constexpr int T[3][3] = {{0, 3, 4}, {3, 1, 5}, {4, 5, 2}};      // tau as xx, yy, zz, xy, xz, yz
+        const float q = fabsf(r.C[3 * c]) + fabsf(r.C[3 * c + 1]) + fabsf(r.C[3 * c + 2]);
+        const float f = MAT == MPM_WATER ? fabsf(gw)
+                                         : cg * (fabsf(r.s[T[c][0]]) + fabsf(r.s[T[c][1]]) + fabsf(r.s[T[c][2]]));
+        s += fmaf(hm, q, fmaf(mat.mass, fabsf(r.v[c]), f));
+    }
+    return s;       // the sum over c: a NaN of any component stays one
+}
+
+// Adds one particle's 27 node contributions to the arena, FAST form.  Node
+// (ox, oy, oz) of its stencil receives, with N the B-spline weights,
+// D = dN/dx, a_c = m v_c - h m C_c fx, B = h m C and G = -dt V tau / h
+// (water: dt V p J / h on the diagonal),
+//   p_c(o) = Nz alpha_c(ox, oy) + Nx Ny zeta_c(oz),  m(o) / m = Nx Ny Nz
+//   alpha_c = Ny (Nx (a_c + ox B_c0) + G_c0 Dx) + Nx (oy Ny B_c1 + G_c1 Dy)
+//   zeta_c  = oz Nz B_c2 + G_c2 Dz
+// in fixed point: momenta times pscale, masses over m times pscale mscale.  The last
+// two products of each value run in FP64 (full rate on this target) and end
+// in the fixed-point sum's own rounding.
+template <int MAT>
+__device__ __forceinline__ void scatter_particle(unsigned long long *node, const GridP &g, const MatP &mat, float dt,
+                                                 const RawP &r, float gw, const float fx[3], double pscale,
+                                                 double mscale, bool in)
+{
+    const float hm = g.h * mat.mass, cg = -dt * mat.vol * g.inv_h;
+    float N[3][3], D[3][3];
+    bspline3_wave(fx, N, D);
+    float sx[3][3], ey[3][3];       // [offset][component]
+    double ez[3][3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        constexpr int T[3][3] = {{0, 3, 4}, {3, 1, 5}, {4, 5, 2}};
+        float B[3], G[3];
+        float a = mat.mass * r.v[c];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            B[k] = hm * r.C[3 * c + k];
+            a = fmaf(-B[k], fx[k], a);
+            if (MAT == MPM_WATER) G[k] = k == c ? gw : 0.0f;
+            else G[k] = cg * r.s[T[c][k]];
+        }
+        // water: G is zero off the diagonal (resolved at compile time)
+#define GZ(k) (MAT == MPM_WATER && (k) != c)
+        const float ax[3] = {a, a + B[0], a + (B[0] + B[0])};
+        const float By[3] = {0.0f, B[1], B[1] + B[1]}, Bz[3] = {0.0f, B[2], B[2] + B[2]};
+#pragma unroll
+        for (int o = 0; o < 3; ++o) {
+            const float gy = GZ(1) ? 0.0f : G[1] * D[1][o], gz = GZ(2) ? 0.0f : G[2] * D[2][o];
+            ey[o][c] = o == 0 ? gy : (GZ(1) ? N[1][o] * By[o] : fmaf(N[1][o], By[o], gy));
+            ez[o][c] = pscale * (double)(o == 0 ? gz : (GZ(2) ? N[2][o] * Bz[o] : fmaf(N[2][o], Bz[o], gz)));
+            const float t = N[0][o] * ax[o];
+            sx[o][c] = GZ(0) ? t : fmaf(G[0], D[0][o], t);
+        }
+#undef GZ
+    }
+    double pz[3];
+#pragma unroll
+    for (int o = 0; o < 3; ++o) pz[o] = pscale * (double)N[2][o];
+    if (!in) return;
+    auto add = [](unsigned long long *s, double v) { atomicAdd(s, (unsigned long long)__double_as_longlong(v)); };
+#pragma unroll
+    for (int ox = 0; ox < 3; ++ox)
+#pragma unroll
+        for (int oy = 0; oy < 3; ++oy) {
+            const double nxy = (double)(N[0][ox] * N[1][oy]), mxy = mscale * nxy;
+            double al[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                al[c] = (double)((MAT == MPM_WATER && c != 1 && oy == 0) ? N[1][oy] * sx[ox][c]
+                                                                        : fmaf(N[1][oy], sx[ox][c], N[0][ox] * ey[oy][c]));
+#pragma unroll
+            for (int oz = 0; oz < 3; ++oz) {
+                unsigned long long *s = node + (ox + AR_Y * oy + AR_Z * oz);
+                add(s, fma(mxy, pz[oz], FIX_MAGIC));
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const double q = (MAT == MPM_WATER && c != 2 && oz == 0) ? FIX_MAGIC : fma(nxy, ez[oz][c], FIX_MAGIC);
+                    add(s + (1 + c) * AR_PLANE, fma(pz[oz], al[c], q));
+                }
+            }
+        }
+}
+
 // One tile (descriptor d = first particle, count, block, staging slot) of
-// the FAST-form P2G, by one wave; returns health bits.  Phase A loads only
-// positions (bin keys); phase C reloads x, v, C and the stored stress of
-// each item's particles, so the tile needs no LDS records (12.5 KB instead
-// of 53 KB) and no barrier, and the register file alone bounds the tiles
-// in flight per CU (8 one-wave tiles instead of 3 two-wave ones with LDS
-// records: 77 vs 106 us per 1M-particle snow step, measured).
-template <int MAT, int CH>
+// the FAST-form P2G, by one workgroup of W waves; returns health bits.  The
+// waves take 64 particles at a time in their stored order -- as of the last
+// sort one particle of each cell of the block, then the next of each
+// (k_rank_tiles) -- so the lanes of an LDS atomic mostly hold different
+// nodes.  The sums are integers, exact and the same in any order; their scale
+// comes from the largest contribution any of the tile's particles can make,
+// so the waves read their particles once for that bound (the last batch stays
+// in registers for the scatter) and once more for the other batches.  A tile
+// with a particle that is not finite goes to the atomic fallback.
+template <int MAT, int W>
 __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, const PartView &pv, const uint4 d,
                                              uint32_t staging_cap, float dt, float4 *__restrict__ staging,
                                              uint32_t *spill, uint32_t *flags, uint32_t *counters, int32_t *blk_tile,
-                                             TileKeys<CH> &L)
+                                             TileArena<W> &L)
 {
     uint32_t bits = 0;
     const TileGeo t = tile_geo(g, d.z);
     const bool staged = d.w < staging_cap;
-    const float hm = (1.0f / g.inv_h) * mat.mass;
     const int lane = threadIdx.x & 63;
-    for (int k = lane; k < A_SLOTS; k += 64) L.arena[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-    constexpr int PASSES = CH / 64;
-    uint32_t lane_faces = 0;    // arena faces this lane's particles' stencils reach (see tile_entry)
-    for (uint32_t c0 = 0; c0 < d.y; c0 += CH) {
-        const int nc = (int)min((uint32_t)CH, d.y - c0);
-        // A: all position loads of the chunk first (lanes past its end reload
-        // its last particle; passes past its end load nothing), then bin keys
-        float xs[PASSES][3];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    float x[3], gw = 0.0f;
+    RawP raw;
+    // lanes past the tile's end reload its last particle
+    auto load = [&](uint32_t s0) {
+        const uint32_t i = d.x + min(s0 + (uint32_t)lane, d.y - 1u);
 #pragma unroll
-        for (int it = 0; it < PASSES; ++it) {
-            if (it * 64 >= nc) break;
-            const uint32_t slot = (uint32_t)min(it * 64 + lane, nc - 1);
-#pragma unroll
-            for (int a = 0; a < 3; ++a) xs[it][a] = ld_plane(pv, PL_X + a, d.x + c0 + slot);
+        for (int a = 0; a < 3; ++a) x[a] = ld_plane(pv, PL_X + a, i);
+        load_vcs<MAT>(pv, (int)i, raw);
+    };
+    const uint32_t first = (uint32_t)wave * 64u;
+    if (first < d.y) load(first);
+    {
+        static_assert(4 * AR_PLANE % 2 == 0, "whole 16-byte stores");
+        float4 *z = (float4 *)&L.sum[0][0];
+        for (int k = threadIdx.x; k < 2 * AR_PLANE; k += 64 * W) z[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float bound = 0.0f;
+    uint32_t s0 = first;
+    if (first < d.y)
+        for (;;) {
+            if (MAT == MPM_WATER) gw = water_force(mat, g, dt, raw.s[0]);
+            const float q = contribution_bound<MAT>(mat, g, dt, raw, gw);
+            bound = q <= bound ? bound : q;         // keeps a NaN
+            if (!(q <= 3e38f)) bound = __int_as_float(0x7f800000);
+            if (s0 + 64u * W >= d.y) break;
+            s0 += 64u * W;
+            load(s0);
         }
+    bound = wave_max_dpp(bound);
+    if (lane == 63) L.bound[wave] = bound;
+    __syncthreads();
+    bound = L.bound[0];
 #pragma unroll
-        for (int it = 0; it < PASSES; ++it) {
-            if (it * 64 >= nc) break;
-            const int slot = it * 64 + lane;
-            const bool active = slot < nc;
-            int b[3] = {0, 0, 0};
+    for (int w = 1; w < W; ++w) bound = fmaxf(bound, L.bound[w]);
+    const uint32_t bb32 = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(bound));
+    const bool finite = bb32 < 0x7f800000u;
+    // contributions below 2^e, at most d.y of them a node: sums below 2^50
+    const int e = (int)(bb32 >> 23) - 126, nbits = FIX_BITS - (32 - __builtin_clz(d.y));
+    const double pscale = pow2(nbits - e), mscale = pow2(e);     // mass: 2^nbits = pscale 2^e
+    uint32_t lane_faces = 0;    // arena faces this lane's particles' stencils reach (see tile_entry)
+    if (first < d.y)
+        for (;;) {
+            const bool active = s0 + (uint32_t)lane < d.y;
+            const uint32_t i = d.x + s0 + (uint32_t)lane;
+            int b[3];
             float f[3];
-            if (active) {
-                bits |= base_fx(g, xs[it], b, f);
-#pragma unroll
-                for (int a = 0; a < 3; ++a) L.fx[a][slot] = f[a];
-            }
-            const bool listed = bin_key(g, L, t, active, slot, (int)(d.x + c0) + slot, b, staged, spill, counters,
-                                        flags);
-            // a base on the arena's first (last) bin position reaches its
-            // face at index 0 (7)
-            if (active && !listed) {
+            const uint32_t ob = base_fx(g, x, b, f);
+            if (active) bits |= ob;
+            const bool listed = list_spill(g, t, active, (int)i, b, staged && finite, spill, counters, flags);
+            const bool in = active && !listed;
+            const int rel[3] = {b[0] - t.ax, b[1] - t.ay, b[2] - t.az};
+            if (in) {
+                // a base on the arena's first (last) bin position reaches its
+                // face at index 0 (7)
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                    const int rel = b[a] - (a == 0 ? t.ax : (a == 1 ? t.ay : t.az));
-                    lane_faces |= (rel == 0 ? 1u : 0u) << (2 * a);
-                    lane_faces |= (rel == ARENA - 3 ? 2u : 0u) << (2 * a);
+                    lane_faces |= (rel[a] == 0 ? 1u : 0u) << (2 * a);
+                    lane_faces |= (rel[a] == ARENA - 3 ? 2u : 0u) << (2 * a);
                 }
             }
+            scatter_particle<MAT>(&L.sum[0][0] + (in ? rel[0] + AR_Y * rel[1] + AR_Z * rel[2] : 0), g, mat, dt, raw, gw,
+                                  f, pscale, mscale, in);
+            if (s0 == first) break;
+            s0 -= 64u * W;
+            load(s0);
+            if (MAT == MPM_WATER) gw = water_force(mat, g, dt, raw.s[0]);
         }
-        __asm__ volatile("" ::: "memory");
-        // B and C
-        sort_chunk_wave(L, nc);
-        const int nb = (int)((L.nitems + 63u) >> 6);
-        for (int b = 0; b < nb; ++b) scatter_items_reload<MAT>(L, L.arena, b, g, mat, pv, (int)(d.x + c0), dt, hm);
-        __asm__ volatile("" ::: "memory");
-    }
     // the arena into the tile's staging slot (logical node order): indices
     // 1..6 of each axis and the faces some stencil reached (every other node
     // is zero); mark the node blocks that received mass
-    if (staged) {
-        uint32_t faces = 0;
+    uint32_t faces = 0;
 #pragma unroll
-        for (int f = 0; f < 6; ++f)
-            if (__ballot((lane_faces >> f) & 1u)) faces |= 1u << f;
+    for (int f = 0; f < 6; ++f)
+        if (__ballot((lane_faces >> f) & 1u)) faces |= 1u << f;
+    if (lane == 0) L.faces[wave] = faces;
+    __syncthreads();
+    if (staged) {
+        faces = 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) faces |= L.faces[w];
+        faces = (uint32_t)__builtin_amdgcn_readfirstlane((int)faces);
+        const double punit = pow2(e - nbits), munit = pow2(-nbits) * (double)mat.mass;
         const int64_t dst = (int64_t)d.w * ARENA_NODES;
         const int lo[3] = {(faces & 1u) ? 0 : 1, (faces & 4u) ? 0 : 1, (faces & 16u) ? 0 : 1};
         const int hi[3] = {(faces & 2u) ? 7 : 6, (faces & 8u) ? 7 : 6, (faces & 32u) ? 7 : 6};
         const int kx = lane & 7, ky = lane >> 3;
         const bool row = kx >= lo[0] && kx <= hi[0] && ky >= lo[1] && ky <= hi[1];
-        // all eight z planes are read from LDS back to back (the accumulators
-        // are dead here), then the planes in range are stored
-        float4 v[ARENA];
 #pragma unroll
-        for (int kz = 0; kz < ARENA; ++kz) v[kz] = L.arena[a_slot(kx, ky, kz)];
-#pragma unroll
-        for (int kz = 0; kz < ARENA; ++kz) {
+        for (int q = 0; q < ARENA / W; ++q) {
+            const int kz = q * W + wave;
             if (!row || kz < lo[2] || kz > hi[2]) continue;
-            gstore4(staging, dst + kz * 64 + lane, v[kz]);
+            const int o = kx + AR_Y * ky + AR_Z * kz;
+            const float4 v = make_float4((float)(munit * fix_value(L.sum[0][o])), (float)(punit * fix_value(L.sum[1][o])),
+                                         (float)(punit * fix_value(L.sum[2][o])), (float)(punit * fix_value(L.sum[3][o])));
+            gstore4(staging, dst + kz * 64 + lane, v);
             const int nx_ = t.ax + kx, ny_ = t.ay + ky, nz_ = t.az + kz;
-            if (v[kz].x != 0.f && nx_ >= 0 && ny_ >= 0 && nz_ >= 0 && nx_ < g.nx && ny_ < g.ny && nz_ < g.nz)
+            if (v.x != 0.f && nx_ >= 0 && ny_ >= 0 && nz_ >= 0 && nx_ < g.nx && ny_ < g.ny && nz_ < g.nz)
                 gp(flags)[((int64_t)(nz_ >> 2) * g.nby + (ny_ >> 2)) * g.nbx + (nx_ >> 2)] = 1u;
         }
-        if (lane == 0) gp(blk_tile)[d.z] = tile_entry(d.w, faces);
+        if (threadIdx.x == 0) gp(blk_tile)[d.z] = tile_entry(d.w, faces);
     }
-    __asm__ volatile("" ::: "memory");
+    __syncthreads();        // the arena is cleared for the workgroup's next tile
     return bits;
 }
 
-template <int MAT, int CH>
-__global__ void __launch_bounds__(P2G_THREADS) __attribute__((amdgpu_waves_per_eu(2))) k_p2g_block(GridP g, MatP mat, PartView pv,
+// Bound by LDS and vector issue together: of a SIMD's cycles the vector units
+// take ~54% and the LDS atomics ~41%, half of these in bank conflicts of
+// uneven cells.  Four waves a SIMD: five or six measured the same or slower.
+// One pass over memory, no turns among lanes, no LDS sort: against one wave a
+// tile that sorted its particles in LDS and summed cells in registers, per
+// launch 26.8 -> 11.6 us (16k snow), 46 -> 26.0 (262k jello), 67 -> 56.6
+// (1M snow), 202 -> 145 (2M water).
+template <int MAT, int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) k_p2g_block(GridP g, MatP mat, PartView pv,
                                                             const uint4 *__restrict__ desc,
                                                             const uint32_t *__restrict__ tile_count, uint32_t desc_cap,
                                                             uint32_t staging_cap, float dt,
@@ -1335,7 +1451,7 @@ __global__ void __launch_bounds__(P2G_THREADS) __attribute__((amdgpu_waves_per_e
                                                             uint32_t *flags, uint32_t *counters, int32_t *blk_tile,
                                                             int clear_active)
 {
-    __shared__ TileKeys<CH> L;
+    __shared__ TileArena<W> L;
     const uint32_t nt = min(*tile_count, desc_cap);
     // the active-block and node counters are not used during P2G: clear
     // them here for the block compaction that follows
@@ -1344,13 +1460,12 @@ __global__ void __launch_bounds__(P2G_THREADS) __attribute__((amdgpu_waves_per_e
         gp(counters)[CT_NODES] = 0u;
     }
     uint32_t bits = 0;
-    const uint32_t nt8 = round_xcd(nt);
     dt = step_dt(g, dt);
+    const uint32_t nt8 = round_xcd(nt);
     for (uint32_t k8 = blockIdx.x; k8 < nt8; k8 += gridDim.x) {
         const uint32_t tt = xcd_spread(k8, nt8);
         if (tt >= nt) continue;
-        bits |= p2g_tile<MAT, CH>(g, mat, pv, desc[tt], staging_cap, dt, staging, spill, flags, counters, blk_tile,
-                                  L);
+        bits |= p2g_tile<MAT, W>(g, mat, pv, desc[tt], staging_cap, dt, staging, spill, flags, counters, blk_tile, L);
     }
     if (bits) atomicOr(counters + CT_HEALTH, bits);
     if (threadIdx.x == 0 && blockIdx.x == 0) counters[CT_TILES] = nt;
@@ -1366,10 +1481,10 @@ __global__ void __launch_bounds__(P2G_THREADS) __attribute__((amdgpu_waves_per_e
 // tile's (256 B; LDS is allocated in granules, so any addition is checked
 // against the workgroups per CU it leaves).
 constexpr int P2G_CHUNK = 64;
-template <int MAT, int CH>
-__global__ void __launch_bounds__(P2G_THREADS) __attribute__((amdgpu_waves_per_eu(2))) k_p2g_batch(const BatchSlice *__restrict__ tab, int nslices)
+template <int MAT, int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) k_p2g_batch(const BatchSlice *__restrict__ tab, int nslices)
 {
-    __shared__ TileKeys<CH> L;
+    __shared__ TileArena<W> L;
     __shared__ uint32_t s_end[P2G_CHUNK];
     __shared__ uint32_t s_total;
     if (threadIdx.x < 64) {
@@ -1388,10 +1503,13 @@ __global__ void __launch_bounds__(P2G_THREADS) __attribute__((amdgpu_waves_per_e
         if (tt >= nt) continue;
         const uint32_t sid = (uint32_t)__builtin_amdgcn_readfirstlane((int)__popcll(__ballot(s_end[lane] <= tt)));
         const BatchSlice &b = tab[sid];
-        const uint4 d = gload_u4(b.desc, tt - (sid ? s_end[sid - 1] : 0u));
-        const uint32_t bits =
-            p2g_tile<MAT, CH>(b.g, b.mat, b.pv, d, b.staging_cap, b.dt, b.staging, b.spill, b.flags, b.counters,
-                              b.blk_tile, L);
+        uint4 d = gload_u4(b.desc, tt - (sid ? s_end[sid - 1] : 0u));
+        d.x = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.x);     // uniform: the tile's loops hold barriers
+        d.y = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.y);
+        d.z = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.z);
+        d.w = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.w);
+        const uint32_t bits = p2g_tile<MAT, W>(b.g, b.mat, b.pv, d, b.staging_cap, b.dt, b.staging, b.spill, b.flags,
+                                               b.counters, b.blk_tile, L);
         if (bits) gatomic_or(b.counters + CT_HEALTH, bits);
     }
     if (blockIdx.x == 0)
@@ -1531,6 +1649,10 @@ static int ensure_fast_buffers(mpm_sim *s)
         s->tile_cap = need;
     }
     if (!s->tile_counts) MPM_HIP(hipMalloc(&s->tile_counts, 256 * 4));
+    if (!s->tiles_host) {
+        MPM_HIP(hipHostMalloc((void **)&s->tiles_host, 256 * 4, hipHostMallocCoherent));
+        std::memset(s->tiles_host, 0, 256 * 4);
+    }
     return MPM_OK;
 }
 
@@ -1576,16 +1698,14 @@ int sort_all(mpm_sim *s, bool defer)
         else
             hipLaunchKernelGGL(k_block_keys_hist<8>, dim3(ntiles), dim3(RS_T), 0, st, s->g, pv, s->keys, dmask0,
                                s->sort_hist, ntiles, s->blk_start, blk_end, s->scan_tmp, nb);
-        // a deferred order goes straight to the G2P's permutation
         RadixResult r{};
         if ((rc = radix_sort_ex(st, s->keys, s->vals, s->keys_alt, s->vals_alt, n, bits, s->sort_hist, s->sort_scan,
-                                true, true, defer ? s->g2p_perm + pv.off : nullptr, r)))
+                                true, true, nullptr, r)))
             return hip_fail((hipError_t)rc, "radix_sort");
-        const uint32_t *perm = r.vals;
+        // a deferred order is left for the G2P; the other one needs only a
+        // buffer the radix sort is done with
+        uint32_t *perm = defer ? s->g2p_perm + pv.off : (r.vals == s->vals ? s->vals_alt : s->vals);
         const uint32_t *skeys = r.keys;
-        if (!defer)
-            hipLaunchKernelGGL(k_permute, dim3(round_xcd((uint32_t)nblk(n, 256))), dim3(256), 0, st, s->P, s->P_alt,
-                               s->cap, pv.off, n, perm, s->pid, s->pid_alt, plane_mask);
         // tiles: one per non-empty block, numbered in block order
         hipLaunchKernelGGL(k_block_runs, dim3(nblk(n, 256)), dim3(256), 0, st, skeys, n, s->blk_start, blk_end,
                            s->scan_tmp);
@@ -1594,6 +1714,12 @@ int sort_all(mpm_sim *s, bool defer)
         hipLaunchKernelGGL(k_emit_tiles, dim3(nblk(nb, 256)), dim3(256), 0, st, s->blk_start, blk_end, s->scan_tmp,
                            nb, (uint4 *)s->tile_desc + s->group_tile_off[k], (uint32_t)tile_bound(s, n),
                            s->blk_tile + (int64_t)k * nb, (uint32_t)s->group_tile_off[k]);
+        const uint32_t bound = (uint32_t)tile_bound(s, n);
+        hipLaunchKernelGGL(k_rank_tiles, dim3(std::min<uint32_t>((bound + 3) / 4, 2048u)), dim3(256), 0, st, skeys, r.vals, n,
+                           (const uint4 *)s->tile_desc + s->group_tile_off[k], s->tile_counts + k, bound, perm, s->tiles_host + k);
+        if (!defer)
+            hipLaunchKernelGGL(k_permute, dim3(round_xcd((uint32_t)nblk(n, 256))), dim3(256), 0, st, s->P, s->P_alt,
+                               s->cap, pv.off, n, perm, s->pid, s->pid_alt, plane_mask);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "sort kernels");
     }
@@ -1727,52 +1853,33 @@ int fast_ready(mpm_sim *s)
     return MPM_OK;
 }
 
-// Launchers of the FAST P2G kernels by material and tile shape.
-using BlockLaunch = void (*)(dim3, dim3, hipStream_t, const GridP &, const MatP &, const PartView &, const uint4 *,
-                             const uint32_t *, uint32_t, uint32_t, float, float4 *, uint32_t *, uint32_t *, uint32_t *,
-                             int32_t *);
-using BatchLaunch = void (*)(dim3, dim3, hipStream_t, const BatchSlice *, int);
-template <int MAT, int CH>
-static void launch_block(dim3 gr, dim3 bl, hipStream_t st, const GridP &g, const MatP &m, const PartView &pv,
+// Waves a tile of the FAST P2G.  Two where a tile has fewer particles on
+// average than two waves take at once (others of a workgroup would idle):
+// 2M particles of water, 77 a tile, took 145 us so and 166 with four; four
+// otherwise (262k jello, 512 a tile: 26.0 against 28.3; 1M snow, 300 a tile:
+// 56.6 against 59.4).  The sums do not depend on it.
+constexpr int P2G_WAVES = 4, P2G_WAVES_SPARSE = 2;
+static int p2g_waves(const mpm_sim *s, int group)
+{
+    // of the last sort that ran, 0 before the first
+    const int64_t tiles = __atomic_load_n(&s->tiles_host[group], __ATOMIC_RELAXED);
+    return s->groups[group].n < tiles * 64 * P2G_WAVES_SPARSE ? P2G_WAVES_SPARSE : P2G_WAVES;
+}
+
+template <int MAT>
+static void launch_block(int waves, dim3 gr, hipStream_t st, const GridP &g, const MatP &m, const PartView &pv,
                          const uint4 *desc, const uint32_t *tc, uint32_t cap, uint32_t scap, float dt,
                          float4 *staging, uint32_t *spill, uint32_t *flags, uint32_t *counters, int32_t *blk_tile)
 {
-    hipLaunchKernelGGL((k_p2g_block<MAT, CH>), gr, bl, 0, st, g, m, pv, desc, tc, cap, scap, dt, staging, spill,
-                       flags, counters, blk_tile, 1);
-}
-template <int MAT, int CH>
-static void launch_batch(dim3 gr, dim3 bl, hipStream_t st, const BatchSlice *tab, int n)
-{
-    hipLaunchKernelGGL((k_p2g_batch<MAT, CH>), gr, bl, 0, st, tab, n);
-}
-static int tile_index(int tile) { return tile == 256 ? 0 : (tile == 512 ? 2 : 1); }
-static int mat_index(int mat) { return mat == MPM_JELLO ? 0 : (mat == MPM_SNOW ? 1 : 2); }
-static BlockLaunch block_launcher(int mat, int tile)
-{
-    static const BlockLaunch t[3][3] = {
-        {launch_block<MPM_JELLO, 256>, launch_block<MPM_JELLO, 384>, launch_block<MPM_JELLO, 512>},
-        {launch_block<MPM_SNOW, 256>, launch_block<MPM_SNOW, 384>, launch_block<MPM_SNOW, 512>},
-        {launch_block<MPM_WATER, 256>, launch_block<MPM_WATER, 384>, launch_block<MPM_WATER, 512>}};
-    return t[mat_index(mat)][tile_index(tile)];
-}
-static BatchLaunch batch_launcher(int mat, int tile)
-{
-    static const BatchLaunch t[3][3] = {
-        {launch_batch<MPM_JELLO, 256>, launch_batch<MPM_JELLO, 384>, launch_batch<MPM_JELLO, 512>},
-        {launch_batch<MPM_SNOW, 256>, launch_batch<MPM_SNOW, 384>, launch_batch<MPM_SNOW, 512>},
-        {launch_batch<MPM_WATER, 256>, launch_batch<MPM_WATER, 384>, launch_batch<MPM_WATER, 512>}};
-    return t[mat_index(mat)][tile_index(tile)];
+    if (waves == P2G_WAVES_SPARSE)
+        hipLaunchKernelGGL((k_p2g_block<MAT, P2G_WAVES_SPARSE>), gr, dim3(64 * P2G_WAVES_SPARSE), 0, st, g, m, pv, desc,
+                           tc, cap, scap, dt, staging, spill, flags, counters, blk_tile, 1);
+    else
+        hipLaunchKernelGGL((k_p2g_block<MAT, P2G_WAVES>), gr, dim3(64 * P2G_WAVES), 0, st, g, m, pv, desc, tc, cap, scap,
+                           dt, staging, spill, flags, counters, blk_tile, 1);
 }
 
-int tile_shape(int tile) { return tile == 0 ? TILE_DEFAULT : tile; }
-
-bool tile_shape_valid(int tile)
-{
-    if (tile == 0) return true;
-    for (int t : TILE_SHAPES)
-        if (t == tile) return true;
-    return false;
-}
+bool tile_shape_valid(int tile) { return tile == 0 || tile == 256 || tile == 384 || tile == 512; }
 
 int launch_p2g_tiles(mpm_sim *s, int group, float dt)
 {
@@ -1792,12 +1899,12 @@ int launch_p2g_tiles(mpm_sim *s, int group, float dt)
     }
     uint32_t *hw = nullptr;
     if ((rc = spill_host_word(s, group, &hw))) return rc;
-    dim3 gr(wg), bl(P2G_THREADS);
+    const auto launch = m.type == MPM_JELLO ? launch_block<MPM_JELLO>
+                        : (m.type == MPM_SNOW ? launch_block<MPM_SNOW> : launch_block<MPM_WATER>);
     {
     PhaseTimer tk(s, TK_P2G);
-    block_launcher(m.type, tile_shape(s->cfg.tile))(gr, bl, s->stream, s->g, m, pv, desc, tc, cap, scap, dt,
-                                                    s->staging, s->spill, s->flags, s->counters,
-                                                    s->blk_tile + (int64_t)group * s->nblocks);
+    launch(p2g_waves(s, group), dim3(wg), s->stream, s->g, m, pv, desc, tc, cap, scap, dt, s->staging, s->spill, s->flags,
+           s->counters, s->blk_tile + (int64_t)group * s->nblocks);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "p2g_block");
@@ -2040,13 +2147,13 @@ int launch_sort_batch(hipStream_t st, const SortSlice *tab, int ns, const SortBa
     for (int pass = 0; pass < pl.passes; ++pass) {
         if (pass) hipLaunchKernelGGL(k_bsort_hist, dim3(pl.tiles), dim3(RS_T), 0, st, tab, ns, pass);
         hipLaunchKernelGGL(k_bsort_spine, dim3(pl.spine), dim3(256), 0, st, tab, ns);
-        hipLaunchKernelGGL(k_bsort_scatter, dim3(pl.tiles), dim3(RS_T), 0, st, tab, ns, pass,
-                           pass == pl.passes - 1 ? 1 : 0);
+        hipLaunchKernelGGL(k_bsort_scatter, dim3(pl.tiles), dim3(RS_T), 0, st, tab, ns, pass);
     }
     hipLaunchKernelGGL(k_bsort_runs, dim3(pl.runs), dim3(256), 0, st, tab, ns, pl.passes & 1);
     hipLaunchKernelGGL(k_bsort_scan_reduce, dim3(pl.scan), dim3(SCAN_T), 0, st, tab, ns);
     hipLaunchKernelGGL(k_bsort_scan_apply, dim3(pl.scan), dim3(SCAN_T), 0, st, tab, ns);
     hipLaunchKernelGGL(k_bsort_emit, dim3(pl.emit), dim3(256), 0, st, tab, ns);
+    hipLaunchKernelGGL(k_bsort_rank, dim3(1024), dim3(256), 0, st, tab, ns, pl.passes & 1);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? MPM_OK : hip_fail(e, "sort_batch");
 }
@@ -2080,18 +2187,17 @@ void fill_batch_slice(mpm_sim *s, BatchSlice &b)
     b.copy_q = s->warm_cnt ? 1 : 0;
 }
 
-// Material `mat` of the scenes [0, nslices) of tab, in chunks of P2G_CHUNK,
-// tiles of `tile` particles per pass.
-int launch_p2g_batch(hipStream_t st, int mat, const BatchSlice *tab, const int *types, int nslices, int wgs,
-                     int tile)
+// Material `mat` of the scenes [0, nslices) of tab, in chunks of P2G_CHUNK.
+int launch_p2g_batch(hipStream_t st, int mat, const BatchSlice *tab, const int *types, int nslices, int wgs)
 {
-    dim3 gr(wgs), bl(P2G_THREADS);
+    const auto kernel = mat == MPM_JELLO ? k_p2g_batch<MPM_JELLO, P2G_WAVES>
+                        : (mat == MPM_SNOW ? k_p2g_batch<MPM_SNOW, P2G_WAVES> : k_p2g_batch<MPM_WATER, P2G_WAVES>);
     for (int c0 = 0; c0 < nslices; c0 += P2G_CHUNK) {
         const int n = std::min(P2G_CHUNK, nslices - c0);
         bool any = false;
         for (int k = c0; k < c0 + n; ++k) any = any || types[k] == mat;
         if (!any) continue;
-        batch_launcher(mat, tile_shape(tile))(gr, bl, st, tab + c0, n);
+        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(64 * P2G_WAVES), 0, st, tab + c0, n);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
     }

@@ -45,8 +45,19 @@ struct GridP {
     float ox, oy, oz;
     float gx, gy, gz;
     int pad, bc_mode;
+    uint32_t div_nbx, div_nby;  // floor(2^32 / nbx), floor(2^32 / nby) (see div_by)
     const float *dtp;   // step-size controller on: the step's dt is read here (device memory), else null
 };
+
+// n / d with recip = floor(2^32 / d) (0xFFFFFFFF for d = 1): the high half of
+// the product is the quotient or one less.  Uniform operands stay in scalar
+// registers.
+__host__ __device__ inline uint32_t div_recip(uint32_t d) { return d <= 1u ? 0xFFFFFFFFu : (uint32_t)((1ull << 32) / d); }
+__host__ __device__ __forceinline__ uint32_t div_by(uint32_t n, uint32_t d, uint32_t recip)
+{
+    const uint32_t q = (uint32_t)(((uint64_t)n * recip) >> 32);
+    return n - q * d >= d ? q + 1u : q;
+}
 
 struct MatP {
     int type, water_c_mode;
@@ -359,6 +370,7 @@ struct mpm_sim {
     int64_t tile_cap = 0;
     std::vector<int64_t> group_tile_off;    // per group: first tile slot
     uint32_t *tile_counts = nullptr;        // per group: tiles built by the last sort
+    uint32_t *tiles_host = nullptr;         // pinned: the same counts as of the last sort that ran
     float4 *staging = nullptr;              // per tile: 8^3-node P2G arena written back without atomics
     int64_t staging_cap = 0;                // tiles the staging buffer holds
     int32_t *blk_tile = nullptr;            // [group][block]: tile_entry of the block (-1: no tile)

@@ -65,11 +65,8 @@ int launch_sort_batch(hipStream_t st, const SortSlice *tab, int ns, const SortBa
 int launch_batch_zero(hipStream_t st, const BatchSlice *tab, int nslices);
 // Warm-start particle lists of a simulator (mpm_api.hip).
 int ensure_warm_lists(mpm_sim *s);
-int launch_p2g_batch(hipStream_t st, int mat, const BatchSlice *tab, const int *types, int nslices, int wgs,
-                     int tile);
-// FAST P2G tile shapes (particles per pass over a tile): 0 = the default.
-int tile_shape(int tile);
-bool tile_shape_valid(int tile);
+int launch_p2g_batch(hipStream_t st, int mat, const BatchSlice *tab, const int *types, int nslices, int wgs);
+bool tile_shape_valid(int tile);              // values of mpm_config.tile and mpm_batch_shape.p2g_tile
 int launch_spill_batch(hipStream_t st, const BatchSlice *tab, int nslices, int wgs);
 int launch_compact_batch(hipStream_t st, const BatchSlice *tab, int nslices, int wgs);
 int launch_permute_batch(hipStream_t st, const BatchSlice *src, const BatchSlice *dst, int nslices, int wgs);
