@@ -247,6 +247,7 @@ struct mpm2d_sim {
     hipGraphExec_t graph = nullptr;
     int graph_len = 0;
     int64_t steps = 0;
+    ReadStage reads;
 };
 
 namespace {
@@ -396,14 +397,7 @@ int mpm2d_read(mpm2d_sim *s, int32_t field, float *out)
     case MPM2D_JP: p0 = Q_J; w = 1; break;
     default: return set_error(MPM_ERR_INVALID, "unknown field");
     }
-    std::vector<float> tmp((size_t)w * s->np);
-    for (int k = 0; k < w; ++k)
-        MPM_HIP(hipMemcpyAsync(tmp.data() + (size_t)k * s->np, s->P + (int64_t)(p0 + k) * s->cap,
-                               (size_t)s->np * sizeof(float), hipMemcpyDeviceToHost, s->stream));
-    MPM_HIP(hipStreamSynchronize(s->stream));
-    for (int64_t i = 0; i < s->np; ++i)
-        for (int k = 0; k < w; ++k) out[i * w + k] = tmp[(size_t)k * s->np + i];
-    return MPM_OK;
+    return read_rows(s->reads, s->stream, s->P + (int64_t)p0 * s->cap, s->cap, s->np, w, nullptr, nullptr, out);
 }
 
 int mpm2d_read_grid(mpm2d_sim *s, float *mass, float *vel)

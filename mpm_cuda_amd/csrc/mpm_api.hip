@@ -437,20 +437,10 @@ int mpm_read_particles(mpm_sim *s, int32_t group, int32_t field, float *out)
         }
         s->tau_valid = true;
     }
-    int64_t n = gi.n;
-    std::vector<float> buf((size_t)n * w);
-    std::vector<uint32_t> ids((size_t)n);
-    for (int c = 0; c < w; ++c)
-        MPM_HIP(hipMemcpyAsync(buf.data() + (size_t)c * n, s->P + (size_t)(p0 + c) * s->cap + gi.off,
-                               (size_t)n * 4, hipMemcpyDeviceToHost, s->stream));
-    MPM_HIP(hipMemcpyAsync(ids.data(), s->pid + gi.off, (size_t)n * 4, hipMemcpyDeviceToHost, s->stream));
-    MPM_HIP(hipStreamSynchronize(s->stream));
-    for (int64_t j = 0; j < n; ++j) {
-        uint32_t i = ids[j];
-        if (i >= (uint32_t)n) return set_error(MPM_ERR_STATE, "particle id table corrupted");
-        for (int c = 0; c < w; ++c) out[(size_t)i * w + c] = buf[(size_t)c * n + j];
-    }
-    return MPM_OK;
+    // the other particle buffer is free between calls
+    static_assert(PL_COUNT > 9, "P_alt holds the rows of any field");
+    return read_rows(s->reads, s->stream, s->P + (size_t)p0 * s->cap + gi.off, s->cap, gi.n, w, s->pid + gi.off,
+                     s->P_alt, out);
 }
 
 int mpm_write_particles(mpm_sim *s, int32_t group, int32_t field, const float *in)

@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include <string>
+#include <mutex>
 #include <vector>
 
 #include "../../include/mpm/mpm.h"
@@ -347,6 +348,19 @@ struct SliceScan {
     }
 };
 
+// Particle reads of one simulator (mpm_read.hip); `lock` is held during one.
+// The pinned buffers belong to the process and are freed with its last
+// simulator.
+constexpr int READ_SLOTS = 4;
+struct ReadStage {
+    std::mutex lock;
+    hipEvent_t ev[READ_SLOTS] = {};
+    ReadStage();
+    ~ReadStage();
+    ReadStage(const ReadStage &) = delete;
+    ReadStage &operator=(const ReadStage &) = delete;
+};
+
 }  // namespace mpm
 
 struct mpm_sim {
@@ -360,6 +374,7 @@ struct mpm_sim {
     float *P = nullptr, *P_alt = nullptr;
     uint32_t *pid = nullptr, *pid_alt = nullptr;
     int64_t cap = 0, total = 0;
+    mpm::ReadStage reads;
     std::vector<mpm::GroupInfo> groups;
     bool tau_valid = false;
     // FAST form: sort and tile buffers

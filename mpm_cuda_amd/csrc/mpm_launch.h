@@ -66,6 +66,11 @@ int launch_batch_zero(hipStream_t st, const BatchSlice *tab, int nslices);
 // Warm-start particle lists of a simulator (mpm_api.hip).
 int ensure_warm_lists(mpm_sim *s);
 int launch_p2g_batch(hipStream_t st, int mat, const BatchSlice *tab, const int *types, int nslices, int wgs);
+// Planes of w floats (plane c at planes + c * stride) of n particles to the
+// host rows out[id][w]; ids NULL: in stored order, else `scratch` holds n * w
+// floats rounded up to 16 bytes (mpm_read.hip).
+int read_rows(ReadStage &rs, hipStream_t st, const float *planes, int64_t stride, int64_t n, int w,
+              const uint32_t *ids, float *scratch, float *out);
 bool tile_shape_valid(int tile);              // values of mpm_config.tile and mpm_batch_shape.p2g_tile
 int launch_spill_batch(hipStream_t st, const BatchSlice *tab, int nslices, int wgs);
 int launch_compact_batch(hipStream_t st, const BatchSlice *tab, int nslices, int wgs);
