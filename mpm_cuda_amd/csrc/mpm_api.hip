@@ -247,11 +247,11 @@ int mpm_create(const mpm_config *cfg, mpm_sim **out)
     if (!rc && (e = hipMalloc(&s->grid_v, gbytes)) != hipSuccess) fail(e, "hipMalloc grid_v");
     if (!rc && (e = hipMalloc(&s->flags, (size_t)s->nblocks * 4)) != hipSuccess) fail(e, "hipMalloc flags");
     if (!rc && (e = hipMalloc(&s->list, (size_t)s->nblocks * 4)) != hipSuccess) fail(e, "hipMalloc list");
-    if (!rc && (e = hipMalloc(&s->counters, CT_COUNT * 4)) != hipSuccess) fail(e, "hipMalloc counters");
+    if (!rc && (e = hipMalloc(&s->counters, CT_WORDS * 4)) != hipSuccess) fail(e, "hipMalloc counters");
     if (!rc && (e = hipMemsetAsync(s->grid_mp, 0, gbytes, s->stream)) != hipSuccess) fail(e, "memset");
     if (!rc && (e = hipMemsetAsync(s->grid_v, 0, gbytes, s->stream)) != hipSuccess) fail(e, "memset");
     if (!rc && (e = hipMemsetAsync(s->flags, 0, (size_t)s->nblocks * 4, s->stream)) != hipSuccess) fail(e, "memset");
-    if (!rc && (e = hipMemsetAsync(s->counters, 0, CT_COUNT * 4, s->stream)) != hipSuccess) fail(e, "memset");
+    if (!rc && (e = hipMemsetAsync(s->counters, 0, CT_WORDS * 4, s->stream)) != hipSuccess) fail(e, "memset");
     if (!rc && cfg->dt_mode != MPM_DT_FIXED) {
         if ((e = hipMalloc(&s->dtc, sizeof(DtCtl))) != hipSuccess) fail(e, "hipMalloc dt state");
         else if ((e = hipMemsetAsync(s->dtc, 0, sizeof(DtCtl), s->stream)) != hipSuccess) fail(e, "memset");
@@ -359,7 +359,7 @@ static int dt_control(mpm_sim *s, double max_dt)
 {
     int rc = MPM_OK;
     if (!s->dt_valid) {
-        rc = check_launch(launch_zero_u32(s->stream, s->counters + CT_SPEED, 2), "zero");
+        rc = check_launch(launch_dt_clear(s->stream, s->counters), "dt_clear");
         for (size_t k = 0; k < s->groups.size() && !rc; ++k)
             rc = check_launch(launch_dt_scan(s->stream, s->groups[k].mat, view_of(s, (int)k), s->counters), "dt_scan");
         if (rc) return rc;
@@ -581,12 +581,23 @@ int mpm_health(mpm_sim *s, uint32_t *bits)
     return MPM_OK;
 }
 
+// The counters with the sums of their workgroup copies.
+static int read_counters(mpm_sim *s, uint32_t c[CT_COUNT])
+{
+    uint32_t all[CT_WORDS];
+    MPM_HIP(hipMemcpyAsync(all, s->counters, sizeof all, hipMemcpyDeviceToHost, s->stream));
+    MPM_HIP(hipStreamSynchronize(s->stream));
+    for (int k = 0; k < CT_COUNT; ++k) c[k] = all[k];
+    for (int w = 1; w <= CT_SPREAD; ++w)
+        for (int k : {CT_FALLBACK, CT_REJECT, CT_SVD, CT_WARM}) c[k] += all[CT_COUNT * w + k];
+    return MPM_OK;
+}
+
 int mpm_stats(mpm_sim *s, double st[8])
 {
     if (!s || !st) return set_error(MPM_ERR_INVALID, "null argument");
     uint32_t c[CT_COUNT];
-    MPM_HIP(hipMemcpyAsync(c, s->counters, sizeof c, hipMemcpyDeviceToHost, s->stream));
-    MPM_HIP(hipStreamSynchronize(s->stream));
+    if (int rc = read_counters(s, c)) return rc;
     st[0] = (double)s->steps;
     st[1] = c[CT_ACTIVE];
     st[2] = c[CT_FALLBACK];
@@ -602,8 +613,7 @@ int mpm_svd_stats(mpm_sim *s, double out[4])
 {
     if (!s || !out) return set_error(MPM_ERR_INVALID, "null argument");
     uint32_t c[CT_COUNT];
-    MPM_HIP(hipMemcpyAsync(c, s->counters, sizeof c, hipMemcpyDeviceToHost, s->stream));
-    MPM_HIP(hipStreamSynchronize(s->stream));
+    if (int rc = read_counters(s, c)) return rc;
     out[0] = c[CT_SVD];
     out[1] = c[CT_WARM];
     out[2] = c[CT_REJECT];

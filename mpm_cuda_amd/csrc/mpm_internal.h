@@ -102,8 +102,12 @@ enum Counter : int {
     CT_DEFORM = 9,      // step-size controller: max_p max(J, 1/J) (float bits)
     CT_SVD = 10,        // G2P particle updates that took the Jacobi SVD (cumulative)
     CT_WARM = 11,       // of those, started from a network quaternion (cumulative)
-    CT_COUNT = 16
+    CT_COUNT = 16       // words of a cache line
 };
+// CT_FALLBACK, CT_REJECT, CT_SVD, CT_WARM (summed when read) and CT_SPEED,
+// CT_DEFORM (their maximum) live in CT_SPREAD copies of the line, one a
+// workgroup (see spread).
+constexpr int CT_SPREAD = 256, CT_WORDS = CT_COUNT * (1 + CT_SPREAD);
 
 // Entry of the block -> staging slot map (blk_tile): -1 when the block has
 // no tile; otherwise the slot in bits 0..23 (slots at or above the staging
@@ -191,11 +195,6 @@ __device__ __forceinline__ void gatomic_or(uint32_t *p, uint32_t v)
 // The step's dt: the controller's value in device memory when it is on.
 __device__ __forceinline__ float step_dt(const GridP &g, float dt) { return g.dtp ? *gp(g.dtp) : dt; }
 
-// Largest v over the wave (all 64 lanes take part; NaN loses), merged into
-// *dst with an atomic max.  Non-negative floats order like their bit
-// patterns as unsigned integers.  The atomic is skipped when *dst already
-// holds at least v (a plain read first: once a large value is posted, most
-// waves of a launch leave the single contended word alone).
 // The active lanes of the wave (divergent code included) add their count of
 // `pred` to *dst with one atomic.
 __device__ __forceinline__ void wave_count(uint32_t *dst, bool pred)
@@ -219,15 +218,23 @@ __device__ __forceinline__ void wave_append(uint32_t *list, uint32_t *count, uin
     gp(list)[base + (uint32_t)__popcll(below)] = v;
 }
 
+// Largest v over the wave (all 64 lanes take part; NaN loses), merged into
+// *dst with an atomic max.  Non-negative floats order like their bit
+// patterns as unsigned integers.
 __device__ __forceinline__ void wave_max_to(uint32_t *dst, float v)
 {
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
-    if ((threadIdx.x & 63) == 0 && v > 0.f) {
-        const uint32_t bits = __float_as_uint(v);
-        if (bits > __hip_atomic_load(gp(dst), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            (void)__hip_atomic_fetch_max(gp(dst), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if ((threadIdx.x & 63) == 0 && v > 0.f)
+        (void)__hip_atomic_fetch_max(gp(dst), __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The workgroup's own copy of the counters that every wave of a launch adds
+// to (CT_SPREAD lines after the shared ones): atomics of many waves to one
+// word take turns, ~10 ns each.
+__device__ __forceinline__ uint32_t *spread(uint32_t *counters)
+{
+    return counters + CT_COUNT * (1 + (int)(blockIdx.x % CT_SPREAD));
 }
 
 // Workgroups are dispatched to the 8 XCDs of the device round-robin

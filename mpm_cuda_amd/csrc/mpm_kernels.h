@@ -127,7 +127,7 @@ __device__ __forceinline__ void svd_checked(const float F[9], float U[9], float 
 #pragma unroll
         for (int k = 0; k < 9; ++k) { U[k] = (float)Ud[k]; V[k] = (float)Vd[k]; }
         s[0] = (float)sd[0]; s[1] = (float)sd[1]; s[2] = (float)sd[2];
-        gatomic_add(counters + CT_FALLBACK, 1u);
+        gatomic_add(spread(counters) + CT_FALLBACK, 1u);
     }
 }
 
@@ -146,7 +146,7 @@ __device__ __forceinline__ void svd_warm(const PartView &pv, int i, const float 
     float q[4] = {ld(pv, PL_Q, i), ld(pv, PL_Q + 1, i), ld(pv, PL_Q + 2, i), ld(pv, PL_Q + 3, i)};
     const float qn2 = q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3];
     const bool has_q = qn2 > 0.0f;
-    wave_count(counters + CT_WARM, has_q);
+    wave_count(spread(counters) + CT_WARM, has_q);
     bool ok = false;
     if (has_q && qn2 > 1e-20f && qn2 < 1e20f) {
         const float inv = r_rsqrt(qn2);
@@ -158,7 +158,7 @@ __device__ __forceinline__ void svd_warm(const PartView &pv, int i, const float 
         ok = off <= kWarmTol && s[2] > kFallbackRatio * s[0];
     }
     if (ok) return;
-    wave_count(counters + CT_REJECT, has_q);
+    wave_count(spread(counters) + CT_REJECT, has_q);
     svd_checked(F, U, s, V, sweeps, counters);
 }
 
@@ -169,7 +169,7 @@ __device__ __forceinline__ void svd_warm(const PartView &pv, int i, const float 
 __device__ __forceinline__ void svd_g2p(const MatP &m, const PartView &pv, int i, int io, const float F[9],
                                         float U[9], float s[3], float V[9], int sweeps, uint32_t *counters)
 {
-    wave_count(counters + CT_SVD, true);
+    wave_count(spread(counters) + CT_SVD, true);
     if (m.warm_sweeps > 0) svd_warm(pv, i, F, U, s, V, m.warm_sweeps, sweeps, counters);
     else svd_checked(F, U, s, V, sweeps, counters);
     if (m.wlist) wave_append(m.wlist, m.wcount, (uint32_t)io);

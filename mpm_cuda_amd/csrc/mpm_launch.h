@@ -36,6 +36,7 @@ int launch_spill_compact(hipStream_t st, const GridP &g, const MatP &m, const Pa
                          uint32_t *flags, int nblocks, uint32_t *list, uint32_t *host_count, uint32_t *host_seq,
                          uint32_t seq);
 int launch_dt_scan(hipStream_t st, const MatP &m, const PartView &pv, uint32_t *counters);
+int launch_dt_clear(hipStream_t st, uint32_t *counters);
 int launch_dt_control(hipStream_t st, DtCtl *c, uint32_t *counters, float max_dt, float cfl_h, int mode);
 
 // FAST form (mpm_fast.hip)

@@ -318,8 +318,8 @@ int mpm_probe_svd(const float *F, int64_t n, int32_t sweeps, float *U, float *s,
     MPM_HIP(b.alloc(&dU, n * 36));
     MPM_HIP(b.alloc(&dV, n * 36));
     MPM_HIP(b.alloc(&ds, n * 12));
-    MPM_HIP(b.alloc(&cnt, CT_COUNT * 4));
-    MPM_HIP(hipMemset(cnt, 0, CT_COUNT * 4));
+    MPM_HIP(b.alloc(&cnt, CT_WORDS * 4));
+    MPM_HIP(hipMemset(cnt, 0, CT_WORDS * 4));
     MPM_HIP(hipMemcpy(dF, F, n * 36, hipMemcpyHostToDevice));
     hipLaunchKernelGGL(k_probe_svd, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, dF, (int)n, sweeps, dU, ds,
                        dV, cnt);
@@ -350,8 +350,8 @@ int mpm_probe_stress(const float *F, const float *Jp, int64_t n, int32_t type, d
     MPM_HIP(b.alloc(&dF, n * 36));
     MPM_HIP(b.alloc(&dJ, n * 4));
     MPM_HIP(b.alloc(&dt, n * 24));
-    MPM_HIP(b.alloc(&cnt, CT_COUNT * 4));
-    MPM_HIP(hipMemset(cnt, 0, CT_COUNT * 4));
+    MPM_HIP(b.alloc(&cnt, CT_WORDS * 4));
+    MPM_HIP(hipMemset(cnt, 0, CT_WORDS * 4));
     MPM_HIP(hipMemcpy(dF, F, n * 36, hipMemcpyHostToDevice));
     if (type == MPM_SNOW) MPM_HIP(hipMemcpy(dJ, Jp, n * 4, hipMemcpyHostToDevice));
     else MPM_HIP(hipMemset(dJ, 0, n * 4));
