@@ -8,10 +8,13 @@
 // initialisation reset :154-162 (F_e = F_p = I, C = 0).
 //
 // FP32 structure of arrays on the device.  The workload is small (thousands
-// of particles on a 128^2 grid), so a step is three short kernels -- P2G
-// with float atomics into a (m, p) grid, the grid update (which also clears
-// the accumulation grid for the next step), G2P -- and the runs replay a
-// hipGraph of `graph_steps` steps to take the launch cost off the host.
+// of particles on a 128^2 grid), so a step is two short kernels -- the grid
+// by tiles of nodes, each summed in LDS from the particles that reach it and
+// turned into velocities at once; G2P -- and the runs replay a hipGraph of
+// `graph_steps` steps to take the launch cost off the host.  Workloads for
+// which every tile looking at every particle is too much (grids beyond
+// 1024^2, see tile_side) take three: P2G with float atomics into a (m, p) grid, the grid update (which
+// also clears that grid for the next step), G2P.
 // J_p = det F_p is stored instead of F_p (the step reads only its
 // determinant, :86): J_p <- J_p (s1 s2) / (s1* s2*), which equals
 // det(F_e^-1 F_trial F_p) of :145.  F_e is written as F_trial + U (S* - S) V^T,
@@ -80,21 +83,9 @@ __device__ __forceinline__ uint32_t base2(float x, float inv_dx, int n, int &b)
     return MPM_H_STENCIL_OOB;
 }
 
-// P2G (:84-103): one thread per particle, 9 nodes x 3 float atomics.
-__global__ void __launch_bounds__(256) k2_p2g(P2 p, const float *__restrict__ P, int64_t cap, int np, float4 *gmp,
-                                              uint32_t *health)
+// FixedCorotatedStress with h mu0, h lam0 (:28-32, :87-89).
+__device__ __forceinline__ void stress2(const P2 &p, const float F[4], float Jp, float tau[4])
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= np) return;
-    const float x[2] = {ld2(P, cap, Q_X, i), ld2(P, cap, Q_X + 1, i)};
-    const float v[2] = {ld2(P, cap, Q_V, i), ld2(P, cap, Q_V + 1, i)};
-    float C[4], F[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { C[k] = ld2(P, cap, Q_C + k, i); F[k] = ld2(P, cap, Q_F + k, i); }
-    const float Jp = ld2(P, cap, Q_J, i);
-    int bx, by;
-    uint32_t bits = base2(x[0], p.inv_dx, p.n, bx) | base2(x[1], p.inv_dx, p.n, by);
-    // FixedCorotatedStress with h mu0, h lam0 (:87-89)
     const float hh = expf(p.xi * (1.0f - Jp));
     float U[4], s[2], V[4];
     svd2(F, U, s, V);
@@ -103,8 +94,20 @@ __global__ void __launch_bounds__(256) k2_p2g(P2 p, const float *__restrict__ P,
     const float J = F[0] * F[3] - F[1] * F[2];
     const float D[4] = {F[0] - R[0], F[1] - R[1], F[2] - R[2], F[3] - R[3]};
     const float mu2 = 2.0f * hh * p.mu0, lj = hh * p.lam0 * (J - 1.0f) * J;
-    const float tau[4] = {mu2 * (D[0] * F[0] + D[1] * F[1]) + lj, mu2 * (D[0] * F[2] + D[1] * F[3]),
-                          mu2 * (D[2] * F[0] + D[3] * F[1]), mu2 * (D[2] * F[2] + D[3] * F[3]) + lj};
+    tau[0] = mu2 * (D[0] * F[0] + D[1] * F[1]) + lj;
+    tau[1] = mu2 * (D[0] * F[2] + D[1] * F[3]);
+    tau[2] = mu2 * (D[2] * F[0] + D[3] * F[1]);
+    tau[3] = mu2 * (D[2] * F[2] + D[3] * F[3]) + lj;
+}
+
+// One particle's mass and momentum at the nodes of its stencil, add(bx + a,
+// by + b, m, px, py) for each; returns health bits.
+template <class Add>
+__device__ __forceinline__ uint32_t scatter2(const P2 &p, const float x[2], const float v[2], const float C[4],
+                                             const float tau[4], const Add &add)
+{
+    int bx, by;
+    uint32_t bits = base2(x[0], p.inv_dx, p.n, bx) | base2(x[1], p.inv_dx, p.n, by);
     const float fs = -p.p_vol * p.dt;
     float tw = 0.0f;
 #pragma unroll
@@ -118,15 +121,148 @@ __global__ void __launch_bounds__(256) k2_p2g(P2 p, const float *__restrict__ P,
             const float dpx = gxp - x[0], dpy = gyp - x[1];
             const float gwx = bs_dN(ux) * ny / p.dx, gwy = nx * bs_dN(uy) / p.dx;
             const float mw = w * p.p_mass;
-            const float px = mw * (v[0] + C[0] * dpx + C[1] * dpy) + fs * (tau[0] * gwx + tau[1] * gwy);
-            const float py = mw * (v[1] + C[2] * dpx + C[3] * dpy) + fs * (tau[2] * gwx + tau[3] * gwy);
-            float *dst = (float *)(gmp + (int64_t)(by + b) * p.n + (bx + a));
-            gatomic_add(dst + 0, mw);
-            gatomic_add(dst + 1, px);
-            gatomic_add(dst + 2, py);
+            add(bx + a, by + b, mw, mw * (v[0] + C[0] * dpx + C[1] * dpy) + fs * (tau[0] * gwx + tau[1] * gwy),
+                mw * (v[1] + C[2] * dpx + C[3] * dpy) + fs * (tau[2] * gwx + tau[3] * gwy));
             tw += w;
         }
     if (fabsf(tw - 1.0f) > 1e-4f) bits |= MPM_H_WEIGHT_SUM;        // :102-103
+    return bits;
+}
+
+// Velocity update of a node with mass a.x and momentum (a.y, a.z)
+// (:105-114): (vx, vy, m).
+__device__ __forceinline__ float4 node_velocity(const P2 &p, const float4 a, int i, int j)
+{
+    if (!(a.x > 0.0f)) return make_float4(0.f, 0.f, 0.f, 0.f);
+    float vx = a.y / a.x + p.dt * p.gx, vy = a.z / a.x + p.dt * p.gy;
+    if (i <= p.wall || i >= p.n - p.wall || j <= p.wall || j >= p.n - p.wall) vx = vy = 0.0f;
+    return make_float4(vx, vy, a.x, 0.f);
+}
+
+// What the tiles read of a particle besides x, v and C: the stress of its
+// state and its base node, bx | by << 16 (n_grid <= 16384).
+struct Tau2 {
+    float *tau;         // 4 planes of cap floats
+    uint32_t *base;     // padded to a multiple of four entries, NO_BASE past the last particle
+};
+constexpr uint32_t NO_BASE = 0xFFFFFFFFu;
+
+__device__ __forceinline__ void store_tau2(const P2 &p, const Tau2 &t, int64_t cap, int i, const float x[2],
+                                           const float F[4], float Jp)
+{
+    float tau[4];
+    stress2(p, F, Jp, tau);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) st2(t.tau, cap, k, i, tau[k]);
+    int bx, by;
+    (void)base2(x[0], p.inv_dx, p.n, bx);
+    (void)base2(x[1], p.inv_dx, p.n, by);
+    gp(t.base)[i] = (uint32_t)bx | ((uint32_t)by << 16);
+}
+
+// P2G and velocity update of a T x T tile of nodes by one workgroup.  Its
+// waves look at every particle's base node, four a lane at a time, and keep a
+// list of those whose stencil reaches the tile; 64 of them at once are added
+// to FP64 sums in LDS (~16 cycles a wave; a float atomic there takes ~200).
+// No global atomics: those of particles a few nodes apart, from all eight
+// XCDs to the same lines, were 31 of the 42 us of a step (9,000 particles,
+// 128^2 nodes).
+constexpr int TILE2_T = 1024, TILE2_WAVES = TILE2_T / 64, TILE2_STRIDE = 256;   // a wave's particles per look
+template <int T>
+__global__ void __launch_bounds__(TILE2_T) k2_tile(P2 p, const float *__restrict__ P, int64_t cap, int np, Tau2 t,
+                                                   float4 *gv, uint32_t *health)
+{
+    __shared__ double sum[3][T * T];
+    __shared__ uint32_t list[TILE2_WAVES][64 + TILE2_STRIDE];
+    for (int k = threadIdx.x; k < 3 * T * T; k += TILE2_T) (&sum[0][0])[k] = 0.0;
+    __syncthreads();
+    const int per_row = (p.n + T - 1) / T;
+    const int X0 = (int)(blockIdx.x % (uint32_t)per_row) * T, Y0 = (int)(blockIdx.x / (uint32_t)per_row) * T;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t bits = 0;
+    auto take = [&](uint32_t i) {
+        const float x[2] = {ld2(P, cap, Q_X, i), ld2(P, cap, Q_X + 1, i)};
+        const float v[2] = {ld2(P, cap, Q_V, i), ld2(P, cap, Q_V + 1, i)};
+        float C[4], tau[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { C[k] = ld2(P, cap, Q_C + k, i); tau[k] = ld2(t.tau, cap, k, i); }
+        bits |= scatter2(p, x, v, C, tau, [&](int ix, int iy, float m, float px, float py) {
+            const uint32_t tx = (uint32_t)(ix - X0), ty = (uint32_t)(iy - Y0);
+            if (tx >= (uint32_t)T || ty >= (uint32_t)T) return;
+            const uint32_t o = tx + T * ty;
+            atomicAdd(&sum[0][o], (double)m);
+            atomicAdd(&sum[1][o], (double)px);
+            atomicAdd(&sum[2][o], (double)py);
+        });
+    };
+    uint32_t cnt = 0;       // of the wave's list
+    for (int i0 = w * TILE2_STRIDE; i0 < np; i0 += TILE2_WAVES * TILE2_STRIDE) {
+        const int i = i0 + 4 * lane;
+        uint4 b = make_uint4(NO_BASE, NO_BASE, NO_BASE, NO_BASE);
+        if (i < np) b = gload_u4((const uint4 *)t.base, i >> 2);
+        const uint32_t bb[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            // stencil [bx, bx + 2] against [X0, X0 + T): bx - (X0 - 2) in [0, T + 2)
+            const bool hit = (bb[k] & 0xFFFFu) + 2u - (uint32_t)X0 < (uint32_t)T + 2u &&
+                             (bb[k] >> 16) + 2u - (uint32_t)Y0 < (uint32_t)T + 2u;
+            const uint64_t m = __ballot(hit);
+            if (hit) list[w][cnt + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)(i + k);
+            cnt += (uint32_t)__popcll(m);
+        }
+        __asm__ volatile("" ::: "memory");      // one wave: its LDS operations execute in order
+        while (cnt >= 64) {
+            cnt -= 64;
+            take(list[w][cnt + lane]);
+        }
+        __asm__ volatile("" ::: "memory");
+    }
+    if ((uint32_t)lane < cnt) take(list[w][lane]);
+    __syncthreads();
+    if (threadIdx.x < T * T) {
+        const int o = threadIdx.x, i = X0 + o % T, j = Y0 + o / T;
+        if (i < p.n && j < p.n)
+            gstore4(gv, (int64_t)j * p.n + i,
+                    node_velocity(p, make_float4((float)sum[0][o], (float)sum[1][o], (float)sum[2][o], 0.f), i, j));
+    }
+    if (bits) gatomic_or(health, bits);
+}
+
+// The tiles' inputs of the state as it was added.
+__global__ void __launch_bounds__(256) k2_tau(P2 p, const float *__restrict__ P, int64_t cap, int np, Tau2 t)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= np) {
+        if (i < (np + 3) / 4 * 4) gp(t.base)[i] = NO_BASE;
+        return;
+    }
+    const float x[2] = {ld2(P, cap, Q_X, i), ld2(P, cap, Q_X + 1, i)};
+    float F[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) F[k] = ld2(P, cap, Q_F + k, i);
+    store_tau2(p, t, cap, i, x, F, ld2(P, cap, Q_J, i));
+}
+
+// P2G (:84-103) by atomics: one thread per particle, 9 nodes x 3 float atomics.
+__global__ void __launch_bounds__(256) k2_p2g(P2 p, const float *__restrict__ P, int64_t cap, int np, float4 *gmp,
+                                              uint32_t *health)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    const float x[2] = {ld2(P, cap, Q_X, i), ld2(P, cap, Q_X + 1, i)};
+    const float v[2] = {ld2(P, cap, Q_V, i), ld2(P, cap, Q_V + 1, i)};
+    float C[4], F[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { C[k] = ld2(P, cap, Q_C + k, i); F[k] = ld2(P, cap, Q_F + k, i); }
+    const float Jp = ld2(P, cap, Q_J, i);
+    float tau[4];
+    stress2(p, F, Jp, tau);
+    const uint32_t bits = scatter2(p, x, v, C, tau, [&](int ix, int iy, float m, float px, float py) {
+        float *dst = (float *)(gmp + (int64_t)iy * p.n + ix);
+        gatomic_add(dst + 0, m);
+        gatomic_add(dst + 1, px);
+        gatomic_add(dst + 2, py);
+    });
     if (bits) gatomic_or(health, bits);
 }
 
@@ -138,18 +274,14 @@ __global__ void __launch_bounds__(256) k2_grid(P2 p, float4 *gmp, float4 *gv)
     if (k >= p.n * p.n) return;
     const float4 a = gload4(gmp, k);
     gstore4(gmp, k, make_float4(0.f, 0.f, 0.f, 0.f));
-    float4 out = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (a.x > 0.0f) {
-        const int i = k % p.n, j = k / p.n;
-        float vx = a.y / a.x + p.dt * p.gx, vy = a.z / a.x + p.dt * p.gy;
-        if (i <= p.wall || i >= p.n - p.wall || j <= p.wall || j >= p.n - p.wall) vx = vy = 0.0f;
-        out = make_float4(vx, vy, a.x, 0.f);
-    }
-    gstore4(gv, k, out);
+    gstore4(gv, k, node_velocity(p, a, k % p.n, k / p.n));
 }
 
-// G2P, plasticity and advection (:116-150), one thread per particle.
-__global__ void __launch_bounds__(256) k2_g2p(P2 p, float *P, int64_t cap, int np, const float4 *gv, uint32_t *health)
+// G2P, plasticity and advection (:116-150), one thread per particle; with
+// TILES also the inputs of the next step's tiles.
+template <bool TILES>
+__global__ void __launch_bounds__(256) k2_g2p(P2 p, float *P, int64_t cap, int np, const float4 *gv, uint32_t *health,
+                                              Tau2 t)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= np) return;
@@ -208,6 +340,7 @@ __global__ void __launch_bounds__(256) k2_g2p(P2 p, float *P, int64_t cap, int n
 #pragma unroll
     for (int k = 0; k < 4; ++k) { st2(P, cap, Q_C + k, i, nC[k]); st2(P, cap, Q_F + k, i, Fn[k]); }
     st2(P, cap, Q_J, i, Jn);
+    if (TILES) store_tau2(p, t, cap, i, x, Fn, Jn);
     if (bits) gatomic_or(health, bits);
 }
 
@@ -233,6 +366,15 @@ __global__ void k2_fill(float4 *p, int n)
 
 inline int blocks(int64_t n, int t) { return (int)((n + t - 1) / t); }
 
+// Side of the node tiles on an n^2 grid, 0: P2G by atomics.  The tiles read
+// all base nodes each, 0.4 us a step per million, and number about one a CU;
+// the atomics cost 1.8 us per thousand particles, so that 3,750 tiles are too
+// many whatever the number of particles (1,025^2 nodes and more).  Measured,
+// us a step with side 8, 16, 32 and by atomics: 10k particles on 64^2 nodes
+// 24, 31, 40, 42; 9k on 128^2 16, 20, 28, 38; 160k on 256^2 138, 76, 152,
+// 426; 160k on 512^2 309, 133, 72, 360; 160k on 1,024^2 1,039, 306, 131, 293.
+inline int tile_side(int n) { return n <= 128 ? 8 : (n <= 256 ? 16 : (n <= 1024 ? 32 : 0)); }
+
 }  // namespace
 
 struct mpm2d_sim {
@@ -244,6 +386,8 @@ struct mpm2d_sim {
     int np = 0;
     float4 *gmp = nullptr, *gv = nullptr;
     uint32_t *health = nullptr;
+    int tile = 0;               // tile_side of the particles
+    Tau2 tau{};                 // with tiles
     hipGraphExec_t graph = nullptr;
     int graph_len = 0;
     int64_t steps = 0;
@@ -256,11 +400,18 @@ int enqueue_steps(mpm2d_sim *s, int k)
 {
     const int nn = s->p.n * s->p.n;
     for (int t = 0; t < k; ++t) {
-        hipLaunchKernelGGL(k2_p2g, dim3(blocks(s->np, 256)), dim3(256), 0, s->stream, s->p, s->P, s->cap, s->np,
-                           s->gmp, s->health);
-        hipLaunchKernelGGL(k2_grid, dim3(blocks(nn, 256)), dim3(256), 0, s->stream, s->p, s->gmp, s->gv);
-        hipLaunchKernelGGL(k2_g2p, dim3(blocks(s->np, 256)), dim3(256), 0, s->stream, s->p, s->P, s->cap, s->np,
-                           s->gv, s->health);
+        const dim3 pg(blocks(s->np, 256)), pt(256);
+        if (s->tile) {
+            const int per_row = blocks(s->p.n, s->tile);
+            const auto grid = s->tile == 8 ? k2_tile<8> : (s->tile == 16 ? k2_tile<16> : k2_tile<32>);
+            hipLaunchKernelGGL(grid, dim3(per_row * per_row), dim3(TILE2_T), 0, s->stream, s->p, s->P, s->cap, s->np,
+                               s->tau, s->gv, s->health);
+            hipLaunchKernelGGL(k2_g2p<true>, pg, pt, 0, s->stream, s->p, s->P, s->cap, s->np, s->gv, s->health, s->tau);
+            continue;
+        }
+        hipLaunchKernelGGL(k2_p2g, pg, pt, 0, s->stream, s->p, s->P, s->cap, s->np, s->gmp, s->health);
+        hipLaunchKernelGGL(k2_grid, dim3(blocks(nn, 256)), pt, 0, s->stream, s->p, s->gmp, s->gv);
+        hipLaunchKernelGGL(k2_g2p<false>, pg, pt, 0, s->stream, s->p, s->P, s->cap, s->np, s->gv, s->health, s->tau);
     }
     MPM_HIP(hipGetLastError());
     return MPM_OK;
@@ -343,12 +494,18 @@ int mpm2d_add_particles(mpm2d_sim *s, int64_t n, const float *xy, const float *v
         if (!(xy[i] >= lo && xy[i] <= hi)) return set_error(MPM_ERR_RANGE, "particle outside [dx, 1 - 2 dx]");
     s->cap = n;
     MPM_HIP(hipMalloc(&s->P, (size_t)Q_COUNT * n * sizeof(float)));
+    if ((s->tile = tile_side(s->p.n))) {
+        MPM_HIP(hipMalloc(&s->tau.tau, (size_t)4 * n * sizeof(float)));
+        MPM_HIP(hipMalloc(&s->tau.base, (size_t)blocks(n, 4) * sizeof(uint4)));
+    }
     float *dxy = nullptr, *dv = nullptr;
     MPM_HIP(hipMalloc(&dxy, (size_t)n * 2 * sizeof(float)));
     if (vel) MPM_HIP(hipMalloc(&dv, (size_t)n * 2 * sizeof(float)));
     MPM_HIP(hipMemcpyAsync(dxy, xy, (size_t)n * 2 * sizeof(float), hipMemcpyHostToDevice, s->stream));
     if (vel) MPM_HIP(hipMemcpyAsync(dv, vel, (size_t)n * 2 * sizeof(float), hipMemcpyHostToDevice, s->stream));
     hipLaunchKernelGGL(k2_init, dim3(blocks(n, 256)), dim3(256), 0, s->stream, s->P, s->cap, (int)n, dxy, dv);
+    if (s->tile)
+        hipLaunchKernelGGL(k2_tau, dim3(blocks(n + 3, 256)), dim3(256), 0, s->stream, s->p, s->P, s->cap, (int)n, s->tau);
     MPM_HIP(hipGetLastError());
     MPM_HIP(hipStreamSynchronize(s->stream));
     (void)hipFree(dxy);
@@ -438,7 +595,7 @@ void mpm2d_destroy(mpm2d_sim *s)
     if (!s) return;
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     if (s->graph) (void)hipGraphExecDestroy(s->graph);
-    void *ptrs[] = {s->P, s->gmp, s->gv, s->health};
+    void *ptrs[] = {s->P, s->gmp, s->gv, s->health, s->tau.tau, s->tau.base};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     if (s->stream) (void)hipStreamDestroy(s->stream);

@@ -134,3 +134,35 @@ def test_errors(gpu):
             s.add_particles(np.array([[0.5, 0.5]], np.float32))
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("n_grid,n", [(9, 1), (16, 63), (33, 257), (128, 4097), (129, 999), (257, 5000), (1024, 3000),
+                                      (1025, 3000)])
+def test_grid_by_tiles(gpu, n_grid, n):
+    """Two steps against the FP64 oracle where the node tiles have remainders,
+    change their side (8, 16, 32 nodes) or give way to the atomics.  Bounds:
+    those of one step on 128^2 nodes, or four roundings of a position of order
+    1 in units of a cell.  (A single particle's C is exactly zero; it is
+    measured against v / dx.)"""
+    rng = np.random.default_rng(n_grid)
+    x = (0.5 + 0.28 * (rng.random((n, 2)) - 0.5)).astype(np.float32)
+    v = (2.0 * rng.normal(size=x.shape)).astype(np.float32)
+    g, o = _pair(x, v, n_grid=n_grid, wall=1, graph_steps=0)
+    try:
+        for _ in range(2):
+            g.run(1)
+            assert o.step(1e-4) == 0
+        m, gv = g.grid()
+        tol = max(1e-5, 4 * 2.0 ** -24 * n_grid)
+        assert rel(m, o.grid_m) < tol
+        assert rel(m[:, None] * gv, o.grid_m[:, None] * o.grid_v.reshape(-1, 2)) < tol
+        gf, of = _fields(g, o)
+        errs = {k: rel(gf[k], of[k]) for k in gf}
+        if n == 1:
+            errs["C"] = np.linalg.norm(gf["C"] - of["C"]) / (n_grid * np.linalg.norm(of["v"]))
+        print("2D tiles", n_grid, n, {k: f"{e:.1e}" for k, e in errs.items()})
+        for k, e in errs.items():
+            assert e < tol, (k, e)
+        assert g.health() == 0
+    finally:
+        g.close()
