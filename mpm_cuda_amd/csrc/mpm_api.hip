@@ -247,10 +247,12 @@ int mpm_create(const mpm_config *cfg, mpm_sim **out)
     if (!rc && (e = hipMalloc(&s->grid_v, gbytes)) != hipSuccess) fail(e, "hipMalloc grid_v");
     if (!rc && (e = hipMalloc(&s->flags, (size_t)s->nblocks * 4)) != hipSuccess) fail(e, "hipMalloc flags");
     if (!rc && (e = hipMalloc(&s->list, (size_t)s->nblocks * 4)) != hipSuccess) fail(e, "hipMalloc list");
+    if (!rc && (e = hipMalloc(&s->act, (size_t)s->nblocks * 4)) != hipSuccess) fail(e, "hipMalloc act");
     if (!rc && (e = hipMalloc(&s->counters, CT_WORDS * 4)) != hipSuccess) fail(e, "hipMalloc counters");
     if (!rc && (e = hipMemsetAsync(s->grid_mp, 0, gbytes, s->stream)) != hipSuccess) fail(e, "memset");
     if (!rc && (e = hipMemsetAsync(s->grid_v, 0, gbytes, s->stream)) != hipSuccess) fail(e, "memset");
     if (!rc && (e = hipMemsetAsync(s->flags, 0, (size_t)s->nblocks * 4, s->stream)) != hipSuccess) fail(e, "memset");
+    if (!rc && (e = hipMemsetAsync(s->act, 0, (size_t)s->nblocks * 4, s->stream)) != hipSuccess) fail(e, "memset");
     if (!rc && (e = hipMemsetAsync(s->counters, 0, CT_WORDS * 4, s->stream)) != hipSuccess) fail(e, "memset");
     if (!rc && cfg->dt_mode != MPM_DT_FIXED) {
         if ((e = hipMalloc(&s->dtc, sizeof(DtCtl))) != hipSuccess) fail(e, "hipMalloc dt state");
@@ -270,7 +272,6 @@ int mpm_add_particles(mpm_sim *s, const mpm_material *mat, int64_t n, const floa
     int rc = validate_material(mat);
     if (rc) return rc;
     if (n <= 0 || !xyz) return set_error(MPM_ERR_INVALID, "no particles");
-    if ((rc = flush_spill(s))) return rc;     // a P2G phase's spill scatter reads the state it saw
     // particle offsets inside a plane are 32-bit byte offsets on the device
     if (s->total + n > MPM_MAX_PARTICLES) return set_error(MPM_ERR_INVALID, "too many particles");
     if ((int64_t)s->groups.size() >= MAX_GROUPS) return set_error(MPM_ERR_INVALID, "at most 256 particle groups");
@@ -450,7 +451,6 @@ int mpm_write_particles(mpm_sim *s, int32_t group, int32_t field, const float *i
     if (field == MPM_P_TAU) return set_error(MPM_ERR_INVALID, "TAU is derived state and read-only");
     int w = width_of(field), p0 = plane_of(field);
     if (w < 0) return set_error(MPM_ERR_INVALID, "unknown particle field");
-    if (int rc = flush_spill(s)) return rc;   // a P2G phase's spill scatter reads the state it saw
     const GroupInfo &gi = s->groups[group];
     int64_t n = gi.n;
     if (field == MPM_P_POS) {
@@ -500,7 +500,6 @@ int mpm_read_grid(mpm_sim *s, int32_t field, float *out)
 {
     if (!s || !out) return set_error(MPM_ERR_INVALID, "null argument");
     if (field < MPM_G_MASS || field > MPM_G_VELOCITY) return set_error(MPM_ERR_INVALID, "unknown grid field");
-    if (int rc = flush_spill(s)) return rc;   // after a P2G phase: its spilled particles' share
     const GridP &g = s->g;
     size_t nslots = (size_t)s->nblocks * BLK_NODES;
     std::vector<float4> mp(nslots), gv(nslots);
@@ -509,13 +508,9 @@ int mpm_read_grid(mpm_sim *s, int32_t field, float *out)
     MPM_HIP(hipMemcpyAsync(gv.data(), s->grid_v, nslots * sizeof(float4), hipMemcpyDeviceToHost, s->stream));
     MPM_HIP(hipMemcpyAsync(cnt.data(), s->counters, CT_COUNT * 4, hipMemcpyDeviceToHost, s->stream));
     MPM_HIP(hipStreamSynchronize(s->stream));
-    uint32_t nact = cnt[CT_ACTIVE];
-    std::vector<uint32_t> lst(nact);
-    if (nact) {
-        MPM_HIP(hipMemcpy(lst.data(), s->list, (size_t)nact * 4, hipMemcpyDeviceToHost));
-    }
-    std::vector<char> active((size_t)s->nblocks, 0);
-    for (uint32_t k = 0; k < nact; ++k) if (lst[k] < (uint32_t)s->nblocks) active[lst[k]] = 1;
+    const uint32_t seq = s->act_seq == BATCH_SEQ ? BATCH_SEQ | cnt[CT_SEQ] : s->act_seq;
+    std::vector<uint32_t> act((size_t)s->nblocks);
+    MPM_HIP(hipMemcpy(act.data(), s->act, act.size() * 4, hipMemcpyDeviceToHost));
     // grid_mp holds (m, p) between P2G and the grid update; grid_v after it
     const bool after_p2g = s->last_phase == MPM_PHASE_P2G;
     if (after_p2g && s->cfg.form != MPM_FORM_PLAIN && s->blk_tile) {
@@ -559,7 +554,7 @@ int mpm_read_grid(mpm_sim *s, int32_t field, float *out)
                 int64_t blk = slot / BLK_NODES;
                 size_t o = ((size_t)z * g.ny + y) * g.nx + x;
                 float4 a = mp[slot];
-                float4 b = active[blk] ? gv[slot] : make_float4(0, 0, 0, 0);
+                float4 b = seq != 0u && act[blk] == seq ? gv[slot] : make_float4(0, 0, 0, 0);
                 if (field == MPM_G_MASS) out[o] = after_p2g ? a.x : b.w;
                 else if (field == MPM_G_MOMENTUM) { out[3 * o] = a.y; out[3 * o + 1] = a.z; out[3 * o + 2] = a.w; }
                 else { out[3 * o] = b.x; out[3 * o + 1] = b.y; out[3 * o + 2] = b.z; }
@@ -597,6 +592,9 @@ int mpm_stats(mpm_sim *s, double st[8])
 {
     if (!s || !st) return set_error(MPM_ERR_INVALID, "null argument");
     uint32_t c[CT_COUNT];
+    if (s->act_seq)
+        if (int rc = check_launch(launch_count_active(s->stream, s->act, s->act_seq, s->nblocks, s->counters, nullptr), "count"))
+            return rc;
     if (int rc = read_counters(s, c)) return rc;
     st[0] = (double)s->steps;
     st[1] = c[CT_ACTIVE];
@@ -729,7 +727,7 @@ void mpm_destroy(mpm_sim *s)
 {
     if (!s) return;
     if (s->stream) (void)hipStreamSynchronize(s->stream);
-    void *ptrs[] = {s->grid_mp, s->grid_v, s->flags, s->list, s->counters, s->P, s->P_alt, s->pid,
+    void *ptrs[] = {s->grid_mp, s->grid_v, s->flags, s->list, s->act, s->counters, s->P, s->P_alt, s->pid,
                     s->pid_alt, s->keys, s->keys_alt, s->vals, s->vals_alt, s->sort_hist, s->sort_scan,
                     s->blk_count, s->blk_start, s->tile_desc, s->scan_tmp, s->tile_counts, s->mlp_w,
                     s->staging, s->blk_tile, s->spill, s->dtc, s->warm_list, s->warm_cnt, s->g2p_perm};
@@ -816,13 +814,11 @@ static int run_phase(mpm_sim *s, int phase, float dt)
     int rc = MPM_OK;
     s->last_phase = phase;
     if (phase == MPM_PHASE_P2G) {
-        // FAST form: the last block compaction cleared the spill counter and
-        // this P2G's spill kernels clear the active-block and node counters
+        // FAST form: the last grid update cleared the spill counter
         const bool clean = s->cfg.form == MPM_FORM_FAST && s->counters_clean && s->total > 0;
         s->counters_clean = false;
-        if ((rc = flush_spill(s))) return rc;
         if (!clean) {
-            rc = check_launch(launch_zero_u32(s->stream, s->counters + CT_ACTIVE, 3), "zero");
+            rc = check_launch(launch_zero_u32(s->stream, s->counters + CT_SPILL, 1), "zero");
             if (rc) return rc;
         }
         if (fast) {
@@ -832,7 +828,7 @@ static int run_phase(mpm_sim *s, int phase, float dt)
             }
             if (rc) return rc;
             PhaseTimer t(s, 1);
-            for (size_t k = 0; k < s->groups.size() && !rc; ++k) rc = launch_p2g_tiles(s, (int)k, dt);
+            rc = launch_p2g_tiles(s, dt);
         } else {
             PhaseTimer t(s, 1), tk(s, TK_P2G);
             for (size_t k = 0; k < s->groups.size() && !rc; ++k)
@@ -844,23 +840,28 @@ static int run_phase(mpm_sim *s, int phase, float dt)
     }
     if (phase == MPM_PHASE_GRID) {
         {
-            PhaseTimer t(s, 2);
-            const bool fused = s->spill_pending;
-            rc = fused ? spill_compact(s)
-                       : check_launch(launch_compact(s->stream, s->flags, (int)s->nblocks, s->list, s->counters),
-                                      "compact");
-            if (rc) return rc;
-            s->counters_clean = true;
+            PhaseTimer t(s, 2), tk(s, TK_GRID);
             const bool staged = fast && s->blk_tile;
-            PhaseTimer tk(s, TK_GRID);
-            rc = check_launch(launch_grid_update(s->stream, s->g, dt, s->list, s->counters, s->grid_mp, s->grid_v,
-                                                 (int)s->nblocks, staged ? s->staging : nullptr,
+            uint32_t *count, *seq, launch;
+            if ((rc = spill_publish(s, &count, &seq, &launch))) return rc;
+            if (++s->grid_seq >= BATCH_SEQ) {
+                if ((rc = check_launch(launch_zero_u32(s->stream, s->act, (int)s->nblocks), "zero"))) return rc;
+                s->grid_seq = 1;
+            }
+            s->act_seq = s->grid_seq;
+            if (!staged &&
+                (rc = check_launch(launch_list_marked(s->stream, s->flags, (int)s->nblocks, s->list, s->counters), "list")))
+                return rc;
+            rc = check_launch(launch_grid_update(s->stream, s->g, dt, s->list, s->flags, s->act, s->act_seq, s->counters,
+                                                 s->grid_mp, s->grid_v, s->nblocks, staged ? s->staging : nullptr,
                                                  staged ? s->blk_tile : nullptr, (int)s->groups.size(),
-                                                 (uint32_t)s->staging_cap, fused ? 1 : 0),
+                                                 (uint32_t)s->staging_cap, count, seq, launch),
                               "grid_update");
             if (rc) return rc;
+            s->counters_clean = true;
         }
-        if (s->timing) rc = check_launch(launch_count_nodes(s->stream, s->list, s->counters, s->grid_v), "count");
+        if (s->timing)
+            rc = check_launch(launch_count_active(s->stream, s->act, s->act_seq, s->nblocks, s->counters, s->grid_v), "count");
         return rc;
     }
     // G2P; a due re-sort of the FAST form is applied by this G2P
@@ -876,13 +877,12 @@ static int run_phase(mpm_sim *s, int phase, float dt)
     }
     {
         PhaseTimer t(s, 3), tk(s, TK_G2P);
-        for (size_t k = 0; k < s->groups.size() && !rc; ++k) {
-            if (fast) rc = launch_g2p_fast(s, (int)k, dt);
-            else
+        if (fast) rc = launch_g2p_fast(s, dt);
+        else
+            for (size_t k = 0; k < s->groups.size() && !rc; ++k)
                 rc = check_launch(launch_g2p(s->stream, s->g, s->groups[k].mat, view_of(s, (int)k), dt, s->grid_v,
                                              0, s->cfg.svd_sweeps, s->counters, thr),
                                   "g2p");
-        }
     }
     if (rc) return rc;          // a failed launch leaves the device state undefined either way
     if ((rc = finish_g2p_move(s, true))) return rc;
@@ -903,9 +903,6 @@ static int fused_step(mpm_sim *s, float dt)
     int rc = MPM_OK;
     if (!s->primed || s->primed_dt != dt) {
         rc = run_phase(s, MPM_PHASE_P2G, dt);
-        if (rc) return rc;
-    } else {
-        rc = check_launch(launch_zero_u32(s->stream, s->counters + CT_ACTIVE, 2), "zero");
         if (rc) return rc;
     }
     rc = run_phase(s, MPM_PHASE_GRID, dt);

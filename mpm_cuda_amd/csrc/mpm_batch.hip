@@ -26,7 +26,6 @@ using namespace mpm;
 
 namespace {
 
-constexpr int SPILL_WGS = 512;
 constexpr int NCAND = 4;
 const int P2G_CAND[NCAND] = {1024, 2048, 4096, 8192};   // one-wave workgroups
 const int GRID_CAND[NCAND] = {1024, 2048, 4096, 8192};
@@ -67,12 +66,10 @@ struct mpm_batch {
     int parity = 0;
     int64_t steps_since_sort = 0;
     int64_t total = 0;
-    int compact_wgs = 0;
     std::vector<int> types;             // material of each scene
     // scenes are kept ordered by material: material m holds table entries
-    // [mat_begin[m], mat_begin[m] + mat_count[m]); its block compaction
-    // takes mat_compact_wgs[m] workgroups
-    int mat_begin[3] = {0, 0, 0}, mat_count[3] = {0, 0, 0}, mat_compact_wgs[3] = {0, 0, 0};
+    // [mat_begin[m], mat_begin[m] + mat_count[m])
+    int mat_begin[3] = {0, 0, 0}, mat_count[3] = {0, 0, 0};
     int permute_wgs = 0;                // workgroups of the batched re-sort move
     SortSlice *stab[2] = {};            // batched re-sort tables of both parities
     SortBatchPlan splan;
@@ -155,17 +152,14 @@ int fork_materials(mpm_batch *b, L launch)
 }
 
 // The step of one material's scenes (table range [s0, s0 + cnt)) on stream
-// ms: counter reset, P2G, spill scatter, block compaction, grid update, the
-// warm-start inference of each weight set among them, G2P.
+// ms: P2G, grid update, the warm-start inference of each weight set among
+// them, G2P.
 int enqueue_material(mpm_batch *b, hipStream_t ms, int m, const BatchSlice *tab, int s0, int cnt, int p2g, int grid,
                      int g2p_threads)
 {
     const BatchSlice *t = tab + s0;
     int rc;
-    if ((rc = check(launch_batch_zero(ms, t, cnt), "batch_zero"))) return rc;
     if ((rc = check(launch_p2g_batch(ms, m, t, b->types.data() + s0, cnt, p2g), "p2g_batch"))) return rc;
-    if ((rc = check(launch_spill_batch(ms, t, cnt, SPILL_WGS), "spill_batch"))) return rc;
-    if ((rc = check(launch_compact_batch(ms, t, cnt, b->mat_compact_wgs[m]), "compact_batch"))) return rc;
     if ((rc = check(launch_grid_batch(ms, t, cnt, grid), "grid_batch"))) return rc;
     for (const auto &ws : b->mat_sets[m])
         if ((rc = check(launch_mlp_infer_batch(ms, b->warm_params[ws.first], t, cnt, ws.first, ws.second),
@@ -191,15 +185,12 @@ int enqueue_step(mpm_batch *b, int p, int p2g, int grid, int g2p_threads, hipEve
         return fork_materials(b, [&](hipStream_t ms, int m) {
             return enqueue_material(b, ms, m, tab, b->mat_begin[m], b->mat_count[m], p2g, grid, g2p_threads);
         });
-    if ((rc = check(launch_batch_zero(st, tab, n), "batch_zero"))) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[0], st));
     rc = fork_materials(b, [&](hipStream_t ms, int m) {
         return check(launch_p2g_batch(ms, m, tab, b->types.data(), n, p2g), "p2g_batch");
     });
     if (rc) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[1], st));
-    if ((rc = check(launch_spill_batch(st, tab, n, SPILL_WGS), "spill_batch"))) return rc;
-    if ((rc = check(launch_compact_batch(st, tab, n, b->compact_wgs), "compact_batch"))) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[2], st));
     if ((rc = check(launch_grid_batch(st, tab, n, grid), "grid_batch"))) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[3], st));
@@ -342,7 +333,7 @@ int build(mpm_batch *b)
             h[k].warm_group = b->warm_group[k];
             if (warm_on(s)) {
                 // the G2P lists the particles that take the SVD; the next
-                // step's inference runs over them (k_batch_zero hands them over)
+                // step's inference runs over them (k_grid_batch hands them over)
                 h[k].mat.wlist = s->warm_list;
                 h[k].mat.wcount = s->warm_cnt + 1;
                 h[k].warm_cnt = s->warm_cnt;
@@ -400,8 +391,10 @@ int prepare(mpm_batch *b)
     const size_t n = b->sims.size();
     for (size_t k = 0; k < n; ++k) {
         mpm_sim *s = b->sims[k];
-        s->counters_clean = false;     // batch steps reset the counters themselves
-        if (int rc = flush_spill(s)) return rc;
+        if (!s->counters_clean)         // a batch's grid update leaves it cleared
+            if (int rc = check(launch_zero_u32(s->stream, s->counters + CT_SPILL, 1), "zero")) return rc;
+        s->counters_clean = true;
+        s->spill_unread = false;
         if (parity_of(b, k) < 0) return set_error(MPM_ERR_INVALID, "a scene's particle storage changed since mpm_batch_create");
         if (s->groups.size() != 1) return set_error(MPM_ERR_INVALID, "a scene of the batch gained a particle group");
         int rc = fast_ready(s);
@@ -466,6 +459,7 @@ void after_step(mpm_batch *b)
         s->steps_since_sort += 1;
         s->tau_valid = true;
         s->last_phase = MPM_PHASE_G2P;
+        s->act_seq = BATCH_SEQ;
     }
     b->steps_since_sort += 1;
 }
@@ -561,7 +555,6 @@ int mpm_batch_create(mpm_sim *const *sims, int32_t n, const mpm_batch_shape *sha
     for (mpm_sim *s : b->sims) {
         b->P0.push_back(s->P); b->P1.push_back(s->P_alt);
         b->pid0.push_back(s->pid); b->pid1.push_back(s->pid_alt);
-        b->compact_wgs += (int)((s->nblocks + 255) / 256);
     }
     uint32_t pblocks = 0;
     for (mpm_sim *s : b->sims) pblocks += (uint32_t)((s->groups[0].n + 255) / 256);
@@ -570,7 +563,6 @@ int mpm_batch_create(mpm_sim *const *sims, int32_t n, const mpm_batch_shape *sha
         const int m = b->types[k];
         if (b->mat_count[m] == 0) b->mat_begin[m] = k;
         b->mat_count[m] += 1;
-        b->mat_compact_wgs[m] += (int)((b->sims[k]->nblocks + 255) / 256);
     }
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking)) != hipSuccess) return fail(hip_fail(e, "stream"));

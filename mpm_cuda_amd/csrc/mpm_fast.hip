@@ -550,15 +550,20 @@ __device__ __forceinline__ void rank_tile(const uint32_t *__restrict__ skeys, co
 }
 
 // One wave per tile; 10-18 us a sort (262k-2M particles).  The number of
-// tiles goes to a pinned host word for the choice of the P2G's width.
+// tiles goes to a pinned host word for the choice of the P2G's width; the
+// list of blocks that follows starts over.
 __global__ void __launch_bounds__(256) k_rank_tiles(const uint32_t *__restrict__ skeys, const uint32_t *__restrict__ sperm,
                                                     int n, const uint4 *__restrict__ desc,
                                                     const uint32_t *__restrict__ tile_count, uint32_t desc_cap,
-                                                    uint32_t *__restrict__ perm, uint32_t *tiles_host)
+                                                    uint32_t *__restrict__ perm, uint32_t *tiles_host,
+                                                    uint32_t *counters)
 {
     __shared__ RankLds L[4];
     const uint32_t w = threadIdx.x >> 6, nt = min(*tile_count, desc_cap);
-    if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(tiles_host, nt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        __hip_atomic_store(tiles_host, nt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        gp(counters)[CT_LIST] = 0u;
+    }
     for (uint32_t t = blockIdx.x * 4 + w; t < nt; t += gridDim.x * 4) rank_tile(skeys, sperm, desc[t], (uint32_t)n, perm, L[w]);
 }
 
@@ -687,6 +692,7 @@ __global__ void __launch_bounds__(256) k_bsort_rank(const SortSlice *__restrict_
     SliceScan sc;
     sc.build(ns, [&](int s) { return min(*gp(tab[s].tile_count), tab[s].desc_cap); });
     const uint32_t w = threadIdx.x >> 6;
+    if (blockIdx.x == 0 && (int)threadIdx.x < ns) gp(tab[threadIdx.x].counters)[CT_LIST] = 0u;
     for (uint32_t k = blockIdx.x * 4 + w; k < sc.total; k += gridDim.x * 4) {
         const uint32_t sid = (uint32_t)__builtin_amdgcn_readfirstlane((int)sc.find(k));
         const SortSlice &t = tab[sid];
@@ -713,7 +719,8 @@ __global__ void __launch_bounds__(256) k_bsort_rank(const SortSlice *__restrict_
 //      lanes of one bin take turns.
 // The arena is written to the tile's staging slot, which the grid update
 // gathers.  Particles whose stencil leaves the arena (or whose tile has no
-// staging slot) are listed for the atomic fallback kernel.
+// staging slot) take the atomic fallback: at the end of their tile (FAST) or
+// listed for a kernel after this one (FUSED).
 constexpr int TILE_WAVES = 2;                    // FUSED form: waves per tile
 constexpr int TILE_THREADS = 64 * TILE_WAVES;
 static_assert(ARENA_NODES % TILE_THREADS == 0, "arena nodes per thread must be whole");
@@ -819,12 +826,11 @@ __device__ __forceinline__ TileGeo tile_geo(const GridP &g, uint32_t blk)
     return TileGeo{bx * BLK - 1, by * BLK - 1, (int)bz * BLK - 1};
 }
 
-// Phase A tail: a particle whose base lies outside the arena's bins (or whose
-// tile has no staging slot) gets an entry in the list of the atomic fallback
-// (its node blocks are flagged here when `flags` is given).  Returns true
-// when the particle was listed.
+// FUSED form phase A tail: a particle whose base lies outside the arena's bins (or whose
+// tile has no staging slot) gets an entry in the list of the atomic fallback.
+// Returns true when the particle was listed.
 __device__ __forceinline__ bool list_spill(const GridP &g, const TileGeo &t, bool active, int i, const int b[3],
-                                           bool staged, uint32_t *spill, uint32_t *counters, uint32_t *flags)
+                                           bool staged, uint32_t *spill, uint32_t *counters)
 {
     const int lane = threadIdx.x & 63;
     const int lx = b[0] - t.ax, ly = b[1] - t.ay, lz = b[2] - t.az;
@@ -838,10 +844,7 @@ __device__ __forceinline__ bool list_spill(const GridP &g, const TileGeo &t, boo
         if (lane == leader) base = gatomic_add(counters + CT_SPILL, (uint32_t)__popcll(sm));
         base = __shfl(base, leader);
         const uint64_t below = lane ? (sm & ((~0ull) >> (64 - lane))) : 0ull;
-        if (spill_me) {
-            gp(spill)[base + __popcll(below)] = (uint32_t)i;
-            if (flags) mark_blocks(g, b, flags);
-        }
+        if (spill_me) gp(spill)[base + __popcll(below)] = (uint32_t)i;
     }
     return spill_me;
 }
@@ -875,7 +878,7 @@ __device__ __forceinline__ bool bin_particle(const GridP &g, TileLds &L, const T
                                              int i, const Stencil &s, const Scatter &sc, bool staged,
                                              uint32_t *spill, uint32_t *counters)
 {
-    const bool spill_me = list_spill(g, t, active, i, s.b, staged, spill, counters, nullptr);
+    const bool spill_me = list_spill(g, t, active, i, s.b, staged, spill, counters);
     if (active) L.key[slot] = spill_me ? (uint8_t)NO_BIN : (uint8_t)bin_of(t, s.b);
     if (active && !spill_me) {
         float q0[3], hB[9], Gs[6];
@@ -1184,7 +1187,8 @@ __device__ __forceinline__ void tile_clear(TileLds &L)
 // Sum the waves' arenas into staging slot `slot` (logical node order) and
 // mark the node blocks that received mass.
 __device__ __forceinline__ void tile_end(const GridP &g, const TileGeo &t, const TileLds &L, float4 *staging,
-                                         uint32_t slot, bool staged, uint32_t *flags, int32_t *blk_entry)
+                                         uint32_t slot, bool staged, uint32_t *flags, uint32_t *list, uint32_t *counters,
+                                         int32_t *blk_entry)
 {
     __syncthreads();
     if (staged) {
@@ -1201,9 +1205,8 @@ __device__ __forceinline__ void tile_end(const GridP &g, const TileGeo &t, const
                 v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
             }
             gstore4(staging, dst + k, v);
-            const int nx_ = t.ax + kx, ny_ = t.ay + ky, nz_ = t.az + kz;
-            if (v.x != 0.f && nx_ >= 0 && ny_ >= 0 && nz_ >= 0 && nx_ < g.nx && ny_ < g.ny && nz_ < g.nz)
-                gp(flags)[((int64_t)(nz_ >> 2) * g.nby + (ny_ >> 2)) * g.nbx + (nx_ >> 2)] = 1u;
+            if (v.x != 0.f)
+                mark_node(g, t.ax + kx, t.ay + ky, t.az + kz, kx == 0 || ky == 0 || kz == 0, flags, list, counters);
         }
     }
     __syncthreads();
@@ -1318,12 +1321,13 @@ __device__ __forceinline__ void scatter_particle(unsigned long long *node, const
 // comes from the largest contribution any of the tile's particles can make,
 // so the waves read their particles once for that bound (the last batch stays
 // in registers for the scatter) and once more for the other batches.  A tile
-// with a particle that is not finite goes to the atomic fallback.
+// with a particle that is not finite goes to the atomic fallback; a wave with
+// particles for it goes through its batches again at the end.
 template <int MAT, int W>
 __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, const PartView &pv, const uint4 d,
                                              uint32_t staging_cap, float dt, float4 *__restrict__ staging,
-                                             uint32_t *spill, uint32_t *flags, uint32_t *counters, int32_t *blk_tile,
-                                             TileArena<W> &L)
+                                             float4 *grid, uint32_t *flags, uint32_t *list, uint32_t *counters,
+                                             int32_t *blk_tile, TileArena<W> &L)
 {
     uint32_t bits = 0;
     const TileGeo t = tile_geo(g, d.z);
@@ -1369,18 +1373,23 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
     // contributions below 2^e, at most d.y of them a node: sums below 2^50
     const int e = (int)(bb32 >> 23) - 126, nbits = FIX_BITS - (32 - __builtin_clz(d.y));
     const double pscale = pow2(nbits - e), mscale = pow2(e);     // mass: 2^nbits = pscale 2^e
+    // base inside the arena's bins (rel: relative to it), and a slot to write the tile to
+    auto in_arena = [&](const int rel[3]) {
+        return staged && finite && (uint32_t)rel[0] <= (uint32_t)(ARENA - 3) &&
+               (uint32_t)rel[1] <= (uint32_t)(ARENA - 3) && (uint32_t)rel[2] <= (uint32_t)(ARENA - 3);
+    };
+    uint64_t out = 0;           // lanes that met a particle for the atomic fallback
     uint32_t lane_faces = 0;    // arena faces this lane's particles' stencils reach (see tile_entry)
     if (first < d.y)
         for (;;) {
             const bool active = s0 + (uint32_t)lane < d.y;
-            const uint32_t i = d.x + s0 + (uint32_t)lane;
             int b[3];
             float f[3];
             const uint32_t ob = base_fx(g, x, b, f);
             if (active) bits |= ob;
-            const bool listed = list_spill(g, t, active, (int)i, b, staged && finite, spill, counters, flags);
-            const bool in = active && !listed;
             const int rel[3] = {b[0] - t.ax, b[1] - t.ay, b[2] - t.az};
+            const bool in = active && in_arena(rel);
+            out |= __ballot(active && !in);
             if (in) {
                 // a base on the arena's first (last) bin position reaches its
                 // face at index 0 (7)
@@ -1425,50 +1434,84 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
             const float4 v = make_float4((float)(munit * fix_value(L.sum[0][o])), (float)(punit * fix_value(L.sum[1][o])),
                                          (float)(punit * fix_value(L.sum[2][o])), (float)(punit * fix_value(L.sum[3][o])));
             gstore4(staging, dst + kz * 64 + lane, v);
-            const int nx_ = t.ax + kx, ny_ = t.ay + ky, nz_ = t.az + kz;
-            if (v.x != 0.f && nx_ >= 0 && ny_ >= 0 && nz_ >= 0 && nx_ < g.nx && ny_ < g.ny && nz_ < g.nz)
-                gp(flags)[((int64_t)(nz_ >> 2) * g.nby + (ny_ >> 2)) * g.nbx + (nx_ >> 2)] = 1u;
+            if (v.x != 0.f)
+                mark_node(g, t.ax + kx, t.ay + ky, t.az + kz, kx == 0 || ky == 0 || kz == 0, flags, list, counters);
         }
         if (threadIdx.x == 0) gp(blk_tile)[d.z] = tile_entry(d.w, faces);
     }
+    if (out)
+        for (s0 = first; s0 < d.y; s0 += 64u * W) {
+            const bool active = s0 + (uint32_t)lane < d.y;
+            const uint32_t i = d.x + min(s0 + (uint32_t)lane, d.y - 1u);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) x[a] = ld_plane(pv, PL_X + a, i);
+            int b[3];
+            (void)base_only(g, x, b);
+            const int rel[3] = {b[0] - t.ax, b[1] - t.ay, b[2] - t.az};
+            const uint64_t m = __ballot(active && !in_arena(rel));
+            if (m && lane == 0) (void)gatomic_add(counters + CT_SPILL, (uint32_t)__popcll(m));
+            if ((m >> lane) & 1ull) spill_particle<MAT>(g, mat, pv, (int)i, dt, counters, grid, flags, list);
+        }
     __syncthreads();        // the arena is cleared for the workgroup's next tile
     return bits;
 }
 
-// Bound by LDS and vector issue together: of a SIMD's cycles the vector units
-// take ~54% and the LDS atomics ~41%, half of these in bank conflicts of
-// uneven cells.  Four waves a SIMD: five or six measured the same or slower.
-// One pass over memory, no turns among lanes, no LDS sort: against one wave a
-// tile that sorted its particles in LDS and summed cells in registers, per
-// launch 26.8 -> 11.6 us (16k snow), 46 -> 26.0 (262k jello), 67 -> 56.6
-// (1M snow), 202 -> 145 (2M water).
-template <int MAT, int W>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) k_p2g_block(GridP g, MatP mat, PartView pv,
-                                                            const uint4 *__restrict__ desc,
-                                                            const uint32_t *__restrict__ tile_count, uint32_t desc_cap,
-                                                            uint32_t staging_cap, float dt,
-                                                            float4 *__restrict__ staging, uint32_t *spill,
-                                                            uint32_t *flags, uint32_t *counters, int32_t *blk_tile,
-                                                            int clear_active)
+__device__ __forceinline__ uint4 uniform_u4(const uint4 v)
+{
+    return make_uint4((uint32_t)__builtin_amdgcn_readfirstlane((int)v.x), (uint32_t)__builtin_amdgcn_readfirstlane((int)v.y),
+                      (uint32_t)__builtin_amdgcn_readfirstlane((int)v.z), (uint32_t)__builtin_amdgcn_readfirstlane((int)v.w));
+}
+
+// A tile of a group or scene of any material that MATS takes: the material is
+// one of the kernel's (MATS) or the tile's own (MAT_ANY).
+template <int MATS, int W>
+__device__ __forceinline__ uint32_t p2g_tile_of(const GridP &g, const MatP &mat, const PartView &pv, const uint4 d,
+                                                uint32_t staging_cap, float dt, float4 *staging, float4 *grid,
+                                                uint32_t *flags, uint32_t *list, uint32_t *counters, int32_t *blk_tile,
+                                                TileArena<W> &L)
+{
+    const int type = MATS == MAT_ANY ? mat.type : MATS;
+    if (type == MPM_JELLO) return p2g_tile<MPM_JELLO, W>(g, mat, pv, d, staging_cap, dt, staging, grid, flags, list, counters, blk_tile, L);
+    if (type == MPM_SNOW) return p2g_tile<MPM_SNOW, W>(g, mat, pv, d, staging_cap, dt, staging, grid, flags, list, counters, blk_tile, L);
+    return p2g_tile<MPM_WATER, W>(g, mat, pv, d, staging_cap, dt, staging, grid, flags, list, counters, blk_tile, L);
+}
+
+// The tiles of up to LAUNCH_GROUPS particle groups, one group's after the
+// other's (ONE: of a single group, whose arguments are then in scalar
+// registers from the start: 2M water 130 us, 135 otherwise).  Jello, snow and
+// water, 100k particles each: 16.8, 15.0 and 15.7 us apart, 28 together.
+// Bound by LDS and vector issue together: of a SIMD's cycles the
+// vector units take ~54% and the LDS atomics ~41%, half of these in bank
+// conflicts of uneven cells.  Four waves a SIMD: five or six measured the same
+// or slower.  One pass over memory, no turns among lanes, no LDS sort: against
+// one wave a tile that sorted its particles in LDS and summed cells in
+// registers, per launch 26.8 -> 11.6 us (16k snow), 46 -> 26.0 (262k jello),
+// 67 -> 56.6 (1M snow), 202 -> 145 (2M water).
+template <int MATS, int W, bool ONE>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) k_p2g_groups(const P2GArgs a)
 {
     __shared__ TileArena<W> L;
-    const uint32_t nt = min(*tile_count, desc_cap);
-    // the active-block and node counters are not used during P2G: clear
-    // them here for the block compaction that follows
-    if (clear_active && blockIdx.x == 0 && threadIdx.x == 0) {
-        gp(counters)[CT_ACTIVE] = 0u;
-        gp(counters)[CT_NODES] = 0u;
-    }
-    uint32_t bits = 0;
-    dt = step_dt(g, dt);
+    // the groups' counts by scalar loads (a scan over lanes and its barrier
+    // before the first tile cost 1M snow 4 of 55 us)
+    auto tiles = [&](int k) { return min(*a.grp[k].tile_count, a.grp[k].desc_cap); };
+    uint32_t nt = 0, last = 0;
+    for (int k = 0; k < (ONE ? 1 : a.ngroups); ++k) nt += last = tiles(k);
+    if (blockIdx.x == 0 && threadIdx.x == 0) gp(a.counters)[CT_TILES] = last;
     const uint32_t nt8 = round_xcd(nt);
+    uint32_t bits = 0;
+    const float dt = step_dt(a.g, a.dt);
     for (uint32_t k8 = blockIdx.x; k8 < nt8; k8 += gridDim.x) {
-        const uint32_t tt = xcd_spread(k8, nt8);
+        uint32_t tt = xcd_spread(k8, nt8);
         if (tt >= nt) continue;
-        bits |= p2g_tile<MAT, W>(g, mat, pv, desc[tt], staging_cap, dt, staging, spill, flags, counters, blk_tile, L);
+        int gi = 0;
+        if (!ONE)
+            for (uint32_t n; tt >= (n = tiles(gi)); ++gi) tt -= n;
+        const P2GGroup &q = a.grp[ONE ? 0 : gi];
+        const uint4 d = uniform_u4(gload_u4(q.desc, tt));    // the tile's loops hold barriers
+        bits |= p2g_tile_of<MATS, W>(a.g, q.mat, q.pv, d, a.staging_cap, dt, a.staging, a.grid, a.flags, a.list,
+                                     a.counters, q.blk_tile, L);
     }
-    if (bits) atomicOr(counters + CT_HEALTH, bits);
-    if (threadIdx.x == 0 && blockIdx.x == 0) counters[CT_TILES] = nt;
+    if (bits) atomicOr(a.counters + CT_HEALTH, bits);
 }
 
 // Batched P2G: the tiles of the scenes of material MAT among up to
@@ -1503,18 +1546,17 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
         if (tt >= nt) continue;
         const uint32_t sid = (uint32_t)__builtin_amdgcn_readfirstlane((int)__popcll(__ballot(s_end[lane] <= tt)));
         const BatchSlice &b = tab[sid];
-        uint4 d = gload_u4(b.desc, tt - (sid ? s_end[sid - 1] : 0u));
-        d.x = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.x);     // uniform: the tile's loops hold barriers
-        d.y = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.y);
-        d.z = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.z);
-        d.w = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.w);
-        const uint32_t bits = p2g_tile<MAT, W>(b.g, b.mat, b.pv, d, b.staging_cap, b.dt, b.staging, b.spill, b.flags,
+        const uint4 d = uniform_u4(gload_u4(b.desc, tt - (sid ? s_end[sid - 1] : 0u)));
+        const uint32_t bits = p2g_tile<MAT, W>(b.g, b.mat, b.pv, d, b.staging_cap, b.dt, b.staging, b.grid_mp, b.flags, b.list,
                                                b.counters, b.blk_tile, L);
         if (bits) gatomic_or(b.counters + CT_HEALTH, bits);
     }
     if (blockIdx.x == 0)
         for (int s = threadIdx.x; s < nslices; s += blockDim.x)
-            if (tab[s].mat.type == MAT) gp(tab[s].counters)[CT_TILES] = min(*gp(tab[s].tile_count), tab[s].desc_cap);
+            if (tab[s].mat.type == MAT) {
+                gp(tab[s].counters)[CT_TILES] = min(*gp(tab[s].tile_count), tab[s].desc_cap);
+                gp(tab[s].counters)[CT_SEQ] = (gp(tab[s].counters)[CT_SEQ] + 1u) & ~BATCH_SEQ;
+            }
 }
 
 // ---------------------------------------------------------------------------
@@ -1531,7 +1573,7 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
                                                               uint32_t desc_cap, uint32_t staging_cap, float dt,
                                                               float dt_next, const float4 *__restrict__ gv,
                                                               float4 *__restrict__ staging, uint32_t *spill,
-                                                              uint32_t *flags, uint32_t *counters, int sweeps,
+                                                              uint32_t *flags, uint32_t *list, uint32_t *counters, int sweeps,
                                                               int32_t *blk_tile)
 {
     __shared__ TileLds L;
@@ -1591,7 +1633,7 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
             }
             scatter_chunk<MAT>(L, nc, g.inv_h, mat.mass);
         }
-        tile_end(g, t, L, staging, d.w, staged, flags, blk_tile + d.z);
+        tile_end(g, t, L, staging, d.w, staged, flags, list, counters, blk_tile + d.z);
     }
     if (bits) atomicOr(counters + CT_HEALTH, bits);
     if (threadIdx.x == 0 && blockIdx.x == 0) counters[CT_TILES] = nt;
@@ -1628,7 +1670,7 @@ static int ensure_fast_buffers(mpm_sim *s)
         MPM_HIP(hipMalloc(&s->blk_start, s->nblocks * 4));
         MPM_HIP(hipMalloc(&s->scan_tmp, s->nblocks * 4));
     }
-    if (!s->spill) MPM_HIP(hipMalloc(&s->spill, s->cap * sizeof(uint32_t)));
+    if (!s->spill && s->cfg.form == MPM_FORM_FUSED) MPM_HIP(hipMalloc(&s->spill, s->cap * sizeof(uint32_t)));
     int64_t need = 0;
     s->group_tile_off.assign(s->groups.size(), 0);
     for (size_t k = 0; k < s->groups.size(); ++k) {
@@ -1716,13 +1758,15 @@ int sort_all(mpm_sim *s, bool defer)
                            s->blk_tile + (int64_t)k * nb, (uint32_t)s->group_tile_off[k]);
         const uint32_t bound = (uint32_t)tile_bound(s, n);
         hipLaunchKernelGGL(k_rank_tiles, dim3(std::min<uint32_t>((bound + 3) / 4, 2048u)), dim3(256), 0, st, skeys, r.vals, n,
-                           (const uint4 *)s->tile_desc + s->group_tile_off[k], s->tile_counts + k, bound, perm, s->tiles_host + k);
+                           (const uint4 *)s->tile_desc + s->group_tile_off[k], s->tile_counts + k, bound, perm, s->tiles_host + k, s->counters);
         if (!defer)
             hipLaunchKernelGGL(k_permute, dim3(round_xcd((uint32_t)nblk(n, 256))), dim3(256), 0, st, s->P, s->P_alt,
                                s->cap, pv.off, n, perm, s->pid, s->pid_alt, plane_mask);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "sort kernels");
     }
+    if ((rc = launch_list_near(st, s->g, s->blk_tile, (int)s->groups.size(), nb, s->flags, s->list, s->counters)))
+        return hip_fail((hipError_t)rc, "list_near");
     if (defer) {
         s->g2p_move_pending = true;
     } else {
@@ -1767,11 +1811,10 @@ static bool sort_due(mpm_sim *s, int ahead = 0)
     if (want < s->sorted_at_launch || !s->spill_host) return false;    // counts of the current order only
     const int slot = (int)(want % mpm_sim::SPILL_SLOTS);
     if (s->spill_launch[slot] != want) return false;
-    // wait until every group's spill kernel of that launch has published its
-    // count (launch number written after the count with release order)
+    // wait until the counts of that launch are written (launch number written after the count with release order)
     const uint32_t *seq = s->spill_host + mpm_sim::SPILL_SLOTS * MAX_GROUPS + slot * MAX_GROUPS;
     const auto t0 = std::chrono::steady_clock::now();
-    for (size_t k = 0; k < s->groups.size(); ++k) {
+    for (int k = 0; k < s->spill_words[slot]; ++k) {
         while (__atomic_load_n(&seq[k], __ATOMIC_ACQUIRE) != (uint32_t)want) {
             if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(2)) return false;
             std::this_thread::yield();
@@ -1779,15 +1822,15 @@ static bool sort_due(mpm_sim *s, int ahead = 0)
     }
     s->spill_launch[slot] = -1;
     uint64_t tot = 0;
-    for (size_t k = 0; k < s->groups.size(); ++k) tot += s->spill_host[slot * MAX_GROUPS + k];
+    for (int k = 0; k < s->spill_words[slot]; ++k) tot += s->spill_host[slot * MAX_GROUPS + k];
     if (tot <= std::max<uint64_t>(64, (uint64_t)s->total / 10000)) return false;
     s->sort_interval = s->sort_safe = std::max<int64_t>(1, s->steps_since_sort - 3);
     s->sort_clean = 0;
     return true;
 }
 
-// Pinned host word that receives the spill count of group `group`'s tile
-// launch (written by the spill kernel itself: no copy in the stream).
+// Pinned host word that receives the spill count of the tile launch (of its
+// group `group`), written by a kernel: no copy in the stream.
 static int spill_host_word(mpm_sim *s, int group, uint32_t **word)
 {
     if (!s->spill_host) {
@@ -1801,16 +1844,32 @@ static int spill_host_word(mpm_sim *s, int group, uint32_t **word)
     return MPM_OK;
 }
 
-// After group `group`'s tile launch: the launch counter advances after the
-// last group.
-static int note_spills(mpm_sim *s, int group)
+// After a tile launch (of its last group): `words` counts will be written.
+static void note_spills(mpm_sim *s, int words)
 {
     const int slot = (int)(s->tile_launches % mpm_sim::SPILL_SLOTS);
-    if (group + 1 == (int)s->groups.size()) {
-        s->spill_launch[slot] = s->tile_launches;
-        s->tile_launches += 1;
-    }
-    return MPM_OK;
+    s->spill_launch[slot] = s->tile_launches;
+    s->spill_words[slot] = words;
+    s->tile_launches += 1;
+}
+
+// The grid phase after a tile P2G writes the P2G's spill count (count null:
+// none is due); a P2G without its grid phase leaves its slot unread.
+int spill_publish(mpm_sim *s, uint32_t **count, uint32_t **seq, uint32_t *launch)
+{
+    *count = *seq = nullptr;
+    *launch = 0;
+    if (!s->spill_unread) return MPM_OK;
+    s->spill_unread = false;
+    s->tile_launches -= 1;
+    uint32_t *hw = nullptr;
+    const int rc = spill_host_word(s, 0, &hw);
+    *launch = (uint32_t)s->tile_launches;
+    if (rc) s->tile_launches += 1;
+    else note_spills(s, 1);
+    *count = hw;
+    *seq = hw ? hw + mpm_sim::SPILL_SLOTS * MAX_GROUPS : nullptr;
+    return rc;
 }
 
 int sort_if_due(mpm_sim *s)
@@ -1859,92 +1918,76 @@ int fast_ready(mpm_sim *s)
 // otherwise (262k jello, 512 a tile: 26.0 against 28.3; 1M snow, 300 a tile:
 // 56.6 against 59.4).  The sums do not depend on it.
 constexpr int P2G_WAVES = 4, P2G_WAVES_SPARSE = 2;
-static int p2g_waves(const mpm_sim *s, int group)
-{
-    // of the last sort that ran, 0 before the first
-    const int64_t tiles = __atomic_load_n(&s->tiles_host[group], __ATOMIC_RELAXED);
-    return s->groups[group].n < tiles * 64 * P2G_WAVES_SPARSE ? P2G_WAVES_SPARSE : P2G_WAVES;
-}
-
-template <int MAT>
-static void launch_block(int waves, dim3 gr, hipStream_t st, const GridP &g, const MatP &m, const PartView &pv,
-                         const uint4 *desc, const uint32_t *tc, uint32_t cap, uint32_t scap, float dt,
-                         float4 *staging, uint32_t *spill, uint32_t *flags, uint32_t *counters, int32_t *blk_tile)
-{
-    if (waves == P2G_WAVES_SPARSE)
-        hipLaunchKernelGGL((k_p2g_block<MAT, P2G_WAVES_SPARSE>), gr, dim3(64 * P2G_WAVES_SPARSE), 0, st, g, m, pv, desc,
-                           tc, cap, scap, dt, staging, spill, flags, counters, blk_tile, 1);
-    else
-        hipLaunchKernelGGL((k_p2g_block<MAT, P2G_WAVES>), gr, dim3(64 * P2G_WAVES), 0, st, g, m, pv, desc, tc, cap, scap,
-                           dt, staging, spill, flags, counters, blk_tile, 1);
-}
 
 bool tile_shape_valid(int tile) { return tile == 0 || tile == 256 || tile == 384 || tile == 512; }
 
-int launch_p2g_tiles(mpm_sim *s, int group, float dt)
+// The tile P2G of groups [first, first + n) (n <= LAUNCH_GROUPS) in one
+// launch.
+static int launch_p2g_groups(mpm_sim *s, int first, int n, float dt)
 {
-    PartView pv = view_of(s, group);
-    if (pv.n <= 0) return MPM_OK;
-    const MatP &m = s->groups[group].mat;
-    int64_t bound = tile_bound(s, pv.n);
-    int wg = (int)std::min<int64_t>(bound, 8192);
-    const uint4 *desc = (const uint4 *)s->tile_desc + s->group_tile_off[group];
-    const uint32_t *tc = s->tile_counts + group;
-    const uint32_t cap = (uint32_t)bound;
-    const uint32_t scap = (uint32_t)s->staging_cap;
-    int rc = MPM_OK;
-    if (group > 0) {        // the step's counter reset cleared group 0's count
-        rc = launch_zero_u32(s->stream, s->counters + CT_SPILL, 1);
-        if (rc) return hip_fail((hipError_t)rc, "zero");
+    P2GArgs a;
+    a.g = s->g;
+    a.dt = dt;
+    a.staging_cap = (uint32_t)s->staging_cap;
+    a.staging = s->staging;
+    a.grid = s->grid_mp;
+    a.flags = s->flags;
+    a.list = s->list;
+    a.counters = s->counters;
+    a.ngroups = 0;
+    int64_t bound = 0, particles = 0, tiles = 0;
+    int mats = -1;
+    for (int k = first; k < first + n; ++k) {
+        const PartView pv = view_of(s, k);
+        if (pv.n <= 0) continue;
+        P2GGroup &q = a.grp[a.ngroups++];
+        q.mat = s->groups[k].mat;
+        q.pv = pv;
+        q.desc = (const uint4 *)s->tile_desc + s->group_tile_off[k];
+        q.tile_count = s->tile_counts + k;
+        q.blk_tile = s->blk_tile + (int64_t)k * s->nblocks;
+        q.desc_cap = (uint32_t)tile_bound(s, pv.n);
+        bound += q.desc_cap;
+        particles += pv.n;
+        tiles += __atomic_load_n(&s->tiles_host[k], __ATOMIC_RELAXED);      // of the last sort that ran, 0 before the first
+        mats = mats < 0 || mats == q.mat.type ? q.mat.type : MAT_ANY;
     }
-    uint32_t *hw = nullptr;
-    if ((rc = spill_host_word(s, group, &hw))) return rc;
-    const auto launch = m.type == MPM_JELLO ? launch_block<MPM_JELLO>
-                        : (m.type == MPM_SNOW ? launch_block<MPM_SNOW> : launch_block<MPM_WATER>);
+    if (!a.ngroups) return MPM_OK;
+    const bool sparse = particles < tiles * 64 * P2G_WAVES_SPARSE;
+    const dim3 gr((uint32_t)std::min<int64_t>(bound, 8192)), bl(64 * (sparse ? P2G_WAVES_SPARSE : P2G_WAVES));
+#define MPM_P2G_LAUNCH(MATS_)                                                                       \
+    do {                                                                                            \
+        const bool one = MATS_ != MAT_ANY && a.ngroups == 1;                                        \
+        const auto k = sparse ? (one ? k_p2g_groups<MATS_, P2G_WAVES_SPARSE, MATS_ != MAT_ANY>       \
+                                     : k_p2g_groups<MATS_, P2G_WAVES_SPARSE, false>)                 \
+                              : (one ? k_p2g_groups<MATS_, P2G_WAVES, MATS_ != MAT_ANY>              \
+                                     : k_p2g_groups<MATS_, P2G_WAVES, false>);                       \
+        hipLaunchKernelGGL(k, gr, bl, 0, s->stream, a);                                             \
+    } while (0)
+    switch (mats) {
+    case MPM_JELLO: MPM_P2G_LAUNCH(MPM_JELLO); break;
+    case MPM_SNOW: MPM_P2G_LAUNCH(MPM_SNOW); break;
+    case MPM_WATER: MPM_P2G_LAUNCH(MPM_WATER); break;
+    default: MPM_P2G_LAUNCH(MAT_ANY); break;
+    }
+#undef MPM_P2G_LAUNCH
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? MPM_OK : hip_fail(e, "p2g_groups");
+}
+
+int launch_p2g_tiles(mpm_sim *s, float dt)
+{
     {
-    PhaseTimer tk(s, TK_P2G);
-    launch(p2g_waves(s, group), dim3(wg), s->stream, s->g, m, pv, desc, tc, cap, scap, dt, s->staging, s->spill, s->flags,
-           s->counters, s->blk_tile + (int64_t)group * s->nblocks);
+        PhaseTimer tk(s, TK_P2G);
+        const int n = (int)s->groups.size();
+        for (int k = 0; k < n; k += LAUNCH_GROUPS)
+            if (int rc = launch_p2g_groups(s, k, std::min(LAUNCH_GROUPS, n - k), dt)) return rc;
     }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return hip_fail(e, "p2g_block");
-    if (s->groups.size() == 1) {
-        // one group: the listed particles are scattered by the block
-        // compaction of the grid phase (the tiles flagged their blocks)
-        s->spill_pending = true;
-        s->spill_dt = dt;
-        s->spill_g = s->g;          // a later scatter takes the dt this launch took
-        s->spill_hw = hw;
-        s->spill_seq = (uint32_t)s->tile_launches;
-        return note_spills(s, group);
-    }
-    rc = launch_p2g_spill(s->stream, s->g, m, pv, dt, s->spill, (uint32_t)pv.n, s->counters, s->grid_mp, s->flags,
-                          hw, hw + mpm_sim::SPILL_SLOTS * MAX_GROUPS, (uint32_t)s->tile_launches);
-    if (rc) return hip_fail((hipError_t)rc, "p2g_spill");
-    return note_spills(s, group);
-}
-
-int spill_compact(mpm_sim *s)
-{
-    if (!s->spill_pending) return hip_fail(hipErrorInvalidValue, "spill_compact");
-    s->spill_pending = false;
-    const PartView pv = view_of(s, 0);
-    const int rc = launch_spill_compact(s->stream, s->spill_g, s->groups[0].mat, pv, s->spill_dt, s->spill,
-                                        (uint32_t)pv.n, s->counters, s->grid_mp, s->flags, (int)s->nblocks,
-                                        s->list, s->spill_hw, s->spill_hw + mpm_sim::SPILL_SLOTS * MAX_GROUPS,
-                                        s->spill_seq);
-    return rc ? hip_fail((hipError_t)rc, "spill_compact") : MPM_OK;
-}
-
-int flush_spill(mpm_sim *s)
-{
-    if (!s->spill_pending) return MPM_OK;
-    s->spill_pending = false;
-    const PartView pv = view_of(s, 0);
-    const int rc = launch_p2g_spill(s->stream, s->spill_g, s->groups[0].mat, pv, s->spill_dt, s->spill, (uint32_t)pv.n,
-                                    s->counters, s->grid_mp, s->flags, s->spill_hw,
-                                    s->spill_hw + mpm_sim::SPILL_SLOTS * MAX_GROUPS, s->spill_seq);
-    return rc ? hip_fail((hipError_t)rc, "p2g_spill") : MPM_OK;
+    if (s->total <= 0) return MPM_OK;
+    s->spill_launch[s->tile_launches % mpm_sim::SPILL_SLOTS] = -1;
+    s->tile_launches += 1;
+    s->spill_unread = true;
+    return MPM_OK;
 }
 
 int launch_g2p2g(mpm_sim *s, int group, float dt, float dt_next)
@@ -1968,17 +2011,18 @@ int launch_g2p2g(mpm_sim *s, int group, float dt, float dt_next)
     {
     PhaseTimer tk(s, TK_G2P);
     switch (m.type) {
-    case MPM_JELLO: hipLaunchKernelGGL(k_g2p2g_block<MPM_JELLO>, gr, bl, 0, s->stream, s->g, m, pv, desc, tc, cap, scap, dt, dt_next, s->grid_v, s->staging, s->spill, s->flags, s->counters, sw, bt); break;
-    case MPM_SNOW: hipLaunchKernelGGL(k_g2p2g_block<MPM_SNOW>, gr, bl, 0, s->stream, s->g, m, pv, desc, tc, cap, scap, dt, dt_next, s->grid_v, s->staging, s->spill, s->flags, s->counters, sw, bt); break;
-    default: hipLaunchKernelGGL(k_g2p2g_block<MPM_WATER>, gr, bl, 0, s->stream, s->g, m, pv, desc, tc, cap, scap, dt, dt_next, s->grid_v, s->staging, s->spill, s->flags, s->counters, sw, bt); break;
+    case MPM_JELLO: hipLaunchKernelGGL(k_g2p2g_block<MPM_JELLO>, gr, bl, 0, s->stream, s->g, m, pv, desc, tc, cap, scap, dt, dt_next, s->grid_v, s->staging, s->spill, s->flags, s->list, s->counters, sw, bt); break;
+    case MPM_SNOW: hipLaunchKernelGGL(k_g2p2g_block<MPM_SNOW>, gr, bl, 0, s->stream, s->g, m, pv, desc, tc, cap, scap, dt, dt_next, s->grid_v, s->staging, s->spill, s->flags, s->list, s->counters, sw, bt); break;
+    default: hipLaunchKernelGGL(k_g2p2g_block<MPM_WATER>, gr, bl, 0, s->stream, s->g, m, pv, desc, tc, cap, scap, dt, dt_next, s->grid_v, s->staging, s->spill, s->flags, s->list, s->counters, sw, bt); break;
     }
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "g2p2g_block");
     rc = launch_p2g_spill(s->stream, s->g, m, pv, dt_next, s->spill, (uint32_t)pv.n, s->counters, s->grid_mp,
-                          s->flags, hw, hw + mpm_sim::SPILL_SLOTS * MAX_GROUPS, (uint32_t)s->tile_launches);
+                          s->flags, s->list, hw, hw + mpm_sim::SPILL_SLOTS * MAX_GROUPS, (uint32_t)s->tile_launches);
     if (rc) return hip_fail((hipError_t)rc, "p2g_spill");
-    return note_spills(s, group);
+    if (group + 1 == (int)s->groups.size()) note_spills(s, (int)s->groups.size());
+    return MPM_OK;
 }
 
 // Stand-alone sort for the probe entry point (own temporaries).
@@ -2113,6 +2157,9 @@ int fill_sort_slice(mpm_sim *s, SortSlice &t)
     t.has = s->scan_tmp;
     t.perm = s->g2p_perm;
     t.tile_count = s->tile_counts;
+    t.flags = s->flags;
+    t.list = s->list;
+    t.counters = s->counters;
     t.warm_cnt = s->warm_cnt;
     t.desc = (uint4 *)s->tile_desc;
     t.blk_tile = s->blk_tile;
@@ -2154,6 +2201,7 @@ int launch_sort_batch(hipStream_t st, const SortSlice *tab, int ns, const SortBa
     hipLaunchKernelGGL(k_bsort_scan_apply, dim3(pl.scan), dim3(SCAN_T), 0, st, tab, ns);
     hipLaunchKernelGGL(k_bsort_emit, dim3(pl.emit), dim3(256), 0, st, tab, ns);
     hipLaunchKernelGGL(k_bsort_rank, dim3(1024), dim3(256), 0, st, tab, ns, pl.passes & 1);
+    if (int rc = launch_bsort_list(st, tab, ns, pl.emit)) return hip_fail((hipError_t)rc, "bsort_list");
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? MPM_OK : hip_fail(e, "sort_batch");
 }
@@ -2175,8 +2223,8 @@ void fill_batch_slice(mpm_sim *s, BatchSlice &b)
     b.staging = s->staging;
     b.flags = s->flags;
     b.list = s->list;
+    b.act = s->act;
     b.counters = s->counters;
-    b.spill = s->spill;
     b.desc = (const uint4 *)s->tile_desc + s->group_tile_off[0];
     b.tile_count = s->tile_counts;
     b.blk_tile = s->blk_tile;
@@ -2204,27 +2252,61 @@ int launch_p2g_batch(hipStream_t st, int mat, const BatchSlice *tab, const int *
     return 0;
 }
 
-// FAST-form G2P of one group; after a deferred re-sort it writes the group
-// in the new order into the other buffer (finish_g2p_move swaps them).
-int launch_g2p_fast(mpm_sim *s, int group, float dt)
+// FAST-form G2P of groups [first, first + n) (n <= LAUNCH_GROUPS); after a
+// deferred re-sort it writes the groups in the new order into the other
+// buffer (finish_g2p_move swaps them).
+static int launch_g2p_range(mpm_sim *s, int first, int n, float dt)
 {
-    const PartView pv = view_of(s, group);
-    G2PMove mv{s->g2p_perm + pv.off, pv, s->pid, s->pid_alt, s->warm_cnt ? 1 : 0};
-    mv.po.P = s->P_alt;
-    mv.po.pid = s->pid_alt;
-    int rc = launch_g2p(s->stream, s->g, s->groups[group].mat, pv, dt, s->grid_v, 1, s->cfg.svd_sweeps, s->counters,
-                        s->cfg.threads, s->g2p_move_pending ? &mv : nullptr);
-    return rc ? hip_fail((hipError_t)rc, "g2p_fast") : MPM_OK;
+    const bool move = s->g2p_move_pending;
+    if (n == 1) {
+        const PartView pv = view_of(s, first);
+        G2PMove mv{s->g2p_perm + pv.off, pv, s->pid, s->pid_alt, s->warm_cnt ? 1 : 0};
+        mv.po.P = s->P_alt;
+        mv.po.pid = s->pid_alt;
+        const int rc = launch_g2p(s->stream, s->g, s->groups[first].mat, pv, dt, s->grid_v, 1, s->cfg.svd_sweeps,
+                                  s->counters, s->cfg.threads, move ? &mv : nullptr);
+        return rc ? hip_fail((hipError_t)rc, "g2p_fast") : MPM_OK;
+    }
+    G2PArgs a;
+    a.g = s->g;
+    a.dt = dt;
+    a.gv = s->grid_v;
+    a.sweeps = s->cfg.svd_sweeps;
+    a.copy_q = s->warm_cnt ? 1 : 0;
+    a.counters = s->counters;
+    a.pid = s->pid;
+    a.pid_out = s->pid_alt;
+    a.ngroups = 0;
+    uint32_t wgs = 0;
+    for (int k = first; k < first + n; ++k) {
+        const PartView pv = view_of(s, k);
+        if (pv.n <= 0) continue;
+        G2PGroup &q = a.grp[a.ngroups++];
+        q.mat = s->groups[k].mat;
+        q.pv = pv;
+        q.P_out = s->P_alt;
+        q.perm = move ? s->g2p_perm + pv.off : nullptr;
+        wgs += (uint32_t)nblk(pv.n, s->cfg.threads);
+        q.end = wgs;
+    }
+    if (!a.ngroups) return MPM_OK;
+    const int rc = launch_g2p_groups(s->stream, a, wgs, s->cfg.threads, move);
+    return rc ? hip_fail((hipError_t)rc, "g2p_groups") : MPM_OK;
 }
 
-// A due FAST-form re-sort, deferred to the G2P about to run (particles that
-// a P2G of this step listed for the atomic fallback are scattered first:
-// the list names slots of the current order).
+int launch_g2p_fast(mpm_sim *s, float dt)
+{
+    const int n = (int)s->groups.size();
+    for (int k = 0; k < n; k += LAUNCH_GROUPS)
+        if (int rc = launch_g2p_range(s, k, std::min(LAUNCH_GROUPS, n - k), dt)) return rc;
+    return MPM_OK;
+}
+
+// A due FAST-form re-sort, deferred to the G2P about to run.
 int sort_for_g2p(mpm_sim *s)
 {
     if (!s->sorted_valid || s->g2p_move_pending || !sort_due(s, 1)) return MPM_OK;
-    int rc = flush_spill(s);
-    return rc ? rc : sort_all(s, true);
+    return sort_all(s, true);
 }
 
 // After every group's G2P of a deferred re-sort: the written buffer becomes

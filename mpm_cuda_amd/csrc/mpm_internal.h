@@ -90,24 +90,35 @@ struct PartView {
 
 // Device counters (one uint32 array).
 enum Counter : int {
-    CT_ACTIVE = 0,      // active grid blocks of the current step
-    CT_NODES = 1,       // grid nodes with mass in the grid update
-    CT_SPILL = 2,       // particles listed for the atomic P2G fallback
+    CT_LIST = 0,        // entries of the list of blocks that the grid update looks at
+    CT_NODES = 1,       // grid nodes with mass in it (counted when timing is on)
+    CT_SPILL = 2,       // particles that took the atomic P2G fallback
     CT_HEALTH = 3,      // MPM_H_* bits
     CT_FALLBACK = 4,    // FP64 SVD fallbacks
     CT_REJECT = 5,      // warm-start rejections
     CT_TILES = 6,       // P2G tiles (FAST / FUSED forms)
-    CT_SPILLED = 7,     // spill count of the last block compaction (CT_SPILL is cleared there)
+    CT_SPILLED = 7,     // spill count of the last grid update (CT_SPILL is cleared there)
     CT_SPEED = 8,       // step-size controller: max_p |v_p| + c_p (float bits), since the last control
     CT_DEFORM = 9,      // step-size controller: max_p max(J, 1/J) (float bits)
     CT_SVD = 10,        // G2P particle updates that took the Jacobi SVD (cumulative)
     CT_WARM = 11,       // of those, started from a network quaternion (cumulative)
+    CT_SEQ = 12,        // batched steps of the scene
+    CT_ACTIVE = 13,     // active grid blocks of the last grid update (counted when read)
     CT_COUNT = 16       // words of a cache line
 };
 // CT_FALLBACK, CT_REJECT, CT_SVD, CT_WARM (summed when read) and CT_SPEED,
 // CT_DEFORM (their maximum) live in CT_SPREAD copies of the line, one a
 // workgroup (see spread).
 constexpr int CT_SPREAD = 256, CT_WORDS = CT_COUNT * (1 + CT_SPREAD);
+
+// A grid block's entry in `flags`: marked by the P2G, cleared by the grid
+// update; on the list of blocks that the grid update looks at.  In the FAST
+// and FUSED forms the list is that of the last sort -- every tile's block and
+// the next one in each axis, which hold the nodes that particles of the block
+// reach -- and the blocks that particles which left theirs have added since
+// (a fifth of the blocks of a 1M-particle body would be idle if the sort
+// listed those too); in the PLAIN form that of the step.
+constexpr uint32_t BF_MARKED = 1u, BF_LISTED = 2u;
 
 // Entry of the block -> staging slot map (blk_tile): -1 when the block has
 // no tile; otherwise the slot in bits 0..23 (slots at or above the staging
@@ -252,11 +263,57 @@ __host__ __device__ inline int64_t node_slot(const GridP &g, int x, int y, int z
     return b * BLK_NODES + (((z & 3) * BLK + (y & 3)) * BLK + (x & 3));
 }
 
+// Step numbers in a simulator's act entries: those of batched steps are the
+// device's own count (CT_SEQ) with the highest bit set.
+constexpr uint32_t BATCH_SEQ = 0x80000000u;
+
 struct GroupInfo {
     mpm_material src;
     MatP mat;
     int64_t off = 0, n = 0;
     double mass = 0, vol = 0;
+};
+
+// The particle groups of one tile P2G or one G2P launch (kernel arguments:
+// read from there when a workgroup knows its group, so that they take no
+// scalar registers before).
+constexpr int LAUNCH_GROUPS = 8;
+constexpr int MAT_ANY = 3;          // kernel for groups of several materials (a single one's: MPM_JELLO, ...)
+struct P2GGroup {
+    MatP mat;
+    PartView pv;
+    const uint4 *desc;              // tiles of the last sort
+    const uint32_t *tile_count;
+    int32_t *blk_tile;
+    uint32_t desc_cap;
+};
+struct P2GArgs {
+    GridP g;
+    float dt;
+    uint32_t staging_cap;
+    float4 *staging, *grid;
+    uint32_t *flags, *list, *counters;
+    int ngroups;
+    P2GGroup grp[LAUNCH_GROUPS];
+};
+
+struct G2PGroup {
+    MatP mat;
+    PartView pv;
+    float *P_out;                   // with perm: the other particle buffer,
+    const uint32_t *perm;           // slot j of it takes particle perm[j] (null: the same slots)
+    uint32_t end;                   // one past the group's last workgroup
+};
+struct G2PArgs {
+    GridP g;
+    float dt;
+    const float4 *gv;
+    int sweeps, copy_q;
+    uint32_t *counters;
+    const uint32_t *pid;
+    uint32_t *pid_out;
+    int ngroups;
+    G2PGroup grp[LAUNCH_GROUPS];
 };
 
 // One scene of a batch (a simulator with one particle group) as the batched
@@ -275,7 +332,7 @@ struct BatchSlice {
     uint32_t *warm_cnt;             // warm start: [0] listed particles the coming inference takes,
                                     // [1] entries the G2P appends (mat.wlist); null when cold
     float4 *grid_mp, *grid_v, *staging;
-    uint32_t *flags, *list, *counters, *spill;
+    uint32_t *flags, *list, *act, *counters;
     const uint4 *desc;              // P2G tiles of the last sort
     const uint32_t *tile_count;
     int32_t *blk_tile;              // tile_entry per block (the P2G updates its faces)
@@ -297,6 +354,7 @@ struct SortSlice {
     uint32_t *blk_start, *blk_end, *has;
     uint32_t *perm;                 // slot j of the new order takes particle perm[j]
     uint32_t *tile_count;
+    uint32_t *flags, *list, *counters;
     uint32_t *warm_cnt;             // warm-start list counts (cleared: the lists name old slots), or null
     uint4 *desc;
     int32_t *blk_tile;
@@ -377,6 +435,9 @@ struct mpm_sim {
     int64_t nblocks = 0;
     float4 *grid_mp = nullptr, *grid_v = nullptr;
     uint32_t *flags = nullptr, *list = nullptr, *counters = nullptr;
+    uint32_t *act = nullptr;                // per block: number of the last grid update it was active in
+    uint32_t act_seq = 0;                   // number of the last grid update (BATCH_SEQ: a batch's), 0 before the first
+    uint32_t grid_seq = 0;                  // grid updates outside batches
     // particles
     float *P = nullptr, *P_alt = nullptr;
     uint32_t *pid = nullptr, *pid_alt = nullptr;
@@ -396,7 +457,7 @@ struct mpm_sim {
     float4 *staging = nullptr;              // per tile: 8^3-node P2G arena written back without atomics
     int64_t staging_cap = 0;                // tiles the staging buffer holds
     int32_t *blk_tile = nullptr;            // [group][block]: tile_entry of the block (-1: no tile)
-    uint32_t *spill = nullptr;              // indices of particles for the atomic P2G fallback
+    uint32_t *spill = nullptr;              // FUSED: indices of particles for the atomic P2G fallback
     bool primed = false;                    // FUSED: staging holds the scatter of the current state
     float primed_dt = 0.f;                  // FUSED: dt the primed scatter used for the force term
     bool sorted_valid = false;
@@ -409,7 +470,7 @@ struct mpm_sim {
     int64_t g2p_perm_cap = 0;
     bool g2p_move_pending = false;
     // spill counts of the tile P2G launches, written to pinned host memory
-    // by the spill kernel with the launch number after them; a re-sort is
+    // by the grid update (FUSED: the spill kernel) with the launch number after them; a re-sort is
     // brought forward when they grow.  Two slots: the count of the launch two
     // steps back is read (usually written by then; waiting for its number
     // keeps at most two steps queued ahead of the device, and no event
@@ -417,14 +478,10 @@ struct mpm_sim {
     static constexpr int SPILL_SLOTS = 2;
     uint32_t *spill_host = nullptr;         // [slot][MAX_GROUPS] counts, then [slot][MAX_GROUPS] launch numbers
     int64_t spill_launch[SPILL_SLOTS] = {-1, -1};   // tile launch number held by the slot
+    int spill_words[SPILL_SLOTS] = {};      // its counts: one, or one per group (FUSED)
     int64_t tile_launches = 0;
     bool counters_clean = false;            // CT_SPILL cleared by the last grid phase (FAST form)
-    // one-group tile P2G: its spill scatter waits for the grid phase
-    bool spill_pending = false;
-    float spill_dt = 0.f;
-    mpm::GridP spill_g{};                      // the grid arguments of that tile launch (its dt source)
-    uint32_t *spill_hw = nullptr;
-    uint32_t spill_seq = 0;
+    bool spill_unread = false;              // a tile P2G whose count the grid phase has not written yet
     int64_t sorted_at_launch = 0;           // tile_launches when the last sort ran
     int64_t sort_interval = 0;              // steps between re-sorts (learned from the spill counts)
     int64_t sort_safe = 0;                  // longest interval since the last spill-forced re-sort (0: sort_every)

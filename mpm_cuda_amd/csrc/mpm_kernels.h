@@ -35,7 +35,7 @@ struct Stencil {
 };
 
 // Flag the (up to 2x2x2) 4^3-node blocks the 3x3x3 stencil of base node b
-// touches.
+// touches (PLAIN form).
 __device__ __forceinline__ void mark_blocks(const GridP &g, const int b[3], uint32_t *flags)
 {
     int bx0 = b[0] >> 2, bx1 = (b[0] + 2) >> 2;
@@ -44,7 +44,41 @@ __device__ __forceinline__ void mark_blocks(const GridP &g, const int b[3], uint
     for (int bz = bz0; bz <= bz1; ++bz)
         for (int by = by0; by <= by1; ++by)
             for (int bx = bx0; bx <= bx1; ++bx)
-                gp(flags)[((int64_t)bz * g.nby + by) * g.nbx + bx] = 1u;
+                gp(flags)[((int64_t)bz * g.nby + by) * g.nbx + bx] = BF_MARKED;
+}
+
+// A block that the sort may not have listed (FAST and FUSED forms): marked,
+// and added to the list once.
+__device__ __forceinline__ void mark_and_list(uint32_t blk, uint32_t *flags, uint32_t *list, uint32_t *counters)
+{
+    if (gp(flags)[blk] & BF_LISTED) {
+        gp(flags)[blk] = BF_MARKED | BF_LISTED;
+        return;
+    }
+    const uint32_t old = __hip_atomic_fetch_or(gp(flags + blk), BF_MARKED | BF_LISTED, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+    if (!(old & BF_LISTED)) gp(list)[gatomic_add(counters + CT_LIST, 1u)] = blk;
+}
+
+// Node (x, y, z) with mass of a tile's arena (on its low faces: outside the
+// blocks that the sort listed for the tile).
+__device__ __forceinline__ void mark_node(const GridP &g, int x, int y, int z, bool low_face, uint32_t *flags,
+                                          uint32_t *list, uint32_t *counters)
+{
+    if (x < 0 || y < 0 || z < 0 || x >= g.nx || y >= g.ny || z >= g.nz) return;
+    const uint32_t blk = (uint32_t)(((int64_t)(z >> 2) * g.nby + (y >> 2)) * g.nbx + (x >> 2));
+    if (low_face) mark_and_list(blk, flags, list, counters);
+    else gp(flags)[blk] = BF_MARKED | BF_LISTED;
+}
+
+// The blocks of a spilled particle's stencil.
+__device__ __forceinline__ void mark_spilled(const GridP &g, const int b[3], uint32_t *flags, uint32_t *list,
+                                             uint32_t *counters)
+{
+    for (int bz = b[2] >> 2; bz <= (b[2] + 2) >> 2; ++bz)
+        for (int by = b[1] >> 2; by <= (b[1] + 2) >> 2; ++by)
+            for (int bx = b[0] >> 2; bx <= (b[0] + 2) >> 2; ++bx)
+                mark_and_list((uint32_t)(((int64_t)bz * g.nby + by) * g.nbx + bx), flags, list, counters);
 }
 
 // The three axes' weights and derivatives: the closed form of
@@ -262,15 +296,15 @@ __device__ __forceinline__ float ld_plane(const PartView &pv, int plane, uint32_
     return *plane_at(pv, plane, i);
 }
 
-// Contribution of one particle to stencil node (ox, oy, oz): out = (m, p).
-__device__ __forceinline__ float4 node_contrib(const GridP &g, const Stencil &s, const Scatter &sc,
-                                               int ox, int oy, int oz)
+// Contribution of one particle to the stencil node at offsets o, given that
+// node's weights and derivatives: out = (m, p).
+__device__ __forceinline__ float4 node_contrib_w(const GridP &g, const float fx[3], const float wt[3], const float dw[3],
+                                                 const Scatter &sc, const int o[3])
 {
-    float wx = s.w[0][ox], wy = s.w[1][oy], wz = s.w[2][oz];
+    float wx = wt[0], wy = wt[1], wz = wt[2];
     float w = wx * wy * wz;
-    float gr[3] = {g.inv_h * s.dw[0][ox] * wy * wz, g.inv_h * wx * s.dw[1][oy] * wz,
-                   g.inv_h * wx * wy * s.dw[2][oz]};
-    float d[3] = {((float)ox - s.fx[0]) * g.h, ((float)oy - s.fx[1]) * g.h, ((float)oz - s.fx[2]) * g.h};
+    float gr[3] = {g.inv_h * dw[0] * wy * wz, g.inv_h * wx * dw[1] * wz, g.inv_h * wx * wy * dw[2]};
+    float d[3] = {((float)o[0] - fx[0]) * g.h, ((float)o[1] - fx[1]) * g.h, ((float)o[2] - fx[2]) * g.h};
     float4 r;
     r.x = w * sc.m;
     float p[3];
@@ -282,6 +316,46 @@ __device__ __forceinline__ float4 node_contrib(const GridP &g, const Stencil &s,
     }
     r.y = p[0]; r.z = p[1]; r.w = p[2];
     return r;
+}
+__device__ __forceinline__ float4 node_contrib(const GridP &g, const Stencil &s, const Scatter &sc,
+                                               int ox, int oy, int oz)
+{
+    const float w[3] = {s.w[0][ox], s.w[1][oy], s.w[2][oz]}, dw[3] = {s.dw[0][ox], s.dw[1][oy], s.dw[2][oz]};
+    const int o[3] = {ox, oy, oz};
+    return node_contrib_w(g, s.fx, w, dw, sc, o);
+}
+
+// A particle whose stencil left its block arena: scatter with global atomics
+// into grid_mp, which the grid update adds in.
+template <int MAT>
+__device__ __forceinline__ void spill_particle(const GridP &g, const MatP &mat, const PartView &pv, int i, float dt,
+                                               uint32_t *counters, float4 *grid, uint32_t *flags, uint32_t *list)
+{
+    float x[3] = {ld(pv, PL_X, i), ld(pv, PL_X + 1, i), ld(pv, PL_X + 2, i)};
+    Stencil s;
+    make_stencil(g, x, s);
+    Scatter sc;
+    load_scatter<MAT>(pv, i, mat, dt, true, 0, sc, counters);
+    // a loop (rare path, inlined in kernels short of registers); the weights
+    // are picked by compares, not by an index into memory
+    auto pick = [](const float w[3], int o) { return o == 0 ? w[0] : (o == 1 ? w[1] : w[2]); };
+#pragma unroll 1
+    for (int k = 0; k < 27; ++k) {
+        const int o[3] = {k / 9, k / 3 % 3, k % 3};
+        float w[3], dw[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            w[a] = pick(s.w[a], o[a]);
+            dw[a] = pick(s.dw[a], o[a]);
+        }
+        const float4 c = node_contrib_w(g, s.fx, w, dw, sc, o);
+        float *dst = (float *)(grid + node_slot(g, s.b[0] + o[0], s.b[1] + o[1], s.b[2] + o[2]));
+        gatomic_add(dst + 0, c.x);
+        gatomic_add(dst + 1, c.y);
+        gatomic_add(dst + 2, c.z);
+        gatomic_add(dst + 3, c.w);
+    }
+    mark_spilled(g, s.b, flags, list, counters);
 }
 
 }  // namespace mpm

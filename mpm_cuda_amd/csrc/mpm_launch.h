@@ -9,11 +9,16 @@ int launch_zero_u32(hipStream_t st, uint32_t *p, int n);
 int launch_p2g_atomic(hipStream_t st, const GridP &g, const MatP &m, const PartView &pv, float dt,
                       int sweeps, int tau_stored, float4 *grid, uint32_t *flags, uint32_t *counters,
                       int threads);
-int launch_compact(hipStream_t st, uint32_t *flags, int nblocks, uint32_t *list, uint32_t *counters);
-int launch_count_nodes(hipStream_t st, const uint32_t *list, uint32_t *counters, const float4 *gv);
-int launch_grid_update(hipStream_t st, const GridP &g, float dt, const uint32_t *list,
-                       uint32_t *counters, float4 *gmp, float4 *gv, int nblocks, const float4 *staging,
-                       const int32_t *blk_tile, int ngroups, uint32_t staging_cap, int clear_spill = 0);
+int launch_count_active(hipStream_t st, const uint32_t *act, uint32_t seq, int64_t nblocks, uint32_t *counters,
+                        const float4 *gv);
+int launch_list_marked(hipStream_t st, const uint32_t *flags, int nblocks, uint32_t *list, uint32_t *counters);
+int launch_list_near(hipStream_t st, const GridP &g, const int32_t *blk_tile, int ngroups, int nblocks, uint32_t *flags,
+                     uint32_t *list, uint32_t *counters);
+int launch_bsort_list(hipStream_t st, const SortSlice *tab, int ns, int wgs);
+int launch_grid_update(hipStream_t st, const GridP &g, float dt, const uint32_t *list, uint32_t *flags, uint32_t *act,
+                       uint32_t seq, uint32_t *counters, float4 *gmp, float4 *gv, int64_t nblocks,
+                       const float4 *staging, const int32_t *blk_tile, int ngroups, uint32_t staging_cap,
+                       uint32_t *host_count, uint32_t *host_seq, uint32_t launch);
 // A G2P that applies a re-sort: slot j of po receives particle perm[j] of
 // the view, its id (pid -> pid_out) and, with copy_q, its quaternion.
 struct G2PMove {
@@ -28,23 +33,18 @@ int launch_g2p(hipStream_t st, const GridP &g, const MatP &m, const PartView &pv
                const G2PMove *mv = nullptr);
 int launch_compute_tau(hipStream_t st, const MatP &m, const PartView &pv, int sweeps, uint32_t *counters);
 int launch_p2g_spill(hipStream_t st, const GridP &g, const MatP &m, const PartView &pv, float dt,
-                     const uint32_t *list, uint32_t list_cap, uint32_t *counters, float4 *grid, uint32_t *flags,
-                     uint32_t *host_count, uint32_t *host_seq = nullptr, uint32_t seq = 0,
-                     int clear_active = 0);
-int launch_spill_compact(hipStream_t st, const GridP &g, const MatP &m, const PartView &pv, float dt,
-                         const uint32_t *spill, uint32_t spill_cap, uint32_t *counters, float4 *grid,
-                         uint32_t *flags, int nblocks, uint32_t *list, uint32_t *host_count, uint32_t *host_seq,
-                         uint32_t seq);
+                     const uint32_t *list, uint32_t list_cap, uint32_t *counters, float4 *grid, uint32_t *flags, uint32_t *blocks,
+                     uint32_t *host_count, uint32_t *host_seq, uint32_t seq);
 int launch_dt_scan(hipStream_t st, const MatP &m, const PartView &pv, uint32_t *counters);
 int launch_dt_clear(hipStream_t st, uint32_t *counters);
 int launch_dt_control(hipStream_t st, DtCtl *c, uint32_t *counters, float max_dt, float cfl_h, int mode);
 
 // FAST form (mpm_fast.hip)
 int fast_prepare(mpm_sim *s);                 // (re)sort particles and build P2G tiles when due
-int launch_p2g_tiles(mpm_sim *s, int group, float dt);
-int spill_compact(mpm_sim *s);                // grid phase after a one-group tile P2G: spill scatter + compaction
-int flush_spill(mpm_sim *s);                  // spill scatter of a tile P2G whose grid phase did not run
-int launch_g2p_fast(mpm_sim *s, int group, float dt);
+int launch_p2g_tiles(mpm_sim *s, float dt);
+int spill_publish(mpm_sim *s, uint32_t **count, uint32_t **seq, uint32_t *launch);   // where the grid phase writes its count
+int launch_g2p_fast(mpm_sim *s, float dt);
+int launch_g2p_groups(hipStream_t st, const G2PArgs &a, uint32_t wgs, int threads, bool move);
 int launch_g2p2g(mpm_sim *s, int group, float dt, float dt_next);   // FUSED form
 int sort_all(mpm_sim *s, bool defer = false);  // sort every group now and rebuild the tiles
 int sort_for_g2p(mpm_sim *s);                 // a due re-sort, applied by the coming FAST G2P
@@ -63,7 +63,6 @@ struct SortBatchPlan {
 void sort_batch_plan(mpm_sim *const *sims, int ns, SortBatchPlan &pl);
 int fill_sort_slice(mpm_sim *s, SortSlice &t);
 int launch_sort_batch(hipStream_t st, const SortSlice *tab, int ns, const SortBatchPlan &pl);
-int launch_batch_zero(hipStream_t st, const BatchSlice *tab, int nslices);
 // Warm-start particle lists of a simulator (mpm_api.hip).
 int ensure_warm_lists(mpm_sim *s);
 int launch_p2g_batch(hipStream_t st, int mat, const BatchSlice *tab, const int *types, int nslices, int wgs);
@@ -73,8 +72,6 @@ int launch_p2g_batch(hipStream_t st, int mat, const BatchSlice *tab, const int *
 int read_rows(ReadStage &rs, hipStream_t st, const float *planes, int64_t stride, int64_t n, int w,
               const uint32_t *ids, float *scratch, float *out);
 bool tile_shape_valid(int tile);              // values of mpm_config.tile and mpm_batch_shape.p2g_tile
-int launch_spill_batch(hipStream_t st, const BatchSlice *tab, int nslices, int wgs);
-int launch_compact_batch(hipStream_t st, const BatchSlice *tab, int nslices, int wgs);
 int launch_permute_batch(hipStream_t st, const BatchSlice *src, const BatchSlice *dst, int nslices, int wgs);
 int launch_grid_batch(hipStream_t st, const BatchSlice *tab, int nslices, int wgs);
 int launch_g2p_batch(hipStream_t st, int mat, const BatchSlice *tab, int nslices, int wgs, int threads);

@@ -7,6 +7,8 @@
 #include "mpm_g2p.h"
 #include "mpm_launch.h"
 
+#include <algorithm>
+
 namespace mpm {
 
 // ---------------------------------------------------------------------------
@@ -51,76 +53,56 @@ __global__ void __launch_bounds__(256) k_p2g_atomic(GridP g, MatP mat, PartView 
 }
 
 // ---------------------------------------------------------------------------
-// Active-block list: compacts the block flags written by P2G (and clears them).
-// One global atomic per workgroup (256 flags): wave counts are combined in LDS.
-// Thread t of the workgroup handles flag b0 + t.  The workgroup of flag 0
-// also moves the step's spill count (consumed by the spill kernel, which ran
-// before) to CT_SPILLED and clears CT_SPILL for the next P2G, when
-// clear_spill is set (else the grid update does it).
-__device__ __forceinline__ void compact_flags(uint32_t *flags, int nblocks, uint32_t *list, uint32_t *counters,
-                                              int b0, bool clear_spill)
-{
-    __shared__ uint32_t wave_cnt[4], wg_base;
-    if (clear_spill && b0 == 0 && threadIdx.x == 0) {
-        gp(counters)[CT_SPILLED] = gp(counters)[CT_SPILL];
-        gp(counters)[CT_SPILL] = 0u;
-    }
-    int b = b0 + (int)threadIdx.x;
-    bool f = b < nblocks && gp(flags)[b] != 0u;
-    if (f) gp(flags)[b] = 0u;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint64_t mask = __ballot(f);
-    if (lane == 0) wave_cnt[w] = (uint32_t)__popcll(mask);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t tot = wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
-        wg_base = tot ? gatomic_add(counters + CT_ACTIVE, tot) : 0u;
-    }
-    __syncthreads();
-    uint32_t off = wg_base;
-    for (int k = 0; k < w; ++k) off += wave_cnt[k];
-    uint64_t below = lane ? (mask & ((~0ull) >> (64 - lane))) : 0ull;
-    if (f) gp(list)[off + __popcll(below)] = (uint32_t)b;
-}
-
-__global__ void __launch_bounds__(256) k_compact_blocks(uint32_t *flags, int nblocks, uint32_t *list,
-                                                        uint32_t *counters)
-{
-    compact_flags(flags, nblocks, list, counters, (int)(blockIdx.x * blockDim.x), true);
-}
-
-// ---------------------------------------------------------------------------
 // Grid velocity update over active blocks (MPMCUDA.cu:435-472): v = p / m,
-// gravity, walls.  One wave per active block, persistent over the active
-// list.  Node (mass, momentum) is the sum of grid_mp (PLAIN-form scatter and
+// gravity, walls.  One wave per active block.  Node (mass, momentum) is the sum of grid_mp (PLAIN-form scatter and
 // FAST-form spills) and, in the FAST form, of the staged P2G arenas of the
 // up to 2x2x2 particle blocks whose arenas cover the node.  grid_mp is
 // cleared for the next step; the result goes to grid_v.
-__device__ __forceinline__ void grid_block(const GridP &g, float dt, uint32_t b, float4 *gmp, float4 *gv,
+// A block of the list is updated when marked, its mark cleared and the step
+// number `seq` put in its act entry.
+// The staging slots are looked up GB groups at a time (1, or 4 where there are
+// more groups).
+template <int GB>
+__device__ __forceinline__ void grid_block(const GridP &g, float dt, uint32_t b, uint32_t *flags, uint32_t *act,
+                                           uint32_t seq, float4 *gmp, float4 *gv,
                                            const float4 *__restrict__ staging, const int32_t *__restrict__ blk_tile,
                                            int ngroups, uint32_t staging_cap, int64_t nblocks)
 {
     const int lane = threadIdx.x & 63;
     const int kx = lane & 3, ky = (lane >> 2) & 3, kz = lane >> 4;
-    const int bx = (int)(b % (uint32_t)g.nbx);
-    const int by = (int)((b / (uint32_t)g.nbx) % (uint32_t)g.nby);
-    const int bz = (int)(b / ((uint32_t)g.nbx * (uint32_t)g.nby));
+    const uint32_t row = div_by(b, (uint32_t)g.nbx, g.div_nbx);
+    const int bz = (int)div_by(row, (uint32_t)g.nby, g.div_nby);
+    const int bx = (int)(b - row * (uint32_t)g.nbx), by = (int)row - bz * g.nby;
     const int64_t idx = (int64_t)b * BLK_NODES + lane;
+    // Lanes 0..26 look up the staging slots of the 27 neighbour blocks at
+    // once; with the mark and the block's own sums these loads are all in
+    // flight together.
+    const int px = bx + lane % 3 - 1, py = by + (lane / 3) % 3 - 1, pz = bz + lane / 9 - 1;
+    const bool near = blk_tile && lane < 27 && px >= 0 && py >= 0 && pz >= 0 && px < g.nbx && py < g.nby && pz < g.nbz;
+    const int32_t *bt = blk_tile + (((int64_t)pz * g.nby + py) * g.nbx + px);
+    int32_t look[GB];
+    auto lookup = [&](int g0) {
+#pragma unroll
+        for (int k = 0; k < GB; ++k) look[k] = near && g0 + k < ngroups ? gp(bt)[(int64_t)(g0 + k) * nblocks] : -1;
+    };
+    lookup(0);
     float4 a = gload4(gmp, idx);
+    const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)gp(flags)[b]);
+    if (!(f & BF_MARKED)) return;
+    if (lane == 0) {
+        gp(flags)[b] = f & ~BF_MARKED;
+        gp(act)[b] = seq;
+    }
     if (a.x != 0.f || a.y != 0.f || a.z != 0.f || a.w != 0.f) gstore4(gmp, idx, make_float4(0.f, 0.f, 0.f, 0.f));
     if (blk_tile) {
-        for (int gi = 0; gi < ngroups; ++gi) {
-            // lanes 0..26 look up the staging slots of the 27 neighbour
-            // blocks at once; the gathers below are then independent
-            const int32_t *bt = blk_tile + (int64_t)gi * nblocks;
-            int32_t my_t = -1;
-            if (lane < 27) {
-                const int px = bx + lane % 3 - 1, py = by + (lane / 3) % 3 - 1, pz = bz + lane / 9 - 1;
-                if (px >= 0 && py >= 0 && pz >= 0 && px < g.nbx && py < g.nby && pz < g.nbz) {
-                    const int32_t t = gp(bt)[((int64_t)pz * g.nby + py) * g.nbx + px];
-                    if (t >= 0 && ((uint32_t)t & TILE_SLOT_MASK) < staging_cap) my_t = t;
-                }
-            }
+        for (int g0 = 0; g0 < ngroups; g0 += GB) {
+            if (g0) lookup(g0);
+#pragma unroll 1
+            for (int gk = 0; gk < GB && g0 + gk < ngroups; ++gk) {
+            int32_t at = look[0];
+#pragma unroll
+            for (int k = 1; k < GB; ++k) at = gk == k ? look[k] : at;
+            const int32_t my_t = at >= 0 && ((uint32_t)at & TILE_SLOT_MASK) < staging_cap ? at : -1;
             // A node lies in exactly 8 of the 27 arenas: per axis its own
             // block's (d = 0) and the one below (d = -1, local k <= 2) or
             // above (d = +1, k = 3).  A neighbour's arena is read at index 7
@@ -144,6 +126,7 @@ __device__ __forceinline__ void grid_block(const GridP &g, float dt, uint32_t b,
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) { a.x += v[e].x; a.y += v[e].y; a.z += v[e].z; a.w += v[e].w; }
+            }
         }
     }
     float4 out = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -167,51 +150,147 @@ __device__ __forceinline__ void grid_block(const GridP &g, float dt, uint32_t b,
     gstore4(gv, idx, out);
 }
 
-__global__ void __launch_bounds__(64) k_grid_update(GridP g, float dt, const uint32_t *list, uint32_t *counters,
-                                                    float4 *gmp, float4 *gv, const float4 *__restrict__ staging,
+// Persistent over the list.  Also moves the step's spill count to CT_SPILLED,
+// clears CT_SPILL for the next P2G and, when host_count (pinned host memory)
+// is given, writes the count there and then the tile launch number to
+// host_seq (a release store: a host that reads its launch's number also reads
+// that launch's count).
+template <int GB>
+__global__ void __launch_bounds__(64) k_grid_update(GridP g, float dt, const uint32_t *list, uint32_t *flags,
+                                                    uint32_t *act, uint32_t seq, uint32_t *counters, float4 *gmp,
+                                                    float4 *gv, const float4 *__restrict__ staging,
                                                     const int32_t *__restrict__ blk_tile, int ngroups,
-                                                    uint32_t staging_cap, int64_t nblocks, int clear_spill)
+                                                    uint32_t staging_cap, int64_t nblocks, uint32_t *host_count,
+                                                    uint32_t *host_seq, uint32_t launch)
 {
-    const uint32_t nact = counters[CT_ACTIVE];
-    const uint32_t nact8 = round_xcd(nact);
-    if (clear_spill && blockIdx.x == 0 && threadIdx.x == 0) {     // see compact_flags
-        gp(counters)[CT_SPILLED] = gp(counters)[CT_SPILL];
+    const uint32_t n = counters[CT_LIST], n8 = round_xcd(n);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const uint32_t spilled = gp(counters)[CT_SPILL];
+        gp(counters)[CT_SPILLED] = spilled;
         gp(counters)[CT_SPILL] = 0u;
+        if (host_count) {
+            *host_count = spilled;
+            __hip_atomic_store(host_seq, launch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
     dt = step_dt(g, dt);
-    for (uint32_t k8 = blockIdx.x; k8 < nact8; k8 += gridDim.x) {
-        const uint32_t k = xcd_spread(k8, nact8);
-        if (k >= nact) continue;
-        const uint32_t b = __builtin_amdgcn_readfirstlane(list[k]);
-        grid_block(g, dt, b, gmp, gv, staging, blk_tile, ngroups, staging_cap, nblocks);
+    for (uint32_t k8 = blockIdx.x; k8 < n8; k8 += gridDim.x) {
+        const uint32_t k = xcd_spread(k8, n8);
+        if (k >= n) continue;
+        const uint32_t b = (uint32_t)__builtin_amdgcn_readfirstlane((int)list[k]);
+        grid_block<GB>(g, dt, b, flags, act, seq, gmp, gv, staging, blk_tile, ngroups, staging_cap, nblocks);
     }
 }
 
-// Nodes with mass after the grid update (statistics only; launched when
-// timing is on).  One atomic per workgroup: same-address atomics from every
-// wave of the grid update would serialize in L2.
-__global__ void __launch_bounds__(256) k_count_nodes(const uint32_t *list, uint32_t *counters,
-                                                     const float4 *__restrict__ gv)
+// Lists 256 consecutive blocks (thread t: block b0 + t) that `want`, with one
+// global atomic: wave counts are combined in LDS.
+__device__ __forceinline__ void list_blocks(bool want, int b0, uint32_t *list, uint32_t *counters)
 {
-    __shared__ uint32_t part[4];
-    const uint32_t nact = counters[CT_ACTIVE];
+    __shared__ uint32_t wave_cnt[4], wg_base;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t nodes = 0;
-    for (uint32_t k = blockIdx.x * 4 + w; k < nact; k += gridDim.x * 4) {
-        const float4 v = gv[(int64_t)list[k] * BLK_NODES + lane];
-        nodes += (uint32_t)__popcll(__ballot(v.w != 0.f));
-    }
-    if (lane == 0) part[w] = nodes;
+    const uint64_t mask = __ballot(want);
+    if (lane == 0) wave_cnt[w] = (uint32_t)__popcll(mask);
     __syncthreads();
     if (threadIdx.x == 0) {
-        const uint32_t t = part[0] + part[1] + part[2] + part[3];
-        if (t) atomicAdd(counters + CT_NODES, t);
+        const uint32_t tot = wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
+        wg_base = tot ? gatomic_add(counters + CT_LIST, tot) : 0u;
+    }
+    __syncthreads();
+    uint32_t off = wg_base;
+    for (int k = 0; k < w; ++k) off += wave_cnt[k];
+    if (want) gp(list)[off + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = (uint32_t)(b0 + (int)threadIdx.x);
+}
+
+// The blocks that the P2G marked (PLAIN form, each step).
+__global__ void __launch_bounds__(256) k_list_marked(const uint32_t *flags, int nblocks, uint32_t *list,
+                                                     uint32_t *counters)
+{
+    const int b0 = (int)(blockIdx.x * 256u), b = b0 + (int)threadIdx.x;
+    list_blocks(b < nblocks && (gp(flags)[b] & BF_MARKED), b0, list, counters);
+}
+
+// Every tile's block and the next one in each axis (at each sort; a list of
+// the marked blocks was a launch of every step, 4.6 us of 42 for 100k
+// particles), and the blocks still marked.
+__device__ __forceinline__ void list_near_tiles(const GridP &g, const int32_t *__restrict__ blk_tile, int ngroups,
+                                                int nblocks, int b0, uint32_t *flags, uint32_t *list,
+                                                uint32_t *counters)
+{
+    const int b = b0 + (int)threadIdx.x;
+    uint32_t f = 0;
+    if (b < nblocks) {
+        const uint32_t row = div_by((uint32_t)b, (uint32_t)g.nbx, g.div_nbx);
+        const int bz = (int)div_by(row, (uint32_t)g.nby, g.div_nby);
+        const int bx = b - (int)row * g.nbx, by = (int)row - bz * g.nby;
+        bool near = false;
+        for (int gi = 0; gi < ngroups && !near; ++gi)
+            for (int z = max(bz - 1, 0); z <= bz; ++z)
+                for (int y = max(by - 1, 0); y <= by; ++y)
+                    for (int x = max(bx - 1, 0); x <= bx; ++x)
+                        near |= gp(blk_tile)[(int64_t)gi * nblocks + ((int64_t)z * g.nby + y) * g.nbx + x] >= 0;
+        const uint32_t old = gp(flags)[b];
+        f = (old & BF_MARKED) | (near || (old & BF_MARKED) ? BF_LISTED : 0u);
+        if (f != old) gp(flags)[b] = f;
+    }
+    list_blocks(f != 0u, b0, list, counters);
+}
+
+__global__ void __launch_bounds__(256) k_list_near(GridP g, const int32_t *__restrict__ blk_tile, int ngroups,
+                                                   int nblocks, uint32_t *flags, uint32_t *list, uint32_t *counters)
+{
+    list_near_tiles(g, blk_tile, ngroups, nblocks, (int)(blockIdx.x * 256u), flags, list, counters);
+}
+
+__global__ void __launch_bounds__(256) k_bsort_list(const SortSlice *__restrict__ tab, int ns)
+{
+    SliceScan sc;
+    sc.build(ns, [&](int s) { return (uint32_t)((tab[s].nblocks + 255) / 256); });
+    if (blockIdx.x >= sc.total) return;
+    const uint32_t sid = (uint32_t)__builtin_amdgcn_readfirstlane((int)sc.find(blockIdx.x));
+    const SortSlice &t = tab[sid];
+    list_near_tiles(t.g, t.blk_tile, 1, t.nblocks, (int)((blockIdx.x - sc.start(sid)) * 256u), t.flags, t.list,
+                    t.counters);
+}
+
+// Blocks whose act entry is `seq` (BATCH_SEQ: the device's own count of a
+// batched scene) into CT_ACTIVE and, with gv, their nodes with mass into
+// CT_NODES (statistics only).  One atomic per workgroup: same-address atomics
+// from every wave would serialize in L2.
+__global__ void __launch_bounds__(256) k_count_active(const uint32_t *act, uint32_t seq, int64_t nblocks,
+                                                      uint32_t *counters, const float4 *__restrict__ gv)
+{
+    __shared__ uint32_t part[2][4];
+    if (seq == BATCH_SEQ) seq |= counters[CT_SEQ];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t blocks = 0, nodes = 0;
+    for (int64_t b0 = ((int64_t)blockIdx.x * 4 + w) * 64; b0 < nblocks; b0 += (int64_t)gridDim.x * 256) {
+        const uint64_t m = __ballot(b0 + lane < nblocks && act[b0 + lane] == seq);
+        blocks += (uint32_t)__popcll(m);
+        if (gv)
+            for (uint64_t r = m; r; r &= r - 1) {
+                const float4 v = gv[(b0 + __ffsll((unsigned long long)r) - 1) * BLK_NODES + lane];
+                nodes += (uint32_t)__popcll(__ballot(v.w != 0.f));
+            }
+    }
+    if (lane == 0) {
+        part[0][w] = blocks;
+        part[1][w] = nodes;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const uint32_t *p = part[threadIdx.x];
+        const uint32_t t = p[0] + p[1] + p[2] + p[3];
+        if (t) atomicAdd(counters + (threadIdx.x ? CT_NODES : CT_ACTIVE), t);
     }
 }
 
-int launch_count_nodes(hipStream_t st, const uint32_t *list, uint32_t *counters, const float4 *gv)
+int launch_count_active(hipStream_t st, const uint32_t *act, uint32_t seq, int64_t nblocks, uint32_t *counters,
+                        const float4 *gv)
 {
-    hipLaunchKernelGGL(k_count_nodes, dim3(256), dim3(256), 0, st, list, counters, gv);
+    if (int rc = launch_zero_u32(st, counters + CT_ACTIVE, 1)) return rc;
+    if (gv)
+        if (int rc = launch_zero_u32(st, counters + CT_NODES, 1)) return rc;
+    hipLaunchKernelGGL(k_count_active, dim3(256), dim3(256), 0, st, act, seq, nblocks, counters, gv);
     return (int)hipGetLastError();
 }
 
@@ -283,95 +362,79 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kG2pWa
     wave_max_to(spread(counters) + CT_DEFORM, sd[1]);
 }
 
-// Particles whose stencil left their block arena (listed by the block
-// kernels): scatter with global atomics into grid_mp, which the grid update
-// adds in.  Persistent over the list.
-template <int MAT>
-__device__ __forceinline__ void spill_particle(const GridP &g, const MatP &mat, const PartView &pv, int i, float dt,
-                                               uint32_t *counters, float4 *grid, uint32_t *flags)
+// The FAST-form G2P of several groups in one launch, each group's particles in
+// workgroups of their own: a launch costs 4.6 us, and 100k particles (12 us)
+// fill no more than a wave a SIMD.  Jello, snow and water, 100k particles
+// each: 8.9, 11.9 and 6.8 us apart, 17.4 together.
+template <bool MOVE, bool CTL>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_g2p_groups(const G2PArgs a)
 {
-    float x[3] = {ld(pv, PL_X, i), ld(pv, PL_X + 1, i), ld(pv, PL_X + 2, i)};
-    Stencil s;
-    make_stencil(g, x, s);
-    Scatter sc;
-    load_scatter<MAT>(pv, i, mat, dt, true, 0, sc, counters);
+    const uint32_t nb = a.grp[a.ngroups - 1].end, blk = xcd_spread(blockIdx.x, round_xcd(nb));
+    if (blk >= nb) return;                                             // whole workgroup
+    int gi = 0;
+    while (a.grp[gi].end <= blk) ++gi;
+    const G2PGroup &q = a.grp[gi];
+    const int j = (int)((blk - (gi ? a.grp[gi - 1].end : 0u)) * blockDim.x + threadIdx.x);
+    int i = j;
+    PartView po = q.pv;
+    if (MOVE) {
+        po.P = q.P_out;
+        if (j < q.pv.n) {
+            const uint32_t src = gp(q.perm)[j];
+            i = src < (uint32_t)q.pv.n ? (int)src : j;     // always a valid index for a permutation
+            gp(a.pid_out)[q.pv.off + j] = gp(a.pid)[q.pv.off + i];
+            if (a.copy_q) {
 #pragma unroll
-    for (int ox = 0; ox < 3; ++ox)
-#pragma unroll
-        for (int oy = 0; oy < 3; ++oy)
-#pragma unroll
-            for (int oz = 0; oz < 3; ++oz) {
-                float4 c = node_contrib(g, s, sc, ox, oy, oz);
-                float *dst = (float *)(grid + node_slot(g, s.b[0] + ox, s.b[1] + oy, s.b[2] + oz));
-                gatomic_add(dst + 0, c.x);
-                gatomic_add(dst + 1, c.y);
-                gatomic_add(dst + 2, c.z);
-                gatomic_add(dst + 3, c.w);
+                for (int k = 0; k < 4; ++k) st(po, PL_Q + k, j, ld(q.pv, PL_Q + k, i));
             }
-    if (flags) mark_blocks(g, s.b, flags);
+        }
+    }
+    const float dt = step_dt(a.g, a.dt);
+    float sd[2] = {0.0f, 0.0f};
+    float *measures = CTL ? sd : nullptr;
+    if (j < q.pv.n) {
+        switch (q.mat.type) {
+        case MPM_JELLO: g2p_particle<MPM_JELLO>(a.g, q.mat, q.pv, i, po, j, dt, a.gv, true, a.sweeps, a.counters, measures); break;
+        case MPM_SNOW: g2p_particle<MPM_SNOW>(a.g, q.mat, q.pv, i, po, j, dt, a.gv, true, a.sweeps, a.counters, measures); break;
+        default: g2p_particle<MPM_WATER>(a.g, q.mat, q.pv, i, po, j, dt, a.gv, true, a.sweeps, a.counters, measures); break;
+        }
+    }
+    if (!CTL) return;
+    wave_max_to(spread(a.counters) + CT_SPEED, sd[0]);
+    wave_max_to(spread(a.counters) + CT_DEFORM, sd[1]);
 }
 
-// host_count (pinned host memory, or null) receives the spill count, then
-// host_seq the tile launch number `seq` (a release store: a host that reads
-// seq == its launch also reads that launch's count).  With clear_active the
-// kernel also clears the active-block and node counters for the block
-// compaction that follows (no kernel between P2G and it touches them), which
-// saves the FAST form its step-start counter reset.
+int launch_g2p_groups(hipStream_t st, const G2PArgs &a, uint32_t wgs, int threads, bool move)
+{
+    const dim3 gr(round_xcd(wgs)), bl(threads);
+    const auto k = a.g.dtp ? (move ? k_g2p_groups<true, true> : k_g2p_groups<false, true>)
+                           : (move ? k_g2p_groups<true, false> : k_g2p_groups<false, false>);
+    hipLaunchKernelGGL(k, gr, bl, 0, st, a);
+    return (int)hipGetLastError();
+}
+
+// FUSED form: the particles a tile kernel listed, persistent over the list.
+// host_count (pinned host memory) receives their number, then host_seq the
+// tile launch number `seq` (a release store: a host that reads seq == its
+// launch also reads that launch's count).
 template <int MAT>
 __global__ void __launch_bounds__(256) k_p2g_spill(GridP g, MatP mat, PartView pv, float dt,
                                                    const uint32_t *__restrict__ list, uint32_t *counters,
-                                                   float4 *grid, uint32_t *flags, uint32_t list_cap,
-                                                   uint32_t *host_count, uint32_t *host_seq, uint32_t seq,
-                                                   int clear_active)
+                                                   float4 *grid, uint32_t *flags, uint32_t *blocks, uint32_t list_cap,
+                                                   uint32_t *host_count, uint32_t *host_seq, uint32_t seq)
 {
     const uint32_t listed = counters[CT_SPILL];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (host_count) {
-            *host_count = listed;
-            if (host_seq) __hip_atomic_store(host_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
-        if (clear_active) {
-            gp(counters)[CT_ACTIVE] = 0u;
-            gp(counters)[CT_NODES] = 0u;
-        }
+        *host_count = listed;
+        __hip_atomic_store(host_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     const uint32_t n = min(listed, list_cap);
     dt = step_dt(g, dt);
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
         const int i = (int)list[k];
         if (i < 0 || i >= pv.n) continue;
-        spill_particle<MAT>(g, mat, pv, i, dt, counters, grid, flags);
+        spill_particle<MAT>(g, mat, pv, i, dt, counters, grid, flags, blocks);
     }
-}
-
-// Spill scatter and block compaction in one launch (FAST form, one particle
-// group): the tile P2G already flagged the blocks of the particles it listed,
-// so the workgroups scatter their share of the list with atomics (into
-// grid_mp, read only by the grid update after this kernel) and compact their
-// 256 block flags without waiting on each other.  CT_SPILL is read by every
-// workgroup here; the grid update clears it.
-template <int MAT>
-__global__ void __launch_bounds__(256) k_spill_compact(GridP g, MatP mat, PartView pv, float dt,
-                                                       const uint32_t *__restrict__ spill, uint32_t spill_cap,
-                                                       uint32_t *counters, float4 *grid, uint32_t *flags,
-                                                       int nblocks, uint32_t *list, uint32_t *host_count,
-                                                       uint32_t *host_seq, uint32_t seq)
-{
-    const uint32_t listed = counters[CT_SPILL];
-    if (host_count && blockIdx.x == 0 && threadIdx.x == 0) {
-        *host_count = listed;
-        __hip_atomic_store(host_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    const uint32_t n = min(listed, spill_cap);
-    if (n) {
-        dt = step_dt(g, dt);
-        for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-            const int i = (int)spill[k];
-            if (i < 0 || i >= pv.n) continue;
-            spill_particle<MAT>(g, mat, pv, i, dt, counters, grid, nullptr);
-        }
-    }
-    compact_flags(flags, nblocks, list, counters, (int)(blockIdx.x * blockDim.x), false);
 }
 
 // Kirchhoff stress of the current state, for the first P2G of the FAST form
@@ -397,70 +460,25 @@ __global__ void k_compute_tau(MatP mat, PartView pv, int sweeps, uint32_t *count
 // reads that scene's parameters with uniform loads and runs the body of the
 // single-scene kernel.  Materials are selected per scene at run time.
 
-__global__ void k_batch_zero(const BatchSlice *__restrict__ tab, int nslices)
-{
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nslices) return;
-    uint32_t *c = tab[s].counters;
-    gp(c)[CT_ACTIVE] = 0u;
-    gp(c)[CT_NODES] = 0u;
-    gp(c)[CT_SPILL] = 0u;
-    // warm start: the particles the last G2P listed go to this step's
-    // inference, and the list starts over for this step's G2P
-    uint32_t *w = tab[s].warm_cnt;
-    if (w) {
-        gp(w)[0] = gp(w)[1];
-        gp(w)[1] = 0u;
-    }
-}
-
-template <int MAT>
-__device__ __forceinline__ void spill_scene(const BatchSlice &b, uint32_t n, uint32_t tid, uint32_t stride)
-{
-    for (uint32_t k = tid; k < n; k += stride) {
-        const int i = (int)gp(b.spill)[k];
-        if (i < 0 || i >= b.pv.n) continue;
-        spill_particle<MAT>(b.g, b.mat, b.pv, i, b.dt, b.counters, b.grid_mp, b.flags);
-    }
-}
-
-// Spilled particles of every scene: the workgroups form groups of `per`,
-// group q takes scenes q, q + groups, ... (the scenes' counter loads then
-// overlap instead of following one another).
-__global__ void __launch_bounds__(256) k_spill_batch(const BatchSlice *__restrict__ tab, int nslices)
-{
-    const uint32_t per = max(1u, gridDim.x / (uint32_t)nslices);
-    const uint32_t groups = gridDim.x / per;
-    if (blockIdx.x / per >= groups) return;
-    const uint32_t tid = (blockIdx.x % per) * blockDim.x + threadIdx.x, stride = per * blockDim.x;
-    for (uint32_t sid = blockIdx.x / per; sid < (uint32_t)nslices; sid += groups) {
-        const BatchSlice &b = tab[sid];
-        const uint32_t n = min(gp(b.counters)[CT_SPILL], (uint32_t)b.pv.n);
-        if (n == 0u) continue;
-        switch (b.mat.type) {
-        case MPM_JELLO: spill_scene<MPM_JELLO>(b, n, tid, stride); break;
-        case MPM_SNOW: spill_scene<MPM_SNOW>(b, n, tid, stride); break;
-        default: spill_scene<MPM_WATER>(b, n, tid, stride); break;
-        }
-    }
-}
-
-// Active-block lists: workgroup w compacts 256 flags of one scene.
-__global__ void __launch_bounds__(256) k_compact_batch(const BatchSlice *__restrict__ tab, int nslices)
-{
-    SliceScan sc;
-    sc.build(nslices, [&](int s) { return (uint32_t)((tab[s].nblocks + 255) / 256); });
-    if (blockIdx.x >= sc.total) return;
-    const uint32_t sid = (uint32_t)__builtin_amdgcn_readfirstlane((int)sc.find(blockIdx.x));
-    const BatchSlice &b = tab[sid];
-    compact_flags(b.flags, (int)b.nblocks, b.list, b.counters, (int)((blockIdx.x - sc.start(sid)) * 256u), true);
-}
-
-// Grid update over the active blocks of every scene (one wave per block).
+// Grid update over the listed blocks of every scene (one wave per block).
+// The first workgroup also does what k_grid_update does with the spill counts
+// and hands the warm start's list over: the particles the last G2P listed go
+// to this step's inference, and the list starts over for this step's G2P.
 __global__ void __launch_bounds__(64) k_grid_batch(const BatchSlice *__restrict__ tab, int nslices)
 {
+    if (blockIdx.x == 0)
+        for (int s = (int)threadIdx.x; s < nslices; s += 64) {
+            const BatchSlice &b = tab[s];
+            gp(b.counters)[CT_SPILLED] = gp(b.counters)[CT_SPILL];
+            gp(b.counters)[CT_SPILL] = 0u;
+            uint32_t *w = b.warm_cnt;
+            if (w) {
+                gp(w)[0] = gp(w)[1];
+                gp(w)[1] = 0u;
+            }
+        }
     SliceScan sc;
-    sc.build(nslices, [&](int s) { return gp(tab[s].counters)[CT_ACTIVE]; });
+    sc.build(nslices, [&](int s) { return gp(tab[s].counters)[CT_LIST]; });
     const uint32_t n = sc.total, n8 = round_xcd(n);
     for (uint32_t k8 = blockIdx.x; k8 < n8; k8 += gridDim.x) {
         const uint32_t k = xcd_spread(k8, n8);
@@ -468,7 +486,8 @@ __global__ void __launch_bounds__(64) k_grid_batch(const BatchSlice *__restrict_
         const uint32_t sid = (uint32_t)__builtin_amdgcn_readfirstlane((int)sc.find(k));
         const BatchSlice &b = tab[sid];
         const uint32_t blk = (uint32_t)__builtin_amdgcn_readfirstlane((int)gp(b.list)[k - sc.start(sid)]);
-        grid_block(b.g, b.dt, blk, b.grid_mp, b.grid_v, b.staging, b.blk_tile, 1, b.staging_cap, b.nblocks);
+        grid_block<1>(b.g, b.dt, blk, b.flags, b.act, BATCH_SEQ | gp(b.counters)[CT_SEQ], b.grid_mp, b.grid_v, b.staging,
+                    b.blk_tile, 1, b.staging_cap, b.nblocks);
     }
 }
 
@@ -540,21 +559,36 @@ int launch_p2g_atomic(hipStream_t st, const GridP &g, const MatP &m, const PartV
     return (int)hipGetLastError();
 }
 
-int launch_compact(hipStream_t st, uint32_t *flags, int nblocks, uint32_t *list, uint32_t *counters)
+int launch_list_marked(hipStream_t st, const uint32_t *flags, int nblocks, uint32_t *list, uint32_t *counters)
 {
-    hipLaunchKernelGGL(k_compact_blocks, dim3(nblk(nblocks, 256)), dim3(256), 0, st, flags, nblocks, list,
-                       counters);
+    if (int rc = launch_zero_u32(st, counters + CT_LIST, 1)) return rc;
+    hipLaunchKernelGGL(k_list_marked, dim3(nblk(nblocks, 256)), dim3(256), 0, st, flags, nblocks, list, counters);
     return (int)hipGetLastError();
 }
 
-int launch_grid_update(hipStream_t st, const GridP &g, float dt, const uint32_t *list,
-                       uint32_t *counters, float4 *gmp, float4 *gv, int nblocks, const float4 *staging,
-                       const int32_t *blk_tile, int ngroups, uint32_t staging_cap, int clear_spill)
+// CT_LIST was cleared (k_rank_tiles, k_bsort_rank).
+int launch_list_near(hipStream_t st, const GridP &g, const int32_t *blk_tile, int ngroups, int nblocks, uint32_t *flags,
+                     uint32_t *list, uint32_t *counters)
 {
-    int wg = nblocks < 8192 ? nblocks : 8192;
-    if (wg < 1) wg = 1;
-    hipLaunchKernelGGL(k_grid_update, dim3(wg), dim3(64), 0, st, g, dt, list, counters, gmp, gv, staging, blk_tile,
-                       ngroups, staging_cap, (int64_t)nblocks, clear_spill);
+    hipLaunchKernelGGL(k_list_near, dim3(nblk(nblocks, 256)), dim3(256), 0, st, g, blk_tile, ngroups, nblocks, flags,
+                       list, counters);
+    return (int)hipGetLastError();
+}
+
+int launch_bsort_list(hipStream_t st, const SortSlice *tab, int ns, int wgs)
+{
+    hipLaunchKernelGGL(k_bsort_list, dim3(wgs), dim3(256), 0, st, tab, ns);
+    return (int)hipGetLastError();
+}
+
+int launch_grid_update(hipStream_t st, const GridP &g, float dt, const uint32_t *list, uint32_t *flags, uint32_t *act,
+                       uint32_t seq, uint32_t *counters, float4 *gmp, float4 *gv, int64_t nblocks,
+                       const float4 *staging, const int32_t *blk_tile, int ngroups, uint32_t staging_cap,
+                       uint32_t *host_count, uint32_t *host_seq, uint32_t launch)
+{
+    hipLaunchKernelGGL(ngroups > 1 ? k_grid_update<4> : k_grid_update<1>, dim3((uint32_t)std::min<int64_t>(nblocks, 8192)), dim3(64), 0, st, g, dt, list,
+                       flags, act, seq, counters, gmp, gv, staging, blk_tile, ngroups, staging_cap, nblocks, host_count,
+                       host_seq, launch);
     return (int)hipGetLastError();
 }
 
@@ -585,15 +619,16 @@ int launch_g2p(hipStream_t st, const GridP &g, const MatP &m, const PartView &pv
 }
 
 int launch_p2g_spill(hipStream_t st, const GridP &g, const MatP &m, const PartView &pv, float dt,
-                     const uint32_t *list, uint32_t list_cap, uint32_t *counters, float4 *grid, uint32_t *flags,
-                     uint32_t *host_count, uint32_t *host_seq, uint32_t seq, int clear_active)
+                     const uint32_t *list, uint32_t list_cap, uint32_t *counters, float4 *grid, uint32_t *flags, uint32_t *blocks,
+                     uint32_t *host_count, uint32_t *host_seq, uint32_t seq)
 {
     if (pv.n <= 0) return 0;
+    if (!host_count || !host_seq) return (int)hipErrorInvalidValue;
     dim3 gr(64), bl(256);
     switch (m.type) {
-    case MPM_JELLO: hipLaunchKernelGGL(k_p2g_spill<MPM_JELLO>, gr, bl, 0, st, g, m, pv, dt, list, counters, grid, flags, list_cap, host_count, host_seq, seq, clear_active); break;
-    case MPM_SNOW: hipLaunchKernelGGL(k_p2g_spill<MPM_SNOW>, gr, bl, 0, st, g, m, pv, dt, list, counters, grid, flags, list_cap, host_count, host_seq, seq, clear_active); break;
-    default: hipLaunchKernelGGL(k_p2g_spill<MPM_WATER>, gr, bl, 0, st, g, m, pv, dt, list, counters, grid, flags, list_cap, host_count, host_seq, seq, clear_active); break;
+    case MPM_JELLO: hipLaunchKernelGGL(k_p2g_spill<MPM_JELLO>, gr, bl, 0, st, g, m, pv, dt, list, counters, grid, flags, blocks, list_cap, host_count, host_seq, seq); break;
+    case MPM_SNOW: hipLaunchKernelGGL(k_p2g_spill<MPM_SNOW>, gr, bl, 0, st, g, m, pv, dt, list, counters, grid, flags, blocks, list_cap, host_count, host_seq, seq); break;
+    default: hipLaunchKernelGGL(k_p2g_spill<MPM_WATER>, gr, bl, 0, st, g, m, pv, dt, list, counters, grid, flags, blocks, list_cap, host_count, host_seq, seq); break;
     }
     return (int)hipGetLastError();
 }
@@ -609,28 +644,10 @@ int launch_compute_tau(hipStream_t st, const MatP &m, const PartView &pv, int sw
     return (int)hipGetLastError();
 }
 
-int launch_batch_zero(hipStream_t st, const BatchSlice *tab, int nslices)
-{
-    hipLaunchKernelGGL(k_batch_zero, dim3(nblk(nslices, 64)), dim3(64), 0, st, tab, nslices);
-    return (int)hipGetLastError();
-}
-
 int launch_permute_batch(hipStream_t st, const BatchSlice *src, const BatchSlice *dst, int nslices, int wgs)
 {
     if (wgs <= 0) return 0;
     hipLaunchKernelGGL(k_permute_batch, dim3(wgs), dim3(256), 0, st, src, dst, nslices);
-    return (int)hipGetLastError();
-}
-
-int launch_spill_batch(hipStream_t st, const BatchSlice *tab, int nslices, int wgs)
-{
-    hipLaunchKernelGGL(k_spill_batch, dim3(wgs), dim3(256), 0, st, tab, nslices);
-    return (int)hipGetLastError();
-}
-
-int launch_compact_batch(hipStream_t st, const BatchSlice *tab, int nslices, int wgs)
-{
-    hipLaunchKernelGGL(k_compact_batch, dim3(wgs), dim3(256), 0, st, tab, nslices);
     return (int)hipGetLastError();
 }
 
@@ -728,21 +745,6 @@ __global__ void __launch_bounds__(CT_SPREAD) k_dt_control(DtCtl *c, uint32_t *co
 int launch_dt_clear(hipStream_t st, uint32_t *counters)
 {
     hipLaunchKernelGGL(k_dt_clear, dim3(1), dim3(CT_SPREAD), 0, st, counters);
-    return (int)hipGetLastError();
-}
-
-int launch_spill_compact(hipStream_t st, const GridP &g, const MatP &m, const PartView &pv, float dt,
-                         const uint32_t *spill, uint32_t spill_cap, uint32_t *counters, float4 *grid,
-                         uint32_t *flags, int nblocks, uint32_t *list, uint32_t *host_count, uint32_t *host_seq,
-                         uint32_t seq)
-{
-    if (!host_count || !host_seq) return (int)hipErrorInvalidValue;
-    dim3 gr(nblk(nblocks, 256)), bl(256);
-    switch (m.type) {
-    case MPM_JELLO: hipLaunchKernelGGL(k_spill_compact<MPM_JELLO>, gr, bl, 0, st, g, m, pv, dt, spill, spill_cap, counters, grid, flags, nblocks, list, host_count, host_seq, seq); break;
-    case MPM_SNOW: hipLaunchKernelGGL(k_spill_compact<MPM_SNOW>, gr, bl, 0, st, g, m, pv, dt, spill, spill_cap, counters, grid, flags, nblocks, list, host_count, host_seq, seq); break;
-    default: hipLaunchKernelGGL(k_spill_compact<MPM_WATER>, gr, bl, 0, st, g, m, pv, dt, spill, spill_cap, counters, grid, flags, nblocks, list, host_count, host_seq, seq); break;
-    }
     return (int)hipGetLastError();
 }
 
