@@ -392,7 +392,7 @@ typedef struct mpm_batch_shape {
     int32_t grid_workgroups;  /* width of the persistent grid-update launch */
     int32_t g2p_threads;      /* G2P workgroup size: 64, 128, 192 or 256 */
     int32_t sort_every;       /* steps between re-sorts of every scene */
-    int32_t use_graph;        /* 1: replay captured hipGraphs; 0: launch the stages directly */
+    int32_t use_graph;        /* 1: replay captured hipGraphs (the re-sort's); 0: launch every stage directly */
     int32_t p2g_tile;         /* 256, 384 or 512 (0 = 384); accepted, selects nothing */
 } mpm_batch_shape;
 

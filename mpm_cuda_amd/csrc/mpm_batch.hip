@@ -4,15 +4,15 @@
 // Each scene is an mpm_sim with one particle group in the FAST form.  The
 // batch keeps a table of the scenes' parameters (BatchSlice) in device memory
 // and advances every scene by one step with one launch per stage for the
-// whole batch -- counters, atomic spill fallback, active-block compaction,
-// grid update -- and one per stage and material for P2G tiles (per 64
-// scenes) and G2P, each a persistent launch over the scenes of that
-// material, plus one warm-start inference launch per set of scenes with
-// equal network weights.  That sequence is recorded once into a hipGraph and replayed.
-// Every `sort_every` steps all scenes are re-sorted by a second graph with
-// one branch per scene, on the scenes' own streams.  Sorting moves particle
-// storage between two buffers, so there is one step graph and one sort graph
-// per buffer parity.  Launch widths come from mpm_batch_autotune, which times
+// whole batch -- P2G tiles (per 64 scenes), grid update, G2P -- each over the
+// scenes of all materials, plus one warm-start inference launch per set of
+// scenes with equal network weights.  (16 scenes of the three materials, 0.9M
+// particles, 48 steps: 6.3 ms with a hipGraph of one branch per material, whose
+// kernels hardly ran side by side; 5.9 with a graph of these three launches;
+// 5.7 launched directly.)
+// Every `sort_every` steps all scenes are re-sorted, one launch per stage of
+// the sort, replayed as a hipGraph.  Sorting moves particle storage between
+// two buffers, so there is one graph per buffer parity.  Launch widths come from mpm_batch_autotune, which times
 // the candidates of each stage on live steps; results do not depend on them
 // (every tile, block and particle is processed by exactly one workgroup).
 #include "mpm_launch.h"
@@ -33,7 +33,7 @@ const int G2P_CAND[NCAND] = {64, 128, 192, 256};
 constexpr int NTILE = 3;
 const int TILE_CAND[NTILE] = {256, 384, 512};            // values of p2g_tile; the P2G is the same with each
 
-// What the captured graphs depend on, per scene.
+// What the tables and the captured graphs depend on, per scene.
 struct SceneSig {
     float *P0, *P1;
     uint32_t *pid0, *pid1;
@@ -61,26 +61,19 @@ struct mpm_batch {
     BatchSlice *tab[2] = {};
     std::vector<SceneSig> sig;          // signature the tables and graphs were built for
     bool built = false;
-    hipGraphExec_t step_exec[2] = {}, sort_exec[2] = {};
-    int captured_p2g = 0, captured_grid = 0, captured_g2p = 0;
+    hipGraphExec_t sort_exec[2] = {};
     int parity = 0;
     int64_t steps_since_sort = 0;
     int64_t total = 0;
-    std::vector<int> types;             // material of each scene
-    // scenes are kept ordered by material: material m holds table entries
-    // [mat_begin[m], mat_begin[m] + mat_count[m])
-    int mat_begin[3] = {0, 0, 0}, mat_count[3] = {0, 0, 0};
+    int mats = -1;                      // the scenes' material, MAT_ANY: several
     int permute_wgs = 0;                // workgroups of the batched re-sort move
     SortSlice *stab[2] = {};            // batched re-sort tables of both parities
     SortBatchPlan splan;
-    // warm-start sets present among each material's scenes, with their
-    // 64-particle chunks there
-    std::vector<std::pair<int, int64_t>> mat_sets[3];
     // warm-start weight sets: scenes with equal weights share one inference launch
     std::vector<const float *> warm_params; // device weights of each set
     std::vector<int64_t> warm_chunks;       // 64-particle chunks of each set
     std::vector<int> warm_group;            // per scene, -1: cold
-    hipEvent_t ev_fork = nullptr, ev_done = nullptr;
+    hipEvent_t ev_done = nullptr;
     std::vector<hipEvent_t> ev_join;
     std::vector<hipEvent_t> tev;        // step timing events
 };
@@ -118,78 +111,27 @@ void set_parity(mpm_batch *b, size_t k, int p)
     s->pid_alt = p ? b->pid0[k] : b->pid1[k];
 }
 
-// G2P workgroups of the scenes of material `mat` (0: none of them).
-int g2p_wgs(const mpm_batch *b, int mat, int threads)
+// G2P workgroups of all scenes.
+int g2p_wgs(const mpm_batch *b, int threads)
 {
     uint32_t w = 0;
-    for (mpm_sim *s : b->sims)
-        if (s->groups[0].mat.type == mat) w += (uint32_t)((s->groups[0].n + threads - 1) / threads);
+    for (mpm_sim *s : b->sims) w += (uint32_t)((s->groups[0].n + threads - 1) / threads);
     return (int)round_xcd(w);
 }
 
-
 int check(int rc, const char *what) { return rc ? hip_fail((hipError_t)rc, what) : MPM_OK; }
 
-// The launches of every material present (`launch(stream, material)`), as
-// parallel branches: forked from the batch stream onto the stream of each
-// material's first scene and joined back (the materials' scenes are
-// disjoint, so one launch's tail overlaps the others' work).
-template <class L>
-int fork_materials(mpm_batch *b, L launch)
-{
-    MPM_HIP(hipEventRecord(b->ev_fork, b->stream));
-    for (int m = MPM_JELLO; m <= MPM_WATER; ++m) {
-        size_t k = 0;
-        while (k < b->types.size() && b->types[k] != m) ++k;
-        if (k == b->types.size()) continue;
-        hipStream_t ms = b->sims[k]->stream;
-        MPM_HIP(hipStreamWaitEvent(ms, b->ev_fork, 0));
-        if (int rc = launch(ms, m)) return rc;
-        MPM_HIP(hipEventRecord(b->ev_join[k], ms));
-        MPM_HIP(hipStreamWaitEvent(b->stream, b->ev_join[k], 0));
-    }
-    return MPM_OK;
-}
-
-// The step of one material's scenes (table range [s0, s0 + cnt)) on stream
-// ms: P2G, grid update, the warm-start inference of each weight set among
-// them, G2P.
-int enqueue_material(mpm_batch *b, hipStream_t ms, int m, const BatchSlice *tab, int s0, int cnt, int p2g, int grid,
-                     int g2p_threads)
-{
-    const BatchSlice *t = tab + s0;
-    int rc;
-    if ((rc = check(launch_p2g_batch(ms, m, t, b->types.data() + s0, cnt, p2g), "p2g_batch"))) return rc;
-    if ((rc = check(launch_grid_batch(ms, t, cnt, grid), "grid_batch"))) return rc;
-    for (const auto &ws : b->mat_sets[m])
-        if ((rc = check(launch_mlp_infer_batch(ms, b->warm_params[ws.first], t, cnt, ws.first, ws.second),
-                        "mlp_infer_batch")))
-            return rc;
-    const int wgs = g2p_wgs(b, m, g2p_threads);
-    if (wgs && (rc = check(launch_g2p_batch(ms, m, t, cnt, wgs, g2p_threads), "g2p_batch"))) return rc;
-    return MPM_OK;
-}
-
-// One step of every scene (parity p tables).  Without `ev` each material's
-// scenes run their whole step as one branch beside the other materials'.
-// With `ev` (6 events, the autotuner's stage timing) the stages follow one
-// another on the batch stream, only the materials' P2G and G2P launches side
-// by side, and the P2G, grid-update and G2P stages are bracketed.
+// One step of every scene (parity p tables): P2G, grid update, the warm-start
+// inference of each weight set, G2P.  With `ev` (6 events, the autotuner's
+// stage timing) the P2G, grid-update and G2P stages are bracketed.
 int enqueue_step(mpm_batch *b, int p, int p2g, int grid, int g2p_threads, hipEvent_t *ev)
 {
     hipStream_t st = b->stream;
     const BatchSlice *tab = b->tab[p];
     const int n = (int)b->sims.size();
     int rc;
-    if (!ev)
-        return fork_materials(b, [&](hipStream_t ms, int m) {
-            return enqueue_material(b, ms, m, tab, b->mat_begin[m], b->mat_count[m], p2g, grid, g2p_threads);
-        });
     if (ev) MPM_HIP(hipEventRecord(ev[0], st));
-    rc = fork_materials(b, [&](hipStream_t ms, int m) {
-        return check(launch_p2g_batch(ms, m, tab, b->types.data(), n, p2g), "p2g_batch");
-    });
-    if (rc) return rc;
+    if ((rc = check(launch_p2g_batch(st, b->mats, tab, n, p2g), "p2g_batch"))) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[1], st));
     if (ev) MPM_HIP(hipEventRecord(ev[2], st));
     if ((rc = check(launch_grid_batch(st, tab, n, grid), "grid_batch"))) return rc;
@@ -199,11 +141,8 @@ int enqueue_step(mpm_batch *b, int p, int p2g, int grid, int g2p_threads, hipEve
                         "mlp_infer_batch")))
             return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[4], st));
-    rc = fork_materials(b, [&](hipStream_t ms, int m) {
-        const int wgs = g2p_wgs(b, m, g2p_threads);
-        return wgs ? check(launch_g2p_batch(ms, m, tab, n, wgs, g2p_threads), "g2p_batch") : MPM_OK;
-    });
-    if (rc) return rc;
+    const int wgs = g2p_wgs(b, g2p_threads);
+    if (wgs && (rc = check(launch_g2p_batch(st, b->mats, tab, n, wgs, g2p_threads), "g2p_batch"))) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[5], st));
     return MPM_OK;
 }
@@ -224,9 +163,8 @@ int enqueue_sort(mpm_batch *b, int p)
 void drop_graphs(mpm_batch *b)
 {
     for (int p = 0; p < 2; ++p) {
-        if (b->step_exec[p]) (void)hipGraphExecDestroy(b->step_exec[p]);
         if (b->sort_exec[p]) (void)hipGraphExecDestroy(b->sort_exec[p]);
-        b->step_exec[p] = b->sort_exec[p] = nullptr;
+        b->sort_exec[p] = nullptr;
     }
 }
 
@@ -245,14 +183,12 @@ void set_book(mpm_sim *s, const SortBook &k)
     s->sorts = k.sorts;
 }
 
-int capture(mpm_batch *b, hipGraphExec_t *out, bool sort, int p)
+int capture_sort(mpm_batch *b, hipGraphExec_t *out, int p)
 {
     std::vector<SortBook> book;
     for (mpm_sim *s : b->sims) book.push_back(book_of(s));
     MPM_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed));
-    int rc = sort ? enqueue_sort(b, p)
-                  : enqueue_step(b, p, b->shape.p2g_workgroups, b->shape.grid_workgroups, b->shape.g2p_threads,
-                                 nullptr);
+    int rc = enqueue_sort(b, p);
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(b->stream, &graph);
     for (size_t k = 0; k < b->sims.size(); ++k) set_book(b->sims[k], book[k]);
@@ -289,17 +225,6 @@ void group_warm(mpm_batch *b)
         }
         b->warm_group[k] = g;
         b->warm_chunks[g] += (s->groups[0].n + 63) / 64;
-    }
-    for (int m = 0; m < 3; ++m) {
-        b->mat_sets[m].clear();
-        for (int k = b->mat_begin[m]; k < b->mat_begin[m] + b->mat_count[m]; ++k) {
-            const int g = b->warm_group[k];
-            if (g < 0) continue;
-            size_t j = 0;
-            while (j < b->mat_sets[m].size() && b->mat_sets[m][j].first != g) ++j;
-            if (j == b->mat_sets[m].size()) b->mat_sets[m].push_back({g, 0});
-            b->mat_sets[m][j].second += (b->sims[k]->groups[0].n + 63) / 64;
-        }
     }
 }
 
@@ -362,14 +287,10 @@ int build(mpm_batch *b)
     for (size_t k = 0; k < n; ++k) par[k] = parity_of(b, k);
     int rc = MPM_OK;
     for (int p = 0; p < 2 && !rc; ++p) {
-        rc = capture(b, &b->sort_exec[p], true, p);
-        if (!rc) rc = capture(b, &b->step_exec[p], false, p);
+        rc = capture_sort(b, &b->sort_exec[p], p);
     }
     for (size_t k = 0; k < n; ++k) set_parity(b, k, par[k]);
     if (rc) { drop_graphs(b); b->built = false; return rc; }
-    b->captured_p2g = b->shape.p2g_workgroups;
-    b->captured_grid = b->shape.grid_workgroups;
-    b->captured_g2p = b->shape.g2p_threads;
     return MPM_OK;
 }
 
@@ -411,9 +332,7 @@ int prepare(mpm_batch *b)
         }
     bool same = b->built && b->sig.size() == n;
     for (size_t k = 0; same && k < n; ++k) same = sig_of(b, k) == b->sig[k];
-    if (same && b->shape.use_graph)
-        same = b->step_exec[0] && b->captured_p2g == b->shape.p2g_workgroups &&
-               b->captured_grid == b->shape.grid_workgroups && b->captured_g2p == b->shape.g2p_threads;
+    if (b->shape.use_graph) same = same && b->sort_exec[0];
     if (!same) {
         for (mpm_sim *s : b->sims) MPM_HIP(hipStreamSynchronize(s->stream));
         int rc = build(b);
@@ -464,7 +383,7 @@ void after_step(mpm_batch *b)
     b->steps_since_sort += 1;
 }
 
-// Sort when due, then one step; graphs or direct launches.
+// Sort when due (by its graph with `graphs`), then one step.
 int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, hipEvent_t *ev, bool graphs)
 {
     if (b->steps_since_sort >= b->shape.sort_every) {
@@ -479,12 +398,8 @@ int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, hipEvent_t *ev, b
         }
         after_sort(b);
     }
-    if (graphs) {
-        MPM_HIP(hipGraphLaunch(b->step_exec[b->parity], b->stream));
-    } else {
-        int rc = enqueue_step(b, b->parity, p2g, grid, g2p_threads, ev);
-        if (rc) return rc;
-    }
+    int rc = enqueue_step(b, b->parity, p2g, grid, g2p_threads, ev);
+    if (rc) return rc;
     after_step(b);
     return MPM_OK;
 }
@@ -551,7 +466,6 @@ int mpm_batch_create(mpm_sim *const *sims, int32_t n, const mpm_batch_shape *sha
     }
     for (mpm_sim *s : b->sims)
         if (hipStreamSynchronize(s->stream) != hipSuccess) return fail(hip_fail(hipErrorUnknown, "scene sync"));
-    for (mpm_sim *s : b->sims) b->types.push_back(s->groups[0].mat.type);
     for (mpm_sim *s : b->sims) {
         b->P0.push_back(s->P); b->P1.push_back(s->P_alt);
         b->pid0.push_back(s->pid); b->pid1.push_back(s->pid_alt);
@@ -559,10 +473,9 @@ int mpm_batch_create(mpm_sim *const *sims, int32_t n, const mpm_batch_shape *sha
     uint32_t pblocks = 0;
     for (mpm_sim *s : b->sims) pblocks += (uint32_t)((s->groups[0].n + 255) / 256);
     b->permute_wgs = (int)round_xcd(pblocks);
-    for (int k = 0; k < n; ++k) {
-        const int m = b->types[k];
-        if (b->mat_count[m] == 0) b->mat_begin[m] = k;
-        b->mat_count[m] += 1;
+    for (const mpm_sim *s : b->sims) {
+        const int t = s->groups[0].mat.type;
+        b->mats = b->mats < 0 || b->mats == t ? t : MAT_ANY;
     }
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking)) != hipSuccess) return fail(hip_fail(e, "stream"));
@@ -571,7 +484,6 @@ int mpm_batch_create(mpm_sim *const *sims, int32_t n, const mpm_batch_shape *sha
     for (int p = 0; p < 2; ++p)
         if ((e = hipMalloc(&b->stab[p], n * sizeof(SortSlice))) != hipSuccess) return fail(hip_fail(e, "hipMalloc"));
     sort_batch_plan(b->sims.data(), n, b->splan);
-    if ((e = hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming)) != hipSuccess) return fail(hip_fail(e, "event"));
     if ((e = hipEventCreateWithFlags(&b->ev_done, hipEventDisableTiming)) != hipSuccess) return fail(hip_fail(e, "event"));
     b->ev_join.assign(n, nullptr);
     for (auto &ev : b->ev_join)
@@ -711,7 +623,6 @@ void mpm_batch_destroy(mpm_batch *b)
         if (b->tab[p]) (void)hipFree(b->tab[p]);
         if (b->stab[p]) (void)hipFree(b->stab[p]);
     }
-    if (b->ev_fork) (void)hipEventDestroy(b->ev_fork);
     if (b->ev_done) (void)hipEventDestroy(b->ev_done);
     for (hipEvent_t e : b->ev_join)
         if (e) (void)hipEventDestroy(e);

@@ -1514,17 +1514,14 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
     if (bits) atomicOr(a.counters + CT_HEALTH, bits);
 }
 
-// Batched P2G: the tiles of the scenes of material MAT among up to
-// P2G_CHUNK scenes of a batch in one persistent launch (one launch per
-// material -- a run-time material switch over the three tile bodies doubles
-// the tile time at this register cap -- and per chunk of P2G_CHUNK scenes).
-// Work index = the tiles of the first such scene, then of the next, ...;
-// workgroups walk it with the XCD-aware stride of the single-scene kernel.
-// The scene map (end of each scene's tile range) sits in LDS beside the
-// tile's (256 B; LDS is allocated in granules, so any addition is checked
+// Batched P2G: the tiles of up to P2G_CHUNK scenes of a batch in one
+// persistent launch.  Work index = the tiles of the first scene, then of the
+// next, ...; workgroups walk it with the XCD-aware stride of the single-scene
+// kernel.  The scene map (end of each scene's tile range) sits in LDS beside
+// the tile's (256 B; LDS is allocated in granules, so any addition is checked
 // against the workgroups per CU it leaves).
 constexpr int P2G_CHUNK = 64;
-template <int MAT, int W>
+template <int MATS, int W>
 __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) k_p2g_batch(const BatchSlice *__restrict__ tab, int nslices)
 {
     __shared__ TileArena<W> L;
@@ -1532,9 +1529,7 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
     __shared__ uint32_t s_total;
     if (threadIdx.x < 64) {
         SliceScan sc;
-        sc.build(nslices, [&](int s) {
-            return tab[s].mat.type == MAT ? min(*gp(tab[s].tile_count), tab[s].desc_cap) : 0u;
-        });
+        sc.build(nslices, [&](int s) { return min(*gp(tab[s].tile_count), tab[s].desc_cap); });
         s_end[threadIdx.x] = sc.end[0];
         if (threadIdx.x == 0) s_total = sc.total;
     }
@@ -1547,16 +1542,15 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
         const uint32_t sid = (uint32_t)__builtin_amdgcn_readfirstlane((int)__popcll(__ballot(s_end[lane] <= tt)));
         const BatchSlice &b = tab[sid];
         const uint4 d = uniform_u4(gload_u4(b.desc, tt - (sid ? s_end[sid - 1] : 0u)));
-        const uint32_t bits = p2g_tile<MAT, W>(b.g, b.mat, b.pv, d, b.staging_cap, b.dt, b.staging, b.grid_mp, b.flags, b.list,
+        const uint32_t bits = p2g_tile_of<MATS, W>(b.g, b.mat, b.pv, d, b.staging_cap, b.dt, b.staging, b.grid_mp, b.flags, b.list,
                                                b.counters, b.blk_tile, L);
         if (bits) gatomic_or(b.counters + CT_HEALTH, bits);
     }
     if (blockIdx.x == 0)
-        for (int s = threadIdx.x; s < nslices; s += blockDim.x)
-            if (tab[s].mat.type == MAT) {
-                gp(tab[s].counters)[CT_TILES] = min(*gp(tab[s].tile_count), tab[s].desc_cap);
-                gp(tab[s].counters)[CT_SEQ] = (gp(tab[s].counters)[CT_SEQ] + 1u) & ~BATCH_SEQ;
-            }
+        for (int s = threadIdx.x; s < nslices; s += blockDim.x) {
+            gp(tab[s].counters)[CT_TILES] = min(*gp(tab[s].tile_count), tab[s].desc_cap);
+            gp(tab[s].counters)[CT_SEQ] = (gp(tab[s].counters)[CT_SEQ] + 1u) & ~BATCH_SEQ;
+        }
 }
 
 // ---------------------------------------------------------------------------
@@ -2235,17 +2229,16 @@ void fill_batch_slice(mpm_sim *s, BatchSlice &b)
     b.copy_q = s->warm_cnt ? 1 : 0;
 }
 
-// Material `mat` of the scenes [0, nslices) of tab, in chunks of P2G_CHUNK.
-int launch_p2g_batch(hipStream_t st, int mat, const BatchSlice *tab, const int *types, int nslices, int wgs)
+// The scenes [0, nslices) of tab, all of material `mats` (MAT_ANY: of
+// several), in chunks of P2G_CHUNK.
+int launch_p2g_batch(hipStream_t st, int mats, const BatchSlice *tab, int nslices, int wgs)
 {
-    const auto kernel = mat == MPM_JELLO ? k_p2g_batch<MPM_JELLO, P2G_WAVES>
-                        : (mat == MPM_SNOW ? k_p2g_batch<MPM_SNOW, P2G_WAVES> : k_p2g_batch<MPM_WATER, P2G_WAVES>);
+    const auto kernel = mats == MPM_JELLO   ? k_p2g_batch<MPM_JELLO, P2G_WAVES>
+                        : mats == MPM_SNOW  ? k_p2g_batch<MPM_SNOW, P2G_WAVES>
+                        : mats == MPM_WATER ? k_p2g_batch<MPM_WATER, P2G_WAVES>
+                                            : k_p2g_batch<MAT_ANY, P2G_WAVES>;
     for (int c0 = 0; c0 < nslices; c0 += P2G_CHUNK) {
-        const int n = std::min(P2G_CHUNK, nslices - c0);
-        bool any = false;
-        for (int k = c0; k < c0 + n; ++k) any = any || types[k] == mat;
-        if (!any) continue;
-        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(64 * P2G_WAVES), 0, st, tab + c0, n);
+        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(64 * P2G_WAVES), 0, st, tab + c0, std::min(P2G_CHUNK, nslices - c0));
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
     }

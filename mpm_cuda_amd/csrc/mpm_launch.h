@@ -65,7 +65,7 @@ int fill_sort_slice(mpm_sim *s, SortSlice &t);
 int launch_sort_batch(hipStream_t st, const SortSlice *tab, int ns, const SortBatchPlan &pl);
 // Warm-start particle lists of a simulator (mpm_api.hip).
 int ensure_warm_lists(mpm_sim *s);
-int launch_p2g_batch(hipStream_t st, int mat, const BatchSlice *tab, const int *types, int nslices, int wgs);
+int launch_p2g_batch(hipStream_t st, int mats, const BatchSlice *tab, int nslices, int wgs);
 // Planes of w floats (plane c at planes + c * stride) of n particles to the
 // host rows out[id][w]; ids NULL: in stored order, else `scratch` holds n * w
 // floats rounded up to 16 bytes (mpm_read.hip).
@@ -74,7 +74,7 @@ int read_rows(ReadStage &rs, hipStream_t st, const float *planes, int64_t stride
 bool tile_shape_valid(int tile);              // values of mpm_config.tile and mpm_batch_shape.p2g_tile
 int launch_permute_batch(hipStream_t st, const BatchSlice *src, const BatchSlice *dst, int nslices, int wgs);
 int launch_grid_batch(hipStream_t st, const BatchSlice *tab, int nslices, int wgs);
-int launch_g2p_batch(hipStream_t st, int mat, const BatchSlice *tab, int nslices, int wgs, int threads);
+int launch_g2p_batch(hipStream_t st, int mats, const BatchSlice *tab, int nslices, int wgs, int threads);
 int launch_mlp_infer(hipStream_t st, const float *params, const PartView &pv);
 int launch_mlp_infer_batch(hipStream_t st, const float *params, const BatchSlice *tab, int nslices, int group,
                            int64_t chunks);

@@ -59,3 +59,31 @@ def test_groups_and_block_list(gpu, ngroups, same, cells_per_step, cfl):
     finally:
         fast.close()
         plain.close()
+
+
+@pytest.mark.parametrize("type_", TYPES)
+def test_batch_of_one_material(gpu, type_):
+    """Scenes of a single material advanced as a batch and one by one."""
+    sims, alone = [], []
+    E, nu, rho = MAT_PARAMS[type_]
+    for out in (sims, alone):
+        for k, n in enumerate((257, 1)):
+            s = capi.Sim(capi.default_config(h=1.0 / N_GRID, nx=N_GRID, ny=N_GRID, nz=N_GRID, dt=DT, bc_pad=3,
+                                             form=capi.FORM_FAST))
+            x = 0.4 + 0.08 * np.random.default_rng(k).random((n, 3))
+            s.add_particles(capi.material(E, nu, rho, type_), x.astype(np.float32), v0=(1.0, -2.0, 0.5),
+                            volume=0.25 / N_GRID ** 3)
+            out.append(s)
+    batch = capi.Batch(sims, capi.batch_shape(sort_every=3))
+    try:
+        batch.run(7)
+        batch.sync()
+        for s, a in zip(sims, alone):
+            a.run(7)
+            assert s.stats()["active_blocks"] == a.stats()["active_blocks"]
+            assert rel(s.read(0, capi.P_POS), a.read(0, capi.P_POS)) < 2e-6 * 7
+            assert rel(s.read(0, capi.P_VEL), a.read(0, capi.P_VEL)) < 2e-5 * 7
+    finally:
+        batch.close()
+        for s in sims + alone:
+            s.close()
