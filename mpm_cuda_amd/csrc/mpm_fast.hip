@@ -309,27 +309,26 @@ struct RadixResult {
     uint32_t *keys, *vals;
 };
 
-// Sorts (keys, vals) of length n by the low `bits` key bits, ping-ponging
+// Sorts (keys, vals) of length n by `bits` key bits from `low` up, ping-ponging
 // with the *_alt buffers.  `hist` holds 512 x ceil(n / RS_TILE) entries,
 // `totals` RS_MAX_DIGITS.  With hist0_ready the first pass's digit
 // histogram is already in `hist` (radix_digit_bits(bits)-bit digits, written
 // by the caller); with iota_vals the values are the input positions (vals is
-// not read); vals_out, when given (distinct from the other buffers), takes
-// the last pass's values.  res names the sorted keys and values.
+// not read).  res names the sorted keys and values.
 static int radix_sort_ex(hipStream_t st, uint32_t *keys, uint32_t *vals, uint32_t *keys_alt, uint32_t *vals_alt,
                          int n, int bits, uint32_t *hist, uint32_t *totals, bool hist0_ready, bool iota_vals,
-                         uint32_t *vals_out, RadixResult &res)
+                         int low, RadixResult &res)
 {
     res = RadixResult{keys, vals};
     if (n <= 0) return 0;
     const int ntiles = (n + RS_TILE - 1) / RS_TILE;
     uint32_t *ka = keys, *va = vals, *kb = keys_alt, *vb = vals_alt;
     const int db = radix_digit_bits(bits);
-    for (int shift = 0; shift < bits; shift += db) {
-        const bool first = shift == 0, last = shift + db >= bits;
-        const int w = std::min(db, bits - shift);
+    for (int done = 0; done < bits; done += db) {
+        const bool first = done == 0;
+        const int w = std::min(db, bits - done), shift = low + done;
         const uint32_t dmask = (w >= 32) ? ~0u : ((1u << w) - 1u);
-        uint32_t *vdst = (last && vals_out) ? vals_out : vb;
+        uint32_t *vdst = vb;
         const uint32_t *vsrc = (first && iota_vals) ? nullptr : va;
         if (db == 9) {
             if (!(first && hist0_ready))
@@ -356,7 +355,7 @@ static int radix_sort(hipStream_t st, uint32_t *keys, uint32_t *vals, uint32_t *
                       int n, int bits, uint32_t *hist, uint32_t *totals, bool &in_alt)
 {
     RadixResult r{};
-    const int rc = radix_sort_ex(st, keys, vals, keys_alt, vals_alt, n, bits, hist, totals, false, false, nullptr, r);
+    const int rc = radix_sort_ex(st, keys, vals, keys_alt, vals_alt, n, bits, hist, totals, false, false, 0, r);
     in_alt = r.keys != keys;
     return rc;
 }
@@ -365,11 +364,11 @@ static int radix_sort(hipStream_t st, uint32_t *keys, uint32_t *vals, uint32_t *
 // Keys, permutation and tiles.
 //
 // Sort key: linear index of the 4^3-node block holding the particle's base
-// node, above KEY_LOW bits of the base node's position inside the block, so
-// that a block's particles are stored cell by cell: the P2G's counting sort
-// of a chunk by base node then finds them nearly in order, and the item
-// gathers of its phase C read neighbouring particles.  P2G still re-bins
-// every chunk by its particles' current base nodes in LDS.
+// node (of several groups sorted together: their blocks one group's after the
+// other's), above KEY_LOW bits of the base node's position inside the block,
+// which the radix sort leaves alone: the order of a block's particles by cells
+// is made tile by tile afterwards (rank_tile).  (Sorting by them too took a
+// third pass, 20-34 us a sort.)
 constexpr int KEY_LOW = 6;
 
 __device__ __forceinline__ void base_of(const GridP &g, const PartView &pv, int i, int b[3])
@@ -383,14 +382,31 @@ __device__ __forceinline__ void base_of(const GridP &g, const PartView &pv, int 
     }
 }
 
-// Block keys of the particles (linear index of the 4^3-node block holding
-// the base node) of tile `tile` (RS_TILE particles) and the radix sort's
+// The particle groups that one sort takes: the particles of group k are those
+// before end[k] and not before end[k - 1], their blocks the keys
+// [k nblocks, (k + 1) nblocks).
+struct SortGroups {
+    int n, nblocks;
+    uint32_t end[LAUNCH_GROUPS];
+    uint32_t tile_off[LAUNCH_GROUPS];       // first tile slot of the group
+    uint32_t cap[LAUNCH_GROUPS];            // and how many it has
+    __host__ __device__ __forceinline__ uint32_t begin(uint32_t k) const { return k ? end[k - 1] : 0u; }
+    __device__ __forceinline__ uint32_t of(uint32_t i) const
+    {
+        uint32_t k = 0;
+#pragma unroll
+        for (int j = 0; j < LAUNCH_GROUPS - 1; ++j) k += (j < n - 1 && i >= end[j]) ? 1u : 0u;
+        return k;
+    }
+};
+
+// Block keys of the particles of tile `tile` (RS_TILE particles) and the radix sort's
 // first digit histogram (DB-bit digits, dmask the first digit's bits) of
 // the tile, laid out as k_rs_hist writes it; h: 2^DB words of LDS.  Before
 // that, the workgroup clears its share (from `first`, every `stride`) of the
 // nb-entry block arrays z0, z1, z2 that the run and tile kernels fill.
 template <int DB>
-__device__ __forceinline__ void keys_hist_tile(const GridP &g, const PartView &pv, uint32_t *keys, uint32_t dmask,
+__device__ __forceinline__ void keys_hist_tile(const GridP &g, const PartView &pv, const SortGroups &sg, uint32_t *keys, uint32_t dmask,
                                                uint32_t *hist, int ntiles, int tile, uint32_t *z0, uint32_t *z1,
                                                uint32_t *z2, int nb, int first, int stride, uint32_t *h)
 {
@@ -412,24 +428,25 @@ __device__ __forceinline__ void keys_hist_tile(const GridP &g, const PartView &p
         if (valid) {
             int b[3];
             base_of(g, pv, i, b);
-            key = ((((uint32_t)(b[2] >> 2) * (uint32_t)g.nby + (uint32_t)(b[1] >> 2)) * (uint32_t)g.nbx +
-                    (uint32_t)(b[0] >> 2)) << KEY_LOW) |
+            const uint32_t blk = ((uint32_t)(b[2] >> 2) * (uint32_t)g.nby + (uint32_t)(b[1] >> 2)) * (uint32_t)g.nbx +
+                                 (uint32_t)(b[0] >> 2);
+            key = ((sg.of((uint32_t)i) * (uint32_t)sg.nblocks + blk) << KEY_LOW) |
                   (uint32_t)((b[0] & 3) | ((b[1] & 3) << 2) | ((b[2] & 3) << 4));
             keys[i] = key;
         }
-        hist_add(h, valid, key & MASK);
+        hist_add(h, valid, (key >> KEY_LOW) & MASK);
     }
     __syncthreads();
     for (int d = threadIdx.x; d < NB; d += RS_T) hist[(int64_t)d * ntiles + tile] = h[d];
 }
 
 template <int DB>
-__global__ void __launch_bounds__(RS_T) k_block_keys_hist(GridP g, PartView pv, uint32_t *keys, uint32_t dmask,
+__global__ void __launch_bounds__(RS_T) k_block_keys_hist(GridP g, PartView pv, SortGroups sg, uint32_t *keys, uint32_t dmask,
                                                           uint32_t *hist, int ntiles, uint32_t *z0, uint32_t *z1,
                                                           uint32_t *z2, int nb)
 {
     __shared__ uint32_t h[1 << DB];
-    keys_hist_tile<DB>(g, pv, keys, dmask, hist, ntiles, (int)blockIdx.x, z0, z1, z2, nb, (int)blockIdx.x * RS_T,
+    keys_hist_tile<DB>(g, pv, sg, keys, dmask, hist, ntiles, (int)blockIdx.x, z0, z1, z2, nb, (int)blockIdx.x * RS_T,
                        (int)gridDim.x * RS_T, h);
 }
 
@@ -472,61 +489,65 @@ __global__ void k_block_runs(const uint32_t *__restrict__ skeys, int n, uint32_t
     block_run_at(skeys, n, (int)(blockIdx.x * blockDim.x + threadIdx.x), blk_start, blk_end, has);
 }
 
-// Block b's tile: (first particle, count, block, tile id); blk_tile maps the
-// block to its global tile id (staging slot), every arena face marked
-// written until the block's first P2G, or -1 for an empty block.
-__device__ __forceinline__ void emit_tile_at(const uint32_t *blk_start, const uint32_t *blk_end,
-                                             const uint32_t *tile_index, int nblocks, int b, uint4 *desc,
-                                             uint32_t desc_cap, int32_t *blk_tile, uint32_t tile_base)
+// The tile of block key kb (block kb % nblocks of group kb / nblocks): (first
+// particle in its group, count, block, tile id); blk_tile maps the block to
+// its global tile id (staging slot), every arena face marked written until the
+// block's first P2G, or -1 for an empty block.  A group's last block also
+// writes its number of tiles.
+__device__ __forceinline__ void emit_tile_at(const SortGroups &sg, const uint32_t *blk_start, const uint32_t *blk_end,
+                                             const uint32_t *tile_index, int kb, uint4 *desc, int32_t *blk_tile,
+                                             uint32_t *tile_counts)
 {
-    if (b >= nblocks) return;
-    const uint32_t c = blk_end[b] - blk_start[b];
-    const uint32_t t = tile_index[b];
-    if (c > 0 && t < desc_cap) {
-        desc[t] = make_uint4(blk_start[b], c, (uint32_t)b, tile_base + t);
-        blk_tile[b] = tile_entry(tile_base + t, TILE_ALL_FACES);
+    if (kb >= sg.n * sg.nblocks) return;
+    uint32_t k = 0;
+    if (sg.n > 1) k = (uint32_t)kb / (uint32_t)sg.nblocks;
+    const uint32_t k0 = k * (uint32_t)sg.nblocks, b = (uint32_t)kb - k0;
+    const uint32_t c = blk_end[kb] - blk_start[kb];
+    const uint32_t t = tile_index[kb] - tile_index[k0], slot = sg.tile_off[k] + t;
+    if (c > 0 && t < sg.cap[k]) {
+        desc[slot] = make_uint4(blk_start[kb] - sg.begin(k), c, b, slot);
+        blk_tile[kb] = tile_entry(slot, TILE_ALL_FACES);
     } else {
-        blk_tile[b] = -1;
+        blk_tile[kb] = -1;
     }
+    if (b + 1 == (uint32_t)sg.nblocks) tile_counts[k] = t + (c > 0 ? 1u : 0u);
 }
 
-__global__ void k_emit_tiles(const uint32_t *blk_start, const uint32_t *blk_end, const uint32_t *tile_index,
-                             int nblocks, uint4 *desc, uint32_t desc_cap, int32_t *blk_tile, uint32_t tile_base)
+__global__ void k_emit_tiles(SortGroups sg, const uint32_t *blk_start, const uint32_t *blk_end,
+                             const uint32_t *tile_index, uint4 *desc, int32_t *blk_tile, uint32_t *tile_counts)
 {
-    emit_tile_at(blk_start, blk_end, tile_index, nblocks, (int)(blockIdx.x * blockDim.x + threadIdx.x), desc,
-                 desc_cap, blk_tile, tile_base);
+    emit_tile_at(sg, blk_start, blk_end, tile_index, (int)(blockIdx.x * blockDim.x + threadIdx.x), desc, blk_tile,
+                 tile_counts);
 }
 
 // Order of a tile's particles inside its block: one particle of every cell
 // (base node of the block) that has one, in cell order, then the second of
 // every cell that has two, and so on, so that 64 consecutive particles hold
 // mostly different cells and a P2G batch scatters them without turns.  One
-// wave; skeys / sperm are the sorted keys and the stable order, the tile's
-// slots [d.x, d.x + d.y) of perm are written.  Particles past RANK_LEVELS of
-// one cell follow cell by cell.
+// wave; skeys / sperm are the keys and particles in the order of their blocks
+// (particle `first` of a group that begins at `begin` is the tile's first),
+// and the tile's slots of perm are written with indices in the group.
+// Particles past RANK_LEVELS of one cell follow cell by cell.
 constexpr uint32_t RANK_LEVELS = 64;
 struct RankLds {
     uint64_t mask[RANK_LEVELS];     // cells with more than r particles
     uint32_t base[RANK_LEVELS];     // place of the first of them
-    uint32_t begin[64], end[64];    // the cells' runs in the sorted order
+    uint32_t cnt[64];               // particles of the cells, all and then those placed
     uint32_t deep[64];              // place of a cell's particle RANK_LEVELS
 };
 __device__ __forceinline__ void rank_tile(const uint32_t *__restrict__ skeys, const uint32_t *__restrict__ sperm,
-                                          const uint4 d, uint32_t n, uint32_t *__restrict__ perm, RankLds &L)
+                                          uint32_t begin, uint32_t first, uint32_t count, uint32_t n,
+                                          uint32_t *__restrict__ perm, RankLds &L)
 {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t first = d.x, last = min(d.x + d.y, n);
+    first += begin;
+    const uint32_t last = min(first + count, n);
     if (first >= last) return;
-    L.begin[lane] = 0u;
-    L.end[lane] = 0u;
+    L.cnt[lane] = 0u;
     __asm__ volatile("" ::: "memory");      // one wave: its LDS operations execute in order
-    for (uint32_t i = first + lane; i < last; i += 64) {
-        const uint32_t c = skeys[i] & 63u;
-        if (i == first || (skeys[i - 1] & 63u) != c) L.begin[c] = i;
-        if (i + 1 == last || (skeys[i + 1] & 63u) != c) L.end[c] = i + 1;
-    }
+    for (uint32_t i = first + lane; i < last; i += 64) atomicAdd(&L.cnt[skeys[i] & 63u], 1u);
     __asm__ volatile("" ::: "memory");
-    const uint32_t begin = L.begin[lane], cnt = L.end[lane] - begin;
+    const uint32_t cnt = L.cnt[lane];
     uint32_t run = 0;
     for (uint32_t r = 0; r < RANK_LEVELS; ++r) {
         const uint64_t m = __ballot(cnt > r);
@@ -539,32 +560,55 @@ __device__ __forceinline__ void rank_tile(const uint32_t *__restrict__ skeys, co
     }
     const uint32_t rest = cnt > RANK_LEVELS ? cnt - RANK_LEVELS : 0u;
     L.deep[lane] = run + wave_incl_scan(rest) - rest;
+    L.cnt[lane] = 0u;
     __asm__ volatile("" ::: "memory");
-    for (uint32_t i = first + lane; i < last; i += 64) {
-        const uint32_t c = skeys[i] & 63u, r = i - L.begin[c];
-        uint32_t at;
-        if (r < RANK_LEVELS) at = L.base[r] + (uint32_t)__popcll(L.mask[r] & ((1ull << c) - 1ull));
-        else at = L.deep[c] + (r - RANK_LEVELS);
-        perm[first + at] = sperm[i];
+    for (uint32_t i0 = first; i0 < last; i0 += 64) {
+        const uint32_t i = i0 + lane;
+        const bool valid = i < last;
+        const uint32_t c = valid ? skeys[i] & 63u : 0u;
+        uint64_t same = __ballot(valid);        // lanes of the same cell
+#pragma unroll
+        for (int b = 0; b < KEY_LOW; ++b) {
+            const bool bit = (c >> b) & 1u;
+            const uint64_t bb = __ballot(bit);
+            same &= bit ? bb : ~bb;
+        }
+        const uint32_t below = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+        const uint32_t r = L.cnt[c] + below;
+        __asm__ volatile("" ::: "memory");
+        if (valid && below == 0) L.cnt[c] = r + (uint32_t)__popcll(same);
+        __asm__ volatile("" ::: "memory");
+        if (valid) {
+            const uint32_t at = r < RANK_LEVELS ? L.base[r] + (uint32_t)__popcll(L.mask[r] & ((1ull << c) - 1ull))
+                                                : L.deep[c] + (r - RANK_LEVELS);
+            perm[first + at] = sperm[i] - begin;
+        }
     }
 }
 
-// One wave per tile; 10-18 us a sort (262k-2M particles).  The number of
-// tiles goes to a pinned host word for the choice of the P2G's width; the
-// list of blocks that follows starts over.
-__global__ void __launch_bounds__(256) k_rank_tiles(const uint32_t *__restrict__ skeys, const uint32_t *__restrict__ sperm,
-                                                    int n, const uint4 *__restrict__ desc,
-                                                    const uint32_t *__restrict__ tile_count, uint32_t desc_cap,
+// One wave per tile.  The number of tiles of each group goes to a pinned host
+// word for the choice of the P2G's width; the list of blocks that follows
+// starts over.
+__global__ void __launch_bounds__(256) k_rank_tiles(SortGroups sg, const uint32_t *__restrict__ skeys,
+                                                    const uint32_t *__restrict__ sperm, int n,
+                                                    const uint4 *__restrict__ desc,
+                                                    const uint32_t *__restrict__ tile_counts,
                                                     uint32_t *__restrict__ perm, uint32_t *tiles_host,
                                                     uint32_t *counters)
 {
     __shared__ RankLds L[4];
-    const uint32_t w = threadIdx.x >> 6, nt = min(*tile_count, desc_cap);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        __hip_atomic_store(tiles_host, nt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        gp(counters)[CT_LIST] = 0u;
+    const uint32_t w = threadIdx.x >> 6;
+    if (blockIdx.x == 0 && (int)threadIdx.x < sg.n)
+        __hip_atomic_store(tiles_host + threadIdx.x, min(tile_counts[threadIdx.x], sg.cap[threadIdx.x]), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    if (blockIdx.x == 0 && threadIdx.x == 0) gp(counters)[CT_LIST] = 0u;
+    for (uint32_t t0 = blockIdx.x * 4 + w, k = 0; ; t0 += gridDim.x * 4, k = 0) {
+        uint32_t t = t0, nt = 0;
+        for (; k < (uint32_t)sg.n && t >= (nt = min(tile_counts[k], sg.cap[k])); ++k) t -= nt;
+        if (k >= (uint32_t)sg.n) break;
+        const uint4 d = desc[sg.tile_off[k] + t];
+        rank_tile(skeys, sperm, sg.begin(k), d.x, d.y, (uint32_t)n, perm, L[w]);
     }
-    for (uint32_t t = blockIdx.x * 4 + w; t < nt; t += gridDim.x * 4) rank_tile(skeys, sperm, desc[t], (uint32_t)n, perm, L[w]);
 }
 
 // ---------------------------------------------------------------------------
@@ -588,6 +632,17 @@ __device__ __forceinline__ bool bsort_locate(const SortSlice *__restrict__ tab, 
     return true;
 }
 
+__device__ __forceinline__ SortGroups scene_group(const SortSlice &t)
+{
+    SortGroups sg;
+    sg.n = 1;
+    sg.nblocks = t.nblocks;
+    sg.end[0] = (uint32_t)t.n;
+    sg.tile_off[0] = 0u;
+    sg.cap[0] = t.desc_cap;
+    return sg;
+}
+
 __global__ void __launch_bounds__(RS_T) k_bsort_keys(const SortSlice *__restrict__ tab, int ns)
 {
     __shared__ uint32_t h[1 << BS_DB];
@@ -595,7 +650,7 @@ __global__ void __launch_bounds__(RS_T) k_bsort_keys(const SortSlice *__restrict
     int tile;
     if (!bsort_locate(tab, ns, [&](int s) { return (uint32_t)tab[s].ntiles; }, sid, tile)) return;
     const SortSlice &t = tab[sid];
-    keys_hist_tile<BS_DB>(t.g, t.pv, t.keys, 0xFFu, t.hist, t.ntiles, tile, t.blk_start, t.blk_end, t.has, t.nblocks,
+    keys_hist_tile<BS_DB>(t.g, t.pv, scene_group(t), t.keys, 0xFFu, t.hist, t.ntiles, tile, t.blk_start, t.blk_end, t.has, t.nblocks,
                           tile * RS_T, t.ntiles * RS_T, h);
 }
 
@@ -606,7 +661,7 @@ __global__ void __launch_bounds__(RS_T) k_bsort_hist(const SortSlice *__restrict
     int tile;
     if (!bsort_locate(tab, ns, [&](int s) { return (uint32_t)tab[s].ntiles; }, sid, tile)) return;
     const SortSlice &t = tab[sid];
-    rs_hist_tile<BS_DB>((pass & 1) ? t.keys_alt : t.keys, t.n, BS_DB * pass, 0xFFu, t.hist, t.ntiles, tile, h);
+    rs_hist_tile<BS_DB>((pass & 1) ? t.keys_alt : t.keys, t.n, KEY_LOW + BS_DB * pass, 0xFFu, t.hist, t.ntiles, tile, h);
 }
 
 // Four digit columns per workgroup, one per wave.
@@ -632,7 +687,7 @@ __global__ void __launch_bounds__(RS_T) k_bsort_scatter(const SortSlice *__restr
     const bool odd = (pass & 1) != 0;
     const uint32_t *vin = pass == 0 ? nullptr : (odd ? t.vals_alt : t.vals);
     uint32_t *vout = odd ? t.vals : t.vals_alt;
-    rs_scatter_tile<BS_DB>(odd ? t.keys_alt : t.keys, vin, odd ? t.keys : t.keys_alt, vout, t.n, BS_DB * pass, 0xFFu,
+    rs_scatter_tile<BS_DB>(odd ? t.keys_alt : t.keys, vin, odd ? t.keys : t.keys_alt, vout, t.n, KEY_LOW + BS_DB * pass, 0xFFu,
                            t.hist, t.scan, t.ntiles, tile, cnt, lds);
 }
 
@@ -668,7 +723,7 @@ __global__ void __launch_bounds__(SCAN_T) k_bsort_scan_apply(const SortSlice *__
                       wg))
         return;
     const SortSlice &t = tab[sid];
-    scan_apply_wg(t.has, t.has, t.nblocks, t.scan, t.tile_count, wg, lds, &wg_base);
+    scan_apply_wg(t.has, t.has, t.nblocks, t.scan, nullptr, wg, lds, &wg_base);
 }
 
 // Tiles, and the warm-start list counts cleared (their lists name old slots).
@@ -680,8 +735,8 @@ __global__ void __launch_bounds__(256) k_bsort_emit(const SortSlice *__restrict_
     const SortSlice &t = tab[sid];
     if (q == 0 && t.warm_cnt)
         for (int j = (int)threadIdx.x; j < 2 * MAX_GROUPS; j += 256) t.warm_cnt[j] = 0u;
-    emit_tile_at(t.blk_start, t.blk_end, t.has, t.nblocks, q * 256 + (int)threadIdx.x, t.desc, t.desc_cap, t.blk_tile,
-                 0u);
+    emit_tile_at(scene_group(t), t.blk_start, t.blk_end, t.has, q * 256 + (int)threadIdx.x, t.desc, t.blk_tile,
+                 t.tile_count);
 }
 
 // The tiles' particle orders (rank_tile) into the scenes' permutations, one
@@ -697,7 +752,7 @@ __global__ void __launch_bounds__(256) k_bsort_rank(const SortSlice *__restrict_
         const uint32_t sid = (uint32_t)__builtin_amdgcn_readfirstlane((int)sc.find(k));
         const SortSlice &t = tab[sid];
         const uint4 d = gload_u4(t.desc, k - sc.start(sid));
-        rank_tile(alt ? t.keys_alt : t.keys, alt ? t.vals_alt : t.vals, d, (uint32_t)t.n, t.perm, L[w]);
+        rank_tile(alt ? t.keys_alt : t.keys, alt ? t.vals_alt : t.vals, 0u, d.x, d.y, (uint32_t)t.n, t.perm, L[w]);
     }
 }
 
@@ -1639,30 +1694,58 @@ static inline int nblk(int64_t n, int t) { return (int)((n + t - 1) / t); }
 
 static int64_t tile_bound(const mpm_sim *s, int64_t n) { return std::min<int64_t>(s->nblocks, n); }
 
+// Groups that one sort takes from group k on: up to LAUNCH_GROUPS whose
+// particles follow one another, with block arrays of no more than 2^22
+// entries (16 MB each), or one group.  Three groups of 100k on 128^3 nodes:
+// 248 us of sort kernels apart, 73 together.
+static int sort_groups_at(const mpm_sim *s, int k)
+{
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>(LAUNCH_GROUPS, ((int64_t)1 << 22) / s->nblocks));
+    int n = 1;
+    while (n < most && k + n < (int)s->groups.size() &&
+           s->groups[k + n].off == s->groups[k + n - 1].off + s->groups[k + n - 1].n)
+        ++n;
+    return n;
+}
+
 static int ensure_fast_buffers(mpm_sim *s)
 {
     if (s->groups.size() > 256) return set_error(MPM_ERR_INVALID, "at most 256 particle groups");
-    int64_t nmax = 0;
-    for (auto &gi : s->groups) nmax = std::max(nmax, gi.n);
+    // sizes of the largest of the sorts that take all groups
+    int64_t nmax = 0, kblocks = s->nblocks;
+    for (int k = 0, n; k < (int)s->groups.size(); k += n) {
+        n = sort_groups_at(s, k);
+        int64_t sum = 0;
+        for (int j = k; j < k + n; ++j) sum += s->groups[j].n;
+        nmax = std::max(nmax, sum);
+        kblocks = std::max(kblocks, n * s->nblocks);
+    }
     if (!s->keys || s->sort_hist_len < nmax) {
-        void *ptrs[] = {s->keys, s->keys_alt, s->vals, s->vals_alt, s->sort_hist, s->sort_scan};
+        void *ptrs[] = {s->keys, s->keys_alt, s->vals, s->vals_alt, s->sort_hist};
         for (void *p : ptrs) if (p) (void)hipFree(p);
         int64_t ntiles = (nmax + RS_TILE - 1) / RS_TILE;
         int64_t hist_len = 512 * ntiles;     // digits of up to 9 bits
-        // scan partials of the tile numbering, or the radix digit totals
-        int64_t scan_words = std::max<int64_t>(RS_MAX_DIGITS, (s->nblocks + SCAN_TILE - 1) / SCAN_TILE + 16);
         MPM_HIP(hipMalloc(&s->keys, nmax * 4));
         MPM_HIP(hipMalloc(&s->keys_alt, nmax * 4));
         MPM_HIP(hipMalloc(&s->vals, nmax * 4));
         MPM_HIP(hipMalloc(&s->vals_alt, nmax * 4));
         MPM_HIP(hipMalloc(&s->sort_hist, hist_len * 4));
-        MPM_HIP(hipMalloc(&s->sort_scan, scan_words * 4));
         s->sort_hist_len = nmax;
     }
-    if (!s->blk_count) {
-        MPM_HIP(hipMalloc(&s->blk_count, s->nblocks * 4));
-        MPM_HIP(hipMalloc(&s->blk_start, s->nblocks * 4));
-        MPM_HIP(hipMalloc(&s->scan_tmp, s->nblocks * 4));
+    if (s->sort_blocks < kblocks) {
+        void **ptrs[] = {(void **)&s->blk_count, (void **)&s->blk_start, (void **)&s->scan_tmp, (void **)&s->sort_scan};
+        for (void **p : ptrs) {
+            if (*p) (void)hipFree(*p);
+            *p = nullptr;
+        }
+        s->sort_blocks = 0;
+        // scan partials of the tile numbering, or the radix digit totals
+        const int64_t scan_words = std::max<int64_t>(RS_MAX_DIGITS, (kblocks + SCAN_TILE - 1) / SCAN_TILE + 16);
+        MPM_HIP(hipMalloc(&s->blk_count, kblocks * 4));
+        MPM_HIP(hipMalloc(&s->blk_start, kblocks * 4));
+        MPM_HIP(hipMalloc(&s->scan_tmp, kblocks * 4));
+        MPM_HIP(hipMalloc(&s->sort_scan, scan_words * 4));
+        s->sort_blocks = kblocks;
     }
     if (!s->spill && s->cfg.form == MPM_FORM_FUSED) MPM_HIP(hipMalloc(&s->spill, s->cap * sizeof(uint32_t)));
     int64_t need = 0;
@@ -1701,8 +1784,6 @@ int sort_all(mpm_sim *s, bool defer)
     int rc = ensure_fast_buffers(s);
     if (rc) return rc;
     hipStream_t st = s->stream;
-    int bits = KEY_LOW + 1;
-    while ((1ll << (bits - KEY_LOW)) < s->nblocks) ++bits;
     uint64_t plane_mask = (1ull << PL_COUNT) - 1ull;
     if (!s->tau_valid) plane_mask &= ~(((1ull << 6) - 1ull) << PL_TAU);
     if (defer && s->g2p_perm_cap < s->cap) {
@@ -1719,24 +1800,41 @@ int sort_all(mpm_sim *s, bool defer)
     if (!s->warm_cnt) plane_mask &= ~(((1ull << 4) - 1ull) << PL_Q);
     else if (!defer && (rc = launch_zero_u32(st, s->warm_cnt, 2 * MAX_GROUPS))) return hip_fail((hipError_t)rc, "zero");
     const int nb = (int)s->nblocks;
-    const int db = radix_digit_bits(bits);
-    const uint32_t dmask0 = (1u << std::min(db, bits)) - 1u;
-    for (size_t k = 0; k < s->groups.size(); ++k) {
-        PartView pv = view_of(s, (int)k);
-        int n = pv.n;
+    for (int k = 0, ng; k < (int)s->groups.size(); k += ng) {
+        ng = sort_groups_at(s, k);
+        // the groups as one range of particles
+        PartView pv = view_of(s, k);
+        SortGroups sg{};
+        sg.n = ng;
+        sg.nblocks = nb;
+        int64_t sum = 0;
+        uint32_t bound = 0;
+        for (int j = 0; j < ng; ++j) {
+            sum += s->groups[k + j].n;
+            sg.end[j] = (uint32_t)sum;
+            sg.tile_off[j] = (uint32_t)s->group_tile_off[k + j];
+            sg.cap[j] = (uint32_t)tile_bound(s, s->groups[k + j].n);
+            bound += sg.cap[j];
+        }
+        pv.n = (int)sum;
+        const int n = pv.n, nk = ng * nb;
+        int bits = 1;
+        while ((1ll << bits) < nk) ++bits;
+        const int db = radix_digit_bits(bits);
+        const uint32_t dmask0 = (1u << std::min(db, bits)) - 1u;
         uint32_t *blk_end = s->blk_count;
         // keys, first digit histogram, cleared block arrays; the sort's
         // values are the particles' current slots
         const int ntiles = nblk(n, RS_TILE);
         if (db == 9)
-            hipLaunchKernelGGL(k_block_keys_hist<9>, dim3(ntiles), dim3(RS_T), 0, st, s->g, pv, s->keys, dmask0,
-                               s->sort_hist, ntiles, s->blk_start, blk_end, s->scan_tmp, nb);
+            hipLaunchKernelGGL(k_block_keys_hist<9>, dim3(ntiles), dim3(RS_T), 0, st, s->g, pv, sg, s->keys, dmask0,
+                               s->sort_hist, ntiles, s->blk_start, blk_end, s->scan_tmp, nk);
         else
-            hipLaunchKernelGGL(k_block_keys_hist<8>, dim3(ntiles), dim3(RS_T), 0, st, s->g, pv, s->keys, dmask0,
-                               s->sort_hist, ntiles, s->blk_start, blk_end, s->scan_tmp, nb);
+            hipLaunchKernelGGL(k_block_keys_hist<8>, dim3(ntiles), dim3(RS_T), 0, st, s->g, pv, sg, s->keys, dmask0,
+                               s->sort_hist, ntiles, s->blk_start, blk_end, s->scan_tmp, nk);
         RadixResult r{};
         if ((rc = radix_sort_ex(st, s->keys, s->vals, s->keys_alt, s->vals_alt, n, bits, s->sort_hist, s->sort_scan,
-                                true, true, nullptr, r)))
+                                true, true, KEY_LOW, r)))
             return hip_fail((hipError_t)rc, "radix_sort");
         // a deferred order is left for the G2P; the other one needs only a
         // buffer the radix sort is done with
@@ -1745,17 +1843,18 @@ int sort_all(mpm_sim *s, bool defer)
         // tiles: one per non-empty block, numbered in block order
         hipLaunchKernelGGL(k_block_runs, dim3(nblk(n, 256)), dim3(256), 0, st, skeys, n, s->blk_start, blk_end,
                            s->scan_tmp);
-        if ((rc = scan_excl(st, s->scan_tmp, s->scan_tmp, nb, s->sort_scan, s->tile_counts + k)))
+        if ((rc = scan_excl(st, s->scan_tmp, s->scan_tmp, nk, s->sort_scan, nullptr)))
             return hip_fail((hipError_t)rc, "scan");
-        hipLaunchKernelGGL(k_emit_tiles, dim3(nblk(nb, 256)), dim3(256), 0, st, s->blk_start, blk_end, s->scan_tmp,
-                           nb, (uint4 *)s->tile_desc + s->group_tile_off[k], (uint32_t)tile_bound(s, n),
-                           s->blk_tile + (int64_t)k * nb, (uint32_t)s->group_tile_off[k]);
-        const uint32_t bound = (uint32_t)tile_bound(s, n);
-        hipLaunchKernelGGL(k_rank_tiles, dim3(std::min<uint32_t>((bound + 3) / 4, 2048u)), dim3(256), 0, st, skeys, r.vals, n,
-                           (const uint4 *)s->tile_desc + s->group_tile_off[k], s->tile_counts + k, bound, perm, s->tiles_host + k, s->counters);
+        hipLaunchKernelGGL(k_emit_tiles, dim3(nblk(nk, 256)), dim3(256), 0, st, sg, s->blk_start, blk_end, s->scan_tmp,
+                           (uint4 *)s->tile_desc, s->blk_tile + (int64_t)k * nb, s->tile_counts + k);
+        hipLaunchKernelGGL(k_rank_tiles, dim3(std::min<uint32_t>((bound + 3) / 4, 2048u)), dim3(256), 0, st, sg, skeys, r.vals,
+                           n, (const uint4 *)s->tile_desc, s->tile_counts + k, perm, s->tiles_host + k, s->counters);
         if (!defer)
-            hipLaunchKernelGGL(k_permute, dim3(round_xcd((uint32_t)nblk(n, 256))), dim3(256), 0, st, s->P, s->P_alt,
-                               s->cap, pv.off, n, perm, s->pid, s->pid_alt, plane_mask);
+            for (int j = 0; j < ng; ++j) {
+                const PartView v = view_of(s, k + j);
+                hipLaunchKernelGGL(k_permute, dim3(round_xcd((uint32_t)nblk(v.n, 256))), dim3(256), 0, st, s->P, s->P_alt,
+                                   s->cap, v.off, v.n, perm + sg.begin((uint32_t)j), s->pid, s->pid_alt, plane_mask);
+            }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "sort kernels");
     }
@@ -2169,8 +2268,8 @@ void sort_batch_plan(mpm_sim *const *sims, int ns, SortBatchPlan &pl)
     pl = SortBatchPlan{};
     for (int k = 0; k < ns; ++k) {
         const mpm_sim *s = sims[k];
-        int bits = KEY_LOW + 1;
-        while ((1ll << (bits - KEY_LOW)) < s->nblocks) ++bits;
+        int bits = 1;
+        while ((1ll << bits) < s->nblocks) ++bits;
         pl.passes = std::max(pl.passes, (bits + BS_DB - 1) / BS_DB);
         const int64_t n = s->groups[0].n;
         pl.tiles += nblk(n, RS_TILE);

@@ -449,6 +449,7 @@ struct mpm_sim {
     uint32_t *keys = nullptr, *keys_alt = nullptr, *vals = nullptr, *vals_alt = nullptr;
     uint32_t *sort_hist = nullptr, *sort_scan = nullptr;
     int64_t sort_hist_len = 0;
+    int64_t sort_blocks = 0;                // entries of the block arrays below
     uint32_t *blk_count = nullptr, *blk_start = nullptr, *tile_desc = nullptr, *scan_tmp = nullptr;
     int64_t tile_cap = 0;
     std::vector<int64_t> group_tile_off;    // per group: first tile slot
