@@ -346,6 +346,7 @@ int mpm_step_phase(mpm_sim *s, int32_t phase, double dt)
     // single phases always take the given dt; the controller re-reduces its
     // maxima at the next full step
     s->dt_valid = false;
+    s->rule = DtRule{};
     const float *dtp = s->g.dtp;
     s->g.dtp = nullptr;
     int rc = run_phase(s, phase, fdt);
@@ -365,9 +366,9 @@ static int dt_control(mpm_sim *s, double max_dt)
             rc = check_launch(launch_dt_scan(s->stream, s->groups[k].mat, view_of(s, (int)k), s->counters), "dt_scan");
         if (rc) return rc;
     }
-    rc = check_launch(launch_dt_control(s->stream, s->dtc, s->counters, (float)max_dt,
-                                        (float)(s->cfg.cfl * s->cfg.h), s->cfg.dt_mode),
-                      "dt_control");
+    const DtRule rule{s->dtc, (float)max_dt, (float)(s->cfg.cfl * s->cfg.h), s->cfg.dt_mode, 1};
+    if (s->cfg.form == MPM_FORM_FAST && s->total > 0) s->rule = rule;         // the P2G's own
+    else rc = check_launch(launch_dt_control(s->stream, rule, s->counters), "dt_control");
     if (!rc) s->dt_valid = true;        // this step's G2P reduces the maxima of the state it writes
     return rc;
 }
@@ -855,9 +856,10 @@ static int run_phase(mpm_sim *s, int phase, float dt)
             rc = check_launch(launch_grid_update(s->stream, s->g, dt, s->list, s->flags, s->act, s->act_seq, s->counters,
                                                  s->grid_mp, s->grid_v, s->nblocks, staged ? s->staging : nullptr,
                                                  staged ? s->blk_tile : nullptr, (int)s->groups.size(),
-                                                 (uint32_t)s->staging_cap, count, seq, launch),
+                                                 (uint32_t)s->staging_cap, count, seq, launch, s->maxima_read ? 1 : 0),
                               "grid_update");
             if (rc) return rc;
+            s->maxima_read = false;
             s->counters_clean = true;
         }
         if (s->timing)

@@ -109,6 +109,8 @@ enum Counter : int {
 // CT_FALLBACK, CT_REJECT, CT_SVD, CT_WARM (summed when read) and CT_SPEED,
 // CT_DEFORM (their maximum) live in CT_SPREAD copies of the line, one a
 // workgroup (see spread).
+// The maxima use the first CT_MAXIMA copies only: a wave reads them at once.
+constexpr int CT_MAXIMA = 64;
 constexpr int CT_SPREAD = 256, CT_WORDS = CT_COUNT * (1 + CT_SPREAD);
 
 // A grid block's entry in `flags`: marked by the P2G, cleared by the grid
@@ -248,6 +250,35 @@ __device__ __forceinline__ uint32_t *spread(uint32_t *counters)
     return counters + CT_COUNT * (1 + (int)(blockIdx.x % CT_SPREAD));
 }
 
+// The same for the step-size controller's maxima.
+__device__ __forceinline__ uint32_t *spread_maxima(uint32_t *counters)
+{
+    return counters + CT_COUNT * (1 + (int)(blockIdx.x % CT_MAXIMA));
+}
+
+// Step-size control: the step's dt from the maxima.
+struct DtRule {
+    DtCtl *ctl;             // null: no control in this launch
+    float max_dt, cfl_h;
+    int mode, advance;      // advance: this launch also writes the state (dt, clock)
+};
+__device__ __forceinline__ float control_dt(const DtRule &r, float speed, float deform)
+{
+    float dt = r.max_dt;
+    if (speed > 0.0f) dt = fminf(dt, r.cfl_h / speed);
+    if (r.mode == MPM_DT_CFL_DEFORM) {
+        const float f = fminf(10.0f, fmaxf(1.0f, deform * deform * deform));
+        dt = fminf(dt, r.max_dt / f);
+    }
+    return dt;
+}
+__device__ __forceinline__ void advance_clock(DtCtl *c, float dt)
+{
+    gp(c)->dt = dt;
+    gp(c)->last = (double)dt;
+    gp(c)->time = gp(c)->time + (double)dt;
+}
+
 // Workgroups are dispatched to the 8 XCDs of the device round-robin
 // (workgroup id k runs on XCD k % 8), and each XCD has its own L2.  Work item
 // xcd_spread(k, n8) gives every XCD a contiguous eighth of [0, n8), so
@@ -293,6 +324,7 @@ struct P2GArgs {
     uint32_t staging_cap;
     float4 *staging, *grid;
     uint32_t *flags, *list, *counters;
+    DtRule rule;
     int ngroups;
     P2GGroup grp[LAUNCH_GROUPS];
 };
@@ -506,6 +538,8 @@ struct mpm_sim {
     // step-size controller (cfg.dt_mode != MPM_DT_FIXED)
     mpm::DtCtl *dtc = nullptr;
     bool dt_valid = false;                  // counters hold the maxima of the current state
+    mpm::DtRule rule{};                     // FAST form: the coming P2G's (ctl null: none), its maxima
+    bool maxima_read = false;               // read and to be cleared by the grid update
     double last_dt = 0;                     // fixed mode: dt of the last step
     // phase timing (HIP events on `stream`): ids 0-3 phases, 4-7 kernels
     static constexpr int TIMED_IDS = 8;

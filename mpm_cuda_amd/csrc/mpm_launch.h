@@ -18,7 +18,7 @@ int launch_bsort_list(hipStream_t st, const SortSlice *tab, int ns, int wgs);
 int launch_grid_update(hipStream_t st, const GridP &g, float dt, const uint32_t *list, uint32_t *flags, uint32_t *act,
                        uint32_t seq, uint32_t *counters, float4 *gmp, float4 *gv, int64_t nblocks,
                        const float4 *staging, const int32_t *blk_tile, int ngroups, uint32_t staging_cap,
-                       uint32_t *host_count, uint32_t *host_seq, uint32_t launch);
+                       uint32_t *host_count, uint32_t *host_seq, uint32_t launch, int clear_maxima);
 // A G2P that applies a re-sort: slot j of po receives particle perm[j] of
 // the view, its id (pid -> pid_out) and, with copy_q, its quaternion.
 struct G2PMove {
@@ -37,7 +37,7 @@ int launch_p2g_spill(hipStream_t st, const GridP &g, const MatP &m, const PartVi
                      uint32_t *host_count, uint32_t *host_seq, uint32_t seq);
 int launch_dt_scan(hipStream_t st, const MatP &m, const PartView &pv, uint32_t *counters);
 int launch_dt_clear(hipStream_t st, uint32_t *counters);
-int launch_dt_control(hipStream_t st, DtCtl *c, uint32_t *counters, float max_dt, float cfl_h, int mode);
+int launch_dt_control(hipStream_t st, const DtRule &rule, uint32_t *counters);
 
 // FAST form (mpm_fast.hip)
 int fast_prepare(mpm_sim *s);                 // (re)sort particles and build P2G tiles when due

@@ -161,8 +161,13 @@ __global__ void __launch_bounds__(64) k_grid_update(GridP g, float dt, const uin
                                                     float4 *gv, const float4 *__restrict__ staging,
                                                     const int32_t *__restrict__ blk_tile, int ngroups,
                                                     uint32_t staging_cap, int64_t nblocks, uint32_t *host_count,
-                                                    uint32_t *host_seq, uint32_t launch)
+                                                    uint32_t *host_seq, uint32_t launch, int clear_maxima)
 {
+    if (clear_maxima && blockIdx.x == 0) {
+        static_assert(CT_MAXIMA == 64, "one copy per thread");
+        gp(counters)[CT_COUNT * (1 + (int)threadIdx.x) + CT_SPEED] = 0u;
+        gp(counters)[CT_COUNT * (1 + (int)threadIdx.x) + CT_DEFORM] = 0u;
+    }
     const uint32_t n = counters[CT_LIST], n8 = round_xcd(n);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         const uint32_t spilled = gp(counters)[CT_SPILL];
@@ -358,8 +363,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kG2pWa
     dt = step_dt(g, dt);
     float sd[2] = {0.0f, 0.0f};
     if (j < pv.n) g2p_particle<MAT>(g, mat, pv, i, out, j, dt, gv, write_tau != 0, sweeps, counters, sd);
-    wave_max_to(spread(counters) + CT_SPEED, sd[0]);
-    wave_max_to(spread(counters) + CT_DEFORM, sd[1]);
+    wave_max_to(spread_maxima(counters) + CT_SPEED, sd[0]);
+    wave_max_to(spread_maxima(counters) + CT_DEFORM, sd[1]);
 }
 
 // The FAST-form G2P of several groups in one launch, each group's particles in
@@ -400,8 +405,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
         }
     }
     if (!CTL) return;
-    wave_max_to(spread(a.counters) + CT_SPEED, sd[0]);
-    wave_max_to(spread(a.counters) + CT_DEFORM, sd[1]);
+    wave_max_to(spread_maxima(a.counters) + CT_SPEED, sd[0]);
+    wave_max_to(spread_maxima(a.counters) + CT_DEFORM, sd[1]);
 }
 
 int launch_g2p_groups(hipStream_t st, const G2PArgs &a, uint32_t wgs, int threads, bool move)
@@ -584,11 +589,11 @@ int launch_bsort_list(hipStream_t st, const SortSlice *tab, int ns, int wgs)
 int launch_grid_update(hipStream_t st, const GridP &g, float dt, const uint32_t *list, uint32_t *flags, uint32_t *act,
                        uint32_t seq, uint32_t *counters, float4 *gmp, float4 *gv, int64_t nblocks,
                        const float4 *staging, const int32_t *blk_tile, int ngroups, uint32_t staging_cap,
-                       uint32_t *host_count, uint32_t *host_seq, uint32_t launch)
+                       uint32_t *host_count, uint32_t *host_seq, uint32_t launch, int clear_maxima)
 {
     hipLaunchKernelGGL(ngroups > 1 ? k_grid_update<4> : k_grid_update<1>, dim3((uint32_t)std::min<int64_t>(nblocks, 8192)), dim3(64), 0, st, g, dt, list,
                        flags, act, seq, counters, gmp, gv, staging, blk_tile, ngroups, staging_cap, nblocks, host_count,
-                       host_seq, launch);
+                       host_seq, launch, clear_maxima);
     return (int)hipGetLastError();
 }
 
@@ -693,8 +698,8 @@ __global__ void __launch_bounds__(256) k_dt_scan(MatP mat, PartView pv, uint32_t
         }
         dt_measures<MAT>(mat, v, J, sd[0], sd[1]);
     }
-    wave_max_to(spread(counters) + CT_SPEED, sd[0]);
-    wave_max_to(spread(counters) + CT_DEFORM, sd[1]);
+    wave_max_to(spread_maxima(counters) + CT_SPEED, sd[0]);
+    wave_max_to(spread_maxima(counters) + CT_DEFORM, sd[1]);
 }
 
 //
@@ -708,7 +713,7 @@ __global__ void __launch_bounds__(CT_SPREAD) k_dt_clear(uint32_t *counters)
     gp(own)[CT_DEFORM] = 0u;
 }
 
-__global__ void __launch_bounds__(CT_SPREAD) k_dt_control(DtCtl *c, uint32_t *counters, float max_dt, float cfl_h, int mode)
+__global__ void __launch_bounds__(CT_SPREAD) k_dt_control(DtRule rule, uint32_t *counters)
 {
     __shared__ float part[2][CT_SPREAD / 64];
     uint32_t *own = counters + CT_COUNT * (1 + threadIdx.x);
@@ -731,15 +736,7 @@ __global__ void __launch_bounds__(CT_SPREAD) k_dt_control(DtCtl *c, uint32_t *co
         speed = fmaxf(speed, part[0][w]);
         deform = fmaxf(deform, part[1][w]);
     }
-    float dt = max_dt;
-    if (speed > 0.0f) dt = fminf(dt, cfl_h / speed);
-    if (mode == MPM_DT_CFL_DEFORM) {
-        const float f = fminf(10.0f, fmaxf(1.0f, deform * deform * deform));
-        dt = fminf(dt, max_dt / f);
-    }
-    gp(c)->dt = dt;
-    gp(c)->last = (double)dt;
-    gp(c)->time = gp(c)->time + (double)dt;
+    advance_clock(rule.ctl, control_dt(rule, speed, deform));
 }
 
 int launch_dt_clear(hipStream_t st, uint32_t *counters)
@@ -760,9 +757,9 @@ int launch_dt_scan(hipStream_t st, const MatP &m, const PartView &pv, uint32_t *
     return (int)hipGetLastError();
 }
 
-int launch_dt_control(hipStream_t st, DtCtl *c, uint32_t *counters, float max_dt, float cfl_h, int mode)
+int launch_dt_control(hipStream_t st, const DtRule &rule, uint32_t *counters)
 {
-    hipLaunchKernelGGL(k_dt_control, dim3(1), dim3(CT_SPREAD), 0, st, c, counters, max_dt, cfl_h, mode);
+    hipLaunchKernelGGL(k_dt_control, dim3(1), dim3(CT_SPREAD), 0, st, rule, counters);
     return (int)hipGetLastError();
 }
 
