@@ -125,6 +125,7 @@ static MatP make_matp(const mpm_material &m, double mass, double vol)
     p.xi = (float)m.xi;
     p.eos_k = (float)m.eos_k;
     p.eos_gamma = (float)m.eos_gamma;
+    if (p.eos_gamma >= 1.0f && p.eos_gamma <= 32.0f && p.eos_gamma == std::floor(p.eos_gamma)) p.eos_n = (int)p.eos_gamma;
     p.warm_sweeps = 0;
     p.polar_steps = polar_steps_for_band(1.0 - m.theta_c, 1.0 + m.theta_s);
     // squared wave speed at rest for the step-size controller: P waves

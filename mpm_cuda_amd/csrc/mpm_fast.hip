@@ -1270,7 +1270,7 @@ __device__ __forceinline__ void tile_end(const GridP &g, const TileGeo &t, const
 // Water: dt V p J / h of a particle.
 __device__ __forceinline__ float water_force(const MatP &mat, const GridP &g, float dt, float J)
 {
-    const float pr = mat.eos_k * (powf(J, -mat.eos_gamma) - 1.0f);   // MPMCUDA.cu:353
+    const float pr = eos_pressure(mat, J);
     return dt * mat.vol * pr * J * g.inv_h;
 }
 

@@ -301,7 +301,7 @@ __device__ __forceinline__ void scatter_from_out(const MatP &mat, const G2POut &
 #pragma unroll
     for (int k = 0; k < 9; ++k) sc.B[k] = mat.mass * o.C[k];
     if (MAT == MPM_WATER) {
-        float pr = mat.eos_k * (powf(o.S, -mat.eos_gamma) - 1.0f);      // MPMCUDA.cu:353
+        float pr = eos_pressure(mat, o.S);
         float c = dt * mat.vol * pr * o.S;
 #pragma unroll
         for (int k = 0; k < 9; ++k) sc.G[k] = (k % 4 == 0) ? c : 0.0f;

@@ -65,6 +65,7 @@ struct MatP {
     float mass, vol, mu, lam;
     float theta_c, theta_s, xi;
     float eos_k, eos_gamma;
+    int eos_n = 0;      // eos_gamma when it is a whole number from 1 to 32, else 0
     int warm_sweeps;    // > 0: G2P SVDs start from the stored quaternion (PL_Q) with this many sweeps
     float c2;           // squared elastic wave speed at rest: (lam + 2 mu) / rho, water k gamma / rho
     // Newton steps of the polar rotation on the snow elastic path (singular

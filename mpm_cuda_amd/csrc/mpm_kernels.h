@@ -148,6 +148,23 @@ __device__ __forceinline__ uint32_t base_only(const GridP &g, const float x[3], 
     return bits;
 }
 
+// Water pressure k (J^-gamma - 1) (MPMCUDA.cu:353).  A whole gamma as FP64
+// products and one division: exact to FP32 rounding also where J^-gamma is
+// near 1, and a fraction of powf's instructions (the P2G of 2M particles of water
+// with gamma 7: 130.5 us with powf, 125.5 so).
+__device__ __forceinline__ float eos_pressure(const MatP &m, float J)
+{
+    if (m.eos_n > 0) {
+        double r = 1.0, b = (double)J;
+        for (int e = m.eos_n; e; e >>= 1) {
+            if (e & 1) r *= b;
+            b *= b;
+        }
+        return m.eos_k * (float)(1.0 / r - 1.0);
+    }
+    return m.eos_k * (powf(J, -m.eos_gamma) - 1.0f);
+}
+
 // FP32 SVD with the FP64 fallback for ill-conditioned / inverted F.
 __device__ __forceinline__ void svd_checked(const float F[9], float U[9], float s[3], float V[9],
                                             int sweeps, uint32_t *counters)
@@ -260,7 +277,7 @@ __device__ __forceinline__ void load_scatter(const PartView &pv, int i, const Ma
     for (int k = 0; k < 9; ++k) sc.B[k] = mat.mass * ld(pv, PL_C + k, i);
     if (MAT == MPM_WATER) {
         float J = ld(pv, PL_S, i);
-        float pr = mat.eos_k * (powf(J, -mat.eos_gamma) - 1.0f);   // MPMCUDA.cu:353
+        float pr = eos_pressure(mat, J);
         float c = dt * mat.vol * pr * J;
 #pragma unroll
         for (int k = 0; k < 9; ++k) sc.G[k] = (k % 4 == 0) ? c : 0.0f;

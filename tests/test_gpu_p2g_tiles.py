@@ -57,3 +57,17 @@ def test_p2g_tile_sizes(gpu, monkeypatch, type_, counts, one_cell, fast):
         assert p.gpu.stats()["tiles"] == len(counts)
     finally:
         p.close()
+
+
+@pytest.mark.parametrize("gamma", [1.0, 2.0, 7.0, 32.0, 33.0, 2.5, 0.5])
+@pytest.mark.parametrize("form", [capi.FORM_PLAIN, capi.FORM_FAST])
+def test_water_pressure_exponents(gpu, form, gamma):
+    """Whole exponents (products) and others (powf); the parity tests' bar."""
+    p = Pair(type_=capi.WATER, form=form, seed=4, eos_gamma=gamma)
+    try:
+        p.gpu.phase(capi.PHASE_P2G, p.dt)
+        p.orc.clear_grid()
+        assert p.orc.p2g(p.dt) == 0
+        assert rel(p.gpu.grid(capi.G_MOMENTUM), p.orc.grid_vec()) < 1e-5
+    finally:
+        p.close()
