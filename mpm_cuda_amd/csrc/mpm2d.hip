@@ -495,6 +495,10 @@ int mpm2d_add_particles(mpm2d_sim *s, int64_t n, const float *xy, const float *v
     s->cap = n;
     MPM_HIP(hipMalloc(&s->P, (size_t)Q_COUNT * n * sizeof(float)));
     if ((s->tile = tile_side(s->p.n))) {
+        // (of an earlier call that failed)
+        if (s->tau.tau) (void)hipFree(s->tau.tau);
+        if (s->tau.base) (void)hipFree(s->tau.base);
+        s->tau = Tau2{};
         MPM_HIP(hipMalloc(&s->tau.tau, (size_t)4 * n * sizeof(float)));
         MPM_HIP(hipMalloc(&s->tau.base, (size_t)blocks(n, 4) * sizeof(uint4)));
     }

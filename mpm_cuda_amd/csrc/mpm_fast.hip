@@ -1537,8 +1537,11 @@ __device__ __forceinline__ uint32_t p2g_tile_of(const GridP &g, const MatP &mat,
 // water, 100k particles each: 16.8, 15.0 and 15.7 us apart, 28 together.
 // Bound by LDS and vector issue together: of a SIMD's cycles the
 // vector units take ~54% and the LDS atomics ~41%, half of these in bank
-// conflicts of uneven cells.  Four waves a SIMD: five or six measured the same
-// or slower.  One pass over memory, no turns among lanes, no LDS sort: against
+// conflicts of uneven cells.  Four waves a SIMD: with five, 1M snow
+// gains 1% and groups of several materials (8 spilled registers) lose 5%.
+// Slower than its predecessor where cells are uneven and bodies drift fast (1M
+// random samples in two colliding bodies: 70 us, 60 with sorted register sums):
+// lanes then share words, and a 64-bit atomic takes ~20 cycles.  One pass over memory, no turns among lanes, no LDS sort: against
 // one wave a tile that sorted its particles in LDS and summed cells in
 // registers, per launch 26.8 -> 11.6 us (16k snow), 46 -> 26.0 (262k jello),
 // 67 -> 56.6 (1M snow), 202 -> 145 (2M water).
@@ -2020,6 +2023,9 @@ int fast_ready(mpm_sim *s)
 // otherwise (262k jello, 512 a tile: 26.0 against 28.3; 1M snow, 300 a tile:
 // 56.6 against 59.4).  The sums do not depend on it.
 constexpr int P2G_WAVES = 4, P2G_WAVES_SPARSE = 2;
+// A batch fills the chip with tiles: two (64 scenes of 8.7M particles 1.05 ->
+// 1.01 ms a step against four, 16 scenes of 0.9M the same).
+constexpr int P2G_WAVES_BATCH = 2;
 
 bool tile_shape_valid(int tile) { return tile == 0 || tile == 256 || tile == 384 || tile == 512; }
 
@@ -2345,12 +2351,12 @@ void fill_batch_slice(mpm_sim *s, BatchSlice &b)
 // several), in chunks of P2G_CHUNK.
 int launch_p2g_batch(hipStream_t st, int mats, const BatchSlice *tab, int nslices, int wgs)
 {
-    const auto kernel = mats == MPM_JELLO   ? k_p2g_batch<MPM_JELLO, P2G_WAVES>
-                        : mats == MPM_SNOW  ? k_p2g_batch<MPM_SNOW, P2G_WAVES>
-                        : mats == MPM_WATER ? k_p2g_batch<MPM_WATER, P2G_WAVES>
-                                            : k_p2g_batch<MAT_ANY, P2G_WAVES>;
+    const auto kernel = mats == MPM_JELLO   ? k_p2g_batch<MPM_JELLO, P2G_WAVES_BATCH>
+                        : mats == MPM_SNOW  ? k_p2g_batch<MPM_SNOW, P2G_WAVES_BATCH>
+                        : mats == MPM_WATER ? k_p2g_batch<MPM_WATER, P2G_WAVES_BATCH>
+                                            : k_p2g_batch<MAT_ANY, P2G_WAVES_BATCH>;
     for (int c0 = 0; c0 < nslices; c0 += P2G_CHUNK) {
-        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(64 * P2G_WAVES), 0, st, tab + c0, std::min(P2G_CHUNK, nslices - c0));
+        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(64 * P2G_WAVES_BATCH), 0, st, tab + c0, std::min(P2G_CHUNK, nslices - c0));
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
     }
