@@ -54,7 +54,7 @@ for _mat, _b in ALG_BYTES.items():
     for _form in ("plain", "fast"):
         KERNEL_BYTES[(_mat, _form)] = dict(_b)
     KERNEL_BYTES[(_mat, "fused")] = {"g2p": (_b["p2g"][0] + _b["g2p"][0], _b["p2g"][1] + _b["g2p"][1])}
-KERNEL_NAME = {("plain", "p2g"): "k_p2g_atomic", ("plain", "g2p"): "k_g2p", ("fast", "p2g"): "k_p2g_block",
+KERNEL_NAME = {("plain", "p2g"): "k_p2g_atomic", ("plain", "g2p"): "k_g2p", ("fast", "p2g"): "k_p2g_groups",
                ("fast", "g2p"): "k_g2p", ("fused", "g2p"): "k_g2p2g_block", ("plain", "grid"): "k_grid_update",
                ("fast", "grid"): "k_grid_update", ("fused", "grid"): "k_grid_update"}
 

@@ -242,14 +242,14 @@ int mpm_synchronize(mpm_sim *sim);
 /* Per-phase device timing with HIP events recorded on the simulator's
  * stream (no reference counterpart; the reference has only an FPS readout,
  * main.cpp:252-253).  Phases: [0] sort + tile build, [1] P2G, [2] grid
- * update (incl. active-block compaction), [3] G2P.  mpm_phase_times returns
+ * update, [3] G2P.  mpm_phase_times returns
  * milliseconds and launch counts accumulated since the previous call and
  * clears them.  stats_nodes (may be NULL) receives the number of grid nodes
  * with mass in the last grid update. */
 int mpm_set_timing(mpm_sim *sim, int32_t enable);
 int mpm_phase_times(mpm_sim *sim, double ms[4], int64_t counts[4], int64_t *stats_nodes);
 /* The main kernel of each phase alone, timed like the phases (events around
- * the single launch): [0] P2G (k_p2g_block, or k_p2g_atomic in the PLAIN
+ * the single launch): [0] P2G (k_p2g_groups, or k_p2g_atomic in the PLAIN
  * form), [1] k_grid_update, [2] G2P (k_g2p, or k_g2p2g_block in the FUSED
  * form), [3] unused.  Accumulated since the previous call, then cleared. */
 int mpm_kernel_times(mpm_sim *sim, double ms[4], int64_t counts[4]);
