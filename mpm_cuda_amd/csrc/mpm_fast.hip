@@ -828,15 +828,24 @@ struct TileLds {
     uint32_t nitems;
 };
 
-// LDS of a FAST-form tile worked by W waves: an 8^3-node arena of 64-bit
+// LDS of a FAST-form tile worked by W waves: an 8^3-node arena (or two) of 64-bit
 // fixed-point sums, one plane per component (mass, then momentum).  Node
 // (x, y, z) of a plane is x + AR_Y y + AR_Z z: linear, so that a stencil's
 // offsets are immediates of the LDS instructions, and AR_Z = 68 spreads the
-// 64 cells of a block evenly over the banks.  17.1 KB.
+// 64 cells of a block evenly over the banks.  17.5 KB a copy.
 constexpr int AR_Y = ARENA, AR_Z = ARENA * ARENA + 4, AR_PLANE = ARENA * AR_Z;
 template <int W>
 struct TileArena {
-    unsigned long long sum[4][AR_PLANE];
+    // With four waves two copies, the lanes of either half of the cells (a
+    // checkerboard of them, as the sort left them) adding to their own: a
+    // particle that drifted into the next cell no longer shares words with that
+    // cell's.  16 words apart from the first copy's banks.  35 KB, which leaves
+    // the four workgroups a CU that the registers allow; with two waves a second
+    // copy would halve the workgroups.  P2G of 1M snow in two colliding bodies
+    // (0.06 cells a step) 70.6 -> 62.7 us; 100 steps of 262k jello 4.58 -> 4.41
+    // ms, 48 steps of 16 scenes 6.07 -> 6.03 ms, a step of 64 scenes 1.04 -> 1.00.
+    static constexpr int COPIES = W >= 4 ? 2 : 1, COPY = 4 * AR_PLANE + 16;
+    unsigned long long sum[COPIES * COPY];
     float bound[W];
     uint32_t faces[W];
 };
@@ -1389,6 +1398,7 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
     const bool staged = d.w < staging_cap;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int copy = TileArena<W>::COPIES > 1 ? ((lane ^ (lane >> 2) ^ (lane >> 4)) & 1) * TileArena<W>::COPY : 0;
     float x[3], gw = 0.0f;
     RawP raw;
     // lanes past the tile's end reload its last particle
@@ -1401,9 +1411,10 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
     const uint32_t first = (uint32_t)wave * 64u;
     if (first < d.y) load(first);
     {
-        static_assert(4 * AR_PLANE % 2 == 0, "whole 16-byte stores");
-        float4 *z = (float4 *)&L.sum[0][0];
-        for (int k = threadIdx.x; k < 2 * AR_PLANE; k += 64 * W) z[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        using A = TileArena<W>;
+        static_assert(A::COPY % 2 == 0, "whole 16-byte stores");
+        float4 *z = (float4 *)&L.sum[0];
+        for (int k = threadIdx.x; k < A::COPIES * A::COPY / 2; k += 64 * W) z[k] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     float bound = 0.0f;
     uint32_t s0 = first;
@@ -1454,7 +1465,7 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
                     lane_faces |= (rel[a] == ARENA - 3 ? 2u : 0u) << (2 * a);
                 }
             }
-            scatter_particle<MAT>(&L.sum[0][0] + (in ? rel[0] + AR_Y * rel[1] + AR_Z * rel[2] : 0), g, mat, dt, raw, gw,
+            scatter_particle<MAT>(&L.sum[0] + copy + (in ? rel[0] + AR_Y * rel[1] + AR_Z * rel[2] : 0), g, mat, dt, raw, gw,
                                   f, pscale, mscale, in);
             if (s0 == first) break;
             s0 -= 64u * W;
@@ -1486,8 +1497,13 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
             const int kz = q * W + wave;
             if (!row || kz < lo[2] || kz > hi[2]) continue;
             const int o = kx + AR_Y * ky + AR_Z * kz;
-            const float4 v = make_float4((float)(munit * fix_value(L.sum[0][o])), (float)(punit * fix_value(L.sum[1][o])),
-                                         (float)(punit * fix_value(L.sum[2][o])), (float)(punit * fix_value(L.sum[3][o])));
+            auto sum = [&](int c) {
+                unsigned long long t = L.sum[c * AR_PLANE + o];
+                if (TileArena<W>::COPIES > 1) t += L.sum[TileArena<W>::COPY + c * AR_PLANE + o];
+                return fix_value(t);
+            };
+            const float4 v = make_float4((float)(munit * sum(0)), (float)(punit * sum(1)), (float)(punit * sum(2)),
+                                         (float)(punit * sum(3)));
             gstore4(staging, dst + kz * 64 + lane, v);
             if (v.x != 0.f)
                 mark_node(g, t.ax + kx, t.ay + ky, t.az + kz, kx == 0 || ky == 0 || kz == 0, flags, list, counters);
@@ -1540,7 +1556,7 @@ __device__ __forceinline__ uint32_t p2g_tile_of(const GridP &g, const MatP &mat,
 // conflicts of uneven cells.  Four waves a SIMD: with five, 1M snow
 // gains 1% and groups of several materials (8 spilled registers) lose 5%.
 // Slower than its predecessor where cells are uneven and bodies drift fast (1M
-// random samples in two colliding bodies: 70 us, 60 with sorted register sums):
+// random samples in two colliding bodies: 63 us, 60 with sorted register sums):
 // lanes then share words, and a 64-bit atomic takes ~20 cycles.  One pass over memory, no turns among lanes, no LDS sort: against
 // one wave a tile that sorted its particles in LDS and summed cells in
 // registers, per launch 26.8 -> 11.6 us (16k snow), 46 -> 26.0 (262k jello),
@@ -2023,9 +2039,6 @@ int fast_ready(mpm_sim *s)
 // otherwise (262k jello, 512 a tile: 26.0 against 28.3; 1M snow, 300 a tile:
 // 56.6 against 59.4).  The sums do not depend on it.
 constexpr int P2G_WAVES = 4, P2G_WAVES_SPARSE = 2;
-// A batch fills the chip with tiles: two (64 scenes of 8.7M particles 1.05 ->
-// 1.01 ms a step against four, 16 scenes of 0.9M the same).
-constexpr int P2G_WAVES_BATCH = 2;
 
 bool tile_shape_valid(int tile) { return tile == 0 || tile == 256 || tile == 384 || tile == 512; }
 
@@ -2351,12 +2364,12 @@ void fill_batch_slice(mpm_sim *s, BatchSlice &b)
 // several), in chunks of P2G_CHUNK.
 int launch_p2g_batch(hipStream_t st, int mats, const BatchSlice *tab, int nslices, int wgs)
 {
-    const auto kernel = mats == MPM_JELLO   ? k_p2g_batch<MPM_JELLO, P2G_WAVES_BATCH>
-                        : mats == MPM_SNOW  ? k_p2g_batch<MPM_SNOW, P2G_WAVES_BATCH>
-                        : mats == MPM_WATER ? k_p2g_batch<MPM_WATER, P2G_WAVES_BATCH>
-                                            : k_p2g_batch<MAT_ANY, P2G_WAVES_BATCH>;
+    const auto kernel = mats == MPM_JELLO   ? k_p2g_batch<MPM_JELLO, P2G_WAVES>
+                        : mats == MPM_SNOW  ? k_p2g_batch<MPM_SNOW, P2G_WAVES>
+                        : mats == MPM_WATER ? k_p2g_batch<MPM_WATER, P2G_WAVES>
+                                            : k_p2g_batch<MAT_ANY, P2G_WAVES>;
     for (int c0 = 0; c0 < nslices; c0 += P2G_CHUNK) {
-        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(64 * P2G_WAVES_BATCH), 0, st, tab + c0, std::min(P2G_CHUNK, nslices - c0));
+        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(64 * P2G_WAVES), 0, st, tab + c0, std::min(P2G_CHUNK, nslices - c0));
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
     }
