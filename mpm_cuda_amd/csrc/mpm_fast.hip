@@ -845,7 +845,7 @@ struct TileArena {
     // (0.06 cells a step) 70.6 -> 62.7 us; 100 steps of 262k jello 4.58 -> 4.41
     // ms, 48 steps of 16 scenes 6.07 -> 6.03 ms, a step of 64 scenes 1.04 -> 1.00.
     static constexpr int COPIES = W >= 4 ? 2 : 1, COPY = 4 * AR_PLANE + 16;
-    unsigned long long sum[COPIES * COPY];
+    alignas(16) unsigned long long sum[COPIES * COPY];     // cleared by 16-byte stores
     float bound[W];
     uint32_t faces[W];
 };
@@ -1412,7 +1412,7 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
     if (first < d.y) load(first);
     {
         using A = TileArena<W>;
-        static_assert(A::COPY % 2 == 0, "whole 16-byte stores");
+        static_assert(A::COPY % 2 == 0 && alignof(A) >= alignof(float4), "whole, aligned 16-byte stores");
         float4 *z = (float4 *)&L.sum[0];
         for (int k = threadIdx.x; k < A::COPIES * A::COPY / 2; k += 64 * W) z[k] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
