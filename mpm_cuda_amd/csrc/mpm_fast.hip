@@ -846,7 +846,7 @@ struct TileArena {
     // ms, 48 steps of 16 scenes 6.07 -> 6.03 ms, a step of 64 scenes 1.04 -> 1.00.
     static constexpr int COPIES = W >= 4 ? 2 : 1, COPY = 4 * AR_PLANE + 16;
     alignas(16) unsigned long long sum[COPIES * COPY];     // cleared by 16-byte stores
-    float bound[W];
+    uint4 bound[W];
     uint32_t faces[W];
 };
 
@@ -854,19 +854,29 @@ struct TileArena {
 // has the integer nearest to x in its low mantissa bits, so its bit pattern
 // is that integer plus a constant whose low 51 bits are zero: patterns are
 // added as they are, and the low 51 bits of the total, sign-extended, are the
-// sum of the integers as long as that stays below 2^50.  A tile's unit is
-// 2^-50 of its particle count times the largest contribution any of them can
-// make to a component: for 512 particles 2^-40 of that, where FP32 sums round
-// at 2^-24 of the node's own value.  What the unit loses at a node of little
-// mass comes back to a particle times that node's weight.
+// sum of the integers as long as that stays below 2^50.  A momentum
+// component's unit is 2^-50 of the tile's particle count times the largest
+// contribution any of its particles can make to that component: for 511
+// particles 2^-41 of that, where FP32 sums round at 2^-24 of the node's own
+// value.  Particles whose largest bound is more than fix_window octaves below
+// the tile's get units of their own in another round over the tile, so that
+// adding one costs at most 2^-26 of its own bound (from 1,024 particles a tile
+// on twice that per doubling: its nodes then sum that many more).  Without the rounds
+// one particle 2^20 times the others left their nodes 2^-20 off, and with one
+// unit for all components a direction 2^30 times slower was lost; the two cost
+// 2M water 2% of a step, the other timing cases less than 1%.  What a unit
+// loses at a node of little mass comes back to a particle times that node's
+// weight.
 constexpr double FIX_MAGIC = 6755399441055744.0;        // 1.5 * 2^52
 constexpr int FIX_BITS = 50;
+__device__ __forceinline__ int fix_window(int nbits) { return max(14, nbits - 26); }
+constexpr uint32_t ALL_BOUNDS = 0x7f800000u;        // limit of a tile's first round
 __device__ __forceinline__ double fix_value(unsigned long long s) { return (double)((long long)(s << 13) >> 13); }
-// Largest of non-negative v over the wave, in lane 63 (DPP moves; lanes
-// without a source keep their own value).
-__device__ __forceinline__ float wave_max_dpp(float v)
+// Largest v over the wave, in lane 63 (DPP moves; lanes without a source take
+// zero).  Non-negative floats order like their bit patterns.
+__device__ __forceinline__ uint32_t wave_max_dpp(uint32_t v)
 {
-#define MPM_MAX_STEP(ctrl, rows)                                                                                         v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), ctrl, rows, 0xf, false)))
+#define MPM_MAX_STEP(ctrl, rows) v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false))
     MPM_MAX_STEP(0x111, 0xf);       // row_shr:1
     MPM_MAX_STEP(0x112, 0xf);
     MPM_MAX_STEP(0x114, 0xf);
@@ -877,6 +887,7 @@ __device__ __forceinline__ float wave_max_dpp(float v)
     return v;
 }
 __device__ __forceinline__ double pow2(int e) { return __hiloint2double((1023 + e) << 20, 0); }
+__device__ __forceinline__ int exp_of(float v) { return ((__float_as_int(v) >> 23) & 255) - 126; }     // |v| < 2^this
 
 struct TileGeo {
     int ax, ay, az;     // arena origin (node index of arena slot 0)
@@ -1283,23 +1294,25 @@ __device__ __forceinline__ float water_force(const MatP &mat, const GridP &g, fl
     return dt * mat.vol * pr * J * g.inv_h;
 }
 
-// A bound on the magnitude of a particle's contribution to any component of
+// Bounds on the magnitudes of a particle's contributions to the components of
 // any node's momentum (see scatter_particle: N <= 3/4, |D| <= 1, offsets at
-// most 2, |fx| <= 1.5; a NaN input gives NaN or infinity).
+// most 2, |fx| <= 1.5), as bit patterns: those of finite floats are below
+// ALL_BOUNDS, and a particle with any that is not has one that is not.  The
+// same bits wherever it is inlined: a tile's rounds are told apart by them.
 template <int MAT>
-__device__ __forceinline__ float contribution_bound(const MatP &mat, const GridP &g, float dt, const RawP &r, float gw)
+__device__ __forceinline__ void contribution_bounds(const MatP &mat, const GridP &g, float dt, const RawP &r, float gw,
+                                                    uint32_t q[3])
 {
+#pragma clang fp contract(off)
     const float hm = 3.5f * g.h * mat.mass, cg = dt * mat.vol * g.inv_h;
-    float s = 0.0f;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         constexpr int T[3][3] = {{0, 3, 4}, {3, 1, 5}, {4, 5, 2}};      // tau as xx, yy, zz, xy, xz, yz
-        const float q = fabsf(r.C[3 * c]) + fabsf(r.C[3 * c + 1]) + fabsf(r.C[3 * c + 2]);
-        const float f = MAT == MPM_WATER ? fabsf(gw)
+        const float a = fabsf(r.C[3 * c]) + fabsf(r.C[3 * c + 1]) + fabsf(r.C[3 * c + 2]);
+        const float f = MAT == MPM_WATER ? gw
                                          : cg * (fabsf(r.s[T[c][0]]) + fabsf(r.s[T[c][1]]) + fabsf(r.s[T[c][2]]));
-        s += fmaf(hm, q, fmaf(mat.mass, fabsf(r.v[c]), f));
+        q[c] = (uint32_t)__float_as_int(fmaf(hm, a, fmaf(mat.mass, fabsf(r.v[c]), fabsf(f)))) & 0x7fffffffu;
     }
-    return s;       // the sum over c: a NaN of any component stays one
 }
 
 // Adds one particle's 27 node contributions to the arena, FAST form.  Node
@@ -1309,15 +1322,14 @@ __device__ __forceinline__ float contribution_bound(const MatP &mat, const GridP
 //   p_c(o) = Nz alpha_c(ox, oy) + Nx Ny zeta_c(oz),  m(o) / m = Nx Ny Nz
 //   alpha_c = Ny (Nx (a_c + ox B_c0) + G_c0 Dx) + Nx (oy Ny B_c1 + G_c1 Dy)
 //   zeta_c  = oz Nz B_c2 + G_c2 Dz
-// in fixed point: momenta times pscale, masses over m times pscale mscale.  The last
+// in fixed point: momenta times 2^k2[c], masses over m times mscale.  The last
 // two products of each value run in FP64 (full rate on this target) and end
 // in the fixed-point sum's own rounding.
 template <int MAT>
 __device__ __forceinline__ void scatter_particle(unsigned long long *node, const GridP &g, const MatP &mat, float dt,
-                                                 const RawP &r, float gw, const float fx[3], double pscale,
+                                                 const RawP &r, float gw, const float fx[3], const int k2[3],
                                                  double mscale, bool in)
 {
-    const float hm = g.h * mat.mass, cg = -dt * mat.vol * g.inv_h;
     float N[3][3], D[3][3];
     bspline3_wave(fx, N, D);
     float sx[3][3], ey[3][3];       // [offset][component]
@@ -1325,13 +1337,16 @@ __device__ __forceinline__ void scatter_particle(unsigned long long *node, const
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         constexpr int T[3][3] = {{0, 3, 4}, {3, 1, 5}, {4, 5, 2}};
+        // powers of two: nothing is lost by scaling first
+        const float m = __builtin_amdgcn_ldexpf(mat.mass, k2[c]), hm = __builtin_amdgcn_ldexpf(g.h * mat.mass, k2[c]),
+                    cg = __builtin_amdgcn_ldexpf(-dt * mat.vol * g.inv_h, k2[c]);
         float B[3], G[3];
-        float a = mat.mass * r.v[c];
+        float a = m * r.v[c];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             B[k] = hm * r.C[3 * c + k];
             a = fmaf(-B[k], fx[k], a);
-            if (MAT == MPM_WATER) G[k] = k == c ? gw : 0.0f;
+            if (MAT == MPM_WATER) G[k] = k == c ? __builtin_amdgcn_ldexpf(gw, k2[c]) : 0.0f;
             else G[k] = cg * r.s[T[c][k]];
         }
         // water: G is zero off the diagonal (resolved at compile time)
@@ -1342,7 +1357,7 @@ __device__ __forceinline__ void scatter_particle(unsigned long long *node, const
         for (int o = 0; o < 3; ++o) {
             const float gy = GZ(1) ? 0.0f : G[1] * D[1][o], gz = GZ(2) ? 0.0f : G[2] * D[2][o];
             ey[o][c] = o == 0 ? gy : (GZ(1) ? N[1][o] * By[o] : fmaf(N[1][o], By[o], gy));
-            ez[o][c] = pscale * (double)(o == 0 ? gz : (GZ(2) ? N[2][o] * Bz[o] : fmaf(N[2][o], Bz[o], gz)));
+            ez[o][c] = (double)(o == 0 ? gz : (GZ(2) ? N[2][o] * Bz[o] : fmaf(N[2][o], Bz[o], gz)));
             const float t = N[0][o] * ax[o];
             sx[o][c] = GZ(0) ? t : fmaf(G[0], D[0][o], t);
         }
@@ -1350,7 +1365,7 @@ __device__ __forceinline__ void scatter_particle(unsigned long long *node, const
     }
     double pz[3];
 #pragma unroll
-    for (int o = 0; o < 3; ++o) pz[o] = pscale * (double)N[2][o];
+    for (int o = 0; o < 3; ++o) pz[o] = (double)N[2][o];
     if (!in) return;
     auto add = [](unsigned long long *s, double v) { atomicAdd(s, (unsigned long long)__double_as_longlong(v)); };
 #pragma unroll
@@ -1376,19 +1391,28 @@ __device__ __forceinline__ void scatter_particle(unsigned long long *node, const
         }
 }
 
+__device__ __forceinline__ uint4 uniform_u4(const uint4 v)
+{
+    return make_uint4((uint32_t)__builtin_amdgcn_readfirstlane((int)v.x), (uint32_t)__builtin_amdgcn_readfirstlane((int)v.y),
+                      (uint32_t)__builtin_amdgcn_readfirstlane((int)v.z), (uint32_t)__builtin_amdgcn_readfirstlane((int)v.w));
+}
+
 // One tile (descriptor d = first particle, count, block, staging slot) of
 // the FAST-form P2G, by one workgroup of W waves; returns health bits.  The
 // waves take 64 particles at a time in their stored order -- as of the last
 // sort one particle of each cell of the block, then the next of each
 // (k_rank_tiles) -- so the lanes of an LDS atomic mostly hold different
-// nodes.  The sums are integers, exact and the same in any order; their scale
-// comes from the largest contribution any of the tile's particles can make,
-// so the waves read their particles once for that bound (the last batch stays
-// in registers for the scatter) and once more for the other batches.  A tile
+// nodes.  The sums are integers, exact and the same in any order; their scales
+// come from the largest contribution any of the tile's particles can make, so
+// the waves read their particles once for those bounds (the last batch stays
+// in registers for the scatter) and once more for the other batches.
+// Particles too small for those scales (fix_window) wait for another call on
+// the same tile, which takes those with bounds below `limit`, adds their sums
+// to the staged ones, and sets `limit` for the next or to ALL_BOUNDS.  A tile
 // with a particle that is not finite goes to the atomic fallback; a wave with
 // particles for it goes through its batches again at the end.
 template <int MAT, int W>
-__device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, const PartView &pv, const uint4 d,
+__device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, const PartView &pv, const uint4 d, uint32_t &limit,
                                              uint32_t staging_cap, float dt, float4 *__restrict__ staging,
                                              float4 *grid, uint32_t *flags, uint32_t *list, uint32_t *counters,
                                              int32_t *blk_tile, TileArena<W> &L)
@@ -1410,42 +1434,61 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
     };
     const uint32_t first = (uint32_t)wave * 64u;
     if (first < d.y) load(first);
+    uint64_t out = 0;           // lanes that met a particle for the atomic fallback
+    uint32_t lane_faces = 0;    // arena faces this lane's particles' stencils reach (see tile_entry)
+    const bool again = limit < ALL_BOUNDS;
     {
         using A = TileArena<W>;
         static_assert(A::COPY % 2 == 0 && alignof(A) >= alignof(float4), "whole, aligned 16-byte stores");
         float4 *z = (float4 *)&L.sum[0];
         for (int k = threadIdx.x; k < A::COPIES * A::COPY / 2; k += 64 * W) z[k] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    float bound = 0.0f;
+    uint32_t bound[3] = {0u, 0u, 0u};
+    uint32_t least = ~0u;       // this lane's least particle bound above zero, less one
     uint32_t s0 = first;
     if (first < d.y)
         for (;;) {
             if (MAT == MPM_WATER) gw = water_force(mat, g, dt, raw.s[0]);
-            const float q = contribution_bound<MAT>(mat, g, dt, raw, gw);
-            bound = q <= bound ? bound : q;         // keeps a NaN
-            if (!(q <= 3e38f)) bound = __int_as_float(0x7f800000);
+            uint32_t q[3];
+            contribution_bounds<MAT>(mat, g, dt, raw, gw, q);
+            uint32_t all = max(max(q[0], q[1]), q[2]);
+            if (again && all >= limit) all = q[0] = q[1] = q[2] = 0u;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) bound[c] = max(bound[c], q[c]);
+            least = min(least, all - 1u);
             if (s0 + 64u * W >= d.y) break;
             s0 += 64u * W;
             load(s0);
         }
-    bound = wave_max_dpp(bound);
-    if (lane == 63) L.bound[wave] = bound;
-    __syncthreads();
-    bound = L.bound[0];
 #pragma unroll
-    for (int w = 1; w < W; ++w) bound = fmaxf(bound, L.bound[w]);
-    const uint32_t bb32 = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(bound));
-    const bool finite = bb32 < 0x7f800000u;
-    // contributions below 2^e, at most d.y of them a node: sums below 2^50
-    const int e = (int)(bb32 >> 23) - 126, nbits = FIX_BITS - (32 - __builtin_clz(d.y));
-    const double pscale = pow2(nbits - e), mscale = pow2(e);     // mass: 2^nbits = pscale 2^e
+    for (int c = 0; c < 3; ++c) bound[c] = wave_max_dpp(bound[c]);
+    if (lane == 63) L.bound[wave] = make_uint4(bound[0], bound[1], bound[2], 0u);
+    __syncthreads();
+    uint4 top = L.bound[0];
+#pragma unroll
+    for (int w = 1; w < W; ++w) {
+        const uint4 u = L.bound[w];
+        top.x = max(top.x, u.x); top.y = max(top.y, u.y); top.z = max(top.z, u.z);
+    }
+    top = uniform_u4(top);
+    top.w = max(max(top.x, top.y), top.z);
+    const bool finite = top.w < ALL_BOUNDS;
+    const int nbits = FIX_BITS - (32 - __builtin_clz(d.y));
+    // contributions to component c are below 2^(nbits - k2[c]), at most d.y of
+    // them a node: sums below 2^50.  No factor of one overflows when scaled.
+    const int most = 120 - max(max(exp_of(mat.mass), exp_of(g.h) + 2 + exp_of(mat.mass)),
+                               exp_of(dt) + exp_of(mat.vol) + exp_of(g.inv_h));
+    const int k2[3] = {min(nbits + 126 - (int)(top.x >> 23), most), min(nbits + 126 - (int)(top.y >> 23), most),
+                       min(nbits + 126 - (int)(top.z >> 23), most)};
+    const double mscale = pow2(nbits);
+    const int low_exp = (int)(top.w >> 23) - fix_window(nbits);
+    const uint32_t low = finite && staged && low_exp > 0 ? (uint32_t)low_exp << 23 : 0u;    // least bound of this round
+    const bool later = low && __any(least < low - 1u), pick = again || later;
     // base inside the arena's bins (rel: relative to it), and a slot to write the tile to
     auto in_arena = [&](const int rel[3]) {
         return staged && finite && (uint32_t)rel[0] <= (uint32_t)(ARENA - 3) &&
                (uint32_t)rel[1] <= (uint32_t)(ARENA - 3) && (uint32_t)rel[2] <= (uint32_t)(ARENA - 3);
     };
-    uint64_t out = 0;           // lanes that met a particle for the atomic fallback
-    uint32_t lane_faces = 0;    // arena faces this lane's particles' stencils reach (see tile_entry)
     if (first < d.y)
         for (;;) {
             const bool active = s0 + (uint32_t)lane < d.y;
@@ -1454,7 +1497,7 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
             const uint32_t ob = base_fx(g, x, b, f);
             if (active) bits |= ob;
             const int rel[3] = {b[0] - t.ax, b[1] - t.ay, b[2] - t.az};
-            const bool in = active && in_arena(rel);
+            bool in = active && in_arena(rel);
             out |= __ballot(active && !in);
             if (in) {
                 // a base on the arena's first (last) bin position reaches its
@@ -1465,8 +1508,14 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
                     lane_faces |= (rel[a] == ARENA - 3 ? 2u : 0u) << (2 * a);
                 }
             }
+            if (pick) {
+                uint32_t q[3];
+                contribution_bounds<MAT>(mat, g, dt, raw, gw, q);
+                const uint32_t all = max(max(q[0], q[1]), q[2]);
+                in = in && all < limit && (all >= low || (all == 0u && !again));
+            }
             scatter_particle<MAT>(&L.sum[0] + copy + (in ? rel[0] + AR_Y * rel[1] + AR_Z * rel[2] : 0), g, mat, dt, raw, gw,
-                                  f, pscale, mscale, in);
+                                  f, k2, mscale, in);
             if (s0 == first) break;
             s0 -= 64u * W;
             load(s0);
@@ -1474,19 +1523,22 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
         }
     // the arena into the tile's staging slot (logical node order): indices
     // 1..6 of each axis and the faces some stencil reached (every other node
-    // is zero); mark the node blocks that received mass
+    // is zero; of several rounds all nodes); mark the node blocks that
+    // received mass
     uint32_t faces = 0;
 #pragma unroll
     for (int f = 0; f < 6; ++f)
         if (__ballot((lane_faces >> f) & 1u)) faces |= 1u << f;
-    if (lane == 0) L.faces[wave] = faces;
+    if (lane == 0) L.faces[wave] = faces | (later ? 64u : 0u);
     __syncthreads();
-    if (staged) {
-        faces = 0;
+    faces = 0;
 #pragma unroll
-        for (int w = 0; w < W; ++w) faces |= L.faces[w];
-        faces = (uint32_t)__builtin_amdgcn_readfirstlane((int)faces);
-        const double punit = pow2(e - nbits), munit = pow2(-nbits) * (double)mat.mass;
+    for (int w = 0; w < W; ++w) faces |= L.faces[w];
+    faces = (uint32_t)__builtin_amdgcn_readfirstlane((int)faces);
+    const bool more = faces & 64u;
+    if (staged) {
+        if (more || again) faces = 63u;
+        const double munit = pow2(-nbits) * (double)mat.mass;
         const int64_t dst = (int64_t)d.w * ARENA_NODES;
         const int lo[3] = {(faces & 1u) ? 0 : 1, (faces & 4u) ? 0 : 1, (faces & 16u) ? 0 : 1};
         const int hi[3] = {(faces & 2u) ? 7 : 6, (faces & 8u) ? 7 : 6, (faces & 32u) ? 7 : 6};
@@ -1502,16 +1554,21 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
                 if (TileArena<W>::COPIES > 1) t += L.sum[TileArena<W>::COPY + c * AR_PLANE + o];
                 return fix_value(t);
             };
-            const float4 v = make_float4((float)(munit * sum(0)), (float)(punit * sum(1)), (float)(punit * sum(2)),
-                                         (float)(punit * sum(3)));
+            float4 v = make_float4((float)(munit * sum(0)), (float)(pow2(-k2[0]) * sum(1)),
+                                   (float)(pow2(-k2[1]) * sum(2)), (float)(pow2(-k2[2]) * sum(3)));
+            if (again) {
+                const float4 u = gload4(staging, dst + kz * 64 + lane);
+                v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
+            }
             gstore4(staging, dst + kz * 64 + lane, v);
             if (v.x != 0.f)
                 mark_node(g, t.ax + kx, t.ay + ky, t.az + kz, kx == 0 || ky == 0 || kz == 0, flags, list, counters);
         }
         if (threadIdx.x == 0) gp(blk_tile)[d.z] = tile_entry(d.w, faces);
     }
-    if (out)
-        for (s0 = first; s0 < d.y; s0 += 64u * W) {
+    limit = more ? low : ALL_BOUNDS;
+    if (out && !again)
+        for (uint32_t s0 = first; s0 < d.y; s0 += 64u * W) {
             const bool active = s0 + (uint32_t)lane < d.y;
             const uint32_t i = d.x + min(s0 + (uint32_t)lane, d.y - 1u);
 #pragma unroll
@@ -1523,28 +1580,22 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
             if (m && lane == 0) (void)gatomic_add(counters + CT_SPILL, (uint32_t)__popcll(m));
             if ((m >> lane) & 1ull) spill_particle<MAT>(g, mat, pv, (int)i, dt, counters, grid, flags, list);
         }
-    __syncthreads();        // the arena is cleared for the workgroup's next tile
+    __syncthreads();        // the arena is cleared for the workgroup's next tile or round
     return bits;
-}
-
-__device__ __forceinline__ uint4 uniform_u4(const uint4 v)
-{
-    return make_uint4((uint32_t)__builtin_amdgcn_readfirstlane((int)v.x), (uint32_t)__builtin_amdgcn_readfirstlane((int)v.y),
-                      (uint32_t)__builtin_amdgcn_readfirstlane((int)v.z), (uint32_t)__builtin_amdgcn_readfirstlane((int)v.w));
 }
 
 // A tile of a group or scene of any material that MATS takes: the material is
 // one of the kernel's (MATS) or the tile's own (MAT_ANY).
 template <int MATS, int W>
-__device__ __forceinline__ uint32_t p2g_tile_of(const GridP &g, const MatP &mat, const PartView &pv, const uint4 d,
+__device__ __forceinline__ uint32_t p2g_tile_of(const GridP &g, const MatP &mat, const PartView &pv, const uint4 d, uint32_t &limit,
                                                 uint32_t staging_cap, float dt, float4 *staging, float4 *grid,
                                                 uint32_t *flags, uint32_t *list, uint32_t *counters, int32_t *blk_tile,
                                                 TileArena<W> &L)
 {
     const int type = MATS == MAT_ANY ? mat.type : MATS;
-    if (type == MPM_JELLO) return p2g_tile<MPM_JELLO, W>(g, mat, pv, d, staging_cap, dt, staging, grid, flags, list, counters, blk_tile, L);
-    if (type == MPM_SNOW) return p2g_tile<MPM_SNOW, W>(g, mat, pv, d, staging_cap, dt, staging, grid, flags, list, counters, blk_tile, L);
-    return p2g_tile<MPM_WATER, W>(g, mat, pv, d, staging_cap, dt, staging, grid, flags, list, counters, blk_tile, L);
+    if (type == MPM_JELLO) return p2g_tile<MPM_JELLO, W>(g, mat, pv, d, limit, staging_cap, dt, staging, grid, flags, list, counters, blk_tile, L);
+    if (type == MPM_SNOW) return p2g_tile<MPM_SNOW, W>(g, mat, pv, d, limit, staging_cap, dt, staging, grid, flags, list, counters, blk_tile, L);
+    return p2g_tile<MPM_WATER, W>(g, mat, pv, d, limit, staging_cap, dt, staging, grid, flags, list, counters, blk_tile, L);
 }
 
 // The tiles of up to LAUNCH_GROUPS particle groups, one group's after the
@@ -1578,12 +1629,13 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
         // every wave takes the step's dt from the controller's maxima itself:
         // a launch that did cost 4.6 us of 40 (100k snow)
         const uint2 m = *(const uint2 *)(a.counters + CT_COUNT * (1 + (threadIdx.x & 63u)) + CT_SPEED);
-        const float speed = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wave_max_dpp(__uint_as_float(m.x))), 63));
-        const float deform = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wave_max_dpp(__uint_as_float(m.y))), 63));
+        const float speed = __int_as_float(__builtin_amdgcn_readlane((int)wave_max_dpp(m.x), 63));
+        const float deform = __int_as_float(__builtin_amdgcn_readlane((int)wave_max_dpp(m.y), 63));
         dt = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(control_dt(a.rule, speed, deform))));
         if (a.rule.advance && blockIdx.x == 0 && threadIdx.x == 0) advance_clock(a.rule.ctl, dt);
     }
-    for (uint32_t k8 = blockIdx.x; k8 < nt8; k8 += gridDim.x) {
+    uint32_t limit = ALL_BOUNDS;       // below it: another round of the same tile
+    for (uint32_t k8 = blockIdx.x; k8 < nt8; k8 += limit < ALL_BOUNDS ? 0u : gridDim.x) {
         uint32_t tt = xcd_spread(k8, nt8);
         if (tt >= nt) continue;
         int gi = 0;
@@ -1591,7 +1643,7 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
             for (uint32_t n; tt >= (n = tiles(gi)); ++gi) tt -= n;
         const P2GGroup &q = a.grp[ONE ? 0 : gi];
         const uint4 d = uniform_u4(gload_u4(q.desc, tt));    // the tile's loops hold barriers
-        bits |= p2g_tile_of<MATS, W>(a.g, q.mat, q.pv, d, a.staging_cap, dt, a.staging, a.grid, a.flags, a.list,
+        bits |= p2g_tile_of<MATS, W>(a.g, q.mat, q.pv, d, limit, a.staging_cap, dt, a.staging, a.grid, a.flags, a.list,
                                      a.counters, q.blk_tile, L);
     }
     if (bits) atomicOr(a.counters + CT_HEALTH, bits);
@@ -1619,13 +1671,14 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
     __syncthreads();
     const uint32_t nt = s_total, nt8 = round_xcd(nt);
     const int lane = threadIdx.x & 63;
-    for (uint32_t k8 = blockIdx.x; k8 < nt8; k8 += gridDim.x) {
+    uint32_t limit = ALL_BOUNDS;
+    for (uint32_t k8 = blockIdx.x; k8 < nt8; k8 += limit < ALL_BOUNDS ? 0u : gridDim.x) {
         const uint32_t tt = xcd_spread(k8, nt8);
         if (tt >= nt) continue;
         const uint32_t sid = (uint32_t)__builtin_amdgcn_readfirstlane((int)__popcll(__ballot(s_end[lane] <= tt)));
         const BatchSlice &b = tab[sid];
         const uint4 d = uniform_u4(gload_u4(b.desc, tt - (sid ? s_end[sid - 1] : 0u)));
-        const uint32_t bits = p2g_tile_of<MATS, W>(b.g, b.mat, b.pv, d, b.staging_cap, b.dt, b.staging, b.grid_mp, b.flags, b.list,
+        const uint32_t bits = p2g_tile_of<MATS, W>(b.g, b.mat, b.pv, d, limit, b.staging_cap, b.dt, b.staging, b.grid_mp, b.flags, b.list,
                                                b.counters, b.blk_tile, L);
         if (bits) gatomic_or(b.counters + CT_HEALTH, bits);
     }
