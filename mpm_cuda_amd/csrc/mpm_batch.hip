@@ -3,18 +3,20 @@
 // No counterpart in the reference (it steps one MPMSimulator per process).
 // Each scene is an mpm_sim with one particle group in the FAST form.  The
 // batch keeps a table of the scenes' parameters (BatchSlice) in device memory
-// and advances every scene by one step with one launch per stage for the
-// whole batch -- P2G tiles (per 64 scenes), grid update, G2P -- each over the
-// scenes of all materials, plus one warm-start inference launch per set of
-// scenes with equal network weights.  (16 scenes of the three materials, 0.9M
-// particles, 48 steps: 6.3 ms with a hipGraph of one branch per material, whose
-// kernels hardly ran side by side; 5.9 with a graph of these three launches;
-// 5.7 launched directly.)
+// and advances every scene by one step with one launch per stage -- P2G tiles
+// (per 64 scenes), grid update, G2P -- each over the scenes of all materials,
+// plus one warm-start inference launch per set of scenes with equal network
+// weights.  (16 scenes of the three materials, 0.9M particles, 48 steps: 6.3 ms
+// with a hipGraph of one branch per material joined at every step, 5.9 with a
+// graph of these three launches, 5.7 launched directly.)  A longer run of more
+// particles takes two such chains of launches, each over half of the scenes
+// (make_chains).
 // Every `sort_every` steps all scenes are re-sorted, one launch per stage of
 // the sort, replayed as a hipGraph.  Sorting moves particle storage between
-// two buffers, so there is one graph per buffer parity.  Launch widths come from mpm_batch_autotune, which times
-// the candidates of each stage on live steps; results do not depend on them
-// (every tile, block and particle is processed by exactly one workgroup).
+// two buffers, so there is one graph per buffer parity.  Launch widths come
+// from mpm_batch_autotune, which times the candidates of each stage on live
+// steps; results do not depend on them (every tile, block and particle is
+// processed by exactly one workgroup).
 #include "mpm_launch.h"
 
 #include <string.h>
@@ -27,7 +29,7 @@ using namespace mpm;
 namespace {
 
 constexpr int NCAND = 4;
-const int P2G_CAND[NCAND] = {1024, 2048, 4096, 8192};   // one-wave workgroups
+const int P2G_CAND[NCAND] = {1024, 2048, 4096, 8192};   // workgroups of four waves
 const int GRID_CAND[NCAND] = {1024, 2048, 4096, 8192};
 const int G2P_CAND[NCAND] = {64, 128, 192, 256};
 constexpr int NTILE = 3;
@@ -49,6 +51,16 @@ struct SceneSig {
     }
 };
 
+// Scenes [begin, begin + count) of the tables, whose steps follow one another
+// on one stream.
+struct Chain {
+    int begin, count;
+    int mats;                           // their material, MAT_ANY: several
+    hipStream_t stream;                 // null: the batch's own
+    hipEvent_t done;
+    std::vector<std::pair<int, int64_t>> warm;      // weight sets among them, 64-particle chunks of each
+};
+
 }  // namespace
 
 struct mpm_batch {
@@ -65,15 +77,16 @@ struct mpm_batch {
     int parity = 0;
     int64_t steps_since_sort = 0;
     int64_t total = 0;
-    int mats = -1;                      // the scenes' material, MAT_ANY: several
+    Chain all{};                        // every scene, on the batch's stream
+    std::vector<Chain> chains;          // two halves side by side (see make_chains), or none
+    bool forked = false;                // the chains' streams are ahead of the batch's
     int permute_wgs = 0;                // workgroups of the batched re-sort move
     SortSlice *stab[2] = {};            // batched re-sort tables of both parities
     SortBatchPlan splan;
     // warm-start weight sets: scenes with equal weights share one inference launch
     std::vector<const float *> warm_params; // device weights of each set
-    std::vector<int64_t> warm_chunks;       // 64-particle chunks of each set
     std::vector<int> warm_group;            // per scene, -1: cold
-    hipEvent_t ev_done = nullptr;
+    hipEvent_t ev_done = nullptr, ev_fork = nullptr;
     std::vector<hipEvent_t> ev_join;
     std::vector<hipEvent_t> tev;        // step timing events
 };
@@ -111,39 +124,62 @@ void set_parity(mpm_batch *b, size_t k, int p)
     s->pid_alt = p ? b->pid0[k] : b->pid1[k];
 }
 
-// G2P workgroups of all scenes.
-int g2p_wgs(const mpm_batch *b, int threads)
+// G2P workgroups of a chain's scenes.
+int g2p_wgs(const mpm_batch *b, const Chain &c, int threads)
 {
     uint32_t w = 0;
-    for (mpm_sim *s : b->sims) w += (uint32_t)((s->groups[0].n + threads - 1) / threads);
+    for (int k = c.begin; k < c.begin + c.count; ++k)
+        w += (uint32_t)((b->sims[k]->groups[0].n + threads - 1) / threads);
     return (int)round_xcd(w);
 }
 
 int check(int rc, const char *what) { return rc ? hip_fail((hipError_t)rc, what) : MPM_OK; }
 
-// One step of every scene (parity p tables): P2G, grid update, the warm-start
-// inference of each weight set, G2P.  With `ev` (6 events, the autotuner's
-// stage timing) the P2G, grid-update and G2P stages are bracketed.
-int enqueue_step(mpm_batch *b, int p, int p2g, int grid, int g2p_threads, hipEvent_t *ev)
+// One step of a chain's scenes (parity p tables): P2G, grid update, the
+// warm-start inference of each weight set, G2P.  With `ev` (6 events, the
+// autotuner's stage timing) the P2G, grid-update and G2P stages are bracketed.
+int enqueue_step(mpm_batch *b, const Chain &c, int p, int p2g, int grid, int g2p_threads, hipEvent_t *ev)
 {
-    hipStream_t st = b->stream;
-    const BatchSlice *tab = b->tab[p];
-    const int n = (int)b->sims.size();
+    hipStream_t st = c.stream ? c.stream : b->stream;
+    const BatchSlice *tab = b->tab[p] + c.begin;
     int rc;
     if (ev) MPM_HIP(hipEventRecord(ev[0], st));
-    if ((rc = check(launch_p2g_batch(st, b->mats, tab, n, p2g), "p2g_batch"))) return rc;
+    if ((rc = check(launch_p2g_batch(st, c.mats, tab, c.count, p2g), "p2g_batch"))) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[1], st));
     if (ev) MPM_HIP(hipEventRecord(ev[2], st));
-    if ((rc = check(launch_grid_batch(st, tab, n, grid), "grid_batch"))) return rc;
+    if ((rc = check(launch_grid_batch(st, tab, c.count, grid), "grid_batch"))) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[3], st));
-    for (size_t w = 0; w < b->warm_params.size(); ++w)
-        if ((rc = check(launch_mlp_infer_batch(st, b->warm_params[w], tab, n, (int)w, b->warm_chunks[w]),
+    for (const auto &w : c.warm)
+        if ((rc = check(launch_mlp_infer_batch(st, b->warm_params[w.first], tab, c.count, w.first, w.second),
                         "mlp_infer_batch")))
             return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[4], st));
-    const int wgs = g2p_wgs(b, g2p_threads);
-    if (wgs && (rc = check(launch_g2p_batch(st, b->mats, tab, n, wgs, g2p_threads), "g2p_batch"))) return rc;
+    const int wgs = g2p_wgs(b, c, g2p_threads);
+    if (wgs && (rc = check(launch_g2p_batch(st, c.mats, tab, c.count, wgs, g2p_threads), "g2p_batch"))) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[5], st));
+    return MPM_OK;
+}
+
+// The chains' streams go on after the batch's, and the batch's after theirs.
+int fork_chains(mpm_batch *b)
+{
+    if (b->forked || b->chains.empty()) return MPM_OK;
+    MPM_HIP(hipEventRecord(b->ev_fork, b->stream));
+    for (Chain &c : b->chains)
+        if (c.stream) MPM_HIP(hipStreamWaitEvent(c.stream, b->ev_fork, 0));
+    b->forked = true;
+    return MPM_OK;
+}
+
+int join_chains(mpm_batch *b)
+{
+    if (!b->forked) return MPM_OK;
+    b->forked = false;
+    for (Chain &c : b->chains)
+        if (c.stream) {
+            MPM_HIP(hipEventRecord(c.done, c.stream));
+            MPM_HIP(hipStreamWaitEvent(b->stream, c.done, 0));
+        }
     return MPM_OK;
 }
 
@@ -208,7 +244,6 @@ int capture_sort(mpm_batch *b, hipGraphExec_t *out, int p)
 void group_warm(mpm_batch *b)
 {
     b->warm_params.clear();
-    b->warm_chunks.clear();
     b->warm_group.assign(b->sims.size(), -1);
     std::vector<size_t> rep;                        // first scene of each set
     for (size_t k = 0; k < b->sims.size(); ++k) {
@@ -221,11 +256,19 @@ void group_warm(mpm_batch *b)
             g = (int)rep.size();
             rep.push_back(k);
             b->warm_params.push_back(s->mlp_w);
-            b->warm_chunks.push_back(0);
         }
         b->warm_group[k] = g;
-        b->warm_chunks[g] += (s->groups[0].n + 63) / 64;
     }
+    auto sets = [&](Chain &c) {
+        std::vector<int64_t> chunks(rep.size(), 0);
+        for (int k = c.begin; k < c.begin + c.count; ++k)
+            if (b->warm_group[k] >= 0) chunks[b->warm_group[k]] += (b->sims[k]->groups[0].n + 63) / 64;
+        c.warm.clear();
+        for (size_t g = 0; g < chunks.size(); ++g)
+            if (chunks[g]) c.warm.push_back({(int)g, chunks[g]});
+    };
+    sets(b->all);
+    for (Chain &c : b->chains) sets(c);
 }
 
 int build(mpm_batch *b)
@@ -292,6 +335,87 @@ int build(mpm_batch *b)
     for (size_t k = 0; k < n; ++k) set_parity(b, k, par[k]);
     if (rc) { drop_graphs(b); b->built = false; return rc; }
     return MPM_OK;
+}
+
+// Waits for *flag, `ticks` of the 100 MHz clock at most.
+__global__ void k_wait_flag(const uint32_t *flag, uint32_t *seen, long long ticks)
+{
+    const long long t0 = wall_clock64();
+    while (!__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        if (wall_clock64() - t0 > ticks) return;
+        __builtin_amdgcn_s_sleep(8);
+    }
+    *seen = 1u;
+}
+__global__ void k_set_flag(uint32_t *flag) { __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// Whether kernels of the two streams run at the same time: not where the
+// streams share a hardware queue, whose kernels then take turns at ~25 us each.
+int streams_overlap(hipStream_t a, hipStream_t b, uint32_t *words, bool &yes)
+{
+    uint32_t seen = 0;
+    if (int rc = check(launch_zero_u32(a, words, 2), "zero")) return rc;
+    MPM_HIP(hipStreamSynchronize(a));
+    hipLaunchKernelGGL(k_wait_flag, dim3(1), dim3(1), 0, a, words, words + 1, 50000ll);      // 0.5 ms
+    hipLaunchKernelGGL(k_set_flag, dim3(1), dim3(1), 0, b, words);
+    MPM_HIP(hipGetLastError());
+    MPM_HIP(hipStreamSynchronize(b));
+    MPM_HIP(hipStreamSynchronize(a));
+    MPM_HIP(hipMemcpy(&seen, words + 1, 4, hipMemcpyDeviceToHost));
+    yes = seen != 0u;
+    return MPM_OK;
+}
+
+Chain chain_of(const mpm_batch *b, int begin, int end)
+{
+    Chain c{begin, end - begin, -1, nullptr, nullptr, {}};
+    for (int k = begin; k < end; ++k) {
+        const int t = b->sims[k]->groups[0].mat.type;
+        c.mats = c.mats < 0 || c.mats == t ? t : MAT_ANY;
+    }
+    return c;
+}
+
+// Two chains of about equal particles on streams that overlap, joined only at
+// a re-sort and at the end of a run: one's launch tails and gather latencies
+// beside the other's LDS work.  ms a step with one chain and two: 64 scenes,
+// 8.7M particles 1.013 and 0.912 (0.925 with the materials as branches of a
+// graph, joined at each step); 16 scenes, 1.9M 0.233 and 0.208; 3 scenes, 0.43M
+// 0.075 and 0.071; 4 scenes, 0.2M 0.051 and 0.046; three chains 0.89, 0.204 and
+// no better than one below 1M.  Fewer particles are the host's launches either
+// way.  A fork and a join cost ~20 us, so a run of a few steps takes one chain.
+constexpr int64_t CHAIN_PARTICLES = 200000;
+constexpr int32_t CHAIN_STEPS = 8;
+int make_chains(mpm_batch *b)
+{
+    const int n = (int)b->sims.size();
+    b->all = chain_of(b, 0, n);
+    if (n < 2 || b->total < CHAIN_PARTICLES) return MPM_OK;
+    int cut = 0;
+    for (int64_t sum = 0; cut < n - 1 && sum < b->total / 2; ++cut) sum += b->sims[cut]->groups[0].n;
+    uint32_t *words = nullptr;
+    MPM_HIP(hipMalloc(&words, 8));
+    std::vector<hipStream_t> tried;     // kept until the end: a queue is given to the next stream in turn
+    int rc = MPM_OK;
+    bool yes = false;
+    while (!rc && !yes && tried.size() < 4) {
+        hipStream_t st = nullptr;
+        const hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+        if (e != hipSuccess) { rc = hip_fail(e, "stream"); break; }
+        tried.push_back(st);
+        rc = streams_overlap(b->stream, st, words, yes);
+    }
+    (void)hipFree(words);
+    if (!rc && yes) {
+        b->chains = {chain_of(b, 0, cut), chain_of(b, cut, n)};
+        b->chains[1].stream = tried.back();
+        tried.pop_back();
+        hipError_t e = hipEventCreateWithFlags(&b->chains[1].done, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming);
+        if (e != hipSuccess) rc = hip_fail(e, "event");
+    }
+    for (hipStream_t st : tried) (void)hipStreamDestroy(st);
+    return rc;
 }
 
 int validate_shape(const mpm_batch_shape &s)
@@ -383,10 +507,12 @@ void after_step(mpm_batch *b)
     b->steps_since_sort += 1;
 }
 
-// Sort when due (by its graph with `graphs`), then one step.
-int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, hipEvent_t *ev, bool graphs)
+// Sort when due (by its graph with `graphs`), then one step: with `chains`
+// chain by chain, else all scenes together.
+int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, hipEvent_t *ev, bool graphs, bool chains)
 {
     if (b->steps_since_sort >= b->shape.sort_every) {
+        if (int rc = join_chains(b)) return rc;
         if (graphs) {
             MPM_HIP(hipGraphLaunch(b->sort_exec[b->parity], b->stream));
         } else {
@@ -398,7 +524,14 @@ int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, hipEvent_t *ev, b
         }
         after_sort(b);
     }
-    int rc = enqueue_step(b, b->parity, p2g, grid, g2p_threads, ev);
+    int rc = MPM_OK;
+    if (!chains) {
+        rc = enqueue_step(b, b->all, b->parity, p2g, grid, g2p_threads, ev);
+    } else {
+        rc = fork_chains(b);
+        for (size_t k = 0; k < b->chains.size() && !rc; ++k)
+            rc = enqueue_step(b, b->chains[k], b->parity, p2g, grid, g2p_threads, nullptr);
+    }
     if (rc) return rc;
     after_step(b);
     return MPM_OK;
@@ -453,8 +586,7 @@ int mpm_batch_create(mpm_sim *const *sims, int32_t n, const mpm_batch_shape *sha
     }
     mpm_batch *b = new mpm_batch();
     b->sims.assign(sims, sims + n);
-    // ordered by material (stable): each material's scenes form one range of
-    // the tables, so a step can run the materials side by side
+    // ordered by material (stable): a chain then holds as few as may be
     std::stable_sort(b->sims.begin(), b->sims.end(), [](const mpm_sim *x, const mpm_sim *y) {
         return x->groups[0].mat.type < y->groups[0].mat.type;
     });
@@ -473,10 +605,6 @@ int mpm_batch_create(mpm_sim *const *sims, int32_t n, const mpm_batch_shape *sha
     uint32_t pblocks = 0;
     for (mpm_sim *s : b->sims) pblocks += (uint32_t)((s->groups[0].n + 255) / 256);
     b->permute_wgs = (int)round_xcd(pblocks);
-    for (const mpm_sim *s : b->sims) {
-        const int t = s->groups[0].mat.type;
-        b->mats = b->mats < 0 || b->mats == t ? t : MAT_ANY;
-    }
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking)) != hipSuccess) return fail(hip_fail(e, "stream"));
     if ((e = hipMalloc(&b->tab[0], n * sizeof(BatchSlice))) != hipSuccess) return fail(hip_fail(e, "hipMalloc"));
@@ -488,6 +616,7 @@ int mpm_batch_create(mpm_sim *const *sims, int32_t n, const mpm_batch_shape *sha
     b->ev_join.assign(n, nullptr);
     for (auto &ev : b->ev_join)
         if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return fail(hip_fail(e, "event"));
+    if ((rc = make_chains(b))) return fail(rc);
     *out = b;
     return MPM_OK;
 }
@@ -518,19 +647,35 @@ int mpm_batch_run(mpm_batch *b, int32_t nsteps, float *step_ms)
     if (nsteps == 0) return MPM_OK;
     int rc = prepare(b);
     if (rc) return rc;
-    hipEvent_t *ev = step_ms ? timing_events(b, (size_t)nsteps + 1) : nullptr;
-    if (step_ms && !ev) return set_error(MPM_ERR_HIP, "hipEventCreate failed");
+    // a step ends where the last of its chains' does: an event per chain after
+    // each (the batch's stream first), all timed from the start
+    const bool chains = !b->chains.empty() && nsteps >= CHAIN_STEPS;
+    const size_t per = step_ms ? (chains ? b->chains.size() : 1) : 0;
+    hipEvent_t *ev = per ? timing_events(b, (size_t)nsteps * per + 1) : nullptr;
+    if (per && !ev) return set_error(MPM_ERR_HIP, "hipEventCreate failed");
     const bool graphs = b->shape.use_graph != 0;
+    if (ev) MPM_HIP(hipEventRecord(ev[0], b->stream));
     for (int32_t k = 0; k < nsteps; ++k) {
-        if (ev) MPM_HIP(hipEventRecord(ev[k], b->stream));
-        rc = one_step(b, b->shape.p2g_workgroups, b->shape.grid_workgroups, b->shape.g2p_threads, nullptr, graphs);
+        rc = one_step(b, b->shape.p2g_workgroups, b->shape.grid_workgroups, b->shape.g2p_threads, nullptr, graphs, chains);
         if (rc) return rc;
+        for (size_t c = 0; c < per; ++c)
+            MPM_HIP(hipEventRecord(ev[1 + k * per + c], c ? b->chains[c].stream : b->stream));
     }
-    if (ev) MPM_HIP(hipEventRecord(ev[nsteps], b->stream));
+    if ((rc = join_chains(b))) return rc;
     if ((rc = release(b))) return rc;
     if (ev) {
-        MPM_HIP(hipEventSynchronize(ev[nsteps]));
-        for (int32_t k = 0; k < nsteps; ++k) MPM_HIP(hipEventElapsedTime(&step_ms[k], ev[k], ev[k + 1]));
+        MPM_HIP(hipStreamSynchronize(b->stream));
+        float before = 0.0f;
+        for (int32_t k = 0; k < nsteps; ++k) {
+            float end = before;
+            for (size_t c = 0; c < per; ++c) {
+                float t = 0.0f;
+                MPM_HIP(hipEventElapsedTime(&t, ev[0], ev[1 + k * per + c]));
+                end = std::max(end, t);
+            }
+            step_ms[k] = end - before;
+            before = end;
+        }
     }
     return MPM_OK;
 }
@@ -554,7 +699,7 @@ int mpm_batch_autotune(mpm_batch *b, int32_t reps, float *ms_out)
     for (int32_t r = 0; r < reps; ++r)
         for (int c = 0; c < NCAND; ++c) {
             hipEvent_t *e = ev + ((size_t)r * NCAND + c) * per;
-            rc = one_step(b, P2G_CAND[c], GRID_CAND[c], G2P_CAND[c], e, false);
+            rc = one_step(b, P2G_CAND[c], GRID_CAND[c], G2P_CAND[c], e, false, false);
             if (rc) return rc;
         }
     MPM_HIP(hipStreamSynchronize(b->stream));
@@ -587,7 +732,7 @@ int mpm_batch_autotune(mpm_batch *b, int32_t reps, float *ms_out)
     for (int32_t r = 0; r < reps; ++r)
         for (int c = 0; c < NTILE; ++c) {
             hipEvent_t *e = ev + (t0 + (size_t)r * NTILE + c) * per;
-            rc = one_step(b, b->shape.p2g_workgroups, b->shape.grid_workgroups, b->shape.g2p_threads, e, false);
+            rc = one_step(b, b->shape.p2g_workgroups, b->shape.grid_workgroups, b->shape.g2p_threads, e, false, false);
             if (rc) return rc;
         }
     if ((rc = release(b))) return rc;
@@ -617,6 +762,8 @@ int mpm_batch_synchronize(mpm_batch *b)
 void mpm_batch_destroy(mpm_batch *b)
 {
     if (!b) return;
+    for (Chain &c : b->chains)
+        if (c.stream) (void)hipStreamSynchronize(c.stream);
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     drop_graphs(b);
     for (int p = 0; p < 2; ++p) {
@@ -624,6 +771,11 @@ void mpm_batch_destroy(mpm_batch *b)
         if (b->stab[p]) (void)hipFree(b->stab[p]);
     }
     if (b->ev_done) (void)hipEventDestroy(b->ev_done);
+    if (b->ev_fork) (void)hipEventDestroy(b->ev_fork);
+    for (Chain &c : b->chains) {
+        if (c.stream) (void)hipStreamDestroy(c.stream);
+        if (c.done) (void)hipEventDestroy(c.done);
+    }
     for (hipEvent_t e : b->ev_join)
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : b->tev)
