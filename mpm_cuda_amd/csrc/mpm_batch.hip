@@ -59,6 +59,9 @@ struct Chain {
     hipStream_t stream;                 // null: the batch's own
     hipEvent_t done;
     std::vector<std::pair<int, int64_t>> warm;      // weight sets among them, 64-particle chunks of each
+    SortBatchPlan sort;                 // their re-sort, and the workgroups of its move
+    int permute_wgs;
+    hipGraphExec_t sort_exec[2];        // per parity
 };
 
 }  // namespace
@@ -73,16 +76,13 @@ struct mpm_batch {
     BatchSlice *tab[2] = {};
     std::vector<SceneSig> sig;          // signature the tables and graphs were built for
     bool built = false;
-    hipGraphExec_t sort_exec[2] = {};
     int parity = 0;
     int64_t steps_since_sort = 0;
     int64_t total = 0;
     Chain all{};                        // every scene, on the batch's stream
-    std::vector<Chain> chains;          // two halves side by side (see make_chains), or none
+    std::vector<Chain> chains;          // two halves side by side (see make_chains), or all
     bool forked = false;                // the chains' streams are ahead of the batch's
-    int permute_wgs = 0;                // workgroups of the batched re-sort move
     SortSlice *stab[2] = {};            // batched re-sort tables of both parities
-    SortBatchPlan splan;
     // warm-start weight sets: scenes with equal weights share one inference launch
     std::vector<const float *> warm_params; // device weights of each set
     std::vector<int> warm_group;            // per scene, -1: cold
@@ -163,7 +163,7 @@ int enqueue_step(mpm_batch *b, const Chain &c, int p, int p2g, int grid, int g2p
 // The chains' streams go on after the batch's, and the batch's after theirs.
 int fork_chains(mpm_batch *b)
 {
-    if (b->forked || b->chains.empty()) return MPM_OK;
+    if (b->forked || b->chains.size() < 2) return MPM_OK;
     MPM_HIP(hipEventRecord(b->ev_fork, b->stream));
     for (Chain &c : b->chains)
         if (c.stream) MPM_HIP(hipStreamWaitEvent(c.stream, b->ev_fork, 0));
@@ -183,25 +183,26 @@ int join_chains(mpm_batch *b)
     return MPM_OK;
 }
 
-// Re-sort every scene from parity p into parity 1 - p on the batch stream:
-// keys, order and tiles of all scenes with one launch per sort stage, then
-// one launch moves every scene's particles into the parity 1 - p buffers in
-// its new order (the warm-start lists, which name old slots, are dropped).
-// The caller points the host views at parity 1 - p.
-int enqueue_sort(mpm_batch *b, int p)
+// Re-sort a chain's scenes from parity p into parity 1 - p: keys, order and
+// tiles of all of them with one launch per sort stage, then one launch moves
+// every scene's particles into the parity 1 - p buffers in its new order (the
+// warm-start lists, which name old slots, are dropped).  The caller points the
+// host views at parity 1 - p.
+int enqueue_sort(mpm_batch *b, const Chain &c, hipStream_t st, int p)
 {
-    const int n = (int)b->sims.size();
-    int rc = launch_sort_batch(b->stream, b->stab[p], n, b->splan);
+    int rc = launch_sort_batch(st, b->stab[p] + c.begin, c.count, c.sort);
     if (rc) return rc;
-    return check(launch_permute_batch(b->stream, b->tab[p], b->tab[p ^ 1], n, b->permute_wgs), "permute_batch");
+    return check(launch_permute_batch(st, b->tab[p] + c.begin, b->tab[p ^ 1] + c.begin, c.count, c.permute_wgs),
+                 "permute_batch");
 }
 
 void drop_graphs(mpm_batch *b)
 {
-    for (int p = 0; p < 2; ++p) {
-        if (b->sort_exec[p]) (void)hipGraphExecDestroy(b->sort_exec[p]);
-        b->sort_exec[p] = nullptr;
-    }
+    for (Chain &c : b->chains)
+        for (int p = 0; p < 2; ++p) {
+            if (c.sort_exec[p]) (void)hipGraphExecDestroy(c.sort_exec[p]);
+            c.sort_exec[p] = nullptr;
+        }
 }
 
 // Scene bookkeeping kept by sort_all, saved around captures and replays.
@@ -219,12 +220,12 @@ void set_book(mpm_sim *s, const SortBook &k)
     s->sorts = k.sorts;
 }
 
-int capture_sort(mpm_batch *b, hipGraphExec_t *out, int p)
+int capture_sort(mpm_batch *b, Chain &c, int p)
 {
     std::vector<SortBook> book;
     for (mpm_sim *s : b->sims) book.push_back(book_of(s));
     MPM_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed));
-    int rc = enqueue_sort(b, p);
+    int rc = enqueue_sort(b, c, b->stream, p);
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(b->stream, &graph);
     for (size_t k = 0; k < b->sims.size(); ++k) set_book(b->sims[k], book[k]);
@@ -233,7 +234,7 @@ int capture_sort(mpm_batch *b, hipGraphExec_t *out, int p)
         return rc;
     }
     if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
-    e = hipGraphInstantiate(out, graph, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&c.sort_exec[p], graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     if (e != hipSuccess) return hip_fail(e, "hipGraphInstantiate");
     return MPM_OK;
@@ -329,9 +330,8 @@ int build(mpm_batch *b)
     std::vector<int> par(n);
     for (size_t k = 0; k < n; ++k) par[k] = parity_of(b, k);
     int rc = MPM_OK;
-    for (int p = 0; p < 2 && !rc; ++p) {
-        rc = capture_sort(b, &b->sort_exec[p], p);
-    }
+    for (Chain &c : b->chains)
+        for (int p = 0; p < 2 && !rc; ++p) rc = capture_sort(b, c, p);
     for (size_t k = 0; k < n; ++k) set_parity(b, k, par[k]);
     if (rc) { drop_graphs(b); b->built = false; return rc; }
     return MPM_OK;
@@ -368,28 +368,34 @@ int streams_overlap(hipStream_t a, hipStream_t b, uint32_t *words, bool &yes)
 
 Chain chain_of(const mpm_batch *b, int begin, int end)
 {
-    Chain c{begin, end - begin, -1, nullptr, nullptr, {}};
+    Chain c{begin, end - begin, -1, nullptr, nullptr, {}, {}, 0, {nullptr, nullptr}};
+    uint32_t wgs = 0;
     for (int k = begin; k < end; ++k) {
         const int t = b->sims[k]->groups[0].mat.type;
         c.mats = c.mats < 0 || c.mats == t ? t : MAT_ANY;
+        wgs += (uint32_t)((b->sims[k]->groups[0].n + 255) / 256);
     }
+    c.permute_wgs = (int)round_xcd(wgs);
+    sort_batch_plan(b->sims.data() + begin, end - begin, c.sort);
     return c;
 }
 
 // Two chains of about equal particles on streams that overlap, joined only at
-// a re-sort and at the end of a run: one's launch tails and gather latencies
-// beside the other's LDS work.  ms a step with one chain and two: 64 scenes,
-// 8.7M particles 1.013 and 0.912 (0.925 with the materials as branches of a
-// graph, joined at each step); 16 scenes, 1.9M 0.233 and 0.208; 3 scenes, 0.43M
-// 0.075 and 0.071; 4 scenes, 0.2M 0.051 and 0.046; three chains 0.89, 0.204 and
-// no better than one below 1M.  Fewer particles are the host's launches either
-// way.  A fork and a join cost ~20 us, so a run of a few steps takes one chain.
+// the end of a run: one's launch tails, gather latencies and re-sort beside the
+// other's LDS work.  ms a step with one chain and two: 64 scenes, 8.7M
+// particles 1.013 and 0.898 (0.925 with the materials as branches of a graph,
+// joined at each step; 0.912 with a join at each re-sort); 16 scenes, 1.9M 0.233
+// and 0.204; 3 scenes, 0.43M 0.075 and 0.069; 4 scenes, 0.2M 0.051 and 0.047.
+// Three chains: 0.89, 0.204 and no better than one below 1M.  Fewer particles
+// are the host's launches either way.  A fork and a join cost ~20 us, so a run
+// of a few steps takes one chain.
 constexpr int64_t CHAIN_PARTICLES = 200000;
 constexpr int32_t CHAIN_STEPS = 8;
 int make_chains(mpm_batch *b)
 {
     const int n = (int)b->sims.size();
     b->all = chain_of(b, 0, n);
+    b->chains = {b->all};
     if (n < 2 || b->total < CHAIN_PARTICLES) return MPM_OK;
     int cut = 0;
     for (int64_t sum = 0; cut < n - 1 && sum < b->total / 2; ++cut) sum += b->sims[cut]->groups[0].n;
@@ -456,7 +462,7 @@ int prepare(mpm_batch *b)
         }
     bool same = b->built && b->sig.size() == n;
     for (size_t k = 0; same && k < n; ++k) same = sig_of(b, k) == b->sig[k];
-    if (b->shape.use_graph) same = same && b->sort_exec[0];
+    if (b->shape.use_graph) same = same && b->chains[0].sort_exec[0];
     if (!same) {
         for (mpm_sim *s : b->sims) MPM_HIP(hipStreamSynchronize(s->stream));
         int rc = build(b);
@@ -507,20 +513,20 @@ void after_step(mpm_batch *b)
     b->steps_since_sort += 1;
 }
 
-// Sort when due (by its graph with `graphs`), then one step: with `chains`
-// chain by chain, else all scenes together.
+// Sort when due (by graphs with `graphs`), then one step: with `chains` each
+// chain on its stream, else all scenes together on the batch's.
 int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, hipEvent_t *ev, bool graphs, bool chains)
 {
+    if (chains)
+        if (int rc = fork_chains(b)) return rc;
     if (b->steps_since_sort >= b->shape.sort_every) {
-        if (int rc = join_chains(b)) return rc;
-        if (graphs) {
-            MPM_HIP(hipGraphLaunch(b->sort_exec[b->parity], b->stream));
-        } else {
-            std::vector<SortBook> book;
-            for (mpm_sim *s : b->sims) book.push_back(book_of(s));
-            int rc = enqueue_sort(b, b->parity);
-            for (size_t k = 0; k < b->sims.size(); ++k) set_book(b->sims[k], book[k]);
-            if (rc) return rc;
+        for (Chain &c : b->chains) {
+            hipStream_t st = chains && c.stream ? c.stream : b->stream;
+            if (graphs) {
+                MPM_HIP(hipGraphLaunch(c.sort_exec[b->parity], st));
+                continue;
+            }
+            if (int rc = enqueue_sort(b, c, st, b->parity)) return rc;
         }
         after_sort(b);
     }
@@ -528,7 +534,6 @@ int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, hipEvent_t *ev, b
     if (!chains) {
         rc = enqueue_step(b, b->all, b->parity, p2g, grid, g2p_threads, ev);
     } else {
-        rc = fork_chains(b);
         for (size_t k = 0; k < b->chains.size() && !rc; ++k)
             rc = enqueue_step(b, b->chains[k], b->parity, p2g, grid, g2p_threads, nullptr);
     }
@@ -602,16 +607,12 @@ int mpm_batch_create(mpm_sim *const *sims, int32_t n, const mpm_batch_shape *sha
         b->P0.push_back(s->P); b->P1.push_back(s->P_alt);
         b->pid0.push_back(s->pid); b->pid1.push_back(s->pid_alt);
     }
-    uint32_t pblocks = 0;
-    for (mpm_sim *s : b->sims) pblocks += (uint32_t)((s->groups[0].n + 255) / 256);
-    b->permute_wgs = (int)round_xcd(pblocks);
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking)) != hipSuccess) return fail(hip_fail(e, "stream"));
     if ((e = hipMalloc(&b->tab[0], n * sizeof(BatchSlice))) != hipSuccess) return fail(hip_fail(e, "hipMalloc"));
     if ((e = hipMalloc(&b->tab[1], n * sizeof(BatchSlice))) != hipSuccess) return fail(hip_fail(e, "hipMalloc"));
     for (int p = 0; p < 2; ++p)
         if ((e = hipMalloc(&b->stab[p], n * sizeof(SortSlice))) != hipSuccess) return fail(hip_fail(e, "hipMalloc"));
-    sort_batch_plan(b->sims.data(), n, b->splan);
     if ((e = hipEventCreateWithFlags(&b->ev_done, hipEventDisableTiming)) != hipSuccess) return fail(hip_fail(e, "event"));
     b->ev_join.assign(n, nullptr);
     for (auto &ev : b->ev_join)
@@ -649,7 +650,7 @@ int mpm_batch_run(mpm_batch *b, int32_t nsteps, float *step_ms)
     if (rc) return rc;
     // a step ends where the last of its chains' does: an event per chain after
     // each (the batch's stream first), all timed from the start
-    const bool chains = !b->chains.empty() && nsteps >= CHAIN_STEPS;
+    const bool chains = b->chains.size() > 1 && nsteps >= CHAIN_STEPS;
     const size_t per = step_ms ? (chains ? b->chains.size() : 1) : 0;
     hipEvent_t *ev = per ? timing_events(b, (size_t)nsteps * per + 1) : nullptr;
     if (per && !ev) return set_error(MPM_ERR_HIP, "hipEventCreate failed");

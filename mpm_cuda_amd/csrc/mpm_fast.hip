@@ -740,7 +740,7 @@ __global__ void __launch_bounds__(256) k_bsort_emit(const SortSlice *__restrict_
 }
 
 // The tiles' particle orders (rank_tile) into the scenes' permutations, one
-// wave per tile of all the scenes' tiles.
+// wave per tile of all the scenes' tiles (2,048 workgroups fill the chip).
 __global__ void __launch_bounds__(256) k_bsort_rank(const SortSlice *__restrict__ tab, int ns, int alt)
 {
     __shared__ RankLds L[4];
@@ -2351,6 +2351,7 @@ int fill_sort_slice(mpm_sim *s, SortSlice &t)
 void sort_batch_plan(mpm_sim *const *sims, int ns, SortBatchPlan &pl)
 {
     pl = SortBatchPlan{};
+    int64_t bound = 0;
     for (int k = 0; k < ns; ++k) {
         const mpm_sim *s = sims[k];
         int bits = 1;
@@ -2361,8 +2362,10 @@ void sort_batch_plan(mpm_sim *const *sims, int ns, SortBatchPlan &pl)
         pl.runs += nblk(n, 256);
         pl.scan += nblk(s->nblocks, SCAN_TILE);
         pl.emit += nblk(s->nblocks, 256);
+        bound += tile_bound(s, n);
     }
     pl.spine = ns * ((1 << BS_DB) / 4);
+    pl.rank = (int)std::min<int64_t>((bound + 3) / 4, 2048);
 }
 
 int launch_sort_batch(hipStream_t st, const SortSlice *tab, int ns, const SortBatchPlan &pl)
@@ -2378,7 +2381,7 @@ int launch_sort_batch(hipStream_t st, const SortSlice *tab, int ns, const SortBa
     hipLaunchKernelGGL(k_bsort_scan_reduce, dim3(pl.scan), dim3(SCAN_T), 0, st, tab, ns);
     hipLaunchKernelGGL(k_bsort_scan_apply, dim3(pl.scan), dim3(SCAN_T), 0, st, tab, ns);
     hipLaunchKernelGGL(k_bsort_emit, dim3(pl.emit), dim3(256), 0, st, tab, ns);
-    hipLaunchKernelGGL(k_bsort_rank, dim3(1024), dim3(256), 0, st, tab, ns, pl.passes & 1);
+    hipLaunchKernelGGL(k_bsort_rank, dim3(pl.rank), dim3(256), 0, st, tab, ns, pl.passes & 1);
     if (int rc = launch_bsort_list(st, tab, ns, pl.emit)) return hip_fail((hipError_t)rc, "bsort_list");
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? MPM_OK : hip_fail(e, "sort_batch");

@@ -58,7 +58,7 @@ void fill_batch_slice(mpm_sim *s, BatchSlice &b);
 // Batched re-sort (mpm_fast.hip): launch sizes of a set of scenes, one
 // scene's table entry in its current parity, and the launches.
 struct SortBatchPlan {
-    int passes = 0, tiles = 0, spine = 0, runs = 0, scan = 0, emit = 0;
+    int passes = 0, tiles = 0, spine = 0, runs = 0, scan = 0, emit = 0, rank = 0;
 };
 void sort_batch_plan(mpm_sim *const *sims, int ns, SortBatchPlan &pl);
 int fill_sort_slice(mpm_sim *s, SortSlice &t);
