@@ -98,7 +98,7 @@ typedef struct mpm_config {
     int32_t warm_start;       /* MPM_WARM_* */
     int32_t warm_sweeps;      /* Jacobi sweeps after a warm start */
     int32_t tile;             /* 0, 256, 384 or 512; accepted, the P2G takes its own passes */
-    int32_t threads;          /* threads per workgroup for particle kernels, 0 = default */
+    int32_t threads;          /* threads per workgroup for particle kernels: 64, 128 or 256 (512: as 256); 0 = 256 */
     int32_t dt_mode;          /* MPM_DT_*; the dt given to mpm_step is max_dt */
     float cfl;                /* CFL number of the controller, in (0, 1] (0.5) */
     int32_t reserved[3];

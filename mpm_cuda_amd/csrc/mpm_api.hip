@@ -221,6 +221,7 @@ int mpm_create(const mpm_config *cfg, mpm_sim **out)
     int threads = cfg->threads ? cfg->threads : 256;
     if (threads != 64 && threads != 128 && threads != 256 && threads != 512)
         return set_error(MPM_ERR_INVALID, "threads must be 64, 128, 256 or 512");
+    threads = std::min(threads, 256);       // the particle kernels' bound; 512 stays accepted
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return set_error(MPM_ERR_HIP, "no HIP device");
     mpm_sim *s = new mpm_sim();
