@@ -843,7 +843,7 @@ static int run_phase(mpm_sim *s, int phase, float dt)
     }
     if (phase == MPM_PHASE_GRID) {
         {
-            PhaseTimer t(s, 2), tk(s, TK_GRID);
+            PhaseTimer t(s, 2);
             const bool staged = fast && s->blk_tile;
             uint32_t *count, *seq, launch;
             if ((rc = spill_publish(s, &count, &seq, &launch))) return rc;
@@ -855,6 +855,7 @@ static int run_phase(mpm_sim *s, int phase, float dt)
             if (!staged &&
                 (rc = check_launch(launch_list_marked(s->stream, s->flags, (int)s->nblocks, s->list, s->counters), "list")))
                 return rc;
+            PhaseTimer tk(s, TK_GRID);
             rc = check_launch(launch_grid_update(s->stream, s->g, dt, s->list, s->flags, s->act, s->act_seq, s->counters,
                                                  s->grid_mp, s->grid_v, s->nblocks, staged ? s->staging : nullptr,
                                                  staged ? s->blk_tile : nullptr, (int)s->groups.size(),
