@@ -136,8 +136,9 @@ int g2p_wgs(const mpm_batch *b, const Chain &c, int threads)
 int check(int rc, const char *what) { return rc ? hip_fail((hipError_t)rc, what) : MPM_OK; }
 
 // One step of a chain's scenes (parity p tables): P2G, grid update, the
-// warm-start inference of each weight set, G2P.  With `ev` (6 events, the
-// autotuner's stage timing) the P2G, grid-update and G2P stages are bracketed.
+// warm-start inference of each weight set, G2P.  With `ev` (STEP_EVENTS, the
+// autotuner's stage timing) an event before the first stage and after each.
+constexpr int STEP_EVENTS = 5, STAGE_BEGIN[3] = {0, 1, 3};      // P2G, grid update, G2P end at the next one
 int enqueue_step(mpm_batch *b, const Chain &c, int p, int p2g, int grid, int g2p_threads, hipEvent_t *ev)
 {
     hipStream_t st = c.stream ? c.stream : b->stream;
@@ -146,17 +147,16 @@ int enqueue_step(mpm_batch *b, const Chain &c, int p, int p2g, int grid, int g2p
     if (ev) MPM_HIP(hipEventRecord(ev[0], st));
     if ((rc = check(launch_p2g_batch(st, c.mats, tab, c.count, p2g), "p2g_batch"))) return rc;
     if (ev) MPM_HIP(hipEventRecord(ev[1], st));
-    if (ev) MPM_HIP(hipEventRecord(ev[2], st));
     if ((rc = check(launch_grid_batch(st, tab, c.count, grid), "grid_batch"))) return rc;
-    if (ev) MPM_HIP(hipEventRecord(ev[3], st));
+    if (ev) MPM_HIP(hipEventRecord(ev[2], st));
     for (const auto &w : c.warm)
         if ((rc = check(launch_mlp_infer_batch(st, b->warm_params[w.first], tab, c.count, w.first, w.second),
                         "mlp_infer_batch")))
             return rc;
-    if (ev) MPM_HIP(hipEventRecord(ev[4], st));
+    if (ev) MPM_HIP(hipEventRecord(ev[3], st));
     const int wgs = g2p_wgs(b, c, g2p_threads);
     if (wgs && (rc = check(launch_g2p_batch(st, c.mats, tab, c.count, wgs, g2p_threads), "g2p_batch"))) return rc;
-    if (ev) MPM_HIP(hipEventRecord(ev[5], st));
+    if (ev) MPM_HIP(hipEventRecord(ev[4], st));
     return MPM_OK;
 }
 
@@ -694,7 +694,7 @@ int mpm_batch_autotune(mpm_batch *b, int32_t reps, float *ms_out)
     if (reps < 1 || reps > 1000) return set_error(MPM_ERR_INVALID, "reps out of range [1,1000]");
     int rc = prepare(b);
     if (rc) return rc;
-    const size_t per = 6;
+    const size_t per = STEP_EVENTS;
     hipEvent_t *ev = timing_events(b, (size_t)reps * (NCAND + NTILE) * per);
     if (!ev) return set_error(MPM_ERR_HIP, "hipEventCreate failed");
     for (int32_t r = 0; r < reps; ++r)
@@ -720,7 +720,7 @@ int mpm_batch_autotune(mpm_batch *b, int32_t reps, float *ms_out)
     float med[3][NCAND];
     for (int c = 0; c < NCAND; ++c)
         for (int j = 0; j < 3; ++j)
-            if ((rc = median((size_t)c, NCAND, 2 * j, med[j][c]))) return rc;
+            if ((rc = median((size_t)c, NCAND, STAGE_BEGIN[j], med[j][c]))) return rc;
     int best[3] = {0, 0, 0};
     for (int j = 0; j < 3; ++j)
         for (int c = 1; c < NCAND; ++c)

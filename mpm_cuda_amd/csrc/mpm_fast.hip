@@ -81,7 +81,7 @@ __device__ __forceinline__ void scan_reduce_wg(const uint32_t *in, int n, uint32
 }
 
 __device__ __forceinline__ void scan_apply_wg(const uint32_t *in, uint32_t *out, int n, const uint32_t *partial,
-                                              uint32_t *total_out, int wg, uint32_t *lds, uint32_t *wg_base)
+                                              int wg, uint32_t *lds, uint32_t *wg_base)
 {
     if (threadIdx.x < 64) {
         uint32_t b = 0;
@@ -103,10 +103,7 @@ __device__ __forceinline__ void scan_apply_wg(const uint32_t *in, uint32_t *out,
     uint32_t run = *wg_base + block_excl_scan(s, tot, lds);
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; ++k) {
-        if (i0 + k < n) {
-            out[i0 + k] = run;
-            if (total_out && i0 + k == n - 1) *total_out = run + v[k];
-        }
+        if (i0 + k < n) out[i0 + k] = run;
         run += v[k];
     }
 }
@@ -118,21 +115,20 @@ __global__ void __launch_bounds__(SCAN_T) k_scan_reduce(const uint32_t *in, int 
 }
 
 __global__ void __launch_bounds__(SCAN_T) k_scan_apply(const uint32_t *in, uint32_t *out, int n,
-                                                       const uint32_t *partial, uint32_t *total_out)
+                                                       const uint32_t *partial)
 {
     __shared__ uint32_t lds[40];
     __shared__ uint32_t wg_base;
-    scan_apply_wg(in, out, n, partial, total_out, (int)blockIdx.x, lds, &wg_base);
+    scan_apply_wg(in, out, n, partial, (int)blockIdx.x, lds, &wg_base);
 }
 
 // out = exclusive scan of in (in-place allowed); partial holds ceil(n / 2048) words.
-static int scan_excl(hipStream_t st, const uint32_t *in, uint32_t *out, int n, uint32_t *partial,
-                     uint32_t *total_out)
+static int scan_excl(hipStream_t st, const uint32_t *in, uint32_t *out, int n, uint32_t *partial)
 {
     int nt = (n + SCAN_TILE - 1) / SCAN_TILE;
     if (nt == 0) return 0;
     hipLaunchKernelGGL(k_scan_reduce, dim3(nt), dim3(SCAN_T), 0, st, in, n, partial);
-    hipLaunchKernelGGL(k_scan_apply, dim3(nt), dim3(SCAN_T), 0, st, in, out, n, partial, total_out);
+    hipLaunchKernelGGL(k_scan_apply, dim3(nt), dim3(SCAN_T), 0, st, in, out, n, partial);
     return (int)hipGetLastError();
 }
 
@@ -723,7 +719,7 @@ __global__ void __launch_bounds__(SCAN_T) k_bsort_scan_apply(const SortSlice *__
                       wg))
         return;
     const SortSlice &t = tab[sid];
-    scan_apply_wg(t.has, t.has, t.nblocks, t.scan, nullptr, wg, lds, &wg_base);
+    scan_apply_wg(t.has, t.has, t.nblocks, t.scan, wg, lds, &wg_base);
 }
 
 // Tiles, and the warm-start list counts cleared (their lists name old slots).
@@ -1924,7 +1920,7 @@ int sort_all(mpm_sim *s, bool defer)
         // tiles: one per non-empty block, numbered in block order
         hipLaunchKernelGGL(k_block_runs, dim3(nblk(n, 256)), dim3(256), 0, st, skeys, n, s->blk_start, blk_end,
                            s->scan_tmp);
-        if ((rc = scan_excl(st, s->scan_tmp, s->scan_tmp, nk, s->sort_scan, nullptr)))
+        if ((rc = scan_excl(st, s->scan_tmp, s->scan_tmp, nk, s->sort_scan)))
             return hip_fail((hipError_t)rc, "scan");
         hipLaunchKernelGGL(k_emit_tiles, dim3(nblk(nk, 256)), dim3(256), 0, st, sg, s->blk_start, blk_end, s->scan_tmp,
                            (uint4 *)s->tile_desc, s->blk_tile + (int64_t)k * nb, s->tile_counts + k);

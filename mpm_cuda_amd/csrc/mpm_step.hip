@@ -677,9 +677,10 @@ int launch_g2p_batch(hipStream_t st, int mats, const BatchSlice *tab, int nslice
 // min(10, max_p max(J, 1/J)^3) after every step and never uses it,
 // MPMCUDA.cu:915-920).  k_dt_scan reduces the controller's maxima over the
 // current state (first step, or after the host rewrote particles); after
-// that every G2P reduces them over the state it writes.  k_dt_control runs
-// first in each step: it turns the maxima into the step's dt, advances the
-// clock and clears the maxima for this step's G2P.
+// that every G2P reduces them over the state it writes.  In the FAST form the
+// P2G's waves turn the maxima into the step's dt themselves; in the PLAIN form
+// k_dt_control does that first in each step, advances the clock and clears the
+// maxima for this step's G2P.
 template <int MAT>
 __global__ void __launch_bounds__(256) k_dt_scan(MatP mat, PartView pv, uint32_t *counters)
 {
