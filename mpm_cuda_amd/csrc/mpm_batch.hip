@@ -198,37 +198,23 @@ int enqueue_sort(mpm_batch *b, const Chain &c, hipStream_t st, int p)
 
 void drop_graphs(mpm_batch *b)
 {
-    for (Chain &c : b->chains)
+    auto drop = [](Chain &c) {
         for (int p = 0; p < 2; ++p) {
             if (c.sort_exec[p]) (void)hipGraphExecDestroy(c.sort_exec[p]);
             c.sort_exec[p] = nullptr;
         }
+    };
+    drop(b->all);
+    for (Chain &c : b->chains) drop(c);
 }
 
-// Scene bookkeeping kept by sort_all, saved around captures and replays.
-struct SortBook {
-    bool sorted_valid;
-    int64_t steps_since_sort, sorted_at_launch, sorts;
-};
-
-SortBook book_of(const mpm_sim *s) { return SortBook{s->sorted_valid, s->steps_since_sort, s->sorted_at_launch, s->sorts}; }
-void set_book(mpm_sim *s, const SortBook &k)
-{
-    s->sorted_valid = k.sorted_valid;
-    s->steps_since_sort = k.steps_since_sort;
-    s->sorted_at_launch = k.sorted_at_launch;
-    s->sorts = k.sorts;
-}
-
+// The graph of a chain's re-sort from parity p, at its first use.
 int capture_sort(mpm_batch *b, Chain &c, int p)
 {
-    std::vector<SortBook> book;
-    for (mpm_sim *s : b->sims) book.push_back(book_of(s));
     MPM_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed));
     int rc = enqueue_sort(b, c, b->stream, p);
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(b->stream, &graph);
-    for (size_t k = 0; k < b->sims.size(); ++k) set_book(b->sims[k], book[k]);
     if (rc) {
         if (graph) (void)hipGraphDestroy(graph);
         return rc;
@@ -240,7 +226,6 @@ int capture_sort(mpm_batch *b, Chain &c, int p)
     return MPM_OK;
 }
 
-// Device tables for both parities; graphs when the shape asks for them.
 // Warm scenes grouped by identical weights.
 void group_warm(mpm_batch *b)
 {
@@ -272,6 +257,7 @@ void group_warm(mpm_batch *b)
     for (Chain &c : b->chains) sets(c);
 }
 
+// Device tables for both parities.
 int build(mpm_batch *b)
 {
     const size_t n = b->sims.size();
@@ -326,14 +312,6 @@ int build(mpm_batch *b)
     for (size_t k = 0; k < n; ++k) b->sig.push_back(sig_of(b, k));
     drop_graphs(b);
     b->built = true;
-    if (!b->shape.use_graph) return MPM_OK;
-    std::vector<int> par(n);
-    for (size_t k = 0; k < n; ++k) par[k] = parity_of(b, k);
-    int rc = MPM_OK;
-    for (Chain &c : b->chains)
-        for (int p = 0; p < 2 && !rc; ++p) rc = capture_sort(b, c, p);
-    for (size_t k = 0; k < n; ++k) set_parity(b, k, par[k]);
-    if (rc) { drop_graphs(b); b->built = false; return rc; }
     return MPM_OK;
 }
 
@@ -390,7 +368,7 @@ Chain chain_of(const mpm_batch *b, int begin, int end)
 // are the host's launches either way.  A fork and a join cost ~20 us, so a run
 // of a few steps takes one chain.
 constexpr int64_t CHAIN_PARTICLES = 200000;
-constexpr int32_t CHAIN_STEPS = 8;
+constexpr int32_t CHAIN_STEPS = 12;
 int make_chains(mpm_batch *b)
 {
     const int n = (int)b->sims.size();
@@ -462,7 +440,6 @@ int prepare(mpm_batch *b)
         }
     bool same = b->built && b->sig.size() == n;
     for (size_t k = 0; same && k < n; ++k) same = sig_of(b, k) == b->sig[k];
-    if (b->shape.use_graph) same = same && b->chains[0].sort_exec[0];
     if (!same) {
         for (mpm_sim *s : b->sims) MPM_HIP(hipStreamSynchronize(s->stream));
         int rc = build(b);
@@ -520,13 +497,16 @@ int one_step(mpm_batch *b, int p2g, int grid, int g2p_threads, hipEvent_t *ev, b
     if (chains)
         if (int rc = fork_chains(b)) return rc;
     if (b->steps_since_sort >= b->shape.sort_every) {
-        for (Chain &c : b->chains) {
-            hipStream_t st = chains && c.stream ? c.stream : b->stream;
-            if (graphs) {
-                MPM_HIP(hipGraphLaunch(c.sort_exec[b->parity], st));
+        Chain *first = chains ? b->chains.data() : &b->all;
+        for (Chain *c = first; c < first + (chains ? b->chains.size() : 1); ++c) {
+            hipStream_t st = c->stream ? c->stream : b->stream;
+            if (!graphs) {
+                if (int rc = enqueue_sort(b, *c, st, b->parity)) return rc;
                 continue;
             }
-            if (int rc = enqueue_sort(b, c, st, b->parity)) return rc;
+            if (!c->sort_exec[b->parity])
+                if (int rc = capture_sort(b, *c, b->parity)) return rc;
+            MPM_HIP(hipGraphLaunch(c->sort_exec[b->parity], st));
         }
         after_sort(b);
     }

@@ -32,15 +32,15 @@ def test_chains_match_single_scenes(gpu, sizes, timed):
     batch = capi.Batch(sims, capi.batch_shape(sort_every=5))
     try:
         assert batch.particles >= 200_000
-        for n in (8, 1, 7, 13):
+        for n in (12, 1, 11, 13):
             ms = batch.run(n, timed=timed)
             assert not timed or (ms.shape == (n,) and np.all(ms > 0))
         sims[1].run(2)                  # on its own stream, after the chains
-        batch.run(9)
+        batch.run(12)
         batch.sync()
         for k, a in enumerate(alone):
-            a.run(40 if k == 1 else 38)
-        _same(sims, alone, 40)
+            a.run(51 if k == 1 else 49)
+        _same(sims, alone, 51)
     finally:
         batch.close()
         for s in sims + alone:
@@ -60,11 +60,11 @@ def test_chains_with_warm_start(gpu):
         s.write(0, capi.P_F, F)
     batch = capi.Batch(sims, capi.batch_shape(sort_every=50))
     try:
-        batch.run(8)
+        batch.run(12)
         batch.sync()
         for a in alone:
-            a.run(8)
-        _same(sims, alone, 8)
+            a.run(12)
+        _same(sims, alone, 12)
         for k, (s, a) in enumerate(zip(sims, alone)):
             if k % 3 != 2:
                 sa, sb = s.svd_stats(), a.svd_stats()
