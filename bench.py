@@ -57,6 +57,9 @@ for _mat, _b in ALG_BYTES.items():
 KERNEL_NAME = {("plain", "p2g"): "k_p2g_atomic", ("plain", "g2p"): "k_g2p", ("fast", "p2g"): "k_p2g_groups",
                ("fast", "g2p"): "k_g2p", ("fused", "g2p"): "k_g2p2g_block", ("plain", "grid"): "k_grid_update",
                ("fast", "grid"): "k_grid_update", ("fused", "grid"): "k_grid_update"}
+# What holds a kernel back where it is not the memory that its roofline is drawn against.
+LIMITED_BY = {"k_p2g_groups": "LDS atomics and vector issue", "k_p2g_atomic": "global float atomics",
+              "k_g2p2g_block": "registers (one wave a SIMD)"}
 
 
 def parse():
@@ -182,8 +185,8 @@ def run_gpu(workload, form, steps, warmup, sort_every=0, tile=0, warm_sweeps=0, 
 
 def run_batch(steps, warmup, warm=False, autotune_reps=2, seq_steps=5):
     """The batched workload: 64 scenes (log-uniform 10k-500k particles, mixed
-    jello / snow / water, 64^3-160^3 grids) advanced together, one launch per
-    stage replayed from hipGraphs, launch widths from the autotuner.  With
+    jello / snow / water, 64^3-160^3 grids) advanced together, two chains of one
+    launch per stage side by side, launch widths from the autotuner.  With
     `warm`, snow scenes use the learned warm start.  Also times every scene
     stepped on its own (the unbatched path) for comparison."""
     from mpm_cuda_amd import capi, workloads, warm_start
@@ -275,7 +278,7 @@ def roofline(res, material, form, steps, workload):
     achieved = bytes_per[dom] / (avg[dom] * 1e-3) / 1e9
     kname = KERNEL_NAME[(form, dom)]
     traffic = measured_traffic(kname) if workload == "snow_spheres" else None
-    return {"kernel": kname, "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+    return {"kernel": kname, "bound": "hbm", "limited_by": LIMITED_BY.get(kname, "hbm"), "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": round(traffic) if traffic else None,
             "kernel_avg_ms": {KERNEL_NAME.get((form, k), k): round(v, 4) for k, v in avg.items() if v > 0},

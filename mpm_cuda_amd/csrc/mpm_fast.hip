@@ -1478,7 +1478,7 @@ __device__ __forceinline__ uint32_t p2g_tile(const GridP &g, const MatP &mat, co
                        min(nbits + 126 - (int)(top.z >> 23), most)};
     const double mscale = pow2(nbits);
     const int low_exp = (int)(top.w >> 23) - fix_window(nbits);
-    const uint32_t low = finite && staged && low_exp > 0 ? (uint32_t)low_exp << 23 : 0u;    // least bound of this round
+    const uint32_t low = finite && staged && low_exp > 0 ? (uint32_t)low_exp << 23 : 0u;    // least bound taken now
     const bool later = low && __any(least < low - 1u), pick = again || later;
     // base inside the arena's bins (rel: relative to it), and a slot to write the tile to
     auto in_arena = [&](const int rel[3]) {
@@ -1597,17 +1597,18 @@ __device__ __forceinline__ uint32_t p2g_tile_of(const GridP &g, const MatP &mat,
 // The tiles of up to LAUNCH_GROUPS particle groups, one group's after the
 // other's (ONE: of a single group, whose arguments are then in scalar
 // registers from the start: 2M water 130 us, 135 otherwise).  Jello, snow and
-// water, 100k particles each: 16.8, 15.0 and 15.7 us apart, 28 together.
-// Bound by LDS and vector issue together: of a SIMD's cycles the
-// vector units take ~54% and the LDS atomics ~41%, half of these in bank
-// conflicts of uneven cells.  Four waves a SIMD: with five, 1M snow
-// gains 1% and groups of several materials (8 spilled registers) lose 5%.
-// Slower than its predecessor where cells are uneven and bodies drift fast (1M
-// random samples in two colliding bodies: 63 us, 60 with sorted register sums):
-// lanes then share words, and a 64-bit atomic takes ~20 cycles.  One pass over memory, no turns among lanes, no LDS sort: against
-// one wave a tile that sorted its particles in LDS and summed cells in
-// registers, per launch 26.8 -> 11.6 us (16k snow), 46 -> 26.0 (262k jello),
-// 67 -> 56.6 (1M snow), 202 -> 145 (2M water).
+// water, 100k particles each: 16.8, 15.0 and 15.7 us apart, 27 together.
+// Bound by LDS and vector issue together: vector instructions are issued in
+// 37 / 59 / 63% of a SIMD's cycles (262k jello, 1M snow, 2M water) and LDS bank
+// conflicts of uneven cells take 30 / 32 / 29% of a CU's.  Four waves a SIMD:
+// with five, 1M snow gains 1% and groups of several materials (8 spilled
+// registers) lose 5%.  Slower than its predecessor where cells are uneven and
+// bodies drift fast (1M random samples in two colliding bodies: 64 us, 60 with
+// sorted register sums): lanes then share words, and a 64-bit atomic takes ~20
+// cycles.  No turns among lanes, no LDS sort: against one wave a tile that
+// sorted its particles in LDS and summed cells in registers, per launch
+// 26.8 -> 11.3 us (16k snow), 46 -> 24.1 (262k jello), 67 -> 55.4 (1M snow),
+// 202 -> 132 (2M water).
 template <int MATS, int W, bool ONE>
 __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) k_p2g_groups(const P2GArgs a)
 {
@@ -2083,10 +2084,11 @@ int fast_ready(mpm_sim *s)
 }
 
 // Waves a tile of the FAST P2G.  Two where a tile has fewer particles on
-// average than two waves take at once (others of a workgroup would idle):
-// 2M particles of water, 77 a tile, took 145 us so and 166 with four; four
-// otherwise (262k jello, 512 a tile: 26.0 against 28.3; 1M snow, 300 a tile:
-// 56.6 against 59.4).  The sums do not depend on it.
+// average than two waves take at once (others of a workgroup would idle, and
+// clear a second arena copy): 2M particles of water, 77 a tile, take 132 us so
+// and 182 with four; four otherwise (262k jello, 512 a tile: 24.1 against 29.6;
+// 1M snow, 300 a tile: 55.4 either way; 100k snow 15.9 against 20.3).  The sums
+// do not depend on it.
 constexpr int P2G_WAVES = 4, P2G_WAVES_SPARSE = 2;
 
 bool tile_shape_valid(int tile) { return tile == 0 || tile == 256 || tile == 384 || tile == 512; }
