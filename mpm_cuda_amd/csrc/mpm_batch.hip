@@ -418,6 +418,7 @@ int validate_shape(const mpm_batch_shape &s)
 int prepare(mpm_batch *b)
 {
     const size_t n = b->sims.size();
+    if (int rc = join_chains(b)) return rc;         // of a run that ended early
     for (size_t k = 0; k < n; ++k) {
         mpm_sim *s = b->sims[k];
         if (!s->counters_clean)         // a batch's grid update leaves it cleared
