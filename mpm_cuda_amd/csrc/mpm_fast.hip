@@ -860,7 +860,7 @@ struct TileArena {
 // on twice that per doubling: its nodes then sum that many more).  Without the rounds
 // one particle 2^20 times the others left their nodes 2^-20 off, and with one
 // unit for all components a direction 2^30 times slower was lost; the two cost
-// 2M water 2% of a step, the other timing cases less than 1%.  What a unit
+// the timing cases 0 to 1.5% of a step.  What a unit
 // loses at a node of little mass comes back to a particle times that node's
 // weight.
 constexpr double FIX_MAGIC = 6755399441055744.0;        // 1.5 * 2^52
@@ -1307,7 +1307,7 @@ __device__ __forceinline__ void contribution_bounds(const MatP &mat, const GridP
         const float a = fabsf(r.C[3 * c]) + fabsf(r.C[3 * c + 1]) + fabsf(r.C[3 * c + 2]);
         const float f = MAT == MPM_WATER ? gw
                                          : cg * (fabsf(r.s[T[c][0]]) + fabsf(r.s[T[c][1]]) + fabsf(r.s[T[c][2]]));
-        q[c] = (uint32_t)__float_as_int(fmaf(hm, a, fmaf(mat.mass, fabsf(r.v[c]), fabsf(f)))) & 0x7fffffffu;
+        q[c] = (uint32_t)__float_as_int(fmaf(hm, a, fmaf(mat.mass, fabsf(r.v[c]), fabsf(f))));
     }
 }
 
@@ -1594,6 +1594,11 @@ __device__ __forceinline__ uint32_t p2g_tile_of(const GridP &g, const MatP &mat,
     return p2g_tile<MPM_WATER, W>(g, mat, pv, d, limit, staging_cap, dt, staging, grid, flags, list, counters, blk_tile, L);
 }
 
+// Waves a SIMD that the registers are to allow: the LDS of two-wave workgroups
+// has room for four and a half, so that water's 98 registers would cost it a
+// workgroup a CU (2M water 129.6 us, 128.1 with 96); more spills elsewhere.
+template <int MATS, int W> constexpr int kP2gWaves = MATS == MPM_WATER && W == 2 ? 5 : 4;
+
 // The tiles of up to LAUNCH_GROUPS particle groups, one group's after the
 // other's (ONE: of a single group, whose arguments are then in scalar
 // registers from the start: 2M water 130 us, 135 otherwise).  Jello, snow and
@@ -1608,9 +1613,9 @@ __device__ __forceinline__ uint32_t p2g_tile_of(const GridP &g, const MatP &mat,
 // cycles.  No turns among lanes, no LDS sort: against one wave a tile that
 // sorted its particles in LDS and summed cells in registers, per launch
 // 26.8 -> 11.3 us (16k snow), 46 -> 24.1 (262k jello), 67 -> 55.4 (1M snow),
-// 202 -> 132 (2M water).
+// 202 -> 130 (2M water).
 template <int MATS, int W, bool ONE>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) k_p2g_groups(const P2GArgs a)
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(kP2gWaves<MATS, W>))) k_p2g_groups(const P2GArgs a)
 {
     __shared__ TileArena<W> L;
     // the groups' counts by scalar loads (a scan over lanes and its barrier
@@ -2085,7 +2090,7 @@ int fast_ready(mpm_sim *s)
 
 // Waves a tile of the FAST P2G.  Two where a tile has fewer particles on
 // average than two waves take at once (others of a workgroup would idle, and
-// clear a second arena copy): 2M particles of water, 77 a tile, take 132 us so
+// clear a second arena copy): 2M particles of water, 77 a tile, take 130 us so
 // and 182 with four; four otherwise (262k jello, 512 a tile: 24.1 against 29.6;
 // 1M snow, 300 a tile: 55.4 either way; 100k snow 15.9 against 20.3).  The sums
 // do not depend on it.
